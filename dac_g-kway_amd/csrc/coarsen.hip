@@ -161,35 +161,365 @@ int launch_jump_round(int32_t n, const int32_t* cand, const int32_t* next_in, co
   return hip_status();
 }
 
-__global__ void __launch_bounds__(256) k_label_max(int32_t n, const int32_t* __restrict__ cand,
-                                                   const int32_t* __restrict__ next,
-                                                   int32_t* __restrict__ compmax) {
-  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
-  if (v >= n) return;
-  const int32_t r = next[v];
-  const int32_t key = max(r, cand[r]);
-  atomicMax(&compmax[key], int32_t(v));
+// One vertex more in the component of key: its largest id in comp[key].x, its
+// members counted in comp[key].y; returns v's (arbitrary) place among them.
+// Components are small, so the atomics rarely collide; lanes that share the
+// first active lane's key (hubs, stars) are added with one atomic pair, since
+// same-address atomics serialise.
+__device__ __forceinline__ int32_t comp_add(int2* __restrict__ comp, int32_t key, int32_t v, bool live) {
+  const uint64_t lm = ballot(live);
+  if (lm == 0) return 0;
+  const int first = __ffsll(static_cast<long long>(lm)) - 1;
+  const uint64_t same = ballot(live && key == __shfl(key, first, 64));
+  int32_t slot = 0;
+  if (popc64(same) > 4) {
+    int32_t base = 0;
+    const int lead = 63 - __clzll(static_cast<long long>(same));  // ids grow with the lane: its id is the largest
+    if (lane_id() == lead) {
+      atomicMax(&comp[key].x, v);
+      base = atomicAdd(&comp[key].y, popc64(same));
+    }
+    base = __shfl(base, lead, 64);
+    if ((same >> lane_id()) & 1ull) return base + popc64(same & lanemask_lt());
+  }
+  if (live) {
+    atomicMax(&comp[key].x, v);
+    slot = atomicAdd(&comp[key].y, 1);
+  }
+  return slot;
 }
 
-__global__ void __launch_bounds__(256) k_label_get(int32_t n, const int32_t* __restrict__ cand,
-                                                   const int32_t* __restrict__ next,
-                                                   const int32_t* __restrict__ compmax,
-                                                   int32_t* __restrict__ label) {
-  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
-  if (v >= n) return;
-  const int32_t r = next[v];
-  label[v] = compmax[max(r, cand[r])];
+// Grouping in one pass: every vertex follows its candidates to the mutual
+// pair at the root of its tree (a self loop for an isolated vertex), counting
+// hops.  Vertices sit on average less than one hop from their pair and
+// rarely more than ten, so the walk reads cand[] about three times per vertex
+// where the jumping rounds read and write pointer and distance arrays four
+// times over.  On a 2^22-vertex mesh numbered at random (every read a cache
+// line): 327 us with the component atomics, which bound it, where init and
+// jumping rounds took 60 + 269 us and the label kernels 148 + 98 us (now 64).  flags[r] is set when some vertex is more than 2^r hops
+// away, which tells the jumping rounds that the walk replaces; a vertex more
+// than kWalkMax hops away sets flags[kWalkBits], and the caller falls back to
+// the jumping rounds (long chains would make the walk linear).
+__global__ void __launch_bounds__(256) k_walk(int32_t n, const int32_t* __restrict__ cand, int2* __restrict__ comp,
+                                              int32_t* __restrict__ key_out, int32_t* __restrict__ dist,
+                                              int32_t* __restrict__ slot, int32_t* __restrict__ flags) {
+  const int64_t i = int64_t(xcd_block()) * 256 + threadIdx.x;
+  const bool live = i < n;
+  const int32_t v = live ? int32_t(i) : 0;
+  int32_t a = v, d = 0, key = 0;
+  if (live) {
+    int32_t b = cand[a], c = cand[b];
+    while (c != a && d <= kWalkMax) {
+      a = b;
+      b = c;
+      c = cand[b];
+      ++d;
+    }
+    key = max(a, b);
+    if (c != a) d = kWalkMax + 1;
+    key_out[v] = key;
+    dist[v] = d;
+  }
+  const int32_t s = comp_add(comp, key, v, live);
+  if (live) slot[v] = s;
+  // highest power of two below the wave's largest distance
+  int r = -1;
+#pragma unroll
+  for (int x = 0; x <= kWalkBits; ++x)
+    if (ballot(d > (1 << x)) != 0) r = x;
+  if (r >= 0 && lane_id() == 0 && flags[r] == 0) flags[r] = 1;
 }
 
-int launch_label(int32_t n, const int32_t* cand, const int32_t* next, int32_t* compmax,
-                 int32_t* label, hipStream_t st) {
+int launch_walk(int32_t n, const int32_t* cand, int2* comp, int32_t* key, int32_t* dist, int32_t* slot,
+                int32_t* flags, hipStream_t st) {
   if (n <= 0) return 0;
-  fill<int32_t>(compmax, 0, n, st);
-  k_label_max<<<grid_for(n, 256), 256, 0, st>>>(n, cand, next, compmax);
-  k_label_get<<<grid_for(n, 256), 256, 0, st>>>(n, cand, next, compmax, label);
+  fill<int2>(comp, int2{0, 0}, n, st);
+  k_walk<<<grid_for(n, 256), 256, 0, st>>>(n, cand, comp, key, dist, slot, flags);
   return hip_status();
 }
 
+// The same from the jumping rounds' root pointers (root pair of every vertex).
+__global__ void __launch_bounds__(256) k_comp_count(int32_t n, const int32_t* __restrict__ cand,
+                                                    const int32_t* __restrict__ next, int2* __restrict__ comp,
+                                                    int32_t* __restrict__ key_out, int32_t* __restrict__ slot) {
+  const int64_t i = int64_t(xcd_block()) * 256 + threadIdx.x;
+  const bool live = i < n;
+  int32_t key = 0;
+  if (live) {
+    const int32_t r = next[i];
+    key = max(r, cand[r]);
+    key_out[i] = key;
+  }
+  const int32_t s = comp_add(comp, key, int32_t(i), live);
+  if (live) slot[i] = s;
+}
+
+int launch_comp_count(int32_t n, const int32_t* cand, const int32_t* next, int2* comp, int32_t* key, int32_t* slot,
+                      hipStream_t st) {
+  if (n <= 0) return 0;
+  fill<int2>(comp, int2{0, 0}, n, st);
+  k_comp_count<<<grid_for(n, 256), 256, 0, st>>>(n, cand, next, comp, key, slot);
+  return hip_status();
+}
+
+// label[v] = the largest id of v's component; size[label] = its member count,
+// 0 for every other index.  key may be label.
+__global__ void __launch_bounds__(256) k_label_size(int32_t n, const int32_t* key, const int2* __restrict__ comp,
+                                                    int32_t* label, int32_t* __restrict__ size) {
+  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
+  if (v >= n) return;
+  const int2 c = comp[key[v]];
+  label[v] = c.x;
+  size[v] = c.x == int32_t(v) ? c.y : 0;
+}
+
+int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* label, int32_t* size,
+                      hipStream_t st) {
+  if (n <= 0) return 0;
+  k_label_size<<<grid_for(n, 256), 256, 0, st>>>(n, key, comp, label, size);
+  return hip_status();
+}
+
+// size[l] = vertices with label l, slot[v] = v's (arbitrary) place among them,
+// for labels that come without a grouping.
+__global__ void __launch_bounds__(256) k_label_count(int32_t n, const int32_t* __restrict__ label,
+                                                     int32_t* __restrict__ size, int32_t* __restrict__ slot) {
+  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
+  const bool live = v < n;
+  const int32_t l = live ? label[v] : -1;
+  const uint64_t same = ballot(live && l == __builtin_amdgcn_readfirstlane(l));
+  if (popc64(same) > 4) {  // one atomic for the lanes that share the first lane's label
+    int32_t base = 0;
+    if (lane_id() == 0) base = atomicAdd(&size[l], popc64(same));
+    base = __shfl(base, 0, 64);
+    if ((same >> lane_id()) & 1ull) {
+      slot[v] = base + popc64(same & lanemask_lt());
+      return;
+    }
+  }
+  if (live) slot[v] = atomicAdd(&size[l], 1);
+}
+
+int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, hipStream_t st) {
+  if (n <= 0) return 0;
+  fill<int32_t>(size, 0, n, st);
+  k_label_count<<<grid_for(n, 256), 256, 0, st>>>(n, label, size, slot);
+  return hip_status();
+}
+
+// --------------------------------------------------------------- members
+// Order of the vertices by (label, stamp, id) and their chunks of at most G,
+// by counting instead of sorting: the member counts are scanned over the
+// labels (first place and first coarse id of every group), every vertex is
+// written to its group's places in arbitrary order, and then finds its rank
+// among its group's members.  Groups average 3 to 6 members, so the quadratic
+// ranking is cheaper than the four 8-bit passes of a radix sort over (label,
+// stamp).  2^22 vertices numbered at random: scan 35, scatter 190, rank 79 us,
+// where keys, passes, chunk flags and ids took 530 us and the gathers of the
+// members' rows and weights, which the records now carry, another 120 us.  The
+// scatter is bound by its random 32-byte writes.  A group of more than kRankMax
+// members sets ctl[1] and the caller sorts instead (at 512 members for every
+// vertex the ranking costs about what the passes cost).
+constexpr int kSizeIPT = 8;
+constexpr int kSizeTile = 256 * kSizeIPT;
+constexpr int64_t kSizeDirect = 8192;  // up to this many tiles every block sums the tiles before it itself
+
+__device__ __forceinline__ int32_t chunks_of(int32_t size, int32_t G) {
+  return size == 0 ? 0 : (size - 1) / G + 1;
+}
+
+// Members and chunks of each tile.
+__global__ void __launch_bounds__(256) k_size_reduce(int32_t n, const int32_t* __restrict__ size, int32_t G,
+                                                     int2* __restrict__ partial, int32_t* __restrict__ ctl) {
+  __shared__ int2 ws[4];
+  const int64_t base = int64_t(blockIdx.x) * kSizeTile;
+  int32_t m = 0, c = 0, big = 0;
+#pragma unroll
+  for (int j = 0; j < kSizeIPT; ++j) {
+    const int64_t i = base + j * 256 + threadIdx.x;
+    if (i < n) {
+      const int32_t s = size[i];
+      m += s;
+      c += chunks_of(s, G);
+      big |= s > kRankMax;
+    }
+  }
+  if (ballot(big) != 0 && lane_id() == 0) ctl[1] = 1;
+  m = wave_sum(m);
+  c = wave_sum(c);
+  if (lane_id() == 0) ws[threadIdx.x >> 6] = make_int2(m, c);
+  __syncthreads();
+  if (threadIdx.x == 0)
+    partial[blockIdx.x] = make_int2(ws[0].x + ws[1].x + ws[2].x + ws[3].x, ws[0].y + ws[1].y + ws[2].y + ws[3].y);
+}
+
+// Many tiles: their exclusive sums, in place, by one block.
+__global__ void __launch_bounds__(256) k_size_mid(int64_t nb, int2* __restrict__ partial) {
+  __shared__ int lds[8];
+  int32_t rm = 0, rc = 0;
+  for (int64_t b0 = 0; b0 < nb; b0 += 256) {
+    const int64_t b = b0 + threadIdx.x;
+    const int2 p = b < nb ? partial[b] : make_int2(0, 0);
+    int tm, tc;
+    const int em = block_excl_scan_256(p.x, &tm, lds);
+    const int ec = block_excl_scan_256(p.y, &tc, lds);
+    if (b < nb) partial[b] = make_int2(rm + em, rc + ec);
+    rm += tm;
+    rc += tc;
+  }
+}
+
+// offc[l] = first place and first coarse id of label l's group, offc[n] the
+// totals; ctl[0] (and the host's copy) = the number of coarse ids; host[1..]
+// = the flags.
+__global__ void __launch_bounds__(256) k_size_apply(int32_t n, const int32_t* __restrict__ size, int32_t G,
+                                                    const int2* __restrict__ partial, int scanned,
+                                                    int2* __restrict__ offc, int32_t* __restrict__ ctl,
+                                                    int32_t* __restrict__ host) {
+  __shared__ int lds[8];
+  int32_t pm = 0, pc = 0;
+  if (scanned) {
+    const int2 p = partial[blockIdx.x];
+    pm = p.x;
+    pc = p.y;
+  } else {
+    int32_t sm = 0, sc = 0;
+    for (int64_t b = threadIdx.x; b < int64_t(blockIdx.x); b += 256) {
+      const int2 p = partial[b];
+      sm += p.x;
+      sc += p.y;
+    }
+    int t;
+    (void)block_excl_scan_256(sm, &t, lds);
+    pm = t;
+    (void)block_excl_scan_256(sc, &t, lds);
+    pc = t;
+  }
+  const int64_t base = int64_t(blockIdx.x) * kSizeTile + int64_t(threadIdx.x) * kSizeIPT;
+  int32_t s[kSizeIPT];
+  int32_t m = 0, c = 0;
+#pragma unroll
+  for (int j = 0; j < kSizeIPT; ++j) {
+    s[j] = base + j < n ? size[base + j] : 0;
+    m += s[j];
+    c += chunks_of(s[j], G);
+  }
+  int t;
+  int32_t rm = pm + block_excl_scan_256(m, &t, lds);
+  int32_t rc = pc + block_excl_scan_256(c, &t, lds);
+#pragma unroll
+  for (int j = 0; j < kSizeIPT; ++j) {
+    if (base + j < n) offc[base + j] = make_int2(rm, rc);
+    rm += s[j];
+    rc += chunks_of(s[j], G);
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) {
+    offc[n] = make_int2(rm, rc);
+    ctl[0] = rc;
+    host[0] = rc;
+#pragma unroll
+    for (int i = 1; i < kCtlInts; ++i) host[i] = ctl[i];
+  }
+}
+
+int64_t size_partials(int64_t n) { return (n + kSizeTile - 1) / kSizeTile; }
+
+int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl, int32_t* host,
+                     hipStream_t st) {
+  if (n <= 0) return 0;
+  const int64_t nb = size_partials(n);
+  k_size_reduce<<<unsigned(nb), 256, 0, st>>>(n, size, G, partial, ctl);
+  const bool mid = nb > kSizeDirect;
+  if (mid) k_size_mid<<<1, 256, 0, st>>>(nb, partial);
+  k_size_apply<<<unsigned(nb), 256, 0, st>>>(n, size, G, partial, mid ? 1 : 0, offc, ctl, host);
+  return hip_status();
+}
+
+// Every vertex to a place of its group, with what its later readers need (its
+// row and weight), so that they read consecutive records: memb[2p] = (vertex,
+// stamp, group's first place, group's first coarse id), memb[2p + 1] = (row
+// start, row length, weight, members of the group).
+__global__ void __launch_bounds__(256) k_member_scatter(int32_t n, const int32_t* __restrict__ label,
+                                                        const int32_t* __restrict__ stamp,
+                                                        const int32_t* __restrict__ slot,
+                                                        const int2* __restrict__ offc,
+                                                        const int32_t* __restrict__ xadj,
+                                                        const int32_t* __restrict__ vw, int4* __restrict__ memb) {
+  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
+  if (v >= n) return;
+  const int32_t l = label[v];
+  const int2 oc = offc[l];
+  const int32_t cnt = offc[l + 1].x - oc.x;
+  int32_t a = 0, d = 0;
+  if (xadj) {
+    a = xadj[v];
+    d = xadj[v + 1] - a;
+  }
+  const int64_t p = int64_t(oc.x) + slot[v];
+  memb[2 * p] = make_int4(int32_t(v), stamp ? stamp[v] : 0, oc.x, oc.y);
+  memb[2 * p + 1] = make_int4(a, d, vw ? vw[v] : 0, cnt);
+}
+
+// Rank of every member in its group, and with it the vertex order, the coarse
+// ids, the first place of every coarse id and the members' rows and weights
+// in that order (each output but cptr may be null).
+__global__ void __launch_bounds__(256) k_member_rank(int32_t n, const int4* __restrict__ memb, int32_t G,
+                                                     const int32_t* __restrict__ ctl, int32_t* __restrict__ order,
+                                                     int32_t* __restrict__ cmap, int32_t* __restrict__ cptr,
+                                                     int2* __restrict__ mrow, int32_t* __restrict__ mvw) {
+  const int64_t i = int64_t(xcd_block()) * 256 + threadIdx.x;
+  if (i >= n) return;
+  if (i == n - 1) cptr[ctl[0]] = n;
+  const int4 a = memb[2 * i], b = memb[2 * i + 1];
+  const int32_t cnt = b.w;
+  if (cnt > kRankMax) return;  // ctl[1] is set: the caller sorts
+  int32_t r = 0;
+  for (int32_t j = 0; j < cnt; ++j) {
+    const int4 o = memb[2 * (int64_t(a.z) + j)];
+    r += (o.y < a.y || (o.y == a.y && o.x < a.x)) ? 1 : 0;
+  }
+  const int32_t p = a.z + r;
+  const int32_t q = r / G;
+  if (cmap) cmap[a.x] = a.w + q;
+  if (r - q * G == 0) cptr[a.w + q] = p;
+  if (order) order[p] = a.x;
+  if (mrow) mrow[p] = make_int2(b.x, b.y);
+  if (mvw) mvw[p] = b.z;
+}
+
+int launch_members(int32_t n, const int32_t* label, const int32_t* stamp, const int32_t* slot, const int2* offc,
+                   const int32_t* xadj, const int32_t* vw, int4* memb, int32_t G, const int32_t* ctl,
+                   int32_t* order, int32_t* cmap, int32_t* cptr, int2* mrow, int32_t* mvw, hipStream_t st) {
+  if (n <= 0) return 0;
+  k_member_scatter<<<grid_for(n, 256), 256, 0, st>>>(n, label, stamp, slot, offc, xadj, vw, memb);
+  k_member_rank<<<grid_for(n, 256), 256, 0, st>>>(n, memb, G, ctl, order, cmap, cptr, mrow, mvw);
+  return hip_status();
+}
+
+// The members' rows and weights in a given vertex order (after a sort).
+__global__ void __launch_bounds__(256) k_member_rows(int32_t n, const int32_t* __restrict__ order,
+                                                     const int32_t* __restrict__ xadj,
+                                                     const int32_t* __restrict__ vw, int2* __restrict__ mrow,
+                                                     int32_t* __restrict__ mvw) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int32_t v = order[i];
+  if (mrow) {
+    const int32_t a = xadj[v];
+    mrow[i] = make_int2(a, xadj[v + 1] - a);
+  }
+  if (mvw) mvw[i] = vw[v];
+}
+
+int launch_member_rows(int32_t n, const int32_t* order, const int32_t* xadj, const int32_t* vw, int2* mrow,
+                       int32_t* mvw, hipStream_t st) {
+  if (n <= 0) return 0;
+  k_member_rows<<<grid_for(n, 256), 256, 0, st>>>(n, order, xadj, vw, mrow, mvw);
+  return hip_status();
+}
+
+// --------------------------------------------------------------- sorted order
+// The order by a radix sort of (label, stamp), for groups too large to rank.
 __global__ void __launch_bounds__(256) k_make_keys(int32_t n, const int32_t* __restrict__ label,
                                                    const int32_t* __restrict__ dist, int sbits,
                                                    uint64_t* __restrict__ keys, int32_t* __restrict__ ids) {
@@ -248,12 +578,9 @@ __global__ void __launch_bounds__(256) k_cmap(int32_t n, const uint64_t* __restr
   if (i == n - 1) cptr[c + 1] = n;
 }
 
-int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sbits,
-                   const int32_t* vwgt, int32_t G, int32_t* gstart, int32_t* flagscan,
-                   int32_t* cmap, int32_t* cptr, int32_t* cvwgt, int32_t* nc_dev,
-                   int32_t* scratch, hipStream_t st) {
-  (void)vwgt;
-  (void)cvwgt;
+int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sbits, int32_t G, int32_t* gstart,
+                   int32_t* flagscan, int32_t* cmap, int32_t* cptr, int32_t* nc_dev, int32_t* scratch,
+                   hipStream_t st) {
   if (n <= 0) return 0;
   k_group_start<<<grid_for(n, 256), 256, 0, st>>>(n, skeys, sbits, gstart);
   int rc = scan(n, ChunkFlag{skeys, gstart, sbits, G}, StoreExcl{flagscan}, nc_dev, scratch, st);
@@ -263,35 +590,33 @@ int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sb
 }
 
 // cal_coarsen_vwgt (gkway/coarsen.hpp:157-171) as an ordered sum over the
-// (at most G) members of each chunk; no atomics, destination fully written.
+// (at most G) members of each chunk, their weights in member order; no
+// atomics, destination fully written.
 __global__ void __launch_bounds__(256) k_cvwgt(int32_t nc, const int32_t* __restrict__ cptr,
-                                               const int32_t* __restrict__ order,
-                                               const int32_t* __restrict__ vw, int32_t* __restrict__ cvw) {
+                                               const int32_t* __restrict__ mvw, int32_t* __restrict__ cvw) {
   const int64_t c = int64_t(xcd_block()) * 256 + threadIdx.x;
   if (c >= nc) return;
   int32_t s = 0;
-  for (int32_t j = cptr[c]; j < cptr[c + 1]; ++j) s += vw[order[j]];
+  for (int32_t j = cptr[c]; j < cptr[c + 1]; ++j) s += mvw[j];
   cvw[c] = s;
 }
 
-int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* order, const int32_t* vw,
-                 int32_t* cvw, hipStream_t st) {
+int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* mvw, int32_t* cvw, hipStream_t st) {
   if (nc <= 0) return 0;
-  k_cvwgt<<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, order, vw, cvw);
+  k_cvwgt<<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, mvw, cvw);
   return hip_status();
 }
 
 // --------------------------------------------------------------- contraction
 // Per coarse row: upper bound of entries (sum of member degrees) and its
 // lane class; row ids appended to one list per class, each with its member
-// range in order[] (desc: first member, member count).  Member m's row start
-// and length are copied to mrow[m] on the way, so that the row kernels reach
-// a member's entries with one load instead of order[] then xadj[].
+// range in member order (desc: first member, member count).  The members'
+// rows (mrow) and weights (mvw, with cvw the coarse weights' destination; both
+// may be null) lie in member order, so a row's members are consecutive reads.
 __global__ void __launch_bounds__(256) k_row_bounds(int32_t nc, const int32_t* __restrict__ cptr,
-                                                    const int32_t* __restrict__ order,
-                                                    const int32_t* __restrict__ xadj,
+                                                    const int2* __restrict__ mrow, const int32_t* __restrict__ mvw,
                                                     int32_t* __restrict__ ub, int32_t* __restrict__ lists,
-                                                    int2* __restrict__ desc, int2* __restrict__ mrow,
+                                                    int2* __restrict__ desc, int32_t* __restrict__ cvw,
                                                     int32_t* __restrict__ cnt) {
   const int64_t c = int64_t(xcd_block()) * 256 + threadIdx.x;
   int cls = -1;
@@ -299,14 +624,13 @@ __global__ void __launch_bounds__(256) k_row_bounds(int32_t nc, const int32_t* _
   if (c < nc) {
     m0 = cptr[c];
     m1 = cptr[c + 1];
-    int32_t s = 0;
+    int32_t s = 0, x = 0;
     for (int32_t j = m0; j < m1; ++j) {
-      const int32_t v = order[j];
-      const int32_t a = xadj[v], d = xadj[v + 1] - a;
-      mrow[j] = make_int2(a, d);
-      s += d;
+      s += mrow[j].y;
+      if (mvw) x += mvw[j];
     }
     ub[c] = s;
+    if (mvw) cvw[c] = x;
     cls = s <= 16 ? 0 : (s <= 32 ? 1 : (s <= 64 ? 2 : 3));
   }
   // Block-aggregated append: per class, wave counts in LDS, one global
@@ -344,12 +668,12 @@ struct UbLoad {
   __device__ int operator()(int64_t i) const { return i < nc ? ub[i] : 0; }
 };
 
-int launch_contract_bounds(const DGraph& g, int32_t nc, const int32_t* cptr, const int32_t* order,
-                           int32_t* ub, int32_t* toff, int32_t* lists, int2* desc, int2* mrow,
-                           int32_t* list_cnt, int32_t* scratch, hipStream_t st) {
+int launch_contract_bounds(int32_t nc, const int32_t* cptr, const int2* mrow, const int32_t* mvw, int32_t* ub,
+                           int32_t* toff, int32_t* lists, int2* desc, int32_t* cvw, int32_t* list_cnt,
+                           int32_t* scratch, hipStream_t st) {
   fill<int32_t>(list_cnt, 0, 4, st);
   if (nc <= 0) return 0;
-  k_row_bounds<<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, order, g.xadj, ub, lists, desc, mrow, list_cnt);
+  k_row_bounds<<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, mrow, mvw, ub, lists, desc, cvw, list_cnt);
   int rc = scan(int64_t(nc) + 1, UbLoad{ub, nc}, StoreExcl{toff}, nullptr, scratch, st);
   return rc ? GK_ERR_HIP : hip_status();
 }
@@ -659,8 +983,7 @@ int launch_big_offsets(const int32_t* rows, int32_t nrows, const int32_t* ub, in
 __global__ void __launch_bounds__(256) k_big_gather(const int32_t* __restrict__ rows,
                                                     const int32_t* __restrict__ boff,
                                                     const int32_t* __restrict__ cptr,
-                                                    const int32_t* __restrict__ order,
-                                                    const int32_t* __restrict__ xadj,
+                                                    const int2* __restrict__ mrow,
                                                     const int32_t* __restrict__ adj,
                                                     const int32_t* __restrict__ w,
                                                     const int32_t* __restrict__ cmap,
@@ -669,8 +992,7 @@ __global__ void __launch_bounds__(256) k_big_gather(const int32_t* __restrict__ 
   const int32_t c = rows[i];
   int32_t o = boff[i];
   for (int32_t m = cptr[c]; m < cptr[c + 1]; ++m) {
-    const int32_t v = order[m];
-    const int32_t s = xadj[v], d = xadj[v + 1] - s;
+    const int32_t s = mrow[m].x, d = mrow[m].y;
     for (int32_t t = threadIdx.x; t < d; t += 256) {
       keys[o + t] = (uint64_t(uint32_t(i)) << 32) | uint64_t(uint32_t(cmap[adj[s + t]]));
       vals[o + t] = w[s + t];
@@ -680,10 +1002,10 @@ __global__ void __launch_bounds__(256) k_big_gather(const int32_t* __restrict__ 
 }
 
 int launch_contract_big_gather(const DGraph& g, const int32_t* rows, int32_t nrows,
-                               const int32_t* boff, const int32_t* cptr, const int32_t* order,
+                               const int32_t* boff, const int32_t* cptr, const int2* mrow,
                                const int32_t* cmap, uint64_t* keys, int32_t* vals, hipStream_t st) {
   if (nrows <= 0) return 0;
-  k_big_gather<<<nrows, 256, 0, st>>>(rows, boff, cptr, order, g.xadj, g.adj, g.w, cmap, keys, vals);
+  k_big_gather<<<nrows, 256, 0, st>>>(rows, boff, cptr, mrow, g.adj, g.w, cmap, keys, vals);
   return hip_status();
 }
 

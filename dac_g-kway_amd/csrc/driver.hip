@@ -46,19 +46,45 @@ constexpr int64_t kTuneMinEntries = int64_t(1) << 20;
 constexpr int32_t kTuneMinRows = 1 << 14;
 
 // ---------------------------------------------------------------- stages
-// Grouping: pointer jumping to the root pair, then the component maximum.
-// Returns label/dist in the given buffers, the jump rounds in *rounds.
-int group_stage(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label,
-                Buf<int32_t>& dist_out, int32_t* rounds) {
+// Labels, hops and member counts of the groups by walking to the root pairs.
+// The control words (zeroed here) hold whether every vertex reached its pair.
+int Groups::walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label) {
   Pool& P = ctx->pool;
-  Buf<int32_t> nx[2], ds[2], flags, compmax;
+  GK_TRY(ctl.alloc(P, gkd::kCtlInts));
+  GK_TRY(comp.alloc(P, int64_t(n) + 1));
+  GK_TRY(dist.alloc(P, n));
+  GK_TRY(slot.alloc(P, n));
+  GK_TRY(size.alloc(P, n));
+  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts, st);
+  GK_STAGE(ctx, GK_ST_GROUP, 52LL * n,
+           (gkd::launch_walk(n, cand, comp.p, label, dist.p, slot.p, ctl.p + gkd::kCtlFlags, st) ||
+                    gkd::launch_label_size(n, label, comp.p, label, size.p, st)
+                ? GK_ERR_HIP
+                : GK_OK));
+  return GK_OK;
+}
+
+// Jumping rounds that the walk's flags (words kCtlFlags.. of the control
+// words) stand for: every round halves the largest distance.
+int32_t Groups::rounds(const int32_t* words) {
+  int32_t r = 0;
+  for (int b = 0; b <= gkd::kWalkBits; ++b)
+    if (words[gkd::kCtlFlags + b]) r = b + 1;
+  return r;
+}
+
+// The same by pointer jumping, for trees deeper than the walk goes; returns
+// the jump rounds in *rounds.
+int Groups::jump(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* rounds) {
+  Pool& P = ctx->pool;
+  Buf<int32_t> nx[2], ds[2], flags;
   GK_TRY(nx[0].alloc(P, n));
   GK_TRY(nx[1].alloc(P, n));
   GK_TRY(ds[0].alloc(P, n));
   GK_TRY(ds[1].alloc(P, n));
   GK_TRY(flags.alloc(P, kMaxJumpRounds + 8));
-  GK_TRY(compmax.alloc(P, n));
   gkd::fill<int32_t>(flags.p, 0, kMaxJumpRounds + 8, st);
+  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts, st);
   GK_STAGE(ctx, GK_ST_GROUP, 16LL * n, gkd::launch_jump_init(n, cand, nx[0].p, ds[0].p, st));
   int32_t f = -1;
   int32_t r = 0;
@@ -83,25 +109,69 @@ int group_stage(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int
     r += cnt;
   }
   // Round f moved nothing: buffers f&1 and (f+1)&1 agree.
-  int32_t* next = nx[f & 1].p;
   // Rounds 0..f ran in full (24 bytes per vertex each); later ones exit early.
   count_stage(ctx, GK_ST_GROUP, 24LL * n * (f + 1));
-  GK_STAGE(ctx, GK_ST_GROUP, 32LL * n, gkd::launch_label(n, cand, next, compmax.p, label, st));
-  dist_out = std::move(ds[f & 1]);
+  GK_STAGE(ctx, GK_ST_GROUP, 40LL * n,
+           (gkd::launch_comp_count(n, cand, nx[f & 1].p, comp.p, label, slot.p, st) ||
+                    gkd::launch_label_size(n, label, comp.p, label, size.p, st)
+                ? GK_ERR_HIP
+                : GK_OK));
+  dist = std::move(ds[f & 1]);
   *rounds = f;
   return GK_OK;
 }
 
-// Sort vertices by (label, stamp, id) and chunk them; fills order (sorted
-// ids), cmap, cptr (nc+1) and *nc.
-int cluster_stage(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* dist,
-                  int32_t max_dist_bits, int32_t G, Buf<int32_t>& order, int32_t* cmap,
-                  Buf<int32_t>& cptr, int32_t* nc) {
+// Labels in [0, n) that come without a grouping: member counts only.
+int Groups::count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label) {
   Pool& P = ctx->pool;
-  const int sbits = max_dist_bits;
+  GK_TRY(ctl.alloc(P, gkd::kCtlInts));
+  GK_TRY(comp.alloc(P, int64_t(n) + 1));
+  GK_TRY(slot.alloc(P, n));
+  GK_TRY(size.alloc(P, n));
+  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts, st);
+  GK_STAGE(ctx, GK_ST_SORT, 16LL * n, gkd::launch_label_count(n, label, size.p, slot.p, st));
+  return GK_OK;
+}
+
+// Order, coarse ids and member records by counting, from the groups' sizes
+// and slots.  words (kCtlInts) receives the control words; words[1] != 0: some
+// group is too large, the results are incomplete and sort_members is needed.
+static int count_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* stamp,
+                         Groups& gr, const int32_t* xadj, const int32_t* vw, int32_t G, const MemberOut& out,
+                         int32_t* words) {
+  Buf<int2> partial;
+  Buf<int4> memb;
+  GK_TRY(partial.alloc(ctx->pool, gkd::size_partials(n)));
+  GK_TRY(memb.alloc(ctx->pool, 2 * int64_t(n)));
+  GK_STAGE(ctx, GK_ST_SORT, 16LL * n,
+           gkd::launch_size_scan(n, gr.size.p, G, partial.p, gr.comp.p, gr.ctl.p, ctx->hctl, st));
+  // The counts come back while the members are ordered.
+  GK_HIP(hipEventRecord(ctx->ev, st));
+  GK_STAGE(ctx, GK_ST_SORT, 120LL * n,
+           gkd::launch_members(n, label, stamp, gr.slot.p, gr.comp.p, xadj, vw, memb.p, G, gr.ctl.p, out.order,
+                               out.cmap, out.cptr, out.mrow, out.mvw, st));
+  GK_HIP(hipEventSynchronize(ctx->ev));
+  std::memcpy(words, ctx->hctl, sizeof(int32_t) * gkd::kCtlInts);
+  return GK_OK;
+}
+
+// The same by a radix sort of (label, stamp), stamps below 2^sbits.
+static int sort_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* stamp, int sbits,
+                        const int32_t* xadj, const int32_t* vw, int32_t G, const MemberOut& out, int32_t* nc) {
+  Pool& P = ctx->pool;
   const int lbits = bits_for(n > 0 ? n - 1 : 0);
   Buf<uint64_t> keys, keys2;
-  Buf<int32_t> ids, ids2, scratch, gstart, flagscan, ncd;
+  Buf<int32_t> ids, ids2, scratch, gstart, flagscan, ncd, zero, cm;
+  if (!stamp) {
+    GK_TRY(zero.alloc(P, n));
+    gkd::fill<int32_t>(zero.p, 0, n, st);
+    stamp = zero.p;
+  }
+  int32_t* cmap = out.cmap;
+  if (!cmap) {
+    GK_TRY(cm.alloc(P, n));
+    cmap = cm.p;
+  }
   GK_TRY(keys.alloc(P, n));
   GK_TRY(keys2.alloc(P, n));
   GK_TRY(ids.alloc(P, n));
@@ -110,39 +180,70 @@ int cluster_stage(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, 
   GK_TRY(gstart.alloc(P, n));
   GK_TRY(flagscan.alloc(P, n));
   GK_TRY(ncd.alloc(P, 1));
-  GK_TRY(cptr.alloc(P, int64_t(n) + 1));
   bool alt = false;
   const int passes = (sbits + lbits + 7) / 8;
   GK_STAGE(ctx, GK_ST_SORT, 20LL * n + 32LL * n * passes,
-           (gkd::launch_make_keys(n, label, dist, sbits, keys.p, ids.p, st) ||
+           (gkd::launch_make_keys(n, label, stamp, sbits, keys.p, ids.p, st) ||
                     gkd::radix_sort_pairs<uint64_t>(keys.p, ids.p, keys2.p, ids2.p, n, 0, sbits + lbits, scratch.p, st, &alt)
                 ? GK_ERR_HIP
                 : GK_OK));
-  uint64_t* sk = alt ? keys2.p : keys.p;
-  Buf<int32_t>& sid = alt ? ids2 : ids;
-  GK_STAGE(ctx, GK_ST_CLUSTER, 64LL * n,
-           gkd::launch_cluster(n, sk, sid.p, sbits, nullptr, G, gstart.p, flagscan.p, cmap, cptr.p,
-                               nullptr, ncd.p, scratch.p, st));
+  const int32_t* sid = alt ? ids2.p : ids.p;
+  GK_STAGE(ctx, GK_ST_CLUSTER, 80LL * n,
+           (gkd::launch_cluster(n, alt ? keys2.p : keys.p, sid, sbits, G, gstart.p, flagscan.p, cmap, out.cptr, ncd.p,
+                                scratch.p, st) ||
+                    (out.mrow || out.mvw ? gkd::launch_member_rows(n, sid, xadj, vw, out.mrow, out.mvw, st) : 0)
+                ? GK_ERR_HIP
+                : GK_OK));
+  if (out.order)
+    GK_HIP(hipMemcpyAsync(out.order, sid, sizeof(int32_t) * size_t(n), hipMemcpyDeviceToDevice, st));
   GK_TRY(fetch(ctx, st, {{nc, ncd.p, sizeof(int32_t)}}));
-  order = std::move(sid);
   return GK_OK;
 }
 
-// Contraction of g under (cmap, cptr, order) into the coarse level c.
+// Coarse ids of the vertices from their candidates: groups, their members in
+// (label, stamp, id) order, chunks of at most G.
+int coarse_ids(gk_ctx* ctx, hipStream_t st, const DGraph& g, const int32_t* cand, int32_t G, bool want_order,
+               int32_t* cmap, Members& m, int32_t* nc, int32_t* rounds) {
+  Pool& P = ctx->pool;
+  const int32_t n = g.n;
+  Buf<int32_t> label;
+  Groups gr;
+  GK_TRY(label.alloc(P, n));
+  if (want_order) GK_TRY(m.order.alloc(P, n));
+  GK_TRY(m.cptr.alloc(P, int64_t(n) + 1));
+  GK_TRY(m.mrow.alloc(P, n));
+  GK_TRY(m.mvw.alloc(P, n));
+  const MemberOut out{m.order.p, cmap, m.cptr.p, m.mrow.p, m.mvw.p};
+  int32_t words[gkd::kCtlInts];
+  GK_TRY(gr.walk(ctx, st, n, cand, label.p));
+  GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, words));
+  *rounds = Groups::rounds(words);
+  if (words[gkd::kCtlFlags + gkd::kWalkBits]) {
+    GK_TRY(gr.jump(ctx, st, n, cand, label.p, rounds));
+    GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, words));
+  }
+  *nc = words[0];
+  // Distances are at most 2^rounds.
+  if (words[1]) GK_TRY(sort_members(ctx, st, n, label.p, gr.dist.p, *rounds + 1, g.xadj, g.vw, G, out, nc));
+  return GK_OK;
+}
+
+// Contraction of g under cmap, with its members by coarse id (cptr; their rows
+// mrow, and their weights mvw), into the coarse level c; with mvw also the
+// coarse weights into c.vw (allocated by the caller).
 int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, const int32_t* cmap,
-                   const int32_t* cptr, const int32_t* order, Level& c) {
+                   const int32_t* cptr, const int2* mrow, const int32_t* mvw, Level& c) {
   Pool& P = ctx->pool;
   Buf<int32_t> ub, toff, lists, lcnt, scratch, tadj, tw, len, cnnzd;
-  Buf<int2> desc, mrow;
+  Buf<int2> desc;
   GK_TRY(ub.alloc(P, nc));
   GK_TRY(toff.alloc(P, int64_t(nc) + 1));
   GK_TRY(lists.alloc(P, int64_t(4) * nc));
   GK_TRY(desc.alloc(P, int64_t(4) * nc));
-  GK_TRY(mrow.alloc(P, g.n));
   GK_TRY(lcnt.alloc(P, 4));
   GK_TRY(scratch.alloc(P, gkd::scan_scratch_ints(int64_t(nc) + 1) + 64));
-  GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 20LL * g.n + 36LL * nc,
-           gkd::launch_contract_bounds(g, nc, cptr, order, ub.p, toff.p, lists.p, desc.p, mrow.p, lcnt.p,
+  GK_STAGE(ctx, GK_ST_CONTRACT_AUX, (mvw ? 12LL : 8LL) * g.n + 40LL * nc,
+           gkd::launch_contract_bounds(nc, cptr, mrow, mvw, ub.p, toff.p, lists.p, desc.p, c.vw.p, lcnt.p,
                                        scratch.p, st));
   int32_t hc[4];
   GK_TRY(fetch(ctx, st, {{hc, lcnt.p, sizeof hc}}));
@@ -159,7 +260,7 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
       const int32_t* rows = lists.p + int64_t(cls) * nc;
       auto run = [&](const Tuner::Shape& x) {
         return gkd::launch_contract_rows(g, x.lanes, x.block, rows, desc.p + int64_t(cls) * nc, hc[cls], nc,
-                                         mrow.p, cmap, toff.p, tadj.p, tw.p, len.p, wide, st, steal_of(ctx));
+                                         mrow, cmap, toff.p, tadj.p, tw.p, len.p, wide, st, steal_of(ctx));
       };
       Tuner::Shape shape{lanes[cls], 256};
       if (ctx->autotune && hc[cls] >= kTuneMinRows) {
@@ -203,7 +304,7 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
     bool alt = false;
     const int bpasses = (32 + bits_for(nbig - 1) + 7) / 8;
     GK_STAGE(ctx, GK_ST_CONTRACT_BIG, 24LL * eb + 36LL * eb * bpasses + 24LL * eb,
-             (gkd::launch_contract_big_gather(g, rows, nbig, boff.p, cptr, order, cmap, k1.p, v1.p, st) ||
+             (gkd::launch_contract_big_gather(g, rows, nbig, boff.p, cptr, mrow, cmap, k1.p, v1.p, st) ||
                       gkd::radix_sort_pairs<uint64_t>(k1.p, v1.p, k2.p, v2.p, eb, 0, 32 + bits_for(nbig - 1),
                                                       sscr.p, st, &alt) ||
                       gkd::launch_contract_big_merge(rows, nbig, boff.p, alt ? k2.p : k1.p, alt ? v2.p : v1.p,
@@ -321,23 +422,20 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     const int32_t n = f.g.n;
     if (!(n > floor_n)) break;
     gk_level_stats& ls = S.levels[L.size() - 1];
-    Buf<int32_t> cand, label, dist, order, cptr, cmap;
+    Buf<int32_t> cand, cmap;
+    Members mem;
     GK_TRY(cand.alloc(P, n));
-    GK_TRY(label.alloc(P, n));
     GK_TRY(cmap.alloc(P, n));
     GK_STAGE(ctx, GK_ST_MATCH, 16LL * f.g.nnz + 8LL * n + 4,
              match_stage(ctx, st, f.g, cand.p));
-    int32_t rounds = 0;
-    GK_TRY(group_stage(ctx, st, n, cand.p, label.p, dist, &rounds));
-    int32_t nc = 0;
-    GK_TRY(cluster_stage(ctx, st, n, label.p, dist.p, rounds + 1, prm.max_group, order, cmap.p, cptr, &nc));
+    int32_t rounds = 0, nc = 0;
+    GK_TRY(coarse_ids(ctx, st, f.g, cand.p, prm.max_group, false, cmap.p, mem, &nc, &rounds));
     if (nc == n || nc < k + 1) break;
     if (prm.coarsen_policy != GK_COARSEN_REF && nc < floor_n) break;
     Level c;
     GK_TRY(c.vw.alloc(P, nc));
-    GK_STAGE(ctx, GK_ST_CLUSTER, 8LL * n + 12LL * nc, gkd::launch_cvwgt(nc, cptr.p, order.p, f.g.vw, c.vw.p, st));
     c.g.vw = c.vw.p;
-    GK_TRY(contract_stage(ctx, st, f.g, nc, cmap.p, cptr.p, order.p, c));
+    GK_TRY(contract_stage(ctx, st, f.g, nc, cmap.p, mem.cptr.p, mem.mrow.p, mem.mvw.p, c));
     ls.sweeps = rounds;
     if (trace) {
       std::vector<int32_t> h;
@@ -736,11 +834,19 @@ int gk_ctx_create(int device, gk_ctx** out) {
     gkh::set_error("hipStreamCreate failed");
     return GK_ERR_HIP;
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&c->hpin), 4096, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->hpin), kPinFetch + kPinCtl, hipHostMallocDefault) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     delete c;
     gkh::set_error("hipHostMalloc failed");
     return GK_ERR_NOMEM;
+  }
+  c->hctl = reinterpret_cast<int32_t*>(c->hpin + kPinFetch);
+  if (hipEventCreateWithFlags(&c->ev, hipEventDisableTiming) != hipSuccess) {
+    (void)hipHostFree(c->hpin);
+    (void)hipStreamDestroy(c->stream);
+    delete c;
+    gkh::set_error("hipEventCreate failed");
+    return GK_ERR_HIP;
   }
   *out = c;
   return GK_OK;
@@ -763,6 +869,7 @@ int gk_ctx_destroy(gk_ctx* c) {
   DeviceGuard dg(c->device);
   (void)hipStreamSynchronize(c->stream);
   c->pool.release_all();
+  (void)hipEventDestroy(c->ev);
   (void)hipHostFree(c->hpin);
   (void)hipStreamDestroy(c->stream);
   delete c;
@@ -873,11 +980,17 @@ int gk_k_group(gk_ctx* ctx, int32_t n, const int32_t* cand, int32_t* label, int3
   DeviceGuard guard(ctx->device);
   hipStream_t st = pick(ctx, stream);
   if (n <= 0) { if (sweeps) *sweeps = 0; return GK_OK; }
-  Buf<int32_t> dist;
-  int32_t rounds = 0;
-  GK_TRY(group_stage(ctx, st, n, cand, label, dist, &rounds));
-  GK_HIP(hipMemcpyAsync(stamp, dist.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
-  GK_HIP(hipStreamSynchronize(st));
+  Groups gr;
+  int32_t words[gkd::kCtlInts];
+  GK_TRY(gr.walk(ctx, st, n, cand, label));
+  GK_HIP(hipMemcpyAsync(stamp, gr.dist.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
+  GK_TRY(fetch(ctx, st, {{words, gr.ctl.p, sizeof words}}));
+  int32_t rounds = Groups::rounds(words);
+  if (words[gkd::kCtlFlags + gkd::kWalkBits]) {
+    GK_TRY(gr.jump(ctx, st, n, cand, label, &rounds));
+    GK_HIP(hipMemcpyAsync(stamp, gr.dist.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
+    GK_HIP(hipStreamSynchronize(st));
+  }
   if (sweeps) *sweeps = rounds;
   return GK_OK;
 }
@@ -892,15 +1005,24 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
   DeviceGuard guard(ctx->device);
   hipStream_t st = pick(ctx, stream);
   if (n <= 0) { *nc = 0; return GK_OK; }
-  // The stamp bit width is taken from the data (max stamp).
-  std::vector<int32_t> hs;
-  GK_TRY(to_host(st, hs, stamp, n));
-  int32_t mx = 0;
-  for (int32_t x : hs) mx = std::max(mx, x);
-  Buf<int32_t> ord, cptr;
-  GK_TRY(cluster_stage(ctx, st, n, label, stamp, bits_for(mx), max_group, ord, cmap, cptr, nc));
-  GK_TRY(gkd::launch_cvwgt(*nc, cptr.p, ord.p, vwgt, cvwgt, st));
-  GK_HIP(hipMemcpyAsync(order, ord.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
+  Groups gr;
+  Buf<int32_t> cptr, mvw;
+  GK_TRY(cptr.alloc(ctx->pool, int64_t(n) + 1));
+  GK_TRY(mvw.alloc(ctx->pool, n));
+  const MemberOut out{order, cmap, cptr.p, nullptr, mvw.p};
+  int32_t words[gkd::kCtlInts];
+  GK_TRY(gr.count(ctx, st, n, label));
+  GK_TRY(count_members(ctx, st, n, label, stamp, gr, nullptr, vwgt, max_group, out, words));
+  *nc = words[0];
+  if (words[1]) {
+    // The stamp bit width is taken from the data (max stamp).
+    std::vector<int32_t> hs;
+    GK_TRY(to_host(st, hs, stamp, n));
+    int32_t mx = 0;
+    for (int32_t x : hs) mx = std::max(mx, x);
+    GK_TRY(sort_members(ctx, st, n, label, stamp, bits_for(mx), nullptr, vwgt, max_group, out, nc));
+  }
+  GK_TRY(gkd::launch_cvwgt(*nc, cptr.p, mvw.p, cvwgt, st));
   GK_HIP(hipStreamSynchronize(st));
   return GK_OK;
 }
@@ -915,21 +1037,26 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   hipStream_t st = pick(ctx, stream);
   Pool& P = ctx->pool;
   const int32_t n = dg->n;
-  // Members of each coarse vertex from a stable sort of (cmap[v], v).
-  Buf<int32_t> zero, order, cptr;
-  Buf<int32_t> cm_as_label;
-  GK_TRY(zero.alloc(P, n));
-  gkd::fill<int32_t>(zero.p, 0, n, st);
+  // Members of each coarse vertex in order of (cmap[v], v).
+  Members m;
+  Groups gr;
+  GK_TRY(m.cptr.alloc(P, int64_t(n) + 1));
+  GK_TRY(m.mrow.alloc(P, n));
+  const MemberOut out{nullptr, nullptr, m.cptr.p, m.mrow.p, nullptr};
+  int32_t words[gkd::kCtlInts];
   int32_t nc2 = 0;
-  Buf<int32_t> scratch_cmap;
-  GK_TRY(scratch_cmap.alloc(P, n));
-  GK_TRY(cluster_stage(ctx, st, n, cmap, zero.p, 1, INT32_MAX, order, scratch_cmap.p, cptr, &nc2));
+  if (n > 0) {
+    GK_TRY(gr.count(ctx, st, n, cmap));
+    GK_TRY(count_members(ctx, st, n, cmap, nullptr, gr, dg->xadj, nullptr, INT32_MAX, out, words));
+    nc2 = words[0];
+    if (words[1]) GK_TRY(sort_members(ctx, st, n, cmap, nullptr, 1, dg->xadj, nullptr, INT32_MAX, out, &nc2));
+  }
   // With G = INT32_MAX every label is one chunk, so chunks are the coarse
   // vertices in id order exactly when cmap is onto [0, nc).
   if (nc2 != nc) { gkh::set_error("cmap is not onto [0, nc)"); return GK_ERR_ARG; }
   Level c;
   DGraph g = dview(dg);
-  GK_TRY(contract_stage(ctx, st, g, nc, cmap, cptr.p, order.p, c));
+  GK_TRY(contract_stage(ctx, st, g, nc, cmap, m.cptr.p, m.mrow.p, nullptr, c));
   GK_HIP(hipMemcpyAsync(cxadj, c.g.xadj, sizeof(int32_t) * (nc + 1), hipMemcpyDeviceToDevice, st));
   if (c.g.nnz) {
     GK_HIP(hipMemcpyAsync(cadjncy, c.g.adj, sizeof(int32_t) * c.g.nnz, hipMemcpyDeviceToDevice, st));

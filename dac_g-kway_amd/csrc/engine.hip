@@ -291,25 +291,21 @@ int Engine::coarsen_step(bool* worked) {
   const Store& F = *pk;
   const DGraph g = F.graph();
   const int32_t n = g.n, J = F.nj;
-  Buf<int32_t> cand, label, dist, order, cptr, ce;
+  Buf<int32_t> cand, ce;
+  Members mem;
   auto cmap = std::make_shared<Buf<int32_t>>();
   GK_TRY(cand.alloc(P_, n));
-  GK_TRY(label.alloc(P_, n));
   GK_TRY(cmap->alloc(P_, n));
   GK_STAGE(ctx_, GK_ST_MATCH, 16LL * g.nnz + 8LL * n + 4,
            match_stage(ctx_, st_, g, cand.p));
-  int32_t rounds = 0;
-  GK_TRY(group_stage(ctx_, st_, n, cand.p, label.p, dist, &rounds));
-  int32_t nc = 0;
-  GK_TRY(cluster_stage(ctx_, st_, n, label.p, dist.p, rounds + 1, G, order, cmap->p, cptr, &nc));
+  int32_t rounds = 0, nc = 0;
+  GK_TRY(coarse_ids(ctx_, st_, g, cand.p, G, true, cmap->p, mem, &nc, &rounds));
   auto C = std::make_shared<Store>();
   GK_TRY(C->dv_off.alloc(P_, int64_t(J) + 1));
-  GK_TRY(gkd::launch_job_offsets(J, F.dv_off.p, order.p, cmap->p, nc, C->dv_off.p, st_));
-  GK_TRY(C->bv.alloc(P_, nc));
-  GK_STAGE(ctx_, GK_ST_CLUSTER, 8LL * n + 12LL * nc,
-           gkd::launch_cvwgt(nc, cptr.p, order.p, g.vw, C->bv.p, st_));
+  GK_TRY(gkd::launch_job_offsets(J, F.dv_off.p, mem.order.p, cmap->p, nc, C->dv_off.p, st_));
   Level c;
-  GK_TRY(contract_stage(ctx_, st_, g, nc, cmap->p, cptr.p, order.p, c));
+  GK_TRY(c.vw.alloc(P_, nc));
+  GK_TRY(contract_stage(ctx_, st_, g, nc, cmap->p, mem.cptr.p, mem.mrow.p, mem.mvw.p, c));
   GK_TRY(ce.alloc(P_, int64_t(J) + 1));
   GK_TRY(gkd::launch_job_eoffsets(J, C->dv_off.p, c.xadj.p, ce.p, st_));
   C->v_off.resize(J + 1);
@@ -322,6 +318,7 @@ int Engine::coarsen_step(bool* worked) {
   C->bx = std::move(c.xadj);
   C->ba = std::move(c.adj);
   C->bw = std::move(c.w);
+  C->bv = std::move(c.vw);
   C->xadj = C->bx.p;
   C->adj = C->ba.p;
   C->w = C->bw.p;

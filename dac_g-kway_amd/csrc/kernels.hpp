@@ -54,25 +54,62 @@ int launch_jump_init(int32_t n, const int32_t* cand, int32_t* next, int32_t* dis
 int launch_jump_round(int32_t n, const int32_t* cand, const int32_t* next_in, const int32_t* dist_in,
                       int32_t* next_out, int32_t* dist_out, int32_t* flags, int32_t round,
                       hipStream_t st);
-// label[v] = largest id of v's component (root pair found via next[]).
-int launch_label(int32_t n, const int32_t* cand, const int32_t* next, int32_t* compmax,
-                 int32_t* label, hipStream_t st);
+// Control words of a coarsening level (zeroed by the caller): [0] coarse ids,
+// [1] some group has more than kRankMax members, [2 + r] flags of the walk:
+// some vertex is more than 2^r hops from its root pair (r = kWalkBits: more
+// than kWalkMax, unresolved).
+constexpr int kWalkBits = 6;
+constexpr int kWalkMax = 1 << kWalkBits;
+constexpr int kCtlFlags = 2;
+constexpr int kCtlInts = kCtlFlags + kWalkBits + 1;
+// Largest group whose members find their order by counting.
+constexpr int32_t kRankMax = 512;
+// Grouping by walking to the root pair: key of v's component, hops, and comp
+// [key] = (largest id, members); slot[v] = v's place among the members
+// (arbitrary).  flags: the control words from kCtlFlags on.
+int launch_walk(int32_t n, const int32_t* cand, int2* comp, int32_t* key, int32_t* dist, int32_t* slot,
+                int32_t* flags, hipStream_t st);
+// The same (without hops) from the pointers of the jumping rounds.
+int launch_comp_count(int32_t n, const int32_t* cand, const int32_t* next, int2* comp, int32_t* key, int32_t* slot,
+                      hipStream_t st);
+// label[v] = largest id of v's component, size[l] = members of label l (0
+// where l is no label).  key may be label.
+int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* label, int32_t* size,
+                      hipStream_t st);
+// size and slot of labels in [0, n) that come without a grouping.
+int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, hipStream_t st);
+// offc[l] = (first place, first coarse id) of label l's group; coarse ids and
+// flags to ctl and to host (pinned, kCtlInts ints).  partial: size_partials(n),
+// offc: n + 1 (the last one the totals).
+int64_t size_partials(int64_t n);
+int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl, int32_t* host,
+                     hipStream_t st);
+// Vertices in (label, stamp, id) order, chunks of at most G, the members' rows
+// and weights in that order.  memb: 2n records; stamp, xadj, vw and the
+// outputs order, cmap, mrow, mvw may be null.  Groups of more than kRankMax members
+// are left out (ctl[1] is set for them).
+int launch_members(int32_t n, const int32_t* label, const int32_t* stamp, const int32_t* slot, const int2* offc,
+                   const int32_t* xadj, const int32_t* vw, int4* memb, int32_t G, const int32_t* ctl,
+                   int32_t* order, int32_t* cmap, int32_t* cptr, int2* mrow, int32_t* mvw, hipStream_t st);
+// mrow and mvw (each may be null) of a given order.
+int launch_member_rows(int32_t n, const int32_t* order, const int32_t* xadj, const int32_t* vw, int2* mrow,
+                       int32_t* mvw, hipStream_t st);
 // keys[v] = (label << sbits) | dist, ids[v] = v.
 int launch_make_keys(int32_t n, const int32_t* label, const int32_t* dist, int sbits,
                      uint64_t* keys, int32_t* ids, hipStream_t st);
-// Chunking of the sorted order: cmap, chunk pointers, coarse weights; nc_dev.
-int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sbits,
-                   const int32_t* vwgt, int32_t G, int32_t* gstart, int32_t* flagscan,
-                   int32_t* cmap, int32_t* cptr, int32_t* cvwgt, int32_t* nc_dev,
-                   int32_t* scratch, hipStream_t st);
+// Chunking of the sorted order: cmap, chunk pointers; nc_dev.
+int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sbits, int32_t G, int32_t* gstart,
+                   int32_t* flagscan, int32_t* cmap, int32_t* cptr, int32_t* nc_dev, int32_t* scratch,
+                   hipStream_t st);
 // Contraction, phase 1: per coarse row the upper bound of its entries
 // (sum of member degrees), its class (16/32/64-lane or big), appended to
-// lists[cls * nc ..] with its member range in desc; mrow[m] = (row start,
-// row length) of the member at order position m; the exclusive scan of the
-// bounds (toff, nc+1 entries).  lists and desc: 4 * nc entries, mrow: n.
-int launch_contract_bounds(const DGraph& g, int32_t nc, const int32_t* cptr, const int32_t* order,
-                           int32_t* ub, int32_t* toff, int32_t* lists, int2* desc, int2* mrow,
-                           int32_t* list_cnt, int32_t* scratch, hipStream_t st);
+// lists[cls * nc ..] with its member range in desc; the exclusive scan of the
+// bounds (toff, nc+1 entries).  lists and desc: 4 * nc entries; mrow[m] = (row
+// start, row length) of the member at place m.  With mvw (the members'
+// weights) also the coarse weights cvw.
+int launch_contract_bounds(int32_t nc, const int32_t* cptr, const int2* mrow, const int32_t* mvw, int32_t* ub,
+                           int32_t* toff, int32_t* lists, int2* desc, int32_t* cvw, int32_t* list_cnt,
+                           int32_t* scratch, hipStream_t st);
 // Phase 2 for the rows of one class (lanes in {16, 32, 64}); block size 64,
 // 128, 256 or 512 threads (launch shape only).  nc: coarse vertex count; the
 // sort packs the lane number beside the coarse id in 32 bits when nc allows,
@@ -84,7 +121,7 @@ int launch_contract_rows(const DGraph& g, int lanes, int block, const int32_t* r
                          const Steal* ws = nullptr);
 // Phase 2 for big rows: gather to (row-rank, neighbour) keys.
 int launch_contract_big_gather(const DGraph& g, const int32_t* rows, int32_t nrows,
-                               const int32_t* boff, const int32_t* cptr, const int32_t* order,
+                               const int32_t* boff, const int32_t* cptr, const int2* mrow,
                                const int32_t* cmap, uint64_t* keys, int32_t* vals, hipStream_t st);
 // Segmented merge of the sorted big-row entries into the temporary rows.
 int launch_contract_big_merge(const int32_t* rows, int32_t nrows, const int32_t* boff,
@@ -158,7 +195,6 @@ int launch_cut(const DGraph& g, int32_t k, const int32_t* part, unsigned long lo
                int64_t max_slots = INT64_MAX);
 
 int launch_sum(const int32_t* a, int64_t n, unsigned long long* out, hipStream_t st);
-int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* order, const int32_t* vw,
-                 int32_t* cvw, hipStream_t st);
+int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* mvw, int32_t* cvw, hipStream_t st);
 
 }  // namespace gkd

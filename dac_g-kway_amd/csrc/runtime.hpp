@@ -365,11 +365,20 @@ class Tuner {
 };
 }  // namespace gkrt
 
+namespace gkrt {
+// Pinned bytes of a context: fetch() staging, then the control words.
+constexpr size_t kPinFetch = 4096;
+constexpr size_t kPinCtl = 256;
+static_assert(sizeof(int32_t) * gkd::kCtlInts <= kPinCtl, "control words fit");
+}  // namespace gkrt
+
 struct gk_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   gkrt::Pool pool;
   char* hpin = nullptr;  // pinned staging for small read-backs
+  int32_t* hctl = nullptr;  // pinned: control words that kernels write to the host themselves
+  hipEvent_t ev = nullptr;  // marks when they are written
   gkrt::StageClock clock;
   gk_stats* cur = nullptr;  // stats of the running partition (stage counters)
   gkrt::Pinned up, dl;      // pinned staging of the batched form (uploads / read-backs)
@@ -532,13 +541,38 @@ inline int to_host(hipStream_t st, std::vector<T>& out, const T* dev, int64_t n)
 // Coarsening stages shared by the plain driver and the batch engine
 // (defined in driver.hip).
 struct Level;
-int group_stage(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label,
-                Buf<int32_t>& dist_out, int32_t* rounds);
-int cluster_stage(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* dist,
-                  int32_t max_dist_bits, int32_t G, Buf<int32_t>& order, int32_t* cmap,
-                  Buf<int32_t>& cptr, int32_t* nc);
+
+// Groups of a level: hops, members' places and sizes by label; comp is
+// scratch (component counts, then each label's first place and coarse id).
+struct Groups {
+  Buf<int32_t> ctl, dist, slot, size;
+  Buf<int2> comp;
+  int walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label);
+  int jump(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* rounds);
+  int count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label);
+  static int32_t rounds(const int32_t* words);
+};
+
+// Members by coarse id: first place of every coarse id, and in member order
+// the vertices, their rows (start, length) and their weights.
+struct Members {
+  Buf<int32_t> order, cptr, mvw;
+  Buf<int2> mrow;
+};
+
+// Where the member order and coarse ids go (all but cptr may be null).
+struct MemberOut {
+  int32_t* order;
+  int32_t* cmap;
+  int32_t* cptr;
+  int2* mrow;
+  int32_t* mvw;
+};
+
+int coarse_ids(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, const int32_t* cand, int32_t G, bool want_order,
+               int32_t* cmap, Members& m, int32_t* nc, int32_t* rounds);
 int contract_stage(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, int32_t nc, const int32_t* cmap,
-                   const int32_t* cptr, const int32_t* order, Level& c);
+                   const int32_t* cptr, const int2* mrow, const int32_t* mvw, Level& c);
 // Lanes per vertex of the gain pass for this graph's average degree.
 int gain_lanes(const gkd::DGraph& g);
 // Candidate matching with the context's tuned launch shape (tuned on first
