@@ -242,10 +242,9 @@ struct BalanceOpt {
 // advances pw and subtracts the prefix's gains from *cut.  Returns pos to
 // every thread.
 __device__ inline int balance_prefix(BalanceLds& L, int32_t* dpw, int32_t k, int32_t B, uint64_t idmask,
-                                     const int32_t* __restrict__ part, const int32_t* __restrict__ dest,
-                                     const int32_t* __restrict__ gain, const int32_t* __restrict__ vw,
-                                     int32_t* __restrict__ pw, long long cap, int32_t* __restrict__ moves,
-                                     int32_t* __restrict__ pos_out, long long* __restrict__ cut,
+                                     const int32_t* part, const int32_t* dest, const int32_t* gain,
+                                     const int32_t* __restrict__ vw, int32_t* pw, long long cap,
+                                     int32_t* __restrict__ moves, int32_t* __restrict__ pos_out, long long* cut,
                                      const BalanceOpt& opt = BalanceOpt{}) {
   const int t = threadIdx.x;
   const int lane = lane_id();

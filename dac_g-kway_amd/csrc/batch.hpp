@@ -93,7 +93,8 @@ int select_scratch_ints(int64_t n);
 // that ran the top-M radix select, rounds whose compressed keys exceeded 32
 // bits, rounds that tested deferred vertices.  order (may be null): per job
 // M + 2 ints, [0] = B, [1] = pos and [2, 2 + B) the ordered moves of the
-// job's latest round that selected any.  abytes (may be null): per job, the
+// job's latest round that selected any; hist (may be null, one job): B and pos
+// of ordering round r at hist[2r].  abytes (may be null): per job, the
 // algorithmic bytes of its rounds are added.
 int launch_select_list(const DGraph& g, const int32_t* vjob, const int32_t* gain, const int32_t* dest,
                        const int32_t* pw, const int32_t* pw_off, const long long* cap, const int32_t* thr,
@@ -103,8 +104,40 @@ int launch_round_b(int32_t nj, int32_t kmax, const int32_t* v_off, int32_t M, co
                    const int32_t* pw_off, const DGraph& g, int32_t* part, const int32_t* dest, const int32_t* gain,
                    int32_t* pw, long long* cut, int32_t* rounds, long long* moved, const SelectBufs& sb,
                    int32_t* xlist, uint32_t* hkey, int32_t* upd, int32_t* wl, int32_t* wlc, int32_t* lastcnt,
-                   int32_t* active, uint64_t* cand, int32_t* thr, long long* paths, int32_t* order,
+                   int32_t* active, uint64_t* cand, int32_t* thr, long long* paths, int32_t* order, int32_t* hist,
                    long long* abytes, hipStream_t st);
+// All of a round, and many rounds, in one launch (one workgroup per job), for
+// k <= kGainInlineK.  A job stops when a round selects nothing (lastcnt[job] =
+// 0), after max_rounds rounds, when a round updates more vertices than one
+// workgroup should (they are appended to wl, count wlc[0]: a gain pass over it
+// must follow), or before its first round when its candidates are too many.
+// status[0] receives the number of jobs not converged, status[1] how many of
+// them had too many candidates (launch_select_list and launch_round_b then do
+// their rounds).  wlc and status are zero before the launch; next_wlc and
+// next_status, the words of the launch after it, are zeroed by it.  hist and
+// order (may be null; one job): every ordering round r's move count and
+// position to hist[2r], and the latest one's moves as in launch_round_b.
+struct RoundsArgs {
+  const int32_t* v_off;
+  int32_t M, max_rounds;
+  const int32_t* kk;
+  const long long* cap;
+  const int32_t* pw_off;
+  const int32_t *xadj, *adj, *w, *vw;
+  int32_t *part, *bnd, *gain, *dest, *pw;
+  long long* cut;
+  int32_t* rounds;
+  long long* moved;
+  uint64_t* cand;
+  int32_t *upd, *wl, *wlc, *next_wlc, *lastcnt, *status, *next_status, *thr;
+  long long *paths, *abytes;
+  int32_t *order, *hist;
+};
+int launch_rounds(const RoundsArgs& a, int32_t nj, int lanes, hipStream_t st);
+// Per-job state before a level's first round (rounds, moved and abytes 0,
+// lastcnt and thr 1) and the 4 words each of wlc and status.
+int launch_rounds_init(int32_t nj, int32_t* lastcnt, int32_t* thr, int32_t* rounds, long long* moved,
+                       long long* abytes, int32_t* wlc, int32_t* status, hipStream_t st);
 // *out = largest row length of g.
 int launch_max_deg(const DGraph& g, int32_t* out, hipStream_t st);
 // Final cut and part weights of the jobs covered by the chunk table: chunk c

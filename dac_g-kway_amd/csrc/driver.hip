@@ -359,6 +359,126 @@ int gain_lanes(const DGraph& g) {
   return s;
 }
 
+// ---------------------------------------------------------------- rounds
+namespace {
+
+// One round by the separate kernels.
+int wide_round(gk_ctx* ctx, hipStream_t st, const RoundState& s) {
+  GK_STAGE(ctx, GK_ST_SELECT, 0,
+           gkd::launch_select_list(s.g, s.vjob, s.gain, s.dest, s.pw, s.pw_off, s.cap, s.thr, s.cand, s.sb, s.hcnt,
+                                   s.active, st));
+  GK_STAGE(ctx, GK_ST_BALANCE, 0,
+           gkd::launch_round_b(s.nj, s.kmax, s.v_off, s.M, s.kk, s.cap, s.pw_off, s.g, s.part, s.dest, s.gain, s.pw,
+                               s.cut, s.rounds, s.moved, s.sb, s.xlist, s.hkey, s.upd, s.wl, s.hcnt, s.lastcnt,
+                               s.active, s.cand, s.thr, s.paths, s.order, s.hist, s.abytes, st));
+  GK_STAGE(ctx, GK_ST_GAIN, 0,
+           gkd::launch_gain_wl(s.g, s.kmax, s.lanes, s.wl, s.hcnt, s.heavy, s.part, s.upd, s.bnd, s.gain, s.dest,
+                               s.work, s.wl_items, s.cand, st, steal_of(ctx)));
+  if (s.heavy_rows)
+    GK_STAGE(ctx, GK_ST_GAIN_HEAVY, 0,
+             gkd::launch_gain_heavy(s.g, s.kmax, s.heavy, s.hcnt, s.part, s.upd, s.bnd, s.gain, s.dest, s.work, s.cand,
+                                    st));
+  return GK_OK;
+}
+
+// A launch of the round loop and the gain pass over what it left; pair: which
+// pair of counts and status words it uses.
+int loop_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, int pair) {
+  const int o = 2 * pair, e = 2 * (1 - pair);
+  const gkd::RoundsArgs a{s.v_off,     s.M,        max_rounds, s.kk,         s.cap,        s.pw_off,  s.g.xadj,
+                          s.g.adj,     s.g.w,      s.g.vw,     s.part,       s.bnd,        s.gain,    s.dest,
+                          s.pw,        s.cut,      s.rounds,   s.moved,      s.cand,       s.upd,     s.wl,
+                          s.hcnt + o,  s.hcnt + e, s.lastcnt,  s.status + o, s.status + e, s.thr,     s.paths,
+                          s.abytes,    s.order,    s.hist};
+  GK_STAGE(ctx, GK_ST_BALANCE, 0, gkd::launch_rounds(a, s.nj, s.lanes, st));
+  GK_STAGE(ctx, GK_ST_GAIN, 0,
+           gkd::launch_gain_wl(s.g, s.kmax, s.lanes, s.wl, s.hcnt + o, s.heavy, s.part, s.upd, s.bnd, s.gain, s.dest,
+                               s.work, s.wl_items, s.cand, st, steal_of(ctx)));
+  return GK_OK;
+}
+
+}  // namespace
+
+// Two ways to run rounds, which leave the same state.  The round loop (one
+// workgroup per job, k <= kGainInlineK) is the faster one while a job has up
+// to some thousand candidates; the separate kernels select over the whole
+// device, and start on graphs so large that their first rounds will have more.
+// The host looks at the end of a round loop's launch, and every 4 rounds of
+// the separate kernels (every 8, 16, then 32 once they ran 32: a look costs a
+// copy and a synchronisation; a round with nothing selected changes nothing).
+int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, bool exact, bool graph, int* ran) {
+  constexpr int kWideRounds = 4;
+  constexpr int kLoopRounds = 64;
+  constexpr int64_t kLoopVertices = int64_t(1) << 20;  // per job, to begin with the loop
+  constexpr int32_t kLoopSelected = 1024;              // selected per round, to come back to it
+  const bool can_loop = s.kmax <= gkd::kGainInlineK;
+  bool loop = can_loop && int64_t(s.g.n) <= kLoopVertices * s.nj;
+  graph = graph && !exact && !ctx->clock.timed(GK_ST_SELECT) && !ctx->clock.timed(GK_ST_BALANCE) &&
+          !ctx->clock.timed(GK_ST_GAIN) && !ctx->clock.timed(GK_ST_GAIN_HEAVY);
+  RoundGraph wide_graph, loop_graph;
+  int pair = 1;  // the compaction before the rounds used pair 0
+  int done = 0, wide_done = 0, per_check = kWideRounds;
+  while (max_rounds <= 0 || done < max_rounds) {
+    if (loop) {
+      const int left = max_rounds > 0 ? max_rounds - done : kLoopRounds;
+      int32_t words[2] = {0, 0}, made = 0;
+      if (graph && left >= kLoopRounds) {
+        // both pairs, so that every replay begins with the same one
+        if (!loop_graph.ready())
+          GK_TRY(loop_graph.capture(ctx, st, [&]() -> int {
+            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, pair));
+            return loop_rounds(ctx, st, s, kLoopRounds / 2, 1 - pair);
+          }));
+        GK_TRY(loop_graph.replay(ctx, st));
+        GK_TRY(fetch(ctx, st, {{words, s.status + 2 * (1 - pair), sizeof words}}));
+        done += kLoopRounds;
+      } else {
+        const int rounds = std::min(left, kLoopRounds);
+        GK_TRY(loop_rounds(ctx, st, s, rounds, pair));
+        if (exact) {  // one job: its ordering rounds so far are the rounds done
+          GK_TRY(fetch(ctx, st, {{words, s.status + 2 * pair, sizeof words}, {&made, s.rounds, sizeof made}}));
+          done = made;
+        } else {
+          GK_TRY(fetch(ctx, st, {{words, s.status + 2 * pair, sizeof words}}));
+          done += rounds;
+        }
+        pair = 1 - pair;
+      }
+      if (words[0] == 0) break;
+      if (words[1] != 0) {
+        loop = false;
+        if (!exact) done -= std::min(done, kLoopRounds);  // jobs left out did none
+      }
+    } else {
+      const int left = max_rounds > 0 ? max_rounds - done : per_check;
+      const int rounds = std::min(left, per_check);
+      if (graph && rounds % kWideRounds == 0) {
+        if (!wide_graph.ready())
+          GK_TRY(wide_graph.capture(ctx, st, [&]() -> int {
+            for (int r = 0; r < kWideRounds; ++r) GK_TRY(wide_round(ctx, st, s));
+            return GK_OK;
+          }));
+        for (int r = 0; r < rounds; r += kWideRounds) GK_TRY(wide_graph.replay(ctx, st));
+      } else {
+        for (int r = 0; r < rounds; ++r) GK_TRY(wide_round(ctx, st, s));
+      }
+      done += rounds;
+      wide_done += rounds;
+      int32_t live = 0;
+      GK_TRY(fetch(ctx, st, {{&live, s.active, sizeof live}}));
+      if (live == 0) break;
+      if (can_loop && live <= kLoopSelected * s.nj) {
+        loop = true;
+        gkd::fill<int32_t>(s.hcnt, 0, 4, st);
+        gkd::fill<int32_t>(s.status, 0, 4, st);
+      }
+      if (wide_done >= 32 && per_check < 32) per_check *= 2;
+    }
+  }
+  if (ran) *ran = done;
+  return GK_OK;
+}
+
 }  // namespace gkrt
 
 namespace {
@@ -532,18 +652,14 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   const auto t2 = clk::now();
 
   // ---------------------------------------------------------- uncoarsening
-  // Rounds run back to back on the device (select_list, round_b with one
-  // job, gain passes); the host reads the last round's move count every
-  // kRoundsPerCheck rounds, every 8, 16, then 32 once a level has run 32
-  // (a check costs a copy and a host sync).  A round with nothing selected
-  // changes nothing.
+  // Rounds run back to back on the device (refine_rounds).
   int32_t* cur_part = partA.p;
   int32_t* cur_bnd = bndA.p;
   int32_t* oth_part = partB.p;
   int32_t* oth_bnd = bndB.p;
   if (nl > 1) {
     const int32_t M = prm.max_moves;
-    Buf<int32_t> xlist, dthr, wpos, sscr;
+    Buf<int32_t> xlist, dthr, wpos, sscr, status;
     Buf<int32_t> gain, dest, upd, heavy, hcnt, wl, list, active, drounds, lastcnt, dvoff, dpw_off, dkk;
     Buf<long long> dcap, dmoved, dpaths, dabytes;
     Buf<uint64_t> cand, movable, selbits, defbits;
@@ -576,7 +692,8 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     GK_TRY(sscr.alloc(P, gkd::select_scratch_ints(n0)));
     GK_TRY(xlist.alloc(P, n0));
     GK_TRY(dthr.alloc(P, 1));
-    GK_TRY(hcnt.alloc(P, 2));  // [0] gain worklist count, [1] heavy-row count
+    GK_TRY(hcnt.alloc(P, 4));  // two pairs: [0] gain worklist count, [1] heavy-row count
+    GK_TRY(status.alloc(P, 4));
     GK_TRY(active.alloc(P, 1));
     // Per-level rounds, moves and cut after the level, read back once at the end.
     Buf<long long> dcutlv;
@@ -596,7 +713,6 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     gkd::fill<int32_t>(dpw_off.p + 1, k, 1, st);
     gkd::fill<int32_t>(dkk.p, k, 1, st);
     gkd::fill<long long>(dcap.p, static_cast<long long>(cap), 1, st);
-    constexpr int kRoundsPerCheck = 4;
     for (int32_t l = nl - 2; l >= 0; --l) {
       Level& f = L[l];
       const DGraph& g = f.g;
@@ -615,13 +731,9 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
       // After projection every gain is 0: no candidate yet.
       gkd::fill<uint64_t>(cand.p, 0ull, (int64_t(g.n) + 63) / 64 + 1, st);
       gkd::fill<int32_t>(dvoff.p + 1, g.n, 1, st);
-      gkd::fill<int32_t>(drounds.p + l, 0, 1, st);
-      gkd::fill<int32_t>(lastcnt.p, 1, 1, st);
-      gkd::fill<int32_t>(dthr.p, 1, 1, st);
-      gkd::fill<long long>(dmoved.p + l, 0, 1, st);
-      gkd::fill<long long>(dabytes.p + l, 0, 1, st);
+      GK_TRY(gkd::launch_rounds_init(1, lastcnt.p, dthr.p, drounds.p + l, dmoved.p + l, dabytes.p + l, hcnt.p, status.p,
+                                     st));
       // The projected boundary becomes the first gain worklist.
-      gkd::fill<int32_t>(hcnt.p, 0, 2, st);
       GK_STAGE(ctx, GK_ST_PROJECT, 4LL * g.n, gkd::launch_compact(g.n, upd.p, wl.p, hcnt.p, st));
       GK_STAGE(ctx, GK_ST_GAIN, 0,
                gkd::launch_gain_wl(g, k, lanes, wl.p, hcnt.p, heavy.p, cur_part, upd.p, cur_bnd, gain.p, dest.p,
@@ -633,46 +745,41 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
       // A round updates at most M movers and their neighbours.
       const int64_t avg_deg = g.n > 0 ? (int64_t(g.nnz) + g.n - 1) / g.n : 0;
       const int64_t wl_items = std::min<int64_t>(g.n, int64_t(M) * (1 + 2 * avg_deg));
-      auto one_round = [&]() -> int {
-        GK_STAGE(ctx, GK_ST_SELECT, 0,
-                 gkd::launch_select_list(g, nullptr, gain.p, dest.p, pw.p, dpw_off.p, dcap.p, dthr.p, cand.p, sb,
-                                         hcnt.p, active.p, st));
-        GK_STAGE(ctx, GK_ST_BALANCE, 0,
-                 gkd::launch_round_b(1, k, dvoff.p, M, dkk.p, dcap.p, dpw_off.p, g, cur_part, dest.p, gain.p, pw.p,
-                                     dcut.p, drounds.p + l, dmoved.p + l, sb, xlist.p, hkey.p, upd.p, wl.p,
-                                     hcnt.p, lastcnt.p, active.p, cand.p, dthr.p, dpaths.p, nullptr,
-                                     dabytes.p + l, st));
-        GK_STAGE(ctx, GK_ST_GAIN, 0,
-                 gkd::launch_gain_wl(g, k, lanes, wl.p, hcnt.p, heavy.p, cur_part, upd.p, cur_bnd, gain.p, dest.p,
-                                     work.p, wl_items, cand.p, st, steal_of(ctx)));
-        if (heavy_rows)
-          GK_STAGE(ctx, GK_ST_GAIN_HEAVY, 0,
-                   gkd::launch_gain_heavy(g, k, heavy.p, hcnt.p, cur_part, upd.p, cur_bnd, gain.p, dest.p, work.p,
-                                          cand.p, st));
-        return GK_OK;
-      };
-      // GK_FLAG_GRAPH_ROUNDS: kRoundsPerCheck rounds are captured once per
-      // level and every check interval (a multiple of it) replays them.
-      RoundGraph rg;
-      if ((prm.flags & GK_FLAG_GRAPH_ROUNDS) && !ctx->clock.timed(GK_ST_SELECT) &&
-          !ctx->clock.timed(GK_ST_BALANCE) && !ctx->clock.timed(GK_ST_GAIN) && !ctx->clock.timed(GK_ST_GAIN_HEAVY))
-        GK_TRY(rg.capture(ctx, st, [&]() -> int {
-          for (int r = 0; r < kRoundsPerCheck; ++r) GK_TRY(one_round());
-          return GK_OK;
-        }));
-      int per_check = kRoundsPerCheck, ran = 0;
-      while (true) {
-        if (rg.ready()) {
-          for (int r = 0; r < per_check; r += kRoundsPerCheck) GK_TRY(rg.replay(ctx, st));
-        } else {
-          for (int r = 0; r < per_check; ++r) GK_TRY(one_round());
-        }
-        ran += per_check;
-        int32_t live = 0;
-        GK_TRY(fetch(ctx, st, {{&live, active.p, sizeof live}}));
-        if (live == 0) break;
-        if (ran >= 32 && per_check < 32) per_check *= 2;
-      }
+      RoundState rs;
+      rs.g = g;
+      rs.kmax = k;
+      rs.M = M;
+      rs.lanes = lanes;
+      rs.heavy_rows = heavy_rows;
+      rs.wl_items = wl_items;
+      rs.v_off = dvoff.p;
+      rs.kk = dkk.p;
+      rs.pw_off = dpw_off.p;
+      rs.cap = dcap.p;
+      rs.part = cur_part;
+      rs.bnd = cur_bnd;
+      rs.gain = gain.p;
+      rs.dest = dest.p;
+      rs.pw = pw.p;
+      rs.upd = upd.p;
+      rs.cut = dcut.p;
+      rs.moved = dmoved.p + l;
+      rs.paths = dpaths.p;
+      rs.abytes = dabytes.p + l;
+      rs.rounds = drounds.p + l;
+      rs.lastcnt = lastcnt.p;
+      rs.thr = dthr.p;
+      rs.active = active.p;
+      rs.cand = cand.p;
+      rs.sb = sb;
+      rs.xlist = xlist.p;
+      rs.wl = wl.p;
+      rs.hcnt = hcnt.p;
+      rs.heavy = heavy.p;
+      rs.status = status.p;
+      rs.hkey = hkey.p;
+      rs.work = work.p;
+      GK_TRY(refine_rounds(ctx, st, rs, 0, false, (prm.flags & GK_FLAG_GRAPH_ROUNDS) != 0, nullptr));
       GK_HIP(hipMemcpyAsync(dcutlv.p + l, dcut.p, sizeof(long long), hipMemcpyDeviceToDevice, st));
       if (trace) {
         std::vector<int32_t> h;
@@ -1223,14 +1330,16 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   const int64_t nwords = (int64_t(n) + 63) / 64;
   // The round state of run_vcycle's refinement, for one job.
   Buf<int32_t> upd, wl, heavy, hcnt, list, xlist, wpos, sscr, dthr, active, drounds, lastcnt, dvoff, dpw_off, dkk,
-      dorder, dmax;
-  Buf<long long> dcap, dcut, dmoved, dpaths;
+      dorder, dmax, status, hist;
+  Buf<long long> dcap, dcut, dmoved, dpaths, dabytes;
   Buf<uint64_t> cand, movable, selbits, defbits;
   Buf<uint32_t> hkey;
   GK_TRY(upd.alloc(P, n));
   GK_TRY(wl.alloc(P, n));
   GK_TRY(heavy.alloc(P, n));
-  GK_TRY(hcnt.alloc(P, 2));
+  GK_TRY(hcnt.alloc(P, 4));
+  GK_TRY(status.alloc(P, 4));
+  GK_TRY(hist.alloc(P, 2 * int64_t(nrounds)));
   GK_TRY(list.alloc(P, n));
   GK_TRY(xlist.alloc(P, n));
   GK_TRY(hkey.alloc(P, n));
@@ -1253,12 +1362,9 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   GK_TRY(dcut.alloc(P, 1));
   GK_TRY(dmoved.alloc(P, 1));
   GK_TRY(dpaths.alloc(P, 3));
+  GK_TRY(dabytes.alloc(P, 1));
   gkd::fill<int32_t>(upd.p, 0, n, st);
-  gkd::fill<int32_t>(hcnt.p, 0, 2, st);
   gkd::fill<uint64_t>(selbits.p, 0ull, nwords + 1, st);
-  gkd::fill<int32_t>(dthr.p, 1, 1, st);
-  gkd::fill<int32_t>(drounds.p, 0, 1, st);
-  gkd::fill<int32_t>(lastcnt.p, 1, 1, st);
   gkd::fill<int32_t>(dvoff.p, 0, 1, st);
   gkd::fill<int32_t>(dvoff.p + 1, n, 1, st);
   gkd::fill<int32_t>(dpw_off.p, 0, 1, st);
@@ -1266,36 +1372,64 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   gkd::fill<int32_t>(dkk.p, k, 1, st);
   gkd::fill<long long>(dcap.p, static_cast<long long>(cap), 1, st);
   gkd::fill<long long>(dcut.p, 0, 1, st);
-  gkd::fill<long long>(dmoved.p, 0, 1, st);
   gkd::fill<long long>(dpaths.p, 0, 3, st);
+  GK_TRY(gkd::launch_rounds_init(1, lastcnt.p, dthr.p, drounds.p, dmoved.p, dabytes.p, hcnt.p, status.p, st));
   GK_TRY(gkd::launch_cand_init(n, bnd, gain, cand.p, st));
-  GK_TRY(gkd::launch_max_deg(g, dmax.p, st));
-  int32_t maxdeg = 0;
-  GK_TRY(fetch(ctx, st, {{&maxdeg, dmax.p, sizeof maxdeg}}));
-  const int lanes = gain_lanes(g);
-  const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, nullptr};
-  for (int32_t r = 0; r < nrounds; ++r) {
-    // B = 0, pos = -1 unless the round orders any move.
-    gkd::fill<int32_t>(dorder.p, 0, 1, st);
-    gkd::fill<int32_t>(dorder.p + 1, -1, 1, st);
-    GK_TRY(gkd::launch_select_list(g, nullptr, gain, dest, pw, dpw_off.p, dcap.p, dthr.p, cand.p, sb, hcnt.p,
-                                   active.p, st));
-    GK_TRY(gkd::launch_round_b(1, k, dvoff.p, M, dkk.p, dcap.p, dpw_off.p, g, part, dest, gain, pw, dcut.p,
-                               drounds.p, dmoved.p, sb, xlist.p, hkey.p, upd.p, wl.p, hcnt.p, lastcnt.p, active.p,
-                               cand.p, dthr.p, dpaths.p, dorder.p, nullptr, st));
-    GK_TRY(gkd::launch_gain_wl(g, k, lanes, wl.p, hcnt.p, heavy.p, part, upd.p, bnd, gain, dest, nullptr, n,
-                                cand.p, st));
-    if (maxdeg > lanes && gkd::gain_heavy_separate(k))
-      GK_TRY(gkd::launch_gain_heavy(g, k, heavy.p, hcnt.p, part, upd.p, bnd, gain, dest, nullptr, cand.p, st));
-    int32_t hdr[2] = {0, -1};
-    GK_TRY(fetch(ctx, st, {{hdr, dorder.p, sizeof hdr}}));
-    if (nmoves) nmoves[r] = hdr[0];
-    if (pos) pos[r] = hdr[1];
-    if (order && hdr[0] > 0)
-      GK_HIP(hipMemcpyAsync(order, dorder.p + 2, sizeof(int32_t) * size_t(hdr[0]), hipMemcpyDeviceToDevice, st));
+  RoundState rs;
+  rs.g = g;
+  rs.kmax = k;
+  rs.M = M;
+  rs.lanes = gain_lanes(g);
+  if (gkd::gain_heavy_separate(k)) {
+    GK_TRY(gkd::launch_max_deg(g, dmax.p, st));
+    int32_t maxdeg = 0;
+    GK_TRY(fetch(ctx, st, {{&maxdeg, dmax.p, sizeof maxdeg}}));
+    rs.heavy_rows = maxdeg > rs.lanes;
   }
+  rs.wl_items = n;
+  rs.v_off = dvoff.p;
+  rs.kk = dkk.p;
+  rs.pw_off = dpw_off.p;
+  rs.cap = dcap.p;
+  rs.part = part;
+  rs.bnd = bnd;
+  rs.gain = gain;
+  rs.dest = dest;
+  rs.pw = pw;
+  rs.upd = upd.p;
+  rs.cut = dcut.p;
+  rs.moved = dmoved.p;
+  rs.paths = dpaths.p;
+  rs.abytes = dabytes.p;
+  rs.rounds = drounds.p;
+  rs.lastcnt = lastcnt.p;
+  rs.thr = dthr.p;
+  rs.active = active.p;
+  rs.cand = cand.p;
+  rs.sb = gkd::SelectBufs{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, nullptr};
+  rs.xlist = xlist.p;
+  rs.wl = wl.p;
+  rs.hcnt = hcnt.p;
+  rs.heavy = heavy.p;
+  rs.status = status.p;
+  rs.hkey = hkey.p;
+  rs.order = dorder.p;
+  rs.hist = hist.p;
+  GK_TRY(refine_rounds(ctx, st, rs, nrounds, true, false, nullptr));
+  // Rounds that ordered no move came after those that did (an unchanged state
+  // stays so): no moves, position -1.
   long long hcut = 0, hp[3] = {0, 0, 0};
-  GK_TRY(fetch(ctx, st, {{&hcut, dcut.p, sizeof hcut}, {hp, dpaths.p, sizeof hp}}));
+  int32_t made = 0;
+  GK_TRY(fetch(ctx, st, {{&hcut, dcut.p, sizeof hcut}, {hp, dpaths.p, sizeof hp}, {&made, drounds.p, sizeof made}}));
+  std::vector<int32_t> hh;
+  GK_TRY(to_host(st, hh, hist.p, 2 * int64_t(made)));
+  for (int32_t r = 0; r < nrounds; ++r) {
+    if (nmoves) nmoves[r] = r < made ? hh[2 * r] : 0;
+    if (pos) pos[r] = r < made ? hh[2 * r + 1] : -1;
+  }
+  if (order && made > 0)
+    GK_HIP(hipMemcpyAsync(order, dorder.p + 2, sizeof(int32_t) * size_t(hh[2 * made - 2]), hipMemcpyDeviceToDevice, st));
+  GK_HIP(hipStreamSynchronize(st));
   *gain_sum = -hcut;
   if (paths)
     for (int i = 0; i < 3; ++i) paths[i] = hp[i];

@@ -571,7 +571,7 @@ int Engine::refine_step(bool* worked) {
   const DGraph g = F.graph();
   const int32_t N = g.n;
   Buf<int32_t> dpw_off, dkk, dpw, upd, wl, heavy, list, hcnt, active, drounds, lastcnt, dmax, xlist, dthr, wpos,
-      sscr;
+      sscr, status;
   Buf<long long> dcap, dcut, dmoved, dpaths;
   Buf<uint64_t> cand, movable, selbits, defbits;
   Buf<uint32_t> hkey;
@@ -603,27 +603,23 @@ int Engine::refine_step(bool* worked) {
   GK_TRY(sscr.alloc(P_, gkd::select_scratch_ints(N)));
   GK_TRY(xlist.alloc(P_, N));
   GK_TRY(dthr.alloc(P_, J));
-  gkd::fill<int32_t>(dthr.p, 1, J, st_);
   gkd::fill<uint64_t>(selbits.p, 0ull, nwords + 1, st_);
   Buf<unsigned long long> selbytes;  // the selection kernels' algorithmic bytes, per block slot
   GK_TRY(selbytes.alloc(P_, gkd::kSelectByteSlots));
   gkd::fill<unsigned long long>(selbytes.p, 0ull, gkd::kSelectByteSlots, st_);
   const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, selbytes.p};
   GK_TRY(hkey.alloc(P_, N));
-  GK_TRY(hcnt.alloc(P_, 2));
+  GK_TRY(hcnt.alloc(P_, 4));
+  GK_TRY(status.alloc(P_, 4));
   GK_TRY(active.alloc(P_, 1));
   GK_TRY(drounds.alloc(P_, J));
   GK_TRY(lastcnt.alloc(P_, J));
-  gkd::fill<int32_t>(lastcnt.p, 1, J, st_);
   GK_TRY(dmax.alloc(P_, 1));
   GK_TRY(dmoved.alloc(P_, J));
-  gkd::fill<int32_t>(drounds.p, 0, J, st_);
-  gkd::fill<long long>(dmoved.p, 0, J, st_);
   GK_TRY(dpaths.alloc(P_, 3LL * J));
   gkd::fill<long long>(dpaths.p, 0, 3LL * J, st_);
   Buf<long long> dab;  // the round kernel's algorithmic bytes per job
   GK_TRY(dab.alloc(P_, J));
-  gkd::fill<long long>(dab.p, 0, J, st_);
   // Gain-pass statistics: a (vertices, entries) pair per block of the gain
   // launches (grids of at most kGainSlots blocks), summed after the rounds
   // into the stage's algorithmic bytes.
@@ -647,7 +643,7 @@ int Engine::refine_step(bool* worked) {
     GK_TRY(fetch(ctx_, st_, {{&maxdeg, dmax.p, sizeof maxdeg}}));
     heavy_rows = maxdeg > lanes;
   }
-  gkd::fill<int32_t>(hcnt.p, 0, 2, st_);
+  GK_TRY(gkd::launch_rounds_init(J, lastcnt.p, dthr.p, drounds.p, dmoved.p, dab.p, hcnt.p, status.p, st_));
   GK_STAGE(ctx_, GK_ST_PROJECT, 4LL * N, gkd::launch_compact(N, upd.p, wl.p, hcnt.p, st_));
   GK_STAGE(ctx_, GK_ST_GAIN, 0,
            gkd::launch_gain_wl(g, kmax, lanes, wl.p, hcnt.p, heavy.p, part->p, upd.p, bnd->p, gain.p, dest.p,
@@ -658,61 +654,53 @@ int Engine::refine_step(bool* worked) {
                                     cand.p, st_));
   const int64_t avg_deg = N > 0 ? (int64_t(g.nnz) + N - 1) / N : 0;
   const int64_t wl_items = std::min<int64_t>(N, int64_t(J) * M * (1 + 2 * avg_deg));
-  // Rounds run back to back on the device; the host reads the last round's
-  // move count every kRoundsPerCheck rounds (every 8, 16, then 32 once the
-  // step has run 32: a check costs a copy and a host sync).  A round in which no job selects
-  // a move changes nothing, so rounds past convergence are harmless.  After
-  // kMaxRounds rounds the step ends; jobs still moving resume their level in
-  // the next step, so one slow job does not hold back the others.  The fixed
-  // cost of a step (pack, projection, candidate set, a host sync) grows with
-  // the pack, so bigger packs run more rounds per step: 16 per 16 Mi
-  // vertices + entries, at most 256.
-  constexpr int kRoundsPerCheck = 4;
+  // A step ends after kMaxRounds rounds (refine_rounds); jobs still moving
+  // resume their level in the next step, so one slow job does not hold back
+  // the others.  The fixed cost of a step (pack, projection, candidate set, a
+  // host sync) grows with the pack, so bigger packs run more rounds per step:
+  // 64 per 16 Mi vertices + entries, at most 256.
   const int64_t pack_items = int64_t(N) + int64_t(g.nnz);
-  const int kMaxRounds = static_cast<int>(std::min<int64_t>(256, 16 * std::max<int64_t>(1, pack_items >> 24)));
-  auto one_round = [&]() -> int {
-    GK_STAGE(ctx_, GK_ST_SELECT, 0,
-             gkd::launch_select_list(g, rs.vjob.p, gain.p, dest.p, dpw.p, dpw_off.p, dcap.p, dthr.p, cand.p, sb,
-                                     hcnt.p, active.p, st_));
-    GK_STAGE(ctx_, GK_ST_BALANCE, 0,
-             gkd::launch_round_b(J, kmax, F.dv_off.p, M, dkk.p, dcap.p, dpw_off.p, g, part->p, dest.p, gain.p,
-                                 dpw.p, dcut.p, drounds.p, dmoved.p, sb, xlist.p, hkey.p, upd.p, wl.p, hcnt.p,
-                                 lastcnt.p, active.p, cand.p, dthr.p, dpaths.p, nullptr, dab.p, st_));
-    GK_STAGE(ctx_, GK_ST_GAIN, 0,
-             gkd::launch_gain_wl(g, kmax, lanes, wl.p, hcnt.p, heavy.p, part->p, upd.p, bnd->p, gain.p, dest.p,
-                                 gwork.p, wl_items, cand.p, st_, steal_of(ctx_)));
-    if (heavy_rows)
-      GK_STAGE(ctx_, GK_ST_GAIN_HEAVY, 0,
-               gkd::launch_gain_heavy(g, kmax, heavy.p, hcnt.p, part->p, upd.p, bnd->p, gain.p, dest.p, gwork.p,
-                                      cand.p, st_));
-    return GK_OK;
-  };
-  // With GK_FLAG_GRAPH_ROUNDS (and no round stage event-timed), the
-  // kRoundsPerCheck rounds are captured once and every check interval
-  // replays that graph (intervals are multiples of it).
-  RoundGraph rg;
-  if (graph_rounds_ && !ctx_->clock.timed(GK_ST_SELECT) && !ctx_->clock.timed(GK_ST_BALANCE) &&
-      !ctx_->clock.timed(GK_ST_GAIN) && !ctx_->clock.timed(GK_ST_GAIN_HEAVY))
-    GK_TRY(rg.capture(ctx_, st_, [&]() -> int {
-      for (int r = 0; r < kRoundsPerCheck; ++r) GK_TRY(one_round());
-      return GK_OK;
-    }));
+  const int kMaxRounds = static_cast<int>(std::min<int64_t>(256, 64 * std::max<int64_t>(1, pack_items >> 24)));
+  RoundState s;
+  s.g = g;
+  s.nj = J;
+  s.kmax = kmax;
+  s.M = M;
+  s.lanes = lanes;
+  s.heavy_rows = heavy_rows;
+  s.wl_items = wl_items;
+  s.vjob = rs.vjob.p;
+  s.v_off = F.dv_off.p;
+  s.kk = dkk.p;
+  s.pw_off = dpw_off.p;
+  s.cap = dcap.p;
+  s.part = part->p;
+  s.bnd = bnd->p;
+  s.gain = gain.p;
+  s.dest = dest.p;
+  s.pw = dpw.p;
+  s.upd = upd.p;
+  s.cut = dcut.p;
+  s.moved = dmoved.p;
+  s.paths = dpaths.p;
+  s.abytes = dab.p;
+  s.rounds = drounds.p;
+  s.lastcnt = lastcnt.p;
+  s.thr = dthr.p;
+  s.active = active.p;
+  s.cand = cand.p;
+  s.sb = sb;
+  s.xlist = xlist.p;
+  s.wl = wl.p;
+  s.hcnt = hcnt.p;
+  s.heavy = heavy.p;
+  s.status = status.p;
+  s.hkey = hkey.p;
+  s.work = gwork.p;
   const double tr0 = now_ms();
-  int done_rounds = 0, per_check = kRoundsPerCheck;
-  while (done_rounds < kMaxRounds) {
-    const int nr = std::min(per_check, kMaxRounds - done_rounds);
-    rounds_ += nr;
-    done_rounds += nr;
-    if (rg.ready() && nr % kRoundsPerCheck == 0) {
-      for (int r = 0; r < nr; r += kRoundsPerCheck) GK_TRY(rg.replay(ctx_, st_));
-    } else {
-      for (int r = 0; r < nr; ++r) GK_TRY(one_round());
-    }
-    int32_t live = 0;
-    GK_TRY(fetch(ctx_, st_, {{&live, active.p, sizeof live}}));
-    if (live == 0) break;
-    if (done_rounds >= 32 && per_check < 32) per_check *= 2;
-  }
+  int ran = 0;
+  GK_TRY(refine_rounds(ctx_, st_, s, kMaxRounds, false, graph_rounds_, &ran));
+  rounds_ += ran;
   prof_ms_[5] += now_ms() - tr0;
   std::vector<long long> hcut(J), hmoved(J), hpaths(3 * size_t(J));
   std::vector<int32_t> hrounds(J), hlast(J);

@@ -9,6 +9,7 @@
 #include "kernels.hpp"
 #include "prim.hpp"
 #include "balance.hpp"
+#include "gain.hpp"
 #include "../../include/gkway.h"
 
 namespace gkd {
@@ -87,22 +88,10 @@ int launch_compact(int32_t n, const int32_t* flags, int32_t* list, int32_t* cnt,
   return hip_status();
 }
 
-// Candidate bitmask of the batched form: bit v set iff v is a boundary vertex
-// with positive gain (the vertices its selection looks at).
-__device__ __forceinline__ void set_cand(uint64_t* cand, int32_t v, bool on) {
-  const uint64_t b = 1ull << (v & 63);
-  if (on) atomicOr(reinterpret_cast<unsigned long long*>(&cand[v >> 6]), (unsigned long long)b);
-  else atomicAnd(reinterpret_cast<unsigned long long*>(&cand[v >> 6]), (unsigned long long)~b);
-}
-
 // update_vertex_info + calculate_gain (gkway/uncoarsen.hpp:175-237, 82-109)
-// over a worklist of updated vertices (wlc[0] entries), S lanes per vertex,
-// grid-stride.  Each lane holds one (part, weight) entry of the row and sums
-// the weights of the lanes with the same part (an O(S) shuffle loop), which
-// gives the connectivity to every adjacent part without a histogram.  Gain is
-// the signed max over the adjacent parts of conn_q - conn_p, floored at 0,
-// lowest q on ties.  Rows longer than S: with k <= kGainInlineK the whole
-// wave takes them one at a time after each pass, with a per-wave LDS
+// over a worklist of updated vertices (wlc[0] entries), S lanes per vertex
+// (gain_pass), grid-stride.  Rows longer than S: with k <= kGainInlineK the
+// whole wave takes them one at a time after each pass, with a per-wave LDS
 // histogram of the k connectivities (as k_gain_heavy); with larger k they are
 // appended to the heavy list (wlc[1] entries) for k_gain_heavy.  Processed
 // vertices get upd[v] = 0.
@@ -137,100 +126,19 @@ __device__ __forceinline__ void gain_wl_body(const int32_t* __restrict__ wl, int
       s = xadj[v];
       d = xadj[v + 1] - s;
     }
-    const bool long_row = e < cnt && d > S;
-    if (long_row && !inline_heavy && sub == 0) heavy[atomicAdd(&wlc[1], 1)] = v;
-    if (e < cnt && d <= S) {
-      const int32_t p = part[v];
-      int32_t q = -1, wj = 0;
-      if (sub < d) {
-        q = part[adj[s + sub]];
-        wj = w[s + sub];
-      }
-      int32_t conn = 0, id = 0;
-#pragma unroll
-      for (int i = 0; i < S; ++i) {
-        const int32_t qi = __shfl(q, i, S);
-        const int32_t wi = __shfl(wj, i, S);
-        conn += (qi == q) ? wi : 0;
-        id += (qi == p) ? wi : 0;
-      }
-      const bool ext = q >= 0 && q != p;
-      int32_t g = ext ? conn - id : INT32_MIN;
-      int32_t bq = ext ? q : INT32_MAX;
-      int32_t anyext = ext ? 1 : 0;
-#pragma unroll
-      for (int o = S / 2; o > 0; o >>= 1) {
-        const int32_t og = __shfl_xor(g, o, S), oq = __shfl_xor(bq, o, S);
-        if (og > g || (og == g && oq < bq)) { g = og; bq = oq; }
-        anyext |= __shfl_xor(anyext, o, S);
-      }
-      if (sub == 0) {
-        bnd[v] = anyext;
-        if (anyext && g > 0) {
-          gain[v] = g;
-          dest[v] = bq;
-        } else {
-          gain[v] = 0;
-          dest[v] = p;
-        }
-        if (cand) set_cand(cand, v, anyext && g > 0);
-        upd[v] = 0;
-        ++done_v;
-        done_e += d;
-      }
-    }
-    if (!inline_heavy) return;
-    // The pass's long rows, one at a time, by the whole wave.
-    int32_t* hist = hh[wv];
-    uint64_t lm = ballot(long_row && sub == 0);
-    while (lm) {
-      const int src = __ffsll(static_cast<long long>(lm)) - 1;
-      lm &= lm - 1;
-      const int32_t hv = __shfl(v, src, 64), hs = __shfl(s, src, 64), he = hs + __shfl(d, src, 64);
-      for (int32_t q = lane; q < k; q += 64) hist[q] = 0;
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      const int32_t p = part[hv];
-      bool ext = false;
-      for (int32_t j = hs + lane; j < he; j += 64) {
-        const int32_t q = part[adj[j]];
-        atomicAdd(&hist[q], w[j]);
-        ext |= (q != p);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      const bool any = ballot(ext) != 0;
-      const int32_t id = hist[p];
-      int32_t g = INT32_MIN, bq = INT32_MAX;
-      for (int32_t q = lane; q < k; q += 64) {
-        const int32_t h = hist[q];
-        if (q != p && h > 0) {
-          const int32_t gq = h - id;
-          if (gq > g || (gq == g && q < bq)) { g = gq; bq = q; }
-        }
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const int32_t og = __shfl_xor(g, o, 64), oq = __shfl_xor(bq, o, 64);
-        if (og > g || (og == g && oq < bq)) { g = og; bq = oq; }
-      }
-      if (lane == 0) {
-        bnd[hv] = any ? 1 : 0;
-        if (any && g > 0) {
-          gain[hv] = g;
-          dest[hv] = bq;
-        } else {
-          gain[hv] = 0;
-          dest[hv] = p;
-        }
-        if (cand) set_cand(cand, hv, any && g > 0);
-        upd[hv] = 0;
-        ++done_v;
-        done_e += he - hs;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
+    const bool has = e < cnt;
+    if (has && d > S && !inline_heavy && sub == 0) heavy[atomicAdd(&wlc[1], 1)] = v;
+    gain_pass<S>(has, v, s, d, adj, w, part, k, inline_heavy ? hh[wv] : nullptr,
+                 [&](int32_t u, int32_t p, bool any, int32_t g, int32_t q, int32_t du) {
+                   const bool up = any && g > 0;
+                   bnd[u] = any ? 1 : 0;
+                   gain[u] = up ? g : 0;
+                   dest[u] = up ? q : p;
+                   if (cand) set_cand(cand, u, up);
+                   upd[u] = 0;
+                   ++done_v;
+                   done_e += du;
+                 });
   };
   if constexpr (Steal) {
     const int64_t sweeps = (int64_t(cnt) + (64 / S) - 1) / (64 / S);

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/gkway.h"
+#include "batch.hpp"
 #include "dev_common.hpp"
 #include "kernels.hpp"
 
@@ -579,6 +580,33 @@ int gain_lanes(const gkd::DGraph& g);
 // use of a degree profile when ctx->autotune is set; the degree table
 // otherwise).
 int match_stage(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, int32_t* cand);
+
+// What the refinement rounds of a level work on: one job (vjob null) or a pack
+// of nj jobs.  hcnt: two pairs of worklist counts (entries, heavy rows), the
+// first of which the separate kernels use; status: two pairs of words of
+// launch_rounds.
+struct RoundState {
+  gkd::DGraph g;
+  int32_t nj = 1, kmax = 1, M = 1;
+  int lanes = 4;            // of the gain pass
+  bool heavy_rows = false;  // some row needs the heavy-row kernel
+  int64_t wl_items = 0;     // worklist entries a round appends, at most
+  const int32_t *vjob = nullptr, *v_off = nullptr, *kk = nullptr, *pw_off = nullptr;
+  const long long* cap = nullptr;
+  int32_t *part = nullptr, *bnd = nullptr, *gain = nullptr, *dest = nullptr, *pw = nullptr, *upd = nullptr;
+  long long *cut = nullptr, *moved = nullptr, *paths = nullptr, *abytes = nullptr;
+  int32_t *rounds = nullptr, *lastcnt = nullptr, *thr = nullptr, *active = nullptr;
+  uint64_t* cand = nullptr;
+  gkd::SelectBufs sb{};
+  int32_t *xlist = nullptr, *wl = nullptr, *hcnt = nullptr, *heavy = nullptr, *status = nullptr;
+  uint32_t* hkey = nullptr;
+  unsigned long long* work = nullptr;
+  int32_t *order = nullptr, *hist = nullptr;
+};
+// Runs rounds until every job has converged, at most about max_rounds per job
+// (0: no bound; with exact, exactly so many at most); *ran gets the rounds
+// launched per job.  graph: replay captured launches (GK_FLAG_GRAPH_ROUNDS).
+int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, bool exact, bool graph, int* ran);
 
 struct Level {
   gkd::DGraph g;
