@@ -27,6 +27,10 @@
 #include <thread>
 #include <vector>
 
+#if defined(__x86_64__)
+#include <immintrin.h>
+#endif
+
 #include "../../include/gkway.h"
 #include "host_graph.hpp"
 
@@ -63,107 +67,187 @@ struct Rng {
   uint32_t below(uint32_t m) { return static_cast<uint32_t>((static_cast<uint64_t>(next() >> 32) * m) >> 32); }
 };
 
+// ------------------------------------------------------------------ memory
+// Per-thread stack of memory for the graphs and work arrays of a bisection:
+// they are made and dropped in last-in first-out order (a task that a waiting
+// thread runs meanwhile begins and ends above what the waiter holds), so
+// nothing is zeroed, returned to the system or faulted in again between
+// levels and trials.
+class Arena {
+ public:
+  static Arena& get() {
+    thread_local Arena a;
+    return a;
+  }
+  template <class T>
+  T* take(size_t count) {
+    const size_t bytes = (count * sizeof(T) + 63) & ~size_t(63);
+    while (cur_ < blocks_.size() && used_ + bytes > blocks_[cur_].size) {
+      ++cur_;
+      used_ = 0;
+    }
+    if (cur_ == blocks_.size()) {
+      const size_t size = std::max(bytes, std::max<size_t>(size_t(1) << 20, 2 * (blocks_.empty() ? 0 : blocks_.back().size)));
+      blocks_.push_back({std::unique_ptr<char[]>(new char[size + 64]), size});
+    }
+    char* base = blocks_[cur_].mem.get();
+    char* p = base + ((64 - (reinterpret_cast<uintptr_t>(base) & 63)) & 63) + used_;
+    used_ += bytes;
+    return reinterpret_cast<T*>(p);
+  }
+  // Gives back the end of the latest take: it keeps `count` elements at p.
+  template <class T>
+  void keep(T* p, size_t count) {
+    char* base = blocks_[cur_].mem.get();
+    base += (64 - (reinterpret_cast<uintptr_t>(base) & 63)) & 63;
+    used_ = static_cast<size_t>(reinterpret_cast<char*>(p) - base) + ((count * sizeof(T) + 63) & ~size_t(63));
+  }
+  // Everything taken while a Scope lives is dropped with it.  A thread keeps
+  // at most kIdle bytes between its outermost scopes.
+  class Scope {
+   public:
+    Scope() : a_(Arena::get()), cur_(a_.cur_), used_(a_.used_) { ++a_.depth_; }
+    ~Scope() {
+      a_.cur_ = cur_;
+      a_.used_ = used_;
+      if (--a_.depth_ == 0) a_.trim();
+    }
+    Scope(const Scope&) = delete;
+    Scope& operator=(const Scope&) = delete;
+
+   private:
+    Arena& a_;
+    size_t cur_, used_;
+  };
+
+ private:
+  static constexpr size_t kIdle = size_t(32) << 20;
+  struct Block {
+    std::unique_ptr<char[]> mem;
+    size_t size;
+  };
+  void trim() {
+    size_t total = 0;
+    for (const Block& b : blocks_) total += b.size;
+    if (total > kIdle) blocks_.clear();
+    cur_ = 0;
+    used_ = 0;
+  }
+  std::vector<Block> blocks_;
+  size_t cur_ = 0, used_ = 0;
+  int depth_ = 0;
+};
+
+struct Edge {
+  int32_t u, w;
+};
+
+// A vertex: its row is the edges [lo, hi), inc their summed weight.
+struct V {
+  int32_t lo, hi, vw, inc;
+};
+
+// A graph in arena memory.
 struct G {
   int32_t n = 0;
-  std::vector<int32_t> xadj, adj, w, vw;
-  int64_t tw = 0;  // total vertex weight
+  V* v = nullptr;
+  Edge* e = nullptr;
+  int64_t tw = 0;    // total vertex weight
+  int64_t rows = 0;  // entries of all rows
 };
 
 // ------------------------------------------------------------------ heap
+// State of a vertex in a two-way refinement: weight to its own side and to
+// the other, place in its side's queue (-1: not queued), side, and whether it
+// has moved in this pass or been listed as a boundary vertex.  One record, so
+// that an update of a neighbour touches one cache line.
+struct FV {
+  int32_t id, ed, pos;
+  uint8_t side, locked, listed, pad;
+};
+
 // Indexed binary max-heap of vertices ordered by (gain desc, vertex asc).
 // Both go into one 64-bit key: the gain in the high 32 bits (a gain is
 // bounded by a vertex's weighted degree, below 2^31) and the complemented
 // vertex id in the low 32, so one integer compare orders two entries.  Keys
 // are distinct, so the order in which vertices leave the heap depends on the
 // keys alone, never on the heap's layout: building it in O(n) by sift-down
-// gives the same sequence as n pushes.
+// gives the same sequence as n pushes.  Places are kept in the vertex records.
 class Heap {
  public:
-  static int64_t pack(int64_t g, int32_t v) {
-    return static_cast<int64_t>(static_cast<uint64_t>(g) << 32) | int64_t(0xFFFFFFFFu - static_cast<uint32_t>(v));
+  static int64_t pack(int32_t g, int32_t v) {
+    return static_cast<int64_t>(static_cast<uint64_t>(static_cast<int64_t>(g)) << 32) |
+           int64_t(0xFFFFFFFFu - static_cast<uint32_t>(v));
   }
   static int32_t vertex(int64_t key) { return static_cast<int32_t>(0xFFFFFFFFu - static_cast<uint32_t>(key)); }
-  // Empties the heap over vertices [0, n); only the positions of vertices
-  // still queued are cleared when the size is unchanged.
-  void reset(int32_t n) {
-    if (static_cast<int32_t>(pos_.size()) != n) {
-      pos_.assign(n, -1);
-    } else {
-      for (int64_t k : h_) pos_[vertex(k)] = -1;
-    }
+  void use(FV* fv) { fv_ = fv; }
+  // Empties the heap, clearing the places of what is still queued.
+  void drop() {
+    for (int64_t k : h_) fv_[vertex(k)].pos = -1;
     h_.clear();
   }
-  // Replaces the contents (heap empty before) by `keys`, heapified in O(n).
-  void build(const std::vector<int64_t>& keys) {
-    h_.assign(keys.begin(), keys.end());
+  std::vector<int64_t>& keys() { return h_; }  // filled by the caller while empty, then heapify()
+  void heapify() {
     const int32_t n = static_cast<int32_t>(h_.size());
     for (int32_t i = n / 2 - 1; i >= 0; --i) sift_down(i);
-    for (int32_t i = 0; i < n; ++i) pos_[vertex(h_[i])] = i;
+    for (int32_t i = 0; i < n; ++i) fv_[vertex(h_[i])].pos = i;
   }
   bool empty() const { return h_.empty(); }
-  bool contains(int32_t v) const { return pos_[v] >= 0; }
   int32_t top() const { return vertex(h_[0]); }
   int64_t top_key() const { return h_[0] >> 32; }  // the gain of the top vertex
-  void push(int32_t v, int64_t g) {
+  void push(int32_t v, int32_t g) {
     const int32_t i = static_cast<int32_t>(h_.size());
-    h_.push_back(pack(g, v));
-    pos_[v] = i;
-    up(i);
+    h_.push_back(0);
+    up(i, pack(g, v));
   }
-  void update(int32_t v, int64_t g) {
-    const int32_t i = pos_[v];
-    const int64_t old = h_[i];
-    h_[i] = pack(g, v);
-    if (h_[i] > old) up(i); else down(i);
+  void update(int32_t v, int32_t g) {
+    const int32_t i = fv_[v].pos;
+    const int64_t k = pack(g, v);
+    if (k > h_[i]) up(i, k); else down(i, k);
   }
   void remove(int32_t v) {
-    const int32_t i = pos_[v];
-    pos_[v] = -1;
-    const int64_t last = h_.back();
+    const int32_t i = fv_[v].pos;
+    fv_[v].pos = -1;
+    const int64_t old = h_[i], last = h_.back();
     h_.pop_back();
     if (i == static_cast<int32_t>(h_.size())) return;
-    h_[i] = last;
-    pos_[vertex(last)] = i;
-    up(i);
-    down(pos_[vertex(last)]);
+    if (last > old) up(i, last); else down(i, last);
   }
 
  private:
-  void up(int32_t i) {
-    const int64_t k = h_[i];
+  void up(int32_t i, int64_t k) {
     while (i > 0) {
       const int32_t p = (i - 1) / 2;
       if (h_[p] >= k) break;
       h_[i] = h_[p];
-      pos_[vertex(h_[i])] = i;
+      fv_[vertex(h_[i])].pos = i;
       i = p;
     }
     h_[i] = k;
-    pos_[vertex(k)] = i;
+    fv_[vertex(k)].pos = i;
   }
-  void down(int32_t i) {
+  void down(int32_t i, int64_t k) {
     const int32_t n = static_cast<int32_t>(h_.size());
-    const int64_t k = h_[i];
     while (true) {
       int32_t c = 2 * i + 1;
       if (c >= n) break;
-      if (c + 1 < n && h_[c + 1] > h_[c]) ++c;
+      if (c + 1 < n) c += h_[c + 1] > h_[c];
       if (h_[c] <= k) break;
       h_[i] = h_[c];
-      pos_[vertex(h_[i])] = i;
+      fv_[vertex(h_[i])].pos = i;
       i = c;
     }
     h_[i] = k;
-    pos_[vertex(k)] = i;
+    fv_[vertex(k)].pos = i;
   }
-  // down() without position updates, for build().
+  // down() without place updates, for heapify().
   void sift_down(int32_t i) {
     const int32_t n = static_cast<int32_t>(h_.size());
     const int64_t k = h_[i];
     while (true) {
       int32_t c = 2 * i + 1;
       if (c >= n) break;
-      if (c + 1 < n && h_[c + 1] > h_[c]) ++c;
+      if (c + 1 < n) c += h_[c + 1] > h_[c];
       if (h_[c] <= k) break;
       h_[i] = h_[c];
       i = c;
@@ -171,20 +255,23 @@ class Heap {
     h_[i] = k;
   }
   std::vector<int64_t> h_;
-  std::vector<int32_t> pos_;
+  FV* fv_ = nullptr;
 };
 
 // ------------------------------------------------------------------ fork-join
 // Process-wide worker threads for the independent pieces of the recursive
 // bisection (the trial bisections of a node and the two halves below it).
-// A thread waiting for its own tasks runs queued tasks meanwhile, so nested
-// fork-join never blocks a worker.  Results never depend on which thread runs
-// a task.
+// A thread waiting for a task that nobody has begun runs it itself; it takes
+// no other task meanwhile, which could hold it up long after its own is done
+// (a 7 ms stall of a node's halves was seen).  Every queued task is so run by
+// its waiter or by a worker.  Threads look for a short while before they
+// sleep: tasks follow each other closely, and a wake-up takes longer than
+// many of them.  Results never depend on which thread runs a task.
 class ForkJoin {
  public:
   struct Task {
     std::function<void()> fn;
-    bool done = false;  // guarded by the pool mutex
+    std::atomic<int> state{0};  // 0 queued, 1 running, 2 done
   };
   static ForkJoin& get() {
     static ForkJoin pool;
@@ -194,44 +281,59 @@ class ForkJoin {
   std::shared_ptr<Task> spawn(std::function<void()> fn) {
     auto t = std::make_shared<Task>();
     t->fn = std::move(fn);
+    bool wake;
     {
       std::lock_guard<std::mutex> lk(m_);
       q_.push_back(t);
+      queued_.store(static_cast<int>(q_.size()));
+      wake = idle_ > 0;
     }
-    cv_.notify_all();
+    if (wake) cv_.notify_one();
     return t;
   }
-  // Runs queued tasks until t is done; sleeps when there is nothing to run.
   void wait(const std::shared_ptr<Task>& t) {
-    while (true) {
-      std::shared_ptr<Task> o;
-      {
-        std::unique_lock<std::mutex> lk(m_);
-        cv_.wait(lk, [&] { return t->done || !q_.empty(); });
-        if (t->done) return;
-        o = q_.back();  // newest first: the waiter's own, most likely
-        q_.pop_back();
-      }
-      run(*o);
+    int queued = 0;
+    if (t->state.compare_exchange_strong(queued, 1)) {
+      run(*t);
+      return;
     }
+    for (int i = 0; i < kSpin; ++i) {
+      if (t->state.load() == 2) return;
+      relax();
+    }
+    std::unique_lock<std::mutex> lk(m_);
+    ++waiters_;
+    done_cv_.wait(lk, [&] { return t->state.load() == 2; });
+    --waiters_;
   }
 
  private:
+  static constexpr int kSpin = 4000;
+  static void relax() {
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+  }
   ForkJoin() {
     const unsigned hw = std::thread::hardware_concurrency();
     const int n = static_cast<int>(hw ? std::min(hw, 16u) : 1u) - 1;
     for (int i = 0; i < n; ++i)
       th_.emplace_back([this] {
         while (true) {
+          for (int s = 0; s < kSpin && queued_.load() == 0; ++s) relax();
           std::shared_ptr<Task> t;
           {
             std::unique_lock<std::mutex> lk(m_);
+            ++idle_;
             cv_.wait(lk, [this] { return stop_ || !q_.empty(); });
+            --idle_;
             if (stop_ && q_.empty()) return;
-            t = q_.front();
+            t = std::move(q_.front());
             q_.pop_front();
+            queued_.store(static_cast<int>(q_.size()));
           }
-          run(*t);
+          int queued = 0;
+          if (t->state.compare_exchange_strong(queued, 1)) run(*t);
         }
       });
   }
@@ -245,16 +347,18 @@ class ForkJoin {
   }
   void run(Task& t) {
     t.fn();
-    {
+    t.state.store(2);
+    if (waiters_.load() > 0) {
       std::lock_guard<std::mutex> lk(m_);
-      t.done = true;
+      done_cv_.notify_all();
     }
-    cv_.notify_all();
   }
   std::vector<std::thread> th_;
   std::deque<std::shared_ptr<Task>> q_;
   std::mutex m_;
-  std::condition_variable cv_;
+  std::condition_variable cv_, done_cv_;
+  std::atomic<int> queued_{0}, waiters_{0};
+  int idle_ = 0;  // guarded by m_
   bool stop_ = false;
 };
 
@@ -273,141 +377,148 @@ void par_chunks(int chunks, const F& fn) {
 }
 
 // ------------------------------------------------------------------ coarsening
-// Heavy-edge matching in a seeded random visiting order.  Ties between equal
-// edge weights go to the lighter neighbour, then the lower id.  cmap gets the
-// coarse id of every vertex; returns the coarse graph.
-G coarsen_hem(const G& g, Rng& rng, int64_t maxvw, std::vector<int32_t>& cmap, bool par) {
-  const int32_t n = g.n;
-  std::vector<int32_t> perm(n);
-  std::iota(perm.begin(), perm.end(), 0);
-  for (int32_t i = n - 1; i > 0; --i) std::swap(perm[i], perm[rng.below(static_cast<uint32_t>(i + 1))]);
-  std::vector<int32_t> match(n, -1);
-  for (int32_t v : perm) {
-    if (match[v] >= 0) continue;
-    int32_t best = -1;
-    int32_t bw = 0, bvw = 0;
-    for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-      int32_t u = g.adj[j];
-      if (match[u] >= 0) continue;
-      if (int64_t(g.vw[v]) + g.vw[u] > maxvw) continue;
-      int32_t w = g.w[j];
-      if (best < 0 || w > bw || (w == bw && (g.vw[u] < bvw || (g.vw[u] == bvw && u < best)))) {
-        best = u; bw = w; bvw = g.vw[u];
-      }
-    }
-    if (best >= 0) { match[v] = best; match[best] = v; }
-    else match[v] = v;
-  }
-  cmap.assign(n, -1);
-  int32_t nc = 0;
-  for (int32_t v = 0; v < n; ++v) {
-    if (cmap[v] >= 0) continue;
-    cmap[v] = nc;
-    if (match[v] != v) cmap[match[v]] = nc;
-    ++nc;
-  }
-  // Coarse rows in coarse-id order: coarse vertex cv is first reached at its
-  // smaller member v (min(v, match[v])); its row lists the neighbours of v,
-  // then of match[v], in order of first appearance, weights summed.
-  G c;
-  c.n = nc;
-  c.vw.assign(nc, 0);
-  c.xadj.assign(nc + 1, 0);
-  c.tw = g.tw;
-  const int chunks = par ? static_cast<int>(std::min<size_t>(8, g.adj.size() / 32768)) : 1;
-  if (chunks > 1) {
-    // Rows are independent: ranges of coarse ids are built on pool threads
-    // into their own buffers and concatenated (the same arrays as below).
-    std::vector<int32_t> firstv(nc);
-    for (int32_t v = 0; v < n; ++v)
-      if (match[v] >= v) firstv[cmap[v]] = v;
-    struct Piece {
-      std::vector<int32_t> adj, w;
-    };
-    std::vector<Piece> pieces(chunks);
-    par_chunks(chunks, [&](int ci) {
-      const int32_t lo = static_cast<int32_t>(int64_t(nc) * ci / chunks);
-      const int32_t hi = static_cast<int32_t>(int64_t(nc) * (ci + 1) / chunks);
-      Piece& pc = pieces[ci];
-      pc.adj.reserve(g.adj.size() / chunks + 1024);
-      pc.w.reserve(g.adj.size() / chunks + 1024);
-      std::vector<int32_t> slot(nc, -1);
-      for (int32_t cv = lo; cv < hi; ++cv) {
-        const int32_t v = firstv[cv], m = match[v];
-        const int32_t start = static_cast<int32_t>(pc.adj.size());
-        const int32_t mem[2] = {v, m};
-        for (int k = 0; k < (m != v ? 2 : 1); ++k) {
-          const int32_t x = mem[k];
-          c.vw[cv] += g.vw[x];
-          for (int32_t j = g.xadj[x]; j < g.xadj[x + 1]; ++j) {
-            const int32_t cu = cmap[g.adj[j]];
-            if (cu == cv) continue;
-            if (slot[cu] >= start) {
-              pc.w[slot[cu]] += g.w[j];
-            } else {
-              slot[cu] = static_cast<int32_t>(pc.adj.size());
-              pc.adj.push_back(cu);
-              pc.w.push_back(g.w[j]);
-            }
-          }
-        }
-        c.xadj[cv + 1] = static_cast<int32_t>(pc.adj.size()) - start;  // row length for now
-      }
-    });
-    for (int32_t cv = 0; cv < nc; ++cv) c.xadj[cv + 1] += c.xadj[cv];
-    c.adj.resize(c.xadj[nc]);
-    c.w.resize(c.xadj[nc]);
-    int64_t off = 0;
-    for (int ci = 0; ci < chunks; ++ci) {
-      std::copy(pieces[ci].adj.begin(), pieces[ci].adj.end(), c.adj.begin() + off);
-      std::copy(pieces[ci].w.begin(), pieces[ci].w.end(), c.w.begin() + off);
-      off += static_cast<int64_t>(pieces[ci].adj.size());
-    }
-    return c;
-  }
-  // Rows are built in per-thread buffers that only ever grow (this path
-  // never waits on the pool, so no other coarsening runs on the thread
-  // meanwhile), then copied out at their exact size.
-  thread_local std::vector<int32_t> tadj, tw, slot;
-  if (tadj.size() < g.adj.size()) {
-    tadj.resize(g.adj.size());
-    tw.resize(g.adj.size());
-  }
-  slot.assign(nc, -1);
-  const int32_t* xa = g.xadj.data();
-  const int32_t* ad = g.adj.data();
-  const int32_t* wt = g.w.data();
-  const int32_t* cm = cmap.data();
-  int32_t* ca = tadj.data();
-  int32_t* cw = tw.data();
-  int32_t* sl = slot.data();
-  int32_t top = 0;
-  for (int32_t v = 0; v < n; ++v) {
+// The rows of coarse vertices [lo, hi): coarse vertex cv is first reached at
+// its smaller member v (v <= match[v]); its row lists the neighbours of v,
+// then of match[v], in order of first appearance, weights summed.  out holds
+// the rows from index `top` on, and one entry more at index trash, where edges
+// between the two members go; slot: c.n ints, all -1.  Returns the end.
+int32_t coarse_rows(const G& g, const int32_t* match, const int32_t* cmap, int32_t v0, int32_t v1, G& c, int32_t top,
+                    int32_t trash, int32_t* slot) {
+  Edge* out = c.e;
+  for (int32_t v = v0; v < v1; ++v) {
     const int32_t m = match[v];
-    if (m < v) continue;  // second member: handled with the first
-    const int32_t cv = cm[v];
+    // the partners' rows lie anywhere: fetched some vertices ahead
+    if (v + 8 < v1) __builtin_prefetch(&g.v[match[v + 8]]);
+    if (v + 4 < v1) __builtin_prefetch(&g.e[g.v[match[v + 4]].lo]);
+    if (m < v) continue;  // second member: taken with the first
+    const int32_t cv = cmap[v];
     const int32_t start = top;
-    const int32_t mem[2] = {v, m};
-    for (int k = 0; k < (m != v ? 2 : 1); ++k) {
-      const int32_t x = mem[k];
-      c.vw[cv] += g.vw[x];
-      for (int32_t j = xa[x]; j < xa[x + 1]; ++j) {
-        const int32_t cu = cm[ad[j]];
-        if (cu == cv) continue;
-        if (sl[cu] >= start) {
-          cw[sl[cu]] += wt[j];
-        } else {
-          sl[cu] = top;
-          ca[top] = cu;
-          cw[top] = wt[j];
-          ++top;
+    out[trash].w = 0;
+    slot[cv] = trash;
+    int32_t x = v;
+    while (true) {
+      for (int32_t j = g.v[x].lo; j < g.v[x].hi; ++j) {
+        const int32_t cu = cmap[g.e[j].u];
+        const int32_t s = slot[cu];
+        const bool seen = s >= start;
+        const int32_t at = seen ? s : top;
+        slot[cu] = at;
+        out[at].u = cu;
+        out[at].w = (seen ? out[at].w : 0) + g.e[j].w;
+        top += !seen;
+      }
+      if (x == m) break;
+      x = m;
+    }
+    slot[cv] = -1;
+    c.v[cv] = V{start, top, g.v[v].vw + (m != v ? g.v[m].vw : 0), g.v[v].inc + (m != v ? g.v[m].inc : 0) - out[trash].w};
+  }
+  return top;
+}
+
+// Heavy-edge matching in a seeded random visiting order.  Ties between equal
+// edge weights go to the lighter neighbour, then the lower id.  cmap (n, in
+// the arena) gets the coarse id of every vertex; returns the coarse graph.
+G coarsen_hem(const G& g, Rng& rng, int64_t maxvw, int32_t* cmap, bool par) {
+  const int32_t n = g.n;
+  Arena& A = Arena::get();
+  // The coarse graph comes first in the arena, its arrays sized for n, so that
+  // the work arrays behind it can be dropped.
+  G c;
+  c.v = A.take<V>(n);
+  c.tw = g.tw;
+  c.e = A.take<Edge>(static_cast<size_t>(g.rows) + 1);
+  int64_t end = 0;  // entries of c.e in use
+  {
+    Arena::Scope work;
+    int32_t* perm = A.take<int32_t>(n);
+    int32_t* match = A.take<int32_t>(n);
+    // what the matching asks of a neighbour: matched already, and its weight
+    struct Free {
+      int32_t matched, vw;
+    };
+    Free* fr = A.take<Free>(n);
+    std::iota(perm, perm + n, 0);
+    for (int32_t i = n - 1; i > 0; --i) std::swap(perm[i], perm[rng.below(static_cast<uint32_t>(i + 1))]);
+    for (int32_t v = 0; v < n; ++v) fr[v] = Free{0, g.v[v].vw};
+    for (int32_t i = 0; i < n; ++i) {
+      const int32_t v = perm[i];
+      // the visits jump: vertices and rows are fetched some visits ahead
+      if (i + 16 < n) __builtin_prefetch(&g.v[perm[i + 16]]);
+      if (i + 8 < n) __builtin_prefetch(&g.e[g.v[perm[i + 8]].lo]);
+      if (fr[v].matched) continue;
+      int32_t best = v;  // alone, if nothing fits
+      int32_t bw = INT32_MIN, bvw = 0;
+      const V me = g.v[v];
+      const int64_t room = maxvw - me.vw;
+      for (int32_t j = me.lo; j < me.hi; ++j) {
+        const int32_t u = g.e[j].u, w = g.e[j].w;
+        if (w < bw) continue;
+        const Free f = fr[u];
+        if (f.matched || f.vw > room) continue;
+        if (w > bw || f.vw < bvw || (f.vw == bvw && u < best)) {
+          best = u;
+          bw = w;
+          bvw = f.vw;
         }
       }
+      fr[v].matched = 1;
+      fr[best].matched = 1;
+      match[v] = best;
+      match[best] = v;
     }
-    c.xadj[cv + 1] = top;
+    int32_t nc = 0;
+    for (int32_t v = 0; v < n; ++v)
+      if (match[v] >= v) cmap[v] = nc++; else cmap[v] = cmap[match[v]];
+    c.n = nc;
+    const int chunks = par ? static_cast<int>(std::min<int64_t>(8, g.rows / 32768)) : 1;
+    if (chunks > 1) {
+      // Rows are independent: vertex ranges are taken by pool threads, each
+      // into the entries that its rows could fill at most (a range's rows read
+      // the rows of its own vertices and of their partners behind them).
+      std::vector<int32_t> first(chunks + 1), at(chunks + 1, 0), tops(chunks);
+      for (int i = 0; i <= chunks; ++i) first[i] = static_cast<int32_t>(int64_t(n) * i / chunks);
+      for (int i = 0; i < chunks; ++i) {
+        int32_t ub = 0;
+        for (int32_t v = first[i]; v < first[i + 1]; ++v) {
+          const int32_t m = match[v];
+          if (m < v) continue;
+          ub += g.v[v].hi - g.v[v].lo + (m != v ? g.v[m].hi - g.v[m].lo : 0);
+        }
+        at[i + 1] = at[i] + ub;
+      }
+      // every range's trash entry in an array of its own behind the rows: the
+      // ranges' rows and trash must be indexes of one array
+      Edge* wide = A.take<Edge>(static_cast<size_t>(g.rows) + chunks);
+      G cw = c;
+      cw.e = wide;
+      par_chunks(chunks, [&](int i) {
+        Arena::Scope own;
+        int32_t* slot = Arena::get().take<int32_t>(nc);
+        std::fill(slot, slot + nc, -1);
+        tops[i] = coarse_rows(g, match, cmap, first[i], first[i + 1], cw, at[i], static_cast<int32_t>(g.rows) + i, slot);
+      });
+      // together, without the gaps
+      par_chunks(chunks, [&](int i) {
+        int64_t to = 0;
+        for (int q = 0; q < i; ++q) to += tops[q] - at[q];
+        std::copy(wide + at[i], wide + tops[i], c.e + to);
+        const int32_t shift = static_cast<int32_t>(to) - at[i];
+        for (int32_t v = first[i]; v < first[i + 1]; ++v)
+          if (match[v] >= v) {
+            c.v[cmap[v]].lo += shift;
+            c.v[cmap[v]].hi += shift;
+          }
+      });
+      for (int q = 0; q < chunks; ++q) end += tops[q] - at[q];
+    } else {
+      int32_t* slot = A.take<int32_t>(nc);
+      std::fill(slot, slot + nc, -1);
+      end = coarse_rows(g, match, cmap, 0, n, c, 0, static_cast<int32_t>(g.rows), slot);
+    }
   }
-  c.adj.assign(ca, ca + top);
-  c.w.assign(cw, cw + top);
+  A.keep(c.e, static_cast<size_t>(end));
+  c.rows = end;
   return c;
 }
 
@@ -420,66 +531,39 @@ inline int64_t overload(const int64_t pw[2], const Bal& b) {
   return std::max<int64_t>(0, pw[0] - b.max[0]) + std::max<int64_t>(0, pw[1] - b.max[1]);
 }
 
-// Boundary FM refinement.  Moves that keep both sides within their maxima
-// (or reduce the overload) are taken in max-gain order; the best prefix of a
-// pass (lowest (overload, cut)) is kept.
 // Buffers of fm2, one set per thread (fm2 never waits on the pool, so no
 // other fm2 call can run on its thread while it holds them).
 struct FmWork {
-  std::vector<int64_t> id, ed, keys[2];
-  std::vector<uint8_t> locked;
-  std::vector<int32_t> moved;
+  std::vector<int32_t> moved, list;
   Heap q[2];
 };
 
-// conn0 / inc (optional): every vertex's edge weight to side 0 and in all,
-// as a growing run leaves them; the degrees then come in O(n).
-void fm2(const G& g, std::vector<uint8_t>& side, const Bal& bal, int passes, int64_t& cut,
-         const int64_t* conn0 = nullptr, const int64_t* inc = nullptr) {
+// Boundary FM refinement.  Moves that keep both sides within their maxima
+// (or reduce the overload) are taken in max-gain order; the best prefix of a
+// pass (lowest (overload, cut)) is kept.  fv holds every vertex's side and
+// degrees (exact on entry, kept exact through the moves of a pass and their
+// rollback), pos -1, locked and listed 0; pw the sides' weights.
+void fm2(const G& g, FV* fv, int64_t pw[2], const Bal& bal, int passes, int64_t& cut) {
   const int32_t n = g.n;
   thread_local FmWork W;
-  std::vector<int64_t>& id = W.id;
-  std::vector<int64_t>& ed = W.ed;
-  id.assign(n, 0);
-  ed.assign(n, 0);
-  int64_t pw[2] = {0, 0};
-  for (int32_t v = 0; v < n; ++v) pw[side[v]] += g.vw[v];
   Heap* q = W.q;
-  std::vector<uint8_t>& locked = W.locked;
+  q[0].use(fv);
+  q[1].use(fv);
   std::vector<int32_t>& moved = W.moved;
-  locked.resize(n);
+  // Vertices that are or were on the boundary: what a pass starts from.
+  std::vector<int32_t>& list = W.list;
+  list.clear();
+  for (int32_t v = 0; v < n; ++v)
+    if (fv[v].ed > 0) {
+      fv[v].listed = 1;
+      list.push_back(v);
+    }
   const int32_t limit = std::max<int32_t>(25, std::min<int32_t>(n / 20, 300));
-  // Internal / external degrees: computed once, then kept exact through the
-  // moves of a pass and their rollback.
-  if (conn0) {
-    for (int32_t v = 0; v < n; ++v) {
-      const int64_t a = side[v] == 0 ? conn0[v] : inc[v] - conn0[v];
-      id[v] = a;
-      ed[v] = inc[v] - a;
-    }
-  } else {
-    for (int32_t v = 0; v < n; ++v) {
-      const uint8_t sv = side[v];
-      int64_t a = 0, t = 0;
-      for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-        const int32_t wj = g.w[j];
-        t += wj;
-        a += side[g.adj[j]] == sv ? wj : 0;
-      }
-      id[v] = a;
-      ed[v] = t - a;
-    }
-  }
   for (int pass = 0; pass < passes; ++pass) {
-    q[0].reset(n);
-    q[1].reset(n);
-    std::fill(locked.begin(), locked.end(), 0);
-    W.keys[0].clear();
-    W.keys[1].clear();
-    for (int32_t v = 0; v < n; ++v)
-      if (ed[v] > 0) W.keys[side[v]].push_back(Heap::pack(ed[v] - id[v], v));
-    q[0].build(W.keys[0]);
-    q[1].build(W.keys[1]);
+    for (int32_t v : list)
+      if (fv[v].ed > 0) q[fv[v].side].keys().push_back(Heap::pack(fv[v].ed - fv[v].id, v));
+    q[0].heapify();
+    q[1].heapify();
     moved.clear();
     int64_t cur_cut = cut, best_cut = cut;
     int64_t best_ol = overload(pw, bal);
@@ -497,7 +581,7 @@ void fm2(const G& g, std::vector<uint8_t>& side, const Bal& bal, int passes, int
         for (int s = 0; s < 2; ++s) {
           if (q[s].empty()) continue;
           int32_t v = q[s].top();
-          if (cur_pw[1 - s] + g.vw[v] > bal.max[1 - s]) continue;
+          if (cur_pw[1 - s] + g.v[v].vw > bal.max[1 - s]) continue;
           if (q[s].top_key() > bg) { bg = q[s].top_key(); from = s; }
         }
       }
@@ -505,27 +589,33 @@ void fm2(const G& g, std::vector<uint8_t>& side, const Bal& bal, int passes, int
       int32_t v = q[from].top();
       q[from].remove(v);
       const int to = 1 - from;
-      if (!(ol0 || ol1) && cur_pw[to] + g.vw[v] > bal.max[to]) continue;
-      cur_cut -= ed[v] - id[v];
-      cur_pw[from] -= g.vw[v];
-      cur_pw[to] += g.vw[v];
-      side[v] = static_cast<uint8_t>(to);
-      locked[v] = 1;
-      std::swap(id[v], ed[v]);
+      if (!(ol0 || ol1) && cur_pw[to] + g.v[v].vw > bal.max[to]) continue;
+      FV& f = fv[v];
+      cur_cut -= f.ed - f.id;
+      cur_pw[from] -= g.v[v].vw;
+      cur_pw[to] += g.v[v].vw;
+      f.side = static_cast<uint8_t>(to);
+      f.locked = 1;
+      std::swap(f.id, f.ed);
       moved.push_back(v);
-      for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-        int32_t u = g.adj[j];
-        int32_t w = g.w[j];
-        if (side[u] == to) { id[u] += w; ed[u] -= w; }
-        else { id[u] -= w; ed[u] += w; }
-        if (locked[u]) continue;
-        int s = side[u];
-        if (q[s].contains(u)) {
-          if (ed[u] > 0) q[s].update(u, ed[u] - id[u]); else q[s].remove(u);
-        } else if (ed[u] > 0) {
-          q[s].push(u, ed[u] - id[u]);
+      for (int32_t j = g.v[v].lo; j < g.v[v].hi; ++j) {
+        const int32_t u = g.e[j].u;
+        FV& x = fv[u];
+        const int32_t w = x.side == to ? g.e[j].w : -g.e[j].w;
+        x.id += w;
+        x.ed -= w;
+        if (x.locked) continue;
+        if (x.pos >= 0) {
+          if (x.ed > 0) q[x.side].update(u, x.ed - x.id); else q[x.side].remove(u);
+        } else if (x.ed > 0) {
+          q[x.side].push(u, x.ed - x.id);
+          if (!x.listed) {
+            x.listed = 1;
+            list.push_back(u);
+          }
         }
       }
+      // a mover that was interior cannot be: it came from a queue, so listed
       int64_t ol = overload(cur_pw, bal);
       if (ol < best_ol || (ol == best_ol && cur_cut < best_cut)) {
         best_ol = ol;
@@ -540,18 +630,22 @@ void fm2(const G& g, std::vector<uint8_t>& side, const Bal& bal, int passes, int
     // degree updates.
     for (int32_t i = static_cast<int32_t>(moved.size()) - 1; i >= best_len; --i) {
       const int32_t v = moved[i];
-      const int to = side[v], from = 1 - to;
-      for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-        const int32_t u = g.adj[j];
-        const int32_t w = g.w[j];
-        if (side[u] == to) { id[u] -= w; ed[u] += w; }
-        else { id[u] += w; ed[u] -= w; }
+      FV& f = fv[v];
+      const int to = f.side, from = 1 - to;
+      for (int32_t j = g.v[v].lo; j < g.v[v].hi; ++j) {
+        FV& x = fv[g.e[j].u];
+        const int32_t w = x.side == to ? g.e[j].w : -g.e[j].w;
+        x.id -= w;
+        x.ed += w;
       }
-      std::swap(id[v], ed[v]);
-      side[v] = static_cast<uint8_t>(from);
-      cur_pw[to] -= g.vw[v];
-      cur_pw[from] += g.vw[v];
+      std::swap(f.id, f.ed);
+      f.side = static_cast<uint8_t>(from);
+      cur_pw[to] -= g.v[v].vw;
+      cur_pw[from] += g.v[v].vw;
     }
+    for (int32_t v : moved) fv[v].locked = 0;
+    q[0].drop();
+    q[1].drop();
     pw[0] = cur_pw[0];
     pw[1] = cur_pw[1];
     bool improved = best_cut < cut || best_len > 0;
@@ -560,79 +654,115 @@ void fm2(const G& g, std::vector<uint8_t>& side, const Bal& bal, int passes, int
   }
 }
 
-// Buffers of the growing trials of one bisection: the incident edge weight
-// of every vertex (computed once), side-0 connectivity, room for one row's
-// side-1 neighbours and the queue.
-struct GrowWork {
-  std::vector<int64_t> inc, conn0;
-  std::vector<int32_t> front;  // side-1 neighbours of the vertex being added
-  Heap q;
-  explicit GrowWork(const G& g) : inc(g.n, 0) {
-    int32_t maxdeg = 1;
-    for (int32_t u = 0; u < g.n; ++u) {
-      for (int32_t k = g.xadj[u]; k < g.xadj[u + 1]; ++k) inc[u] += g.w[k];
-      maxdeg = std::max(maxdeg, g.xadj[u + 1] - g.xadj[u]);
-    }
-    front.resize(maxdeg);
-  }
-};
+// First index of the largest of a[0, n), n a multiple of 8.
+int32_t first_max(const int32_t* a, int32_t n) {
+  int32_t at = 0;
+  for (int32_t i = 1; i < n; ++i)
+    if (a[i] > a[at]) at = i;
+  return at;
+}
 
-// Greedy graph growing from `seedv`: side 0 grows by max gain until it
-// reaches its target weight.  Returns the cut of the result (each added
-// vertex turns its edges to side 0 internal and the rest cut).  gw.conn0
-// ends as every vertex's edge weight to side 0.
-int64_t grow(const G& g, GrowWork& gw, int32_t seedv, int64_t target0, std::vector<uint8_t>& side) {
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) int32_t first_max_avx2(const int32_t* a, int32_t n) {
+  __m256i m = _mm256_loadu_si256(reinterpret_cast<const __m256i*>(a));
+  for (int32_t i = 8; i < n; i += 8) m = _mm256_max_epi32(m, _mm256_loadu_si256(reinterpret_cast<const __m256i*>(a + i)));
+  __m128i h = _mm_max_epi32(_mm256_castsi256_si128(m), _mm256_extracti128_si256(m, 1));
+  h = _mm_max_epi32(h, _mm_shuffle_epi32(h, 0x4E));
+  h = _mm_max_epi32(h, _mm_shuffle_epi32(h, 0xB1));
+  const __m256i x = _mm256_broadcastd_epi32(h);
+  for (int32_t i = 0;; i += 8) {
+    const int b = _mm256_movemask_ps(
+        _mm256_castsi256_ps(_mm256_cmpeq_epi32(x, _mm256_loadu_si256(reinterpret_cast<const __m256i*>(a + i)))));
+    if (b) return i + __builtin_ctz(static_cast<unsigned>(b));
+  }
+}
+const auto kFirstMax = __builtin_cpu_supports("avx2") ? first_max_avx2 : first_max;
+#else
+const auto kFirstMax = first_max;
+#endif
+
+// Growing takes the best vertex by a scan of all gains instead of from a heap
+// on graphs of up to kFlatMax vertices with kFlatDegree entries a row or more:
+// the coarsest graphs have about 60 to 120 vertices, and one vector scan costs
+// less than a heap's pop and the key changes of a row (64 coarsest graphs of a
+// batch: growing 25% -> 15% of the time).  On road networks, with two entries
+// a row, the heap holds a handful of vertices and stays cheaper.
+constexpr int32_t kFlatMax = 256;
+constexpr int32_t kFlatDegree = 4;
+
+// Greedy graph growing from `seedv`: side 0 grows by max gain (then lowest
+// id) until it reaches its target weight.  Leaves side and degrees of every
+// vertex in fv and the sides' weights in pw; returns the cut of the result
+// (each added vertex turns its edges to side 0 internal and the rest cut).
+int64_t grow(const G& g, FV* fv, int32_t seedv, int64_t target0, int64_t pw[2]) {
   const int32_t n = g.n;
-  Heap& q = gw.q;
-  side.assign(n, 1);
-  std::vector<int64_t>& conn0 = gw.conn0;
-  conn0.assign(n, 0);
-  const std::vector<int64_t>& inc = gw.inc;
-  int32_t* front = gw.front.data();
-  q.reset(n);
+  const bool flat = n <= kFlatMax && g.rows >= int64_t(kFlatDegree) * n;
+  thread_local Heap q;  // growing never waits on the pool
+  q.use(fv);
+  // While growing, id is the vertex's weight to side 0; gains[v] (flat) the
+  // gain of a side-1 vertex next to side 0, kNone for the others.
+  constexpr int32_t kNone = INT32_MIN;
+  int32_t gains[kFlatMax];
+  const int32_t n8 = (n + 7) & ~7;
+  if (flat) std::fill(gains, gains + n8, kNone);
+  for (int32_t v = 0; v < n; ++v) fv[v] = FV{0, 0, -1, 1, 0, 0, 0};
   int64_t w0 = 0, cut = 0;
   int32_t next_unreached = 0;
   auto add = [&](int32_t v) {
-    side[v] = 0;
-    w0 += g.vw[v];
-    cut += inc[v] - 2 * conn0[v];
-    // connectivity of every neighbour; the side-1 ones are listed without a
-    // branch and their queue keys raised after
-    int32_t nf = 0;
-    for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-      const int32_t u = g.adj[j];
-      conn0[u] += g.w[j];
-      front[nf] = u;
-      nf += side[u] != 0;
-    }
-    for (int32_t i = 0; i < nf; ++i) {
-      const int32_t u = front[i];
-      // gain of moving u to side 0: 2*conn0 - total incident weight
-      const int64_t gain = 2 * conn0[u] - inc[u];
-      if (q.contains(u)) q.update(u, gain); else q.push(u, gain);
+    fv[v].side = 0;
+    const V me = g.v[v];
+    w0 += me.vw;
+    cut += me.inc - 2 * int64_t(fv[v].id);
+    for (int32_t j = me.lo; j < me.hi; ++j) {
+      const int32_t u = g.e[j].u;
+      FV& x = fv[u];
+      x.id += g.e[j].w;
+      // gain of moving u to side 0: 2 * its weight to side 0 - its weight
+      const int32_t gain = static_cast<int32_t>(2 * int64_t(x.id) - g.v[u].inc);
+      if (flat) gains[u] = x.side != 0 ? gain : kNone;
+      else if (x.side == 0) continue;
+      else if (x.pos >= 0) q.update(u, gain);
+      else q.push(u, gain);
     }
   };
   add(seedv);
   while (w0 < target0) {
     int32_t v = -1;
-    if (!q.empty()) { v = q.top(); q.remove(v); }
-    else {
-      while (next_unreached < n && side[next_unreached] == 0) ++next_unreached;
+    if (flat) {
+      v = kFirstMax(gains, n8);
+      if (gains[v] == kNone) v = -1;
+      else gains[v] = kNone;
+    } else if (!q.empty()) {
+      v = q.top();
+      q.remove(v);
+    }
+    if (v < 0) {
+      while (next_unreached < n && fv[next_unreached].side == 0) ++next_unreached;
       if (next_unreached >= n) break;
       v = next_unreached;
     }
-    if (side[v] == 0) continue;
     // Stop before overshooting by more than half the vertex weight.
-    if (w0 + g.vw[v] > target0 && (w0 + g.vw[v] - target0) > (target0 - w0)) break;
+    if (w0 + g.v[v].vw > target0 && (w0 + g.v[v].vw - target0) > (target0 - w0)) break;
     add(v);
   }
+  if (!flat) q.drop();
+  for (int32_t v = 0; v < n; ++v) {
+    FV& f = fv[v];
+    const int32_t own = f.side == 0 ? f.id : g.v[v].inc - f.id;
+    f.id = own;
+    f.ed = g.v[v].inc - own;
+  }
+  pw[0] = w0;
+  pw[1] = g.tw - w0;
   return cut;
 }
 
-
-// Multilevel bisection of g.  target0 = desired weight of side 0.  Returns
-// the cut of the result (tracked exactly through growth, FM and projection).
-int64_t ml_bisect(const G& g, int64_t target0, double tol, uint64_t seed, std::vector<uint8_t>& side, bool par) {
+// Multilevel bisection of g.  target0 = desired weight of side 0.  side[v]
+// (n) receives the result; returns its cut (tracked exactly through growth,
+// FM and projection), and its side-0 weight in *w0.
+int64_t ml_bisect(const G& g, int64_t target0, double tol, uint64_t seed, uint8_t* side, int64_t* w0, bool par) {
+  Arena::Scope all;
+  Arena& A = Arena::get();
   Rng rng(seed);
   const int64_t t1 = g.tw - target0;
   Bal bal;
@@ -640,76 +770,114 @@ int64_t ml_bisect(const G& g, int64_t target0, double tol, uint64_t seed, std::v
   bal.max[1] = static_cast<int64_t>(std::floor(double(t1) * (1.0 + tol)));
   // Coarsen.
   std::vector<G> levels;
-  std::vector<std::vector<int32_t>> cmaps;
+  std::vector<int32_t*> cmaps;
+  levels.reserve(64);
   const G* cur = &g;
   const int64_t maxvw = std::max<int64_t>(1, static_cast<int64_t>(1.5 * double(g.tw) / 60.0));
   while (cur->n > 120) {
-    std::vector<int32_t> cm;
+    int32_t* cm = A.take<int32_t>(cur->n);
     G c = coarsen_hem(*cur, rng, maxvw, cm, par);
     if (c.n > 0.92 * cur->n) break;
-    cmaps.push_back(std::move(cm));
-    levels.push_back(std::move(c));
+    cmaps.push_back(cm);
+    levels.push_back(c);
     cur = &levels.back();
   }
   // Initial bisection: best of several grown regions.
   const G& cg = *cur;
-  std::vector<uint8_t> best, trial;
+  FV* best = A.take<FV>(cg.n);
+  FV* trial = A.take<FV>(cg.n);
   int64_t best_cut = INT64_MAX, best_ol = INT64_MAX;
+  int64_t pw[2] = {0, 0};
   const int trials = cg.n <= 1 ? 1 : GKIP_TRIALS;
-  GrowWork gw(cg);
   for (int t = 0; t < trials; ++t) {
     int32_t s = static_cast<int32_t>(rng.below(static_cast<uint32_t>(std::max(1, cg.n))));
-    int64_t c = grow(cg, gw, s, target0, trial);
-    fm2(cg, trial, bal, 4, c, gw.conn0.data(), gw.inc.data());
-    int64_t pw[2] = {0, 0};
-    for (int32_t v = 0; v < cg.n; ++v) pw[trial[v]] += cg.vw[v];
-    int64_t ol = overload(pw, bal);
-    if (ol < best_ol || (ol == best_ol && c < best_cut)) { best_ol = ol; best_cut = c; best = trial; }
+    int64_t tpw[2];
+    int64_t c = grow(cg, trial, s, target0, tpw);
+    fm2(cg, trial, tpw, bal, 4, c);
+    int64_t ol = overload(tpw, bal);
+    if (ol < best_ol || (ol == best_ol && c < best_cut)) {
+      best_ol = ol;
+      best_cut = c;
+      std::swap(best, trial);
+      pw[0] = tpw[0];
+      pw[1] = tpw[1];
+    }
   }
-  // Uncoarsen with refinement.
-  side = std::move(best);
+  // Uncoarsen with refinement.  A vertex whose coarse vertex has no cut edge
+  // has none either: only the rows of the others are read for their degrees.
+  FV* coarse = best;
   for (int32_t l = static_cast<int32_t>(levels.size()) - 1; l >= 0; --l) {
     const G& fine = (l == 0) ? g : levels[l - 1];
-    const std::vector<int32_t>& cm = cmaps[l];
-    std::vector<uint8_t> fs(fine.n);
-    for (int32_t v = 0; v < fine.n; ++v) fs[v] = side[cm[v]];
-    side = std::move(fs);
-    int64_t c = best_cut;  // projection preserves the cut
-    fm2(fine, side, bal, GKIP_FMPASS, c);
-    best_cut = c;
+    const int32_t* cm = cmaps[l];
+    FV* fv = A.take<FV>(fine.n);
+    uint8_t* sd = A.take<uint8_t>(fine.n);
+    for (int32_t v = 0; v < fine.n; ++v) {
+      const FV& c = coarse[cm[v]];
+      sd[v] = c.side;
+      fv[v] = FV{fine.v[v].inc, c.ed, -1, c.side, 0, 0, 0};
+    }
+    for (int32_t v = 0; v < fine.n; ++v) {
+      if (fv[v].ed == 0) continue;
+      const uint8_t sv = sd[v];
+      int32_t a = 0;
+      for (int32_t j = fine.v[v].lo; j < fine.v[v].hi; ++j) a += sd[fine.e[j].u] == sv ? fine.e[j].w : 0;
+      fv[v].ed = fv[v].id - a;
+      fv[v].id = a;
+    }
+    fm2(fine, fv, pw, bal, GKIP_FMPASS, best_cut);  // projection preserves the cut
+    coarse = fv;
   }
+  for (int32_t v = 0; v < g.n; ++v) side[v] = coarse[v].side;
+  *w0 = pw[0];
   return best_cut;
 }
 
-// Induced subgraph of the vertices with side[v] == s.
-G induced(const G& g, const std::vector<uint8_t>& side, uint8_t s, std::vector<int32_t>& map_back) {
-  std::vector<int32_t> loc(g.n, -1);
-  map_back.clear();
+// Induced subgraph (in the arena) of the vertices with side[v] == s; ids (its
+// vertices' numbers, in the arena) from the parent's.
+G induced(const G& g, const uint8_t* side, uint8_t s, const int32_t* parent_ids, int32_t** ids) {
+  Arena& A = Arena::get();
+  int32_t cnt = 0;
   int64_t ub = 0;  // entries of the kept rows: room for the induced rows
   for (int32_t v = 0; v < g.n; ++v)
     if (side[v] == s) {
-      loc[v] = static_cast<int32_t>(map_back.size());
-      map_back.push_back(v);
-      ub += g.xadj[v + 1] - g.xadj[v];
+      ++cnt;
+      ub += g.v[v].hi - g.v[v].lo;
     }
   G h;
-  h.n = static_cast<int32_t>(map_back.size());
-  h.adj.reserve(ub);
-  h.w.reserve(ub);
-  h.xadj.assign(h.n + 1, 0);
-  h.vw.resize(h.n);
-  for (int32_t i = 0; i < h.n; ++i) {
-    int32_t v = map_back[i];
-    h.vw[i] = g.vw[v];
-    h.tw += g.vw[v];
-    for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-      int32_t u = loc[g.adj[j]];
-      if (u < 0) continue;
-      h.adj.push_back(u);
-      h.w.push_back(g.w[j]);
+  h.n = cnt;
+  h.v = A.take<V>(cnt);
+  *ids = A.take<int32_t>(cnt);
+  h.e = A.take<Edge>(static_cast<size_t>(ub));
+  int32_t top = 0;
+  {
+    Arena::Scope work;
+    int32_t* loc = A.take<int32_t>(g.n);
+    int32_t i = 0;
+    for (int32_t v = 0; v < g.n; ++v) loc[v] = side[v] == s ? i++ : -1;
+    i = 0;
+    for (int32_t v = 0; v < g.n; ++v) {
+      if (side[v] != s) continue;
+      (*ids)[i] = parent_ids[v];
+      h.v[i].vw = g.v[v].vw;
+      h.tw += g.v[v].vw;
+      h.v[i].lo = top;
+      int32_t sum = 0;
+      for (int32_t j = g.v[v].lo; j < g.v[v].hi; ++j) {
+        const int32_t u = loc[g.e[j].u];
+        const bool in = u >= 0;
+        if (in) {
+          h.e[top] = Edge{u, g.e[j].w};
+          sum += g.e[j].w;
+        }
+        top += in;
+      }
+      h.v[i].hi = top;
+      h.v[i].inc = sum;
+      ++i;
     }
-    h.xadj[i + 1] = static_cast<int32_t>(h.adj.size());
   }
+  A.keep(h.e, static_cast<size_t>(top));
+  h.rows = top;
   return h;
 }
 
@@ -720,36 +888,31 @@ struct RBCtx {
   bool parallel;  // use the fork-join pool
 };
 
-void rb(const G& g, int32_t k, int32_t part0, int depth, RBCtx& ctx, int32_t* out,
-        const std::vector<int32_t>& ids) {
-  if (k == 1 || g.n == 0) {
+void rb(const G& g, int32_t k, int32_t part0, int depth, RBCtx& ctx, int32_t* out, const int32_t* ids) {
+  if (k == 1 || g.n <= 1) {
     for (int32_t i = 0; i < g.n; ++i) out[ids[i]] = part0;
     return;
   }
-  if (g.n == 1) {
-    out[ids[0]] = part0;
-    return;
-  }
+  Arena::Scope all;
   const int32_t k0 = k / 2, k1 = k - k0;
   const int64_t target0 = g.tw * k0 / k;
-  std::vector<uint8_t> side;
   const uint64_t s = ctx.seed * 0x9E3779B97F4A7C15ull ^ (uint64_t(depth) << 40) ^ uint64_t(part0) * 0xD1B54A32D192ED03ull;
   // Several independent multilevel bisections (more near the root, where a
   // bisection decides the most); keep the lowest (overload, cut, trial).
   // Trials run on spare threads; the pick does not depend on scheduling.
   const int ncuts = depth == 0 ? ctx.ncuts0 : (depth < 3 ? ctx.ncuts1 : ctx.ncuts2);
-  std::vector<std::vector<uint8_t>> trial(ncuts);
+  uint8_t* trial = Arena::get().take<uint8_t>(size_t(ncuts) * g.n);
   std::vector<int64_t> key_ol(ncuts), key_cut(ncuts);
   auto run_trial = [&](int c) {
-    key_cut[c] = ml_bisect(g, target0, ctx.tol, s + 0x51ED2701ull * uint64_t(c), trial[c], ctx.parallel);
     int64_t pw0 = 0;
-    for (int32_t v = 0; v < g.n; ++v) if (trial[c][v] == 0) pw0 += g.vw[v];
+    key_cut[c] = ml_bisect(g, target0, ctx.tol, s + 0x51ED2701ull * uint64_t(c), trial + size_t(c) * g.n, &pw0, ctx.parallel);
     const int64_t t1 = g.tw - target0;
     const int64_t m0 = static_cast<int64_t>(std::floor(double(target0) * (1.0 + ctx.tol)));
     const int64_t m1 = static_cast<int64_t>(std::floor(double(t1) * (1.0 + ctx.tol)));
     key_ol[c] = std::max<int64_t>(0, pw0 - m0) + std::max<int64_t>(0, (g.tw - pw0) - m1);
   };
-  if (ctx.parallel && g.n > GKIP_SPAWN_MIN) {
+  const bool spawn = ctx.parallel && g.n > GKIP_SPAWN_MIN;
+  if (spawn) {
     std::vector<std::shared_ptr<ForkJoin::Task>> ts;
     for (int c = 1; c < ncuts; ++c) ts.push_back(ForkJoin::get().spawn([&, c] { run_trial(c); }));
     run_trial(0);
@@ -760,71 +923,117 @@ void rb(const G& g, int32_t k, int32_t part0, int depth, RBCtx& ctx, int32_t* ou
   int bc = 0;
   for (int c = 1; c < ncuts; ++c)
     if (key_ol[c] < key_ol[bc] || (key_ol[c] == key_ol[bc] && key_cut[c] < key_cut[bc])) bc = c;
-  side.swap(trial[bc]);
-  std::vector<int32_t> mb0, mb1;
-  G g0, g1;
-  if (ctx.parallel && g.n > GKIP_SPAWN_MIN) {
-    auto t = ForkJoin::get().spawn([&] { g1 = induced(g, side, 1, mb1); });
-    g0 = induced(g, side, 0, mb0);
+  const uint8_t* side = trial + size_t(bc) * g.n;
+  // The two halves are independent: each makes its own graph, one may run on
+  // another thread.
+  auto half = [&](uint8_t x) {
+    Arena::Scope own;
+    int32_t* hid = nullptr;
+    const G h = induced(g, side, x, ids, &hid);
+    if (x == 0) rb(h, k0, part0, depth + 1, ctx, out, hid);
+    else rb(h, k1, part0 + k0, depth + 1, ctx, out, hid);
+  };
+  if (spawn) {
+    auto t = ForkJoin::get().spawn([&] { half(0); });
+    half(1);
     ForkJoin::get().wait(t);
   } else {
-    g0 = induced(g, side, 0, mb0);
-    g1 = induced(g, side, 1, mb1);
-  }
-  std::vector<int32_t> ids0(mb0.size()), ids1(mb1.size());
-  for (size_t i = 0; i < mb0.size(); ++i) ids0[i] = ids[mb0[i]];
-  for (size_t i = 0; i < mb1.size(); ++i) ids1[i] = ids[mb1[i]];
-  // The two halves are independent: one may run on another thread.
-  if (ctx.parallel && g.n > GKIP_SPAWN_MIN) {
-    auto t = ForkJoin::get().spawn([&] { rb(g0, k0, part0, depth + 1, ctx, out, ids0); });
-    rb(g1, k1, part0 + k0, depth + 1, ctx, out, ids1);
-    ForkJoin::get().wait(t);
-  } else {
-    rb(g0, k0, part0, depth + 1, ctx, out, ids0);
-    rb(g1, k1, part0 + k0, depth + 1, ctx, out, ids1);
+    half(0);
+    half(1);
   }
 }
 
 // k-way greedy boundary pass: repair parts above cap, then positive-gain
 // moves that respect the cap.  Vertices are visited in id order each sweep.
-void kway_polish(const G& g, int32_t k, int64_t cap, int32_t* part, int sweeps) {
+// A visit changes nothing, and will not until a neighbour moves, unless the
+// vertex's part is above the cap or some part would give a positive gain (only
+// the cap can then hold it back): after the first sweep only such vertices and
+// the movers' neighbours are visited.  With par the first sweep's vertices are
+// picked on the pool threads beforehand.
+void kway_polish(const G& g, int32_t k, int64_t cap, int32_t* part, int sweeps, bool par) {
+  Arena::Scope all;
+  const int32_t n = g.n;
   std::vector<int64_t> pw(k, 0);
-  for (int32_t v = 0; v < g.n; ++v) pw[part[v]] += g.vw[v];
-  std::vector<int64_t> conn(k, 0);
-  std::vector<int32_t> touched;
+  for (int32_t v = 0; v < n; ++v) pw[part[v]] += g.v[v].vw;
+  const int32_t words = (n + 63) / 64;
+  uint64_t* due = Arena::get().take<uint64_t>(words);
+  // Weights of v to the parts around it (conn, all 0 before; touched lists
+  // them); false when every neighbour is in v's own part.
+  auto connect = [&](int32_t v, int32_t* conn, std::vector<int32_t>& touched) -> bool {
+    const int32_t p = part[v];
+    int32_t j = g.v[v].lo;
+    while (j < g.v[v].hi && part[g.e[j].u] == p) ++j;
+    if (j == g.v[v].hi) return false;
+    touched.clear();
+    for (j = g.v[v].lo; j < g.v[v].hi; ++j) {
+      const int32_t q = part[g.e[j].u];
+      if (conn[q] == 0) touched.push_back(q);
+      conn[q] += g.e[j].w;
+    }
+    return true;
+  };
+  auto may_move = [&](int32_t v, const int32_t* conn, const std::vector<int32_t>& touched) -> bool {
+    const int32_t p = part[v];
+    if (pw[p] > cap) return true;
+    for (int32_t q : touched)
+      if (q != p && conn[q] > conn[p]) return true;
+    return false;
+  };
+  const int chunks = par ? static_cast<int>(std::min<int64_t>(16, g.rows / 8192)) : 1;
+  if (chunks > 1) {
+    par_chunks(chunks, [&](int c) {
+      std::vector<int32_t> conn(k, 0), touched;
+      for (int32_t w = int32_t(int64_t(words) * c / chunks); w < int32_t(int64_t(words) * (c + 1) / chunks); ++w) {
+        uint64_t b = 0;
+        for (int32_t v = 64 * w; v < std::min(n, 64 * w + 64); ++v) {
+          if (!connect(v, conn.data(), touched)) continue;
+          if (may_move(v, conn.data(), touched)) b |= 1ull << (v & 63);
+          for (int32_t q : touched) conn[q] = 0;
+        }
+        due[w] = b;
+      }
+    });
+  } else {
+    for (int32_t w = 0; w < words; ++w) due[w] = w + 1 < words || n % 64 == 0 ? ~0ull : (1ull << (n % 64)) - 1;
+  }
+  std::vector<int32_t> conn(k, 0), touched;
   for (int s = 0; s < sweeps; ++s) {
     int64_t moves = 0;
-    for (int32_t v = 0; v < g.n; ++v) {
-      const int32_t p = part[v];
-      touched.clear();
-      bool boundary = false;
-      for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j) {
-        int32_t q = part[g.adj[j]];
-        if (conn[q] == 0) touched.push_back(q);
-        conn[q] += g.w[j];
-        if (q != p) boundary = true;
-      }
-      if (boundary) {
+    for (int32_t w = 0; w < words; ++w) {
+      // Bits set meanwhile: those behind the current vertex are still visited
+      // in this sweep, those before it in the next one.
+      uint64_t seen = 0;
+      while (uint64_t left = due[w] & ~seen) {
+        const int bit = __builtin_ctzll(left);
+        const int32_t v = 64 * w + bit;
+        seen |= bit == 63 ? ~0ull : (2ull << bit) - 1;
+        due[w] &= ~(1ull << bit);
+        if (!connect(v, conn.data(), touched)) continue;
+        const int32_t p = part[v];
         const bool over = pw[p] > cap;
         int32_t bestq = -1;
         int64_t bestg = 0;
         for (int32_t q : touched) {
           if (q == p) continue;
-          if (pw[q] + g.vw[v] > cap) continue;
-          int64_t gain = conn[q] - conn[p];
+          if (pw[q] + g.v[v].vw > cap) continue;
+          int64_t gain = int64_t(conn[q]) - conn[p];
           bool better;
           if (over) better = bestq < 0 || gain > bestg || (gain == bestg && (pw[q] < pw[bestq] || (pw[q] == pw[bestq] && q < bestq)));
           else better = gain > bestg || (gain == bestg && gain > 0 && q < bestq);
           if (better) { bestq = q; bestg = gain; }
         }
         if (bestq >= 0 && (over || bestg > 0)) {
-          pw[p] -= g.vw[v];
-          pw[bestq] += g.vw[v];
+          pw[p] -= g.v[v].vw;
+          pw[bestq] += g.v[v].vw;
           part[v] = bestq;
           ++moves;
+          due[w] |= 1ull << bit;
+          for (int32_t j = g.v[v].lo; j < g.v[v].hi; ++j) due[g.e[j].u >> 6] |= 1ull << (g.e[j].u & 63);
+        } else if (may_move(v, conn.data(), touched)) {
+          due[w] |= 1ull << bit;
         }
+        for (int32_t q : touched) conn[q] = 0;
       }
-      for (int32_t q : touched) conn[q] = 0;
     }
     if (moves == 0) break;
   }
@@ -842,20 +1051,35 @@ extern "C" int64_t gk_part_cap(int64_t total_vwgt, int32_t k, int32_t ubfactor) 
 extern "C" int gk_initpart(const gk_csr* hg, int32_t k, int64_t cap, int32_t seed,
                            int32_t nthreads, int32_t* part, int64_t* cut) {
   if (!hg || !part || k < 1 || hg->n < 0) return GK_ERR_ARG;
-  G g;
-  g.n = hg->n;
-  g.xadj.assign(hg->xadj, hg->xadj + hg->n + 1);
-  const int32_t nnz = g.xadj[g.n];
-  g.adj.assign(hg->adjncy, hg->adjncy + nnz);
-  if (hg->adjwgt) g.w.assign(hg->adjwgt, hg->adjwgt + nnz); else g.w.assign(nnz, 1);
-  if (hg->vwgt) g.vw.assign(hg->vwgt, hg->vwgt + g.n); else g.vw.assign(g.n, 1);
-  g.tw = 0;
-  for (int32_t v = 0; v < g.n; ++v) g.tw += g.vw[v];
+  const int32_t n = hg->n;
   if (k == 1) {
-    std::fill(part, part + g.n, 0);
+    std::fill(part, part + n, 0);
     if (cut) *cut = 0;
     return GK_OK;
   }
+  Arena::Scope all;
+  Arena& A = Arena::get();
+  const bool parallel = nthreads != 1 && ForkJoin::get().workers() > 0;
+  G g;
+  g.n = n;
+  g.rows = hg->xadj[n];
+  g.v = A.take<V>(n);
+  g.e = A.take<Edge>(static_cast<size_t>(g.rows));
+  const int chunks = parallel ? static_cast<int>(std::min<int64_t>(16, std::max<int64_t>(1, g.rows / 16384))) : 1;
+  std::vector<int64_t> tw(chunks, 0);
+  par_chunks(chunks, [&](int c) {
+    for (int32_t v = int32_t(int64_t(n) * c / chunks); v < int32_t(int64_t(n) * (c + 1) / chunks); ++v) {
+      int32_t sum = 0;
+      for (int32_t j = hg->xadj[v]; j < hg->xadj[v + 1]; ++j) {
+        const int32_t w = hg->adjwgt ? hg->adjwgt[j] : 1;
+        g.e[j] = Edge{hg->adjncy[j], w};
+        sum += w;
+      }
+      g.v[v] = V{hg->xadj[v], hg->xadj[v + 1], hg->vwgt ? hg->vwgt[v] : 1, sum};
+      tw[c] += g.v[v].vw;
+    }
+  });
+  for (int64_t x : tw) g.tw += x;
   // Per-bisection tolerance: (cap / (T/k))^(1/levels) - 1, slightly tightened
   // so that rounding of the recursive targets stays inside the cap.
   const int levels = static_cast<int>(std::ceil(std::log2(double(k))));
@@ -870,17 +1094,22 @@ extern "C" int gk_initpart(const gk_csr* hg, int32_t k, int64_t cap, int32_t see
   ctx.seed = static_cast<uint64_t>(seed) + 1;
   // nthreads == 1: everything on the calling thread; otherwise the
   // process-wide pool (up to 16 threads) helps.
-  ctx.parallel = nthreads != 1 && ForkJoin::get().workers() > 0;
-  std::vector<int32_t> ids(g.n);
-  std::iota(ids.begin(), ids.end(), 0);
+  ctx.parallel = parallel;
+  int32_t* ids = A.take<int32_t>(n);
+  std::iota(ids, ids + n, 0);
   rb(g, k, 0, 0, ctx, part, ids);
-  kway_polish(g, k, cap, part, 4);
+  kway_polish(g, k, cap, part, 4, parallel);
   if (cut) {
-    int64_t c = 0;
-    for (int32_t v = 0; v < g.n; ++v)
-      for (int32_t j = g.xadj[v]; j < g.xadj[v + 1]; ++j)
-        if (v < g.adj[j] && part[v] != part[g.adj[j]]) c += g.w[j];
-    *cut = c;
+    std::vector<int64_t> cs(chunks, 0);
+    par_chunks(chunks, [&](int c) {
+      int64_t x = 0;
+      for (int32_t v = int32_t(int64_t(n) * c / chunks); v < int32_t(int64_t(n) * (c + 1) / chunks); ++v)
+        for (int32_t j = g.v[v].lo; j < g.v[v].hi; ++j)
+          x += v < g.e[j].u && part[v] != part[g.e[j].u] ? g.e[j].w : 0;
+      cs[c] = x;
+    });
+    *cut = 0;
+    for (int64_t x : cs) *cut += x;
   }
   return GK_OK;
 }
