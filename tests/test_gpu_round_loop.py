@@ -66,3 +66,27 @@ def test_batch_more_jobs_than_compute_units(gk, ctx):
         parts, stats = ctx.partition_batch(graphs, ks, flags=flags)
         for i in list(range(0, 300, 37)) + [0, 30, 60]:
             assert np.array_equal(parts[i], ctx.partition(graphs[i], ks[i])[0]), i
+
+
+# The short way of the V-cycle's rounds (the best movable vertices, applied one
+# after another by one wave, with the proof that no later prefix is balanced)
+# against the oracle, level by level: unit weights (hundreds of equal gains in
+# one class), weights over several orders of magnitude, hubs, a tight and a
+# loose cap, move caps below and above a round's movable vertices.
+def weighted(gk, g, top, seed):
+    """g with symmetric edge weights 1..top, spread over their logarithm."""
+    rng = np.random.default_rng(seed)
+    src = np.repeat(np.arange(g.n), g.degrees())
+    key = np.minimum(src, g.adjncy) * np.int64(g.n) + np.maximum(src, g.adjncy)
+    _, inv = np.unique(key, return_inverse=True)
+    w = np.exp(rng.uniform(0, np.log(top), inv.max() + 1)).astype(np.int64)[inv]
+    return gk.Graph(g.xadj, g.adjncy, np.maximum(w, 1), rng.integers(1, 9, g.n))
+
+
+@pytest.mark.parametrize("k,ub,moves", [(2, 30, 1024), (8, 0, 1024), (64, 5, 1024), (256, 30, 1024), (32, 30, 300), (16, 100, 40)])
+@pytest.mark.parametrize("name", ["mesh", "weighted", "dag", "hubs"])
+def test_vcycle_rounds(gk, oracle, ctx, name, k, ub, moves):
+    from test_gpu_parity import compare
+    g = {"mesh": lambda: gk.delaunay(70000, 21), "weighted": lambda: weighted(gk, gk.delaunay(30000, 22), 20000, 1),
+         "dag": lambda: gk.dag(40000, 120, 23), "hubs": lambda: hub_graph(gk, n=12000, hubs=40, fan=200, seed=24)}[name]()
+    compare(gk, oracle, ctx, g, k, ubfactor=ub, max_moves=moves)
