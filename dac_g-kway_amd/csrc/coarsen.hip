@@ -5,6 +5,8 @@
 // writes results that do not depend on the launch schedule: atomics are used
 // only for commutative integer max/add or for slot reservation whose order is
 // discarded by a later sort.
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "prim.hpp"
 #include "steal.hpp"
@@ -496,6 +498,31 @@ int launch_members(int32_t n, const int32_t* label, const int32_t* stamp, const 
   return hip_status();
 }
 
+// The members' rows by group, in arbitrary order inside a group, and each
+// group's first place, for readers to whom that order is all the same.
+__global__ void __launch_bounds__(256) k_member_place(int32_t n, const int32_t* __restrict__ label,
+                                                      const int32_t* __restrict__ slot,
+                                                      const int2* __restrict__ offc,
+                                                      const int32_t* __restrict__ xadj,
+                                                      const int32_t* __restrict__ ctl, int32_t* __restrict__ cptr,
+                                                      int2* __restrict__ mrow) {
+  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
+  if (v >= n) return;
+  const int32_t a = xadj[v];
+  mrow[int64_t(offc[label[v]].x) + slot[v]] = make_int2(a, xadj[v + 1] - a);
+  // index v as a label: the first place of its group, if it has members
+  const int2 o = offc[v];
+  if (offc[v + 1].x > o.x) cptr[o.y] = o.x;
+  if (v == n - 1) cptr[ctl[0]] = n;
+}
+
+int launch_member_place(int32_t n, const int32_t* label, const int32_t* slot, const int2* offc, const int32_t* xadj,
+                        const int32_t* ctl, int32_t* cptr, int2* mrow, hipStream_t st) {
+  if (n <= 0) return 0;
+  k_member_place<<<grid_for(n, 256), 256, 0, st>>>(n, label, slot, offc, xadj, ctl, cptr, mrow);
+  return hip_status();
+}
+
 // The members' rows and weights in a given vertex order (after a sort).
 __global__ void __launch_bounds__(256) k_member_rows(int32_t n, const int32_t* __restrict__ order,
                                                      const int32_t* __restrict__ xadj,
@@ -608,74 +635,106 @@ int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* mvw, int32_t* c
 }
 
 // --------------------------------------------------------------- contraction
-// Per coarse row: upper bound of entries (sum of member degrees) and its
-// lane class; row ids appended to one list per class, each with its member
-// range in member order (desc: first member, member count).  The members'
-// rows (mrow) and weights (mvw, with cvw the coarse weights' destination; both
-// may be null) lie in member order, so a row's members are consecutive reads.
+// Per coarse row: the upper bound of its entries (sum of member degrees), its
+// class (16, 32 or 64 lanes, a workgroup, or the global sort), and room for
+// them in the temporary rows (toff).  Row ids are appended to one list per
+// class, each with its member range in member order (desc: first member,
+// member count); a row of the last two classes leaves its bound in len until
+// it is merged.  The members' rows (mrow) and weights (mvw, with cvw the
+// coarse weights' destination; both may be null) lie in member order, so a
+// row's members are consecutive reads.  A block takes kBoundsPer rows a thread
+// and adds to the class counters and the room once: same-address atomics
+// serialise, and with one row a thread they, not the reads, were the time
+// (2^22 vertices, 1 M rows: 52 us with one, 23 us with four rows a thread and
+// the counters kRowCtlStride ints apart).  Up to kRowsAllMax rows there are few
+// blocks, and one row a thread is the shorter chain (20000 rows: 9 us with
+// four).
+template <int kBoundsPer>
 __global__ void __launch_bounds__(256) k_row_bounds(int32_t nc, const int32_t* __restrict__ cptr,
                                                     const int2* __restrict__ mrow, const int32_t* __restrict__ mvw,
-                                                    int32_t* __restrict__ ub, int32_t* __restrict__ lists,
-                                                    int2* __restrict__ desc, int32_t* __restrict__ cvw,
-                                                    int32_t* __restrict__ cnt) {
-  const int64_t c = int64_t(xcd_block()) * 256 + threadIdx.x;
-  int cls = -1;
-  int32_t m0 = 0, m1 = 0;
-  if (c < nc) {
-    m0 = cptr[c];
-    m1 = cptr[c + 1];
-    int32_t s = 0, x = 0;
-    for (int32_t j = m0; j < m1; ++j) {
-      s += mrow[j].y;
-      if (mvw) x += mvw[j];
-    }
-    ub[c] = s;
-    if (mvw) cvw[c] = x;
-    cls = s <= 16 ? 0 : (s <= 32 ? 1 : (s <= 64 ? 2 : 3));
-  }
-  // Block-aggregated append: per class, wave counts in LDS, one global
-  // atomic per block and class.
-  __shared__ int wcnt[4][4];
-  __shared__ int bbase[4];
+                                                    int32_t* __restrict__ toff, int32_t* __restrict__ lists,
+                                                    int2* __restrict__ desc, int32_t* __restrict__ len,
+                                                    int32_t* __restrict__ cvw, int32_t* __restrict__ cnt) {
+  // per class: rows of each wave and pass; then entries likewise
+  __shared__ int wcnt[kRowClasses][4 * kBoundsPer];
+  __shared__ int wub[4 * kBoundsPer];
+  __shared__ int base[kRowClasses + 1];
   const int wave = threadIdx.x >> 6;
   const uint64_t lt = lanemask_lt();
-  uint64_t m[4];
+  const int64_t c0 = int64_t(xcd_block()) * (256 * kBoundsPer) + threadIdx.x;
+  int32_t m0[kBoundsPer], nm[kBoundsPer], ub[kBoundsPer], pre[kBoundsPer];
+  int cls[kBoundsPer];
+  int big = 0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    m[k] = ballot(cls == k);
-    if (lane_id() == 0) wcnt[k][wave] = popc64(m[k]);
+  for (int r = 0; r < kBoundsPer; ++r) {
+    const int64_t c = c0 + r * 256;
+    cls[r] = -1;
+    m0[r] = nm[r] = ub[r] = 0;
+    if (c < nc) {
+      m0[r] = cptr[c];
+      nm[r] = cptr[c + 1] - m0[r];
+      int32_t s = 0, x = 0;
+      for (int32_t j = m0[r]; j < m0[r] + nm[r]; ++j) {
+        s += mrow[j].y;
+        if (mvw) x += mvw[j];
+      }
+      if (mvw) cvw[c] = x;
+      ub[r] = s;
+      cls[r] = s <= 16 ? 0 : (s <= 32 ? 1 : (s <= 64 ? 2 : (s <= kMidMax ? 3 : 4)));
+      if (cls[r] == 4) big += s;
+      if (cls[r] >= 3) len[c] = s;
+    }
+    const int incl = wave_incl_scan(ub[r]);
+    pre[r] = incl - ub[r];
+    if (lane_id() == 63) wub[r * 4 + wave] = incl;
+#pragma unroll
+    for (int k = 0; k < kRowClasses; ++k) {
+      const int x = popc64(ballot(cls[r] == k));
+      if (lane_id() == 0) wcnt[k][r * 4 + wave] = x;
+    }
+  }
+  if (ballot(big > 0) != 0) {
+    big = wave_sum(big);
+    if (lane_id() == 0) atomicAdd(&cnt[kRowBigEntries * kRowCtlStride], big);
   }
   __syncthreads();
-  if (threadIdx.x < 4) {
-    const int k = threadIdx.x;
-    const int t = wcnt[k][0] + wcnt[k][1] + wcnt[k][2] + wcnt[k][3];
-    bbase[k] = t ? atomicAdd(&cnt[k], t) : 0;
+  if (threadIdx.x <= kRowClasses) {
+    int* w = threadIdx.x < kRowClasses ? wcnt[threadIdx.x] : wub;
+    int run = 0;
+#pragma unroll
+    for (int i = 0; i < 4 * kBoundsPer; ++i) {
+      const int q = w[i];
+      w[i] = run;
+      run += q;
+    }
+    base[threadIdx.x] = run ? atomicAdd(&cnt[threadIdx.x * kRowCtlStride], run) : 0;
   }
   __syncthreads();
-  if (cls >= 0) {
-    int off = bbase[cls];
-    for (int w = 0; w < wave; ++w) off += wcnt[cls][w];
-    const uint64_t mine = cls == 0 ? m[0] : (cls == 1 ? m[1] : (cls == 2 ? m[2] : m[3]));
-    const int64_t slot = int64_t(cls) * nc + off + popc64(mine & lt);
+#pragma unroll
+  for (int r = 0; r < kBoundsPer; ++r) {
+    const int64_t c = c0 + r * 256;
+    uint64_t mine = 0;
+#pragma unroll
+    for (int k = 0; k < kRowClasses; ++k) {
+      const uint64_t m = ballot(cls[r] == k);
+      if (cls[r] == k) mine = m;
+    }
+    if (c >= nc) continue;
+    toff[c] = base[kRowClasses] + wub[r * 4 + wave] + pre[r];
+    const int64_t slot = int64_t(cls[r]) * nc + base[cls[r]] + wcnt[cls[r]][r * 4 + wave] + popc64(mine & lt);
     lists[slot] = int32_t(c);
-    desc[slot] = make_int2(m0, m1 - m0);
+    desc[slot] = make_int2(m0[r], nm[r]);
   }
 }
 
-struct UbLoad {
-  const int32_t* ub;
-  int32_t nc;
-  __device__ int operator()(int64_t i) const { return i < nc ? ub[i] : 0; }
-};
-
-int launch_contract_bounds(int32_t nc, const int32_t* cptr, const int2* mrow, const int32_t* mvw, int32_t* ub,
-                           int32_t* toff, int32_t* lists, int2* desc, int32_t* cvw, int32_t* list_cnt,
-                           int32_t* scratch, hipStream_t st) {
-  fill<int32_t>(list_cnt, 0, 4, st);
+int launch_contract_bounds(int32_t nc, const int32_t* cptr, const int2* mrow, const int32_t* mvw, int32_t* toff,
+                           int32_t* lists, int2* desc, int32_t* len, int32_t* cvw, int32_t* cnt, hipStream_t st) {
   if (nc <= 0) return 0;
-  k_row_bounds<<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, mrow, mvw, ub, lists, desc, cvw, list_cnt);
-  int rc = scan(int64_t(nc) + 1, UbLoad{ub, nc}, StoreExcl{toff}, nullptr, scratch, st);
-  return rc ? GK_ERR_HIP : hip_status();
+  if (nc <= kRowsAllMax)
+    k_row_bounds<1><<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, mrow, mvw, toff, lists, desc, len, cvw, cnt);
+  else
+    k_row_bounds<4><<<grid_for(nc, 1024), 256, 0, st>>>(nc, cptr, mrow, mvw, toff, lists, desc, len, cvw, cnt);
+  return hip_status();
 }
 
 // Rows whose upper bound fits S lanes, any coarse id width: one entry per
@@ -965,6 +1024,153 @@ int launch_contract_rows(const DGraph& g, int lanes, int block, const int32_t* r
   return hip_status();
 }
 
+// The rows of all three lane classes in one launch, their counts read on the
+// device: the waves stride over the classes' waves one after another.  For
+// levels of up to kRowsAllMax coarse rows, whose launches and the read-back of
+// the counts took longer than the rows (mesh of 60000 vertices, 3 levels: 7 us
+// a level here; three launches of 4 us and a read-back of 15 us before).
+__global__ void __launch_bounds__(256) k_contract_rows_all(int32_t nc, const int32_t* __restrict__ cnt,
+                                                           const int32_t* __restrict__ lists,
+                                                           const int2* __restrict__ desc,
+                                                           const int2* __restrict__ mrow,
+                                                           const int32_t* __restrict__ adj,
+                                                           const int32_t* __restrict__ w,
+                                                           const int32_t* __restrict__ cmap,
+                                                           const int32_t* __restrict__ toff,
+                                                           int32_t* __restrict__ tadj, int32_t* __restrict__ tw,
+                                                           int32_t* __restrict__ len) {
+  __shared__ int32_t mark[256];
+  int32_t* wm = mark + (threadIdx.x & ~63u);
+  const int32_t r0 = cnt[0], r1 = cnt[kRowCtlStride], r2 = cnt[2 * kRowCtlStride];
+  const int32_t w0 = (r0 + 3) / 4, w1 = (r1 + 1) / 2;
+  const int32_t total = w0 + w1 + r2;
+  for (int32_t u = int32_t(blockIdx.x) * 4 + int32_t(threadIdx.x >> 6); u < total; u += int32_t(gridDim.x) * 4) {
+    if (u < w0)
+      contract_row_slot<16>(int64_t(u) * 64 + lane_id(), wm, lists, desc, r0, mrow, adj, w, cmap, toff, tadj, tw, len);
+    else if (u < w0 + w1)
+      contract_row_slot<32>(int64_t(u - w0) * 64 + lane_id(), wm, lists + nc, desc + nc, r1, mrow, adj, w, cmap, toff,
+                            tadj, tw, len);
+    else
+      contract_row_slot<64>(int64_t(u - w0 - w1) * 64 + lane_id(), wm, lists + 2 * int64_t(nc), desc + 2 * int64_t(nc),
+                            r2, mrow, adj, w, cmap, toff, tadj, tw, len);
+  }
+}
+
+// Rows of 65 to kMidMax entries: a workgroup per row sums the entries by
+// coarse neighbour in an LDS hash table, collects the (distinct) neighbours
+// and sorts them.  The rows of a weighted DAG's coarse levels are of this kind;
+// sorting all their entries in global memory took a read-back, 69 + 35 us of
+// scatters and histograms and 70 us of scans on a DAG of 1 M vertices, which is
+// 11 us here.  Grid-stride over
+// the class's list, whose count is read on the device.
+constexpr int kMidThreads = 256;
+
+__global__ void __launch_bounds__(kMidThreads) k_contract_mid(const int32_t* __restrict__ cnt,
+                                                              const int32_t* __restrict__ rows,
+                                                              const int2* __restrict__ desc,
+                                                              const int2* __restrict__ mrow,
+                                                              const int32_t* __restrict__ adj,
+                                                              const int32_t* __restrict__ w,
+                                                              const int32_t* __restrict__ cmap,
+                                                              const int32_t* __restrict__ toff,
+                                                              int32_t* __restrict__ tadj, int32_t* __restrict__ tw,
+                                                              int32_t* __restrict__ len) {
+  __shared__ int32_t key[2 * kMidMax];
+  __shared__ int32_t sum[2 * kMidMax];
+  __shared__ uint64_t srt[kMidMax];
+  __shared__ int32_t m;
+  const int t = threadIdx.x;
+  const int32_t nrows = cnt[3 * kRowCtlStride];
+  for (int32_t i = blockIdx.x; i < nrows; i += gridDim.x) {
+    const int32_t c = rows[i];
+    const int2 d = desc[i];
+    // entries of the row, and the table: a power of two, at least twice as many
+    const int32_t ub = len[c];
+    int32_t tab = 256;
+    while (tab < 2 * ub) tab <<= 1;
+    const int shift = __clz(tab) + 1;  // 32 - log2(tab)
+    for (int32_t x = t; x < tab; x += kMidThreads) {
+      key[x] = -1;
+      sum[x] = 0;
+    }
+    if (t == 0) m = 0;
+    __syncthreads();
+    // a wave per member in turn: its entries are consecutive reads
+    for (int32_t x = d.x + (t >> 6); x < d.x + d.y; x += kMidThreads / 64) {
+      const int2 r = mrow[x];
+      for (int32_t e = r.x + lane_id(); e < r.x + r.y; e += 64) {
+        const int32_t q = cmap[adj[e]];
+        if (q == c) continue;
+        const int32_t we = w[e];
+        uint32_t s = (uint32_t(q) * 0x9E3779B1u) >> shift;
+        while (true) {
+          const int32_t o = atomicCAS(&key[s], -1, q);
+          if (o == -1 || o == q) break;
+          s = (s + 1) & uint32_t(tab - 1);
+        }
+        atomicAdd(&sum[s], we);
+      }
+    }
+    __syncthreads();
+    // the distinct neighbours with their sums
+    for (int32_t x0 = 0; x0 < tab; x0 += kMidThreads) {
+      const int32_t q = key[x0 + t];
+      const uint64_t b = ballot(q >= 0);
+      int32_t o = 0;
+      if (lane_id() == 0 && b) o = atomicAdd(&m, popc64(b));
+      o = __shfl(o, 0, 64);
+      if (q >= 0) srt[o + popc64(b & lanemask_lt())] = (uint64_t(uint32_t(q)) << 32) | uint32_t(sum[x0 + t]);
+    }
+    __syncthreads();
+    const int32_t cntc = m;
+    int32_t P = 64;
+    while (P < cntc) P <<= 1;
+    for (int32_t x = cntc + t; x < P; x += kMidThreads) srt[x] = ~0ull;
+    __syncthreads();
+    for (int32_t k2 = 2; k2 <= P; k2 <<= 1)
+      for (int32_t j2 = k2 >> 1; j2 > 0; j2 >>= 1) {
+        for (int32_t p = t; p < (P >> 1); p += kMidThreads) {
+          const int32_t lo = ((p & ~(j2 - 1)) << 1) | (p & (j2 - 1));
+          const int32_t hi = lo + j2;
+          const uint64_t a = srt[lo], b = srt[hi];
+          if ((lo & k2) == 0 ? a > b : a < b) {
+            srt[lo] = b;
+            srt[hi] = a;
+          }
+        }
+        __syncthreads();
+      }
+    const int32_t to = toff[c];
+    for (int32_t x = t; x < cntc; x += kMidThreads) {
+      const uint64_t e = srt[x];
+      tadj[to + x] = int32_t(e >> 32);
+      tw[to + x] = int32_t(uint32_t(e));
+    }
+    if (t == 0) len[c] = cntc;
+    __syncthreads();  // the table and the sorted row are read
+  }
+}
+
+int launch_contract_rows_all(const DGraph& g, int32_t nc, const int32_t* cnt, const int32_t* lists, const int2* desc,
+                             const int2* mrow, const int32_t* cmap, const int32_t* toff, int32_t* tadj, int32_t* tw,
+                             int32_t* len, hipStream_t st) {
+  if (nc <= 0) return 0;
+  gk_launch(k_contract_rows_all, dim3(std::min<unsigned>(grid_for(nc, 4), 4096)), dim3(256), 0, st, nc, cnt, lists,
+            desc, mrow, g.adj, g.w, cmap, toff, tadj, tw, len);
+  return hip_status();
+}
+
+int launch_contract_mid(const DGraph& g, int32_t nc, int32_t max_rows, const int32_t* cnt, const int32_t* lists,
+                        const int2* desc, const int2* mrow, const int32_t* cmap, const int32_t* toff, int32_t* tadj,
+                        int32_t* tw, int32_t* len, hipStream_t st) {
+  // More than 64 entries a row: no more rows than that.
+  const int64_t rows = std::min<int64_t>(std::min<int64_t>(max_rows, nc), int64_t(g.nnz) / 65);
+  if (rows <= 0) return 0;
+  gk_launch(k_contract_mid, dim3(unsigned(std::min<int64_t>(rows, 2048))), dim3(kMidThreads), 0, st, cnt,
+            lists + 3 * int64_t(nc), desc + 3 * int64_t(nc), mrow, g.adj, g.w, cmap, toff, tadj, tw, len);
+  return hip_status();
+}
+
 struct BigUbLoad {
   const int32_t* rows;
   const int32_t* ub;
@@ -972,9 +1178,9 @@ struct BigUbLoad {
   __device__ int operator()(int64_t i) const { return i < nrows ? ub[rows[i]] : 0; }
 };
 
-int launch_big_offsets(const int32_t* rows, int32_t nrows, const int32_t* ub, int32_t* boff,
-                       int32_t* total, int32_t* scratch, hipStream_t st) {
-  int rc = scan(int64_t(nrows) + 1, BigUbLoad{rows, ub, nrows}, StoreExcl{boff}, total, scratch, st);
+int launch_big_offsets(const int32_t* rows, const int32_t* ub, int32_t nrows, int32_t* boff, int32_t* scratch,
+                       hipStream_t st) {
+  int rc = scan(int64_t(nrows) + 1, BigUbLoad{rows, ub, nrows}, StoreExcl{boff}, nullptr, scratch, st);
   return rc ? GK_ERR_HIP : hip_status();
 }
 
@@ -1068,16 +1274,82 @@ int launch_contract_big_merge(const int32_t* rows, int32_t nrows, const int32_t*
   return hip_status();
 }
 
-struct LenLoad {
-  const int32_t* len;
-  int32_t nc;
-  __device__ int operator()(int64_t i) const { return i < nc ? len[i] : 0; }
-};
+// Row starts of the coarse CSR from the rows' lengths: per-tile sums, then
+// every tile adds up the sums before it (many tiles: scanned by one block).
+// The last tile writes the entry count and the row class counters to the host.
+__global__ void __launch_bounds__(256) k_len_reduce(int32_t nc, const int32_t* __restrict__ len,
+                                                    int32_t* __restrict__ partial) {
+  __shared__ int ws[4];
+  const int64_t base = int64_t(blockIdx.x) * kSizeTile;
+  int32_t s = 0;
+#pragma unroll
+  for (int j = 0; j < kSizeIPT; ++j) {
+    const int64_t i = base + j * 256 + threadIdx.x;
+    if (i < nc) s += len[i];
+  }
+  s = wave_sum(s);
+  if (lane_id() == 0) ws[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) partial[blockIdx.x] = ws[0] + ws[1] + ws[2] + ws[3];
+}
 
-int launch_len_scan(int32_t nc, const int32_t* len, int32_t* cxadj, int32_t* cnnz,
-                    int32_t* scratch, hipStream_t st) {
-  int rc = scan(int64_t(nc) + 1, LenLoad{len, nc}, StoreExcl{cxadj}, cnnz, scratch, st);
-  return rc ? GK_ERR_HIP : hip_status();
+__global__ void __launch_bounds__(256) k_len_mid(int64_t nb, int32_t* __restrict__ partial) {
+  __shared__ int lds[8];
+  int32_t run = 0;
+  for (int64_t b0 = 0; b0 < nb; b0 += 256) {
+    const int64_t b = b0 + threadIdx.x;
+    int t;
+    const int e = block_excl_scan_256(b < nb ? partial[b] : 0, &t, lds);
+    if (b < nb) partial[b] = run + e;
+    run += t;
+  }
+}
+
+__global__ void __launch_bounds__(256) k_len_apply(int32_t nc, const int32_t* __restrict__ len,
+                                                   const int32_t* __restrict__ partial, int scanned,
+                                                   int32_t* __restrict__ cxadj, const int32_t* __restrict__ cnt,
+                                                   int32_t* __restrict__ host) {
+  __shared__ int lds[8];
+  int32_t pre = 0;
+  int t;
+  if (scanned) {
+    pre = partial[blockIdx.x];
+  } else {
+    int32_t s = 0;
+    for (int64_t b = threadIdx.x; b < int64_t(blockIdx.x); b += 256) s += partial[b];
+    (void)block_excl_scan_256(s, &t, lds);
+    pre = t;
+  }
+  const int64_t base = int64_t(blockIdx.x) * kSizeTile + int64_t(threadIdx.x) * kSizeIPT;
+  int32_t l[kSizeIPT];
+  int32_t s = 0;
+#pragma unroll
+  for (int j = 0; j < kSizeIPT; ++j) {
+    l[j] = base + j < nc ? len[base + j] : 0;
+    s += l[j];
+  }
+  int32_t run = pre + block_excl_scan_256(s, &t, lds);
+#pragma unroll
+  for (int j = 0; j < kSizeIPT; ++j) {
+    if (base + j < nc) cxadj[base + j] = run;
+    run += l[j];
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) {
+    cxadj[nc] = run;
+    host[0] = run;
+#pragma unroll
+    for (int k = 0; k < kRowCtlWords; ++k) host[1 + k] = cnt[k * kRowCtlStride];
+  }
+}
+
+int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt, int32_t* host,
+                    hipStream_t st) {
+  const int64_t nb = std::max<int64_t>(1, size_partials(nc));
+  k_len_reduce<<<unsigned(nb), 256, 0, st>>>(nc, len, partial);
+  const bool mid = nb > kSizeDirect;
+  if (mid) k_len_mid<<<1, 256, 0, st>>>(nb, partial);
+  k_len_apply<<<unsigned(nb), 256, 0, st>>>(nc, len, partial, mid ? 1 : 0, cxadj, cnt, host);
+  return hip_status();
 }
 
 // Copy merged rows to the final CSR (8 lanes per row).

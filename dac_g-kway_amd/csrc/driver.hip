@@ -50,12 +50,12 @@ constexpr int32_t kTuneMinRows = 1 << 14;
 // The control words (zeroed here) hold whether every vertex reached its pair.
 int Groups::walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label) {
   Pool& P = ctx->pool;
-  GK_TRY(ctl.alloc(P, gkd::kCtlInts));
+  GK_TRY(ctl.alloc(P, gkd::kCtlInts + gkd::kRowCtlInts));
   GK_TRY(comp.alloc(P, int64_t(n) + 1));
   GK_TRY(dist.alloc(P, n));
   GK_TRY(slot.alloc(P, n));
   GK_TRY(size.alloc(P, n));
-  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts, st);
+  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts + gkd::kRowCtlInts, st);
   GK_STAGE(ctx, GK_ST_GROUP, 52LL * n,
            (gkd::launch_walk(n, cand, comp.p, label, dist.p, slot.p, ctl.p + gkd::kCtlFlags, st) ||
                     gkd::launch_label_size(n, label, comp.p, label, size.p, st)
@@ -124,11 +124,11 @@ int Groups::jump(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, in
 // Labels in [0, n) that come without a grouping: member counts only.
 int Groups::count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label) {
   Pool& P = ctx->pool;
-  GK_TRY(ctl.alloc(P, gkd::kCtlInts));
+  GK_TRY(ctl.alloc(P, gkd::kCtlInts + gkd::kRowCtlInts));
   GK_TRY(comp.alloc(P, int64_t(n) + 1));
   GK_TRY(slot.alloc(P, n));
   GK_TRY(size.alloc(P, n));
-  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts, st);
+  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts + gkd::kRowCtlInts, st);
   GK_STAGE(ctx, GK_ST_SORT, 16LL * n, gkd::launch_label_count(n, label, size.p, slot.p, st));
   return GK_OK;
 }
@@ -225,75 +225,100 @@ int coarse_ids(gk_ctx* ctx, hipStream_t st, const DGraph& g, const int32_t* cand
   *nc = words[0];
   // Distances are at most 2^rounds.
   if (words[1]) GK_TRY(sort_members(ctx, st, n, label.p, gr.dist.p, *rounds + 1, g.xadj, g.vw, G, out, nc));
+  m.ctl = std::move(gr.ctl);
   return GK_OK;
 }
 
-// Contraction of g under cmap, with its members by coarse id (cptr; their rows
-// mrow, and their weights mvw), into the coarse level c; with mvw also the
-// coarse weights into c.vw (allocated by the caller).
-int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, const int32_t* cmap,
-                   const int32_t* cptr, const int2* mrow, const int32_t* mvw, Level& c) {
+// Contraction of g under cmap, with its members by coarse id (m: first places,
+// rows, and, unless null, weights), into the coarse level c; with weights also
+// the coarse weights into c.vw (allocated by the caller).
+int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, const int32_t* cmap, const Members& m,
+                   Level& c) {
   Pool& P = ctx->pool;
-  Buf<int32_t> ub, toff, lists, lcnt, scratch, tadj, tw, len, cnnzd;
+  Buf<int32_t> toff, lists, scratch, tadj, tw, len;
   Buf<int2> desc;
-  GK_TRY(ub.alloc(P, nc));
-  GK_TRY(toff.alloc(P, int64_t(nc) + 1));
-  GK_TRY(lists.alloc(P, int64_t(4) * nc));
-  GK_TRY(desc.alloc(P, int64_t(4) * nc));
-  GK_TRY(lcnt.alloc(P, 4));
-  GK_TRY(scratch.alloc(P, gkd::scan_scratch_ints(int64_t(nc) + 1) + 64));
-  GK_STAGE(ctx, GK_ST_CONTRACT_AUX, (mvw ? 12LL : 8LL) * g.n + 40LL * nc,
-           gkd::launch_contract_bounds(nc, cptr, mrow, mvw, ub.p, toff.p, lists.p, desc.p, c.vw.p, lcnt.p,
-                                       scratch.p, st));
-  int32_t hc[4];
-  GK_TRY(fetch(ctx, st, {{hc, lcnt.p, sizeof hc}}));
+  const int32_t* cnt = m.ctl.p + gkd::kCtlInts;
+  GK_TRY(toff.alloc(P, nc));
+  GK_TRY(lists.alloc(P, int64_t(gkd::kRowClasses) * nc));
+  GK_TRY(desc.alloc(P, int64_t(gkd::kRowClasses) * nc));
   GK_TRY(tadj.alloc(P, g.nnz));
   GK_TRY(tw.alloc(P, g.nnz));
   GK_TRY(len.alloc(P, nc));
-  const int lanes[3] = {16, 32, 64};
+  GK_TRY(scratch.alloc(P, gkd::size_partials(nc)));
+  GK_TRY(c.xadj.alloc(P, int64_t(nc) + 1));
+  GK_STAGE(ctx, GK_ST_CONTRACT_AUX, (m.mvw.p ? 12LL : 8LL) * g.n + 28LL * nc,
+           gkd::launch_contract_bounds(nc, m.cptr.p, m.mrow.p, m.mvw.p, toff.p, lists.p, desc.p, len.p,
+                                       c.vw.p, m.ctl.p + gkd::kCtlInts, st));
   // GK_CONTRACT_WIDE=1 runs the row kernels that sort (id, weight) pairs,
   // which otherwise serve only coarse graphs of 2^26 - 1 vertices or more.
   const char* wide_env = std::getenv("GK_CONTRACT_WIDE");
   const bool wide = wide_env && wide_env[0] == '1';
-  auto row_classes = [&]() -> int {
-    for (int cls = 0; cls < 3; ++cls) {
-      const int32_t* rows = lists.p + int64_t(cls) * nc;
-      auto run = [&](const Tuner::Shape& x) {
-        return gkd::launch_contract_rows(g, x.lanes, x.block, rows, desc.p + int64_t(cls) * nc, hc[cls], nc,
-                                         mrow, cmap, toff.p, tadj.p, tw.p, len.p, wide, st, steal_of(ctx));
-      };
-      Tuner::Shape shape{lanes[cls], 256};
-      if (ctx->autotune && hc[cls] >= kTuneMinRows) {
-        // Block size per row class; the lanes of a class are fixed by its rows.
-        const uint64_t key = Tuner::key(1 + cls, g.n, g.nnz);
-        if (const Tuner::Shape* s = ctx->tuner.find(key)) {
-          shape = *s;
-        } else {
-          const int L = lanes[cls];
-          GK_TRY(ctx->tuner.tune(key, {{L, 256}, {L, 64}, {L, 128}, {L, 512}}, st, run, &shape));
-          continue;  // every candidate wrote the rows
+  int32_t words[1 + gkd::kRowCtlWords];  // entries, then the class counters
+  const int32_t* hc = words + 1;
+  if (nc <= gkd::kRowsAllMax && !wide && !ctx->autotune && !steal_of(ctx)) {
+    GK_STAGE(ctx, GK_ST_CONTRACT, 0,
+             gkd::launch_contract_rows_all(g, nc, cnt, lists.p, desc.p, m.mrow.p, cmap, toff.p, tadj.p, tw.p, len.p,
+                                           st));
+    GK_STAGE(ctx, GK_ST_CONTRACT_BIG, 0,
+             gkd::launch_contract_mid(g, nc, nc, cnt, lists.p, desc.p, m.mrow.p, cmap, toff.p, tadj.p, tw.p, len.p,
+                                      st));
+  } else {
+    std::vector<int32_t> h(gkd::kRowCtlInts);
+    GK_TRY(fetch(ctx, st, {{h.data(), cnt, sizeof(int32_t) * gkd::kRowCtlInts}}));
+    for (int i = 0; i < gkd::kRowCtlWords; ++i) words[1 + i] = h[i * gkd::kRowCtlStride];
+    const int lanes[3] = {16, 32, 64};
+    auto row_classes = [&]() -> int {
+      for (int cls = 0; cls < 3; ++cls) {
+        const int32_t* rows = lists.p + int64_t(cls) * nc;
+        auto run = [&](const Tuner::Shape& x) {
+          return gkd::launch_contract_rows(g, x.lanes, x.block, rows, desc.p + int64_t(cls) * nc, hc[cls], nc,
+                                           m.mrow.p, cmap, toff.p, tadj.p, tw.p, len.p, wide, st, steal_of(ctx));
+        };
+        Tuner::Shape shape{lanes[cls], 256};
+        if (ctx->autotune && hc[cls] >= kTuneMinRows) {
+          // Block size per row class; the lanes of a class are fixed by its rows.
+          const uint64_t key = Tuner::key(1 + cls, g.n, g.nnz);
+          if (const Tuner::Shape* s = ctx->tuner.find(key)) {
+            shape = *s;
+          } else {
+            const int L = lanes[cls];
+            GK_TRY(ctx->tuner.tune(key, {{L, 256}, {L, 64}, {L, 128}, {L, 512}}, st, run, &shape));
+            continue;  // every candidate wrote the rows
+          }
         }
+        GK_TRY(run(shape));
       }
-      GK_TRY(run(shape));
-    }
+      return GK_OK;
+    };
+    ctx->clock.begin(GK_ST_CONTRACT);
+    const int rc_rows = row_classes();
+    ctx->clock.end(GK_ST_CONTRACT);
+    if (rc_rows != GK_OK) return rc_rows;
+    count_stage(ctx, GK_ST_CONTRACT, 0);  // bytes added once the coarse entry count is known
+    if (hc[3] > 0)
+      GK_STAGE(ctx, GK_ST_CONTRACT_BIG, 0,
+               gkd::launch_contract_mid(g, nc, hc[3], cnt, lists.p, desc.p, m.mrow.p, cmap, toff.p, tadj.p, tw.p,
+                                        len.p, st));
+  }
+  // The entry count comes back with the class counters; rows for the global
+  // sort, if there are any, are merged then, and the lengths scanned again.
+  auto scan_lengths = [&]() -> int {
+    GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc,
+             gkd::launch_len_scan(nc, len.p, scratch.p, c.xadj.p, cnt, ctx->hctl, st));
+    GK_HIP(hipEventRecord(ctx->ev, st));
+    GK_HIP(hipEventSynchronize(ctx->ev));
+    std::memcpy(words, ctx->hctl, sizeof words);
     return GK_OK;
   };
-  ctx->clock.begin(GK_ST_CONTRACT);
-  const int rc_rows = row_classes();
-  ctx->clock.end(GK_ST_CONTRACT);
-  if (rc_rows != GK_OK) return rc_rows;
-  count_stage(ctx, GK_ST_CONTRACT, 0);  // bytes added once the coarse entry count is known
-  if (hc[3] > 0) {
-    const int32_t nbig = hc[3];
-    const int32_t* rows = lists.p + int64_t(3) * nc;
-    Buf<int32_t> boff, btot, bscr;
+  GK_TRY(scan_lengths());
+  if (hc[4] > 0) {
+    const int32_t nbig = hc[4], eb = hc[gkd::kRowBigEntries];
+    const int32_t* rows = lists.p + int64_t(4) * nc;
+    Buf<int32_t> boff, bscr;
     GK_TRY(boff.alloc(P, int64_t(nbig) + 1));
-    GK_TRY(btot.alloc(P, 1));
     GK_TRY(bscr.alloc(P, gkd::scan_scratch_ints(int64_t(nbig) + 1) + 64));
     GK_STAGE(ctx, GK_ST_CONTRACT_BIG, 16LL * nbig,
-             gkd::launch_big_offsets(rows, nbig, ub.p, boff.p, btot.p, bscr.p, st));
-    int32_t eb = 0;
-    GK_TRY(fetch(ctx, st, {{&eb, btot.p, sizeof eb}}));
+             gkd::launch_big_offsets(rows, len.p, nbig, boff.p, bscr.p, st));
     Buf<uint64_t> k1, k2;
     Buf<int32_t> v1, v2, sscr;
     GK_TRY(k1.alloc(P, eb));
@@ -304,19 +329,16 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
     bool alt = false;
     const int bpasses = (32 + bits_for(nbig - 1) + 7) / 8;
     GK_STAGE(ctx, GK_ST_CONTRACT_BIG, 24LL * eb + 36LL * eb * bpasses + 24LL * eb,
-             (gkd::launch_contract_big_gather(g, rows, nbig, boff.p, cptr, mrow, cmap, k1.p, v1.p, st) ||
+             (gkd::launch_contract_big_gather(g, rows, nbig, boff.p, m.cptr.p, m.mrow.p, cmap, k1.p, v1.p, st) ||
                       gkd::radix_sort_pairs<uint64_t>(k1.p, v1.p, k2.p, v2.p, eb, 0, 32 + bits_for(nbig - 1),
                                                       sscr.p, st, &alt) ||
                       gkd::launch_contract_big_merge(rows, nbig, boff.p, alt ? k2.p : k1.p, alt ? v2.p : v1.p,
                                                      toff.p, tadj.p, tw.p, len.p, st)
                   ? GK_ERR_HIP
                   : GK_OK));
+    GK_TRY(scan_lengths());
   }
-  GK_TRY(cnnzd.alloc(P, 1));
-  GK_TRY(c.xadj.alloc(P, int64_t(nc) + 1));
-  GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc, gkd::launch_len_scan(nc, len.p, c.xadj.p, cnnzd.p, scratch.p, st));
-  int32_t cnnz = 0;
-  GK_TRY(fetch(ctx, st, {{&cnnz, cnnzd.p, sizeof cnnz}}));
+  const int32_t cnnz = words[0];
   GK_TRY(c.adj.alloc(P, cnnz));
   GK_TRY(c.w.alloc(P, cnnz));
   // Row merge: member rows and the cmap gathers read once, merged rows
@@ -555,7 +577,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     Level c;
     GK_TRY(c.vw.alloc(P, nc));
     c.g.vw = c.vw.p;
-    GK_TRY(contract_stage(ctx, st, f.g, nc, cmap.p, mem.cptr.p, mem.mrow.p, mem.mvw.p, c));
+    GK_TRY(contract_stage(ctx, st, f.g, nc, cmap.p, mem, c));
     ls.sweeps = rounds;
     if (trace) {
       std::vector<int32_t> h;
@@ -1144,26 +1166,29 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   hipStream_t st = pick(ctx, stream);
   Pool& P = ctx->pool;
   const int32_t n = dg->n;
-  // Members of each coarse vertex in order of (cmap[v], v).
+  // Members of each coarse vertex, in any order (the rows are sorted).
   Members m;
   Groups gr;
+  Buf<int2> partial;
   GK_TRY(m.cptr.alloc(P, int64_t(n) + 1));
   GK_TRY(m.mrow.alloc(P, n));
-  const MemberOut out{nullptr, nullptr, m.cptr.p, m.mrow.p, nullptr};
-  int32_t words[gkd::kCtlInts];
+  GK_TRY(partial.alloc(P, gkd::size_partials(n)));
   int32_t nc2 = 0;
+  GK_TRY(gr.count(ctx, st, n, cmap));
   if (n > 0) {
-    GK_TRY(gr.count(ctx, st, n, cmap));
-    GK_TRY(count_members(ctx, st, n, cmap, nullptr, gr, dg->xadj, nullptr, INT32_MAX, out, words));
-    nc2 = words[0];
-    if (words[1]) GK_TRY(sort_members(ctx, st, n, cmap, nullptr, 1, dg->xadj, nullptr, INT32_MAX, out, &nc2));
+    GK_TRY(gkd::launch_size_scan(n, gr.size.p, INT32_MAX, partial.p, gr.comp.p, gr.ctl.p, ctx->hctl, st));
+    GK_HIP(hipEventRecord(ctx->ev, st));
+    GK_TRY(gkd::launch_member_place(n, cmap, gr.slot.p, gr.comp.p, dg->xadj, gr.ctl.p, m.cptr.p, m.mrow.p, st));
+    GK_HIP(hipEventSynchronize(ctx->ev));
+    nc2 = ctx->hctl[0];
   }
+  m.ctl = std::move(gr.ctl);
   // With G = INT32_MAX every label is one chunk, so chunks are the coarse
   // vertices in id order exactly when cmap is onto [0, nc).
   if (nc2 != nc) { gkh::set_error("cmap is not onto [0, nc)"); return GK_ERR_ARG; }
   Level c;
   DGraph g = dview(dg);
-  GK_TRY(contract_stage(ctx, st, g, nc, cmap, m.cptr.p, m.mrow.p, nullptr, c));
+  GK_TRY(contract_stage(ctx, st, g, nc, cmap, m, c));
   GK_HIP(hipMemcpyAsync(cxadj, c.g.xadj, sizeof(int32_t) * (nc + 1), hipMemcpyDeviceToDevice, st));
   if (c.g.nnz) {
     GK_HIP(hipMemcpyAsync(cadjncy, c.g.adj, sizeof(int32_t) * c.g.nnz, hipMemcpyDeviceToDevice, st));

@@ -305,7 +305,7 @@ int Engine::coarsen_step(bool* worked) {
   GK_TRY(gkd::launch_job_offsets(J, F.dv_off.p, mem.order.p, cmap->p, nc, C->dv_off.p, st_));
   Level c;
   GK_TRY(c.vw.alloc(P_, nc));
-  GK_TRY(contract_stage(ctx_, st_, g, nc, cmap->p, mem.cptr.p, mem.mrow.p, mem.mvw.p, c));
+  GK_TRY(contract_stage(ctx_, st_, g, nc, cmap->p, mem, c));
   GK_TRY(ce.alloc(P_, int64_t(J) + 1));
   GK_TRY(gkd::launch_job_eoffsets(J, C->dv_off.p, c.xadj.p, ce.p, st_));
   C->v_off.resize(J + 1);

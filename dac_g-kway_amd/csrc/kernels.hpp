@@ -62,6 +62,18 @@ constexpr int kWalkBits = 6;
 constexpr int kWalkMax = 1 << kWalkBits;
 constexpr int kCtlFlags = 2;
 constexpr int kCtlInts = kCtlFlags + kWalkBits + 1;
+// Row class counters of a contraction (zeroed by the caller, kRowCtlStride ints
+// apart): rows per class -- up to 16, 32, 64 entries, up to kMidMax (a workgroup
+// each), more (global sort) -- entries handed out in the temporary rows,
+// entries of the last class.
+constexpr int kRowClasses = 5;
+constexpr int kRowBigEntries = kRowClasses + 1;
+constexpr int kRowCtlWords = kRowClasses + 2;
+constexpr int kRowCtlStride = 32;
+constexpr int kRowCtlInts = kRowCtlWords * kRowCtlStride;
+constexpr int32_t kMidMax = 2048;
+// Coarse rows up to which all lane classes go in one launch.
+constexpr int32_t kRowsAllMax = 1 << 16;
 // Largest group whose members find their order by counting.
 constexpr int32_t kRankMax = 512;
 // Grouping by walking to the root pair: key of v's component, hops, and comp
@@ -91,6 +103,10 @@ int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, i
 int launch_members(int32_t n, const int32_t* label, const int32_t* stamp, const int32_t* slot, const int2* offc,
                    const int32_t* xadj, const int32_t* vw, int4* memb, int32_t G, const int32_t* ctl,
                    int32_t* order, int32_t* cmap, int32_t* cptr, int2* mrow, int32_t* mvw, hipStream_t st);
+// Rows of the members by group (any order inside a group) and the groups'
+// first places, for labels whose coarse ids are those of the size scan.
+int launch_member_place(int32_t n, const int32_t* label, const int32_t* slot, const int2* offc, const int32_t* xadj,
+                        const int32_t* ctl, int32_t* cptr, int2* mrow, hipStream_t st);
 // mrow and mvw (each may be null) of a given order.
 int launch_member_rows(int32_t n, const int32_t* order, const int32_t* xadj, const int32_t* vw, int2* mrow,
                        int32_t* mvw, hipStream_t st);
@@ -101,15 +117,24 @@ int launch_make_keys(int32_t n, const int32_t* label, const int32_t* dist, int s
 int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sbits, int32_t G, int32_t* gstart,
                    int32_t* flagscan, int32_t* cmap, int32_t* cptr, int32_t* nc_dev, int32_t* scratch,
                    hipStream_t st);
-// Contraction, phase 1: per coarse row the upper bound of its entries
-// (sum of member degrees), its class (16/32/64-lane or big), appended to
-// lists[cls * nc ..] with its member range in desc; the exclusive scan of the
-// bounds (toff, nc+1 entries).  lists and desc: 4 * nc entries; mrow[m] = (row
-// start, row length) of the member at place m.  With mvw (the members'
-// weights) also the coarse weights cvw.
-int launch_contract_bounds(int32_t nc, const int32_t* cptr, const int2* mrow, const int32_t* mvw, int32_t* ub,
-                           int32_t* toff, int32_t* lists, int2* desc, int32_t* cvw, int32_t* list_cnt,
-                           int32_t* scratch, hipStream_t st);
+// Contraction, phase 1: per coarse row the upper bound of its entries (sum of
+// member degrees), room for them in the temporary rows (toff), its class,
+// appended to lists[cls * nc ..] with its member range in desc.  lists and
+// desc: kRowClasses * nc entries; mrow[m] = (row start, row length) of the
+// member at place m.  Rows of the last two classes: their bound in len.  With mvw (the members' weights) also the coarse weights
+// cvw.  cnt: the row class counters.
+int launch_contract_bounds(int32_t nc, const int32_t* cptr, const int2* mrow, const int32_t* mvw, int32_t* toff,
+                           int32_t* lists, int2* desc, int32_t* len, int32_t* cvw, int32_t* cnt, hipStream_t st);
+// Phase 2 for the three lane classes in one launch (32-bit keys: nc below
+// 2^26 - 1), counts read on the device.
+int launch_contract_rows_all(const DGraph& g, int32_t nc, const int32_t* cnt, const int32_t* lists, const int2* desc,
+                             const int2* mrow, const int32_t* cmap, const int32_t* toff, int32_t* tadj, int32_t* tw,
+                             int32_t* len, hipStream_t st);
+// Phase 2 for rows of 65 to kMidMax entries (count read on the device; max_rows
+// bounds it).
+int launch_contract_mid(const DGraph& g, int32_t nc, int32_t max_rows, const int32_t* cnt, const int32_t* lists,
+                        const int2* desc, const int2* mrow, const int32_t* cmap, const int32_t* toff, int32_t* tadj,
+                        int32_t* tw, int32_t* len, hipStream_t st);
 // Phase 2 for the rows of one class (lanes in {16, 32, 64}); block size 64,
 // 128, 256 or 512 threads (launch shape only).  nc: coarse vertex count; the
 // sort packs the lane number beside the coarse id in 32 bits when nc allows,
@@ -131,12 +156,14 @@ int launch_contract_big_merge(const int32_t* rows, int32_t nrows, const int32_t*
 int launch_contract_copy(int32_t nc, const int32_t* toff, const int32_t* len, const int32_t* cxadj,
                          const int32_t* tadj, const int32_t* tw, int32_t* cadj, int32_t* cw,
                          hipStream_t st);
-// Big-row prefix (boff = exclusive scan of ub over the big rows).
-int launch_big_offsets(const int32_t* rows, int32_t nrows, const int32_t* ub, int32_t* boff,
-                       int32_t* total, int32_t* scratch, hipStream_t st);
-// cxadj = exclusive scan of len (nc + 1 entries), total into *cnnz.
-int launch_len_scan(int32_t nc, const int32_t* len, int32_t* cxadj, int32_t* cnnz,
-                    int32_t* scratch, hipStream_t st);
+// Big-row prefix (boff = exclusive scan of the big rows' bounds ub).
+int launch_big_offsets(const int32_t* rows, const int32_t* ub, int32_t nrows, int32_t* boff, int32_t* scratch,
+                       hipStream_t st);
+// cxadj = exclusive scan of len (nc + 1 entries); the entry count and the
+// kRowCtlWords class counters to host (pinned).  partial: size_partials(nc)
+// ints (at least one).
+int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt, int32_t* host,
+                    hipStream_t st);
 
 // ---- refinement (refine.hip)
 int launch_project(int32_t n, const int32_t* cmap, const int32_t* cpart, const int32_t* cbnd,

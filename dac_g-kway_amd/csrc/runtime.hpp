@@ -370,7 +370,8 @@ namespace gkrt {
 // Pinned bytes of a context: fetch() staging, then the control words.
 constexpr size_t kPinFetch = 4096;
 constexpr size_t kPinCtl = 256;
-static_assert(sizeof(int32_t) * gkd::kCtlInts <= kPinCtl, "control words fit");
+static_assert(sizeof(int32_t) * gkd::kCtlInts <= kPinCtl && sizeof(int32_t) * (1 + gkd::kRowCtlWords) <= kPinCtl,
+              "control words fit");
 }  // namespace gkrt
 
 struct gk_ctx {
@@ -555,9 +556,10 @@ struct Groups {
 };
 
 // Members by coarse id: first place of every coarse id, and in member order
-// the vertices, their rows (start, length) and their weights.
+// the vertices, their rows (start, length) and their weights; ctl: the
+// grouping's control words, then a contraction's row class counters (zero).
 struct Members {
-  Buf<int32_t> order, cptr, mvw;
+  Buf<int32_t> order, cptr, mvw, ctl;
   Buf<int2> mrow;
 };
 
@@ -573,7 +575,7 @@ struct MemberOut {
 int coarse_ids(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, const int32_t* cand, int32_t G, bool want_order,
                int32_t* cmap, Members& m, int32_t* nc, int32_t* rounds);
 int contract_stage(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, int32_t nc, const int32_t* cmap,
-                   const int32_t* cptr, const int2* mrow, const int32_t* mvw, Level& c);
+                   const Members& m, Level& c);
 // Lanes per vertex of the gain pass for this graph's average degree.
 int gain_lanes(const gkd::DGraph& g);
 // Candidate matching with the context's tuned launch shape (tuned on first
