@@ -403,18 +403,24 @@ int wide_round(gk_ctx* ctx, hipStream_t st, const RoundState& s) {
   return GK_OK;
 }
 
-// A launch of the round loop and the gain pass over what it left; pair: which
-// pair of counts and status words it uses.
+// A launch of the round loop; pair: which pair of counts and status words it
+// uses.
 int loop_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, int pair) {
   const int o = 2 * pair, e = 2 * (1 - pair);
   const gkd::RoundsArgs a{s.v_off,     s.M,        max_rounds, s.kk,         s.cap,        s.pw_off,  s.g.xadj,
                           s.g.adj,     s.g.w,      s.g.vw,     s.part,       s.bnd,        s.gain,    s.dest,
                           s.pw,        s.cut,      s.rounds,   s.moved,      s.cand,       s.upd,     s.wl,
                           s.hcnt + o,  s.hcnt + e, s.lastcnt,  s.status + o, s.status + e, s.thr,     s.paths,
-                          s.abytes,    s.order,    s.hist};
+                          s.abytes,    s.order,    s.hist,     s.nj == 1 ? ctx->hctl : nullptr};
   GK_STAGE(ctx, GK_ST_BALANCE, 0, gkd::launch_rounds(a, s.nj, s.lanes, st));
+  return GK_OK;
+}
+
+// The gain pass over what a launch of the round loop left; none is needed
+// after one in which every job converged.
+int loop_gains(gk_ctx* ctx, hipStream_t st, const RoundState& s, int pair) {
   GK_STAGE(ctx, GK_ST_GAIN, 0,
-           gkd::launch_gain_wl(s.g, s.kmax, s.lanes, s.wl, s.hcnt + o, s.heavy, s.part, s.upd, s.bnd, s.gain, s.dest,
+           gkd::launch_gain_wl(s.g, s.kmax, s.lanes, s.wl, s.hcnt + 2 * pair, s.heavy, s.part, s.upd, s.bnd, s.gain, s.dest,
                                s.work, s.wl_items, s.cand, st, steal_of(ctx)));
   return GK_OK;
 }
@@ -440,30 +446,40 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
   RoundGraph wide_graph, loop_graph;
   int pair = 1;  // the compaction before the rounds used pair 0
   int done = 0, wide_done = 0, per_check = kWideRounds;
+  // Jobs that go on, jobs left out, and with one job the ordering rounds so
+  // far, which its kernel writes to pinned memory: a wait instead of a copy.
+  const bool one = s.nj == 1;
+  auto status = [&](int p, int32_t* words) -> int {
+    if (!one) return fetch(ctx, st, {{words, s.status + 2 * p, 2 * sizeof(int32_t)}});
+    GK_HIP(hipEventRecord(ctx->ev, st));
+    GK_HIP(hipEventSynchronize(ctx->ev));
+    std::memcpy(words, ctx->hctl, 3 * sizeof(int32_t));
+    return GK_OK;
+  };
   while (max_rounds <= 0 || done < max_rounds) {
     if (loop) {
       const int left = max_rounds > 0 ? max_rounds - done : kLoopRounds;
-      int32_t words[2] = {0, 0}, made = 0;
+      int32_t words[3] = {0, 0, 0};
       if (graph && left >= kLoopRounds) {
         // both pairs, so that every replay begins with the same one
         if (!loop_graph.ready())
           GK_TRY(loop_graph.capture(ctx, st, [&]() -> int {
             GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, pair));
-            return loop_rounds(ctx, st, s, kLoopRounds / 2, 1 - pair);
+            GK_TRY(loop_gains(ctx, st, s, pair));
+            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, 1 - pair));
+            return loop_gains(ctx, st, s, 1 - pair);
           }));
         GK_TRY(loop_graph.replay(ctx, st));
-        GK_TRY(fetch(ctx, st, {{words, s.status + 2 * (1 - pair), sizeof words}}));
+        GK_TRY(status(1 - pair, words));
         done += kLoopRounds;
       } else {
         const int rounds = std::min(left, kLoopRounds);
         GK_TRY(loop_rounds(ctx, st, s, rounds, pair));
-        if (exact) {  // one job: its ordering rounds so far are the rounds done
-          GK_TRY(fetch(ctx, st, {{words, s.status + 2 * pair, sizeof words}, {&made, s.rounds, sizeof made}}));
-          done = made;
-        } else {
-          GK_TRY(fetch(ctx, st, {{words, s.status + 2 * pair, sizeof words}}));
-          done += rounds;
-        }
+        // Of several jobs some usually go on, and the wait is the longer part.
+        if (!one) GK_TRY(loop_gains(ctx, st, s, pair));
+        GK_TRY(status(pair, words));
+        if (one && words[0] != 0) GK_TRY(loop_gains(ctx, st, s, pair));
+        done = exact ? words[2] : done + rounds;  // exact: one job
         pair = 1 - pair;
       }
       if (words[0] == 0) break;
@@ -519,12 +535,18 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   ctx->clock.start((prm.flags & GK_FLAG_STAGE_TIME) != 0, st);
   struct Reset {
     gk_ctx* c;
+    hipStream_t st;
+    bool done = false;
     ~Reset() {
+      // An error may leave launches that read the staging memory.
+      if (!done) (void)hipStreamSynchronize(st);
+      c->dl.drained();
+      c->up.drained();
       c->cur = nullptr;
       c->clock.start(false, nullptr);
       gkrt::clear_launch_options(c);
     }
-  } reset{ctx};
+  } reset{ctx, st};
   GK_TRY(gkrt::set_launch_options(ctx, prm.flags));
 
   std::vector<Level> L;
@@ -542,21 +564,12 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     gkd::fill<int32_t>(L[0].vw.p, 1, n0, st);
     L[0].g.vw = L[0].vw.p;
   }
-  int64_t T = 0;
-  {
-    Buf<unsigned long long> tw;
-    GK_TRY(tw.alloc(P, 1));
-    GK_TRY(gkd::launch_sum(L[0].g.vw, n0, tw.p, st));
-    unsigned long long ht = 0;
-    GK_TRY(fetch(ctx, st, {{&ht, tw.p, sizeof ht}}));
-    T = static_cast<int64_t>(ht);
-  }
-  if (T >= (int64_t(1) << 31)) { gkh::set_error("total vertex weight >= 2^31"); return GK_ERR_LIMIT; }
-  const int64_t cap = gk_part_cap(T, k, prm.ubfactor);
+  // The total weight comes back with the coarsest graph.
+  Buf<unsigned long long> tw;
+  GK_TRY(tw.alloc(P, 1));
+  GK_TRY(gkd::launch_sum(L[0].g.vw, n0, tw.p, st));
   const int32_t floor_n = gk_coarsen_floor(n0, k, prm.coarsen_policy, prm.coarsen_to);
   const int32_t maxlv = prm.max_levels > 0 ? std::min(prm.max_levels, GK_MAX_LEVELS) : GK_MAX_LEVELS;
-  S.total_vwgt = T;
-  S.cap = cap;
 
   // ---------------------------------------------------------- coarsening
   while (static_cast<int32_t>(L.size()) < maxlv) {
@@ -596,35 +609,47 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     L.push_back(std::move(c));
   }
   const int32_t nl = static_cast<int32_t>(L.size());
-  GK_HIP(hipStreamSynchronize(st));
-  const auto t1 = clk::now();
 
   // ---------------------------------------------------------- initial partition
   Level& top = L.back();
   const int32_t nt = top.g.n;
-  // Largest row of every level refined later (it decides whether a level
-  // needs the heavy-row gain kernel and the long-row selection pass): read
-  // back with the initial partition's upload, not one host sync per level.
+  // The largest row of every level refined later decides whether a level
+  // needs the heavy-row gain kernel, which serves only large k.
+  const bool heavy_k = gkd::gain_heavy_separate(k) && nl > 1;
   Buf<int32_t> dmaxall;
-  std::vector<int32_t> hmaxdeg(nl, 0);
-  GK_TRY(dmaxall.alloc(P, nl));
-  for (int32_t l = 0; l + 1 < nl; ++l) GK_TRY(gkd::launch_max_deg(L[l].g, dmaxall.p + l, st));
-  // The coarsest graph comes back through the context's pinned staging in
-  // one piece (four copies, one host sync) and is partitioned from there.
-  const int64_t tn = top.g.nnz;
-  void* hdn = nullptr;
-  GK_TRY(ctx->dl.get(st, sizeof(int32_t) * (2 * size_t(nt) + 1 + 2 * size_t(tn)), &hdn));
-  int32_t* hx = static_cast<int32_t*>(hdn);
-  int32_t* ha = hx + nt + 1;
-  int32_t* hw = ha + tn;
-  int32_t* hv = hw + tn;
-  GK_HIP(hipMemcpyAsync(hx, top.g.xadj, sizeof(int32_t) * (size_t(nt) + 1), hipMemcpyDeviceToHost, st));
-  if (tn > 0) {
-    GK_HIP(hipMemcpyAsync(ha, top.g.adj, sizeof(int32_t) * size_t(tn), hipMemcpyDeviceToHost, st));
-    GK_HIP(hipMemcpyAsync(hw, top.g.w, sizeof(int32_t) * size_t(tn), hipMemcpyDeviceToHost, st));
+  if (heavy_k) {
+    GK_TRY(dmaxall.alloc(P, nl));
+    for (int32_t l = 0; l + 1 < nl; ++l) GK_TRY(gkd::launch_max_deg(L[l].g, dmaxall.p + l, st));
   }
-  if (nt > 0) GK_HIP(hipMemcpyAsync(hv, top.g.vw, sizeof(int32_t) * size_t(nt), hipMemcpyDeviceToHost, st));
+  // The coarsest graph comes back through the context's pinned staging in one
+  // launch, which writes there, and is partitioned from there.
+  const int64_t tn = top.g.nnz;
+  auto up4 = [](size_t ints) { return (ints + 3) & ~size_t(3); };  // 16-byte places
+  void* hdn = nullptr;
+  GK_TRY(ctx->dl.get(st, sizeof(int32_t) * (4 + up4(nl) + up4(size_t(nt) + 1) + 2 * up4(tn) + up4(nt)), &hdn));
+  unsigned long long* ht = static_cast<unsigned long long*>(hdn);
+  int32_t* hmaxdeg = reinterpret_cast<int32_t*>(ht + 2);
+  int32_t* hx = hmaxdeg + up4(nl);
+  int32_t* ha = hx + up4(size_t(nt) + 1);
+  int32_t* hw = ha + up4(tn);
+  int32_t* hv = hw + up4(tn);
+  std::memset(hmaxdeg, 0, sizeof(int32_t) * size_t(nl));
+  gkd::Copies dn;
+  dn.add(ht, tw.p, sizeof *ht);
+  if (heavy_k) dn.add(hmaxdeg, dmaxall.p, sizeof(int32_t) * size_t(nl - 1));
+  dn.add(hx, top.g.xadj, sizeof(int32_t) * (size_t(nt) + 1));
+  dn.add(ha, top.g.adj, sizeof(int32_t) * size_t(tn));
+  dn.add(hw, top.g.w, sizeof(int32_t) * size_t(tn));
+  dn.add(hv, top.g.vw, sizeof(int32_t) * size_t(nt));
+  GK_TRY(gkd::launch_copies(dn, st));
   GK_HIP(hipStreamSynchronize(st));
+  const std::vector<int32_t> maxdeg_of(hmaxdeg, hmaxdeg + nl);
+  const auto t1 = clk::now();
+  const int64_t T = static_cast<int64_t>(*ht);
+  if (T >= (int64_t(1) << 31)) { gkh::set_error("total vertex weight >= 2^31"); return GK_ERR_LIMIT; }
+  const int64_t cap = gk_part_cap(T, k, prm.ubfactor);
+  S.total_vwgt = T;
+  S.cap = cap;
   gk_csr hc;
   hc.n = nt;
   hc.nnz = tn;
@@ -632,24 +657,46 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   hc.adjncy = ha;
   hc.adjwgt = hw;
   hc.vwgt = hv;
-  // Initial part, boundary flags, part weights and cut go up through pinned
-  // staging as well.
+  // The initial part goes up through pinned staging, and with it the words
+  // of the refinement's state (64-bit, then 32-bit ones): per level cut after
+  // the level, moves and algorithmic bytes, rounds, worklist counts and round
+  // loop status; what the kernels take as one job's tables.
+  const int nl64 = 3 * nl + 4, nl32 = 11 * nl + 7;
+  const size_t state_bytes = sizeof(long long) * nl64 + sizeof(int32_t) * up4(nl32);
+  struct State {
+    long long *cut, *moved, *abytes, *paths, *cap;
+    int32_t *rounds, *hcnt, *status, *voff, *pwoff, *kk, *thr, *lastcnt, *active;
+  };
+  auto state_at = [&](void* base) {
+    State s;
+    s.cut = static_cast<long long*>(base);
+    s.moved = s.cut + nl;
+    s.abytes = s.moved + nl;
+    s.paths = s.abytes + nl;
+    s.cap = s.paths + 3;
+    s.rounds = reinterpret_cast<int32_t*>(s.cut + nl64);
+    s.hcnt = s.rounds + nl;      // 4 per level: two pairs of (worklist, heavy rows)
+    s.status = s.hcnt + 4 * nl;  // 4 per level
+    s.voff = s.status + 4 * nl;  // 2 per level
+    s.pwoff = s.voff + 2 * nl;
+    s.kk = s.pwoff + 2;
+    s.thr = s.kk + 1;
+    s.lastcnt = s.thr + 1;
+    s.active = s.lastcnt + 1;
+    return s;
+  };
   void* hup = nullptr;
-  GK_TRY(ctx->up.get(st, sizeof(int32_t) * (2 * size_t(nt) + size_t(k)) + sizeof(long long), &hup));
-  long long* hcut0 = static_cast<long long*>(hup);
-  int32_t* hp = reinterpret_cast<int32_t*>(hcut0 + 1);
-  int32_t* hb = hp + nt;
-  int32_t* hpw = hb + nt;
+  GK_TRY(ctx->up.get(st, state_bytes + 16 + sizeof(int32_t) * size_t(nt), &hup));
+  int32_t* hp = reinterpret_cast<int32_t*>(static_cast<char*>(hup) + ((state_bytes + 15) & ~size_t(15)));
   int64_t cut0 = 0;
   GK_TRY(gk_initpart(&hc, k, cap, prm.seed, prm.initpart_threads, hp, &cut0));
-  std::fill(hb, hb + nt, 0);
-  std::fill(hpw, hpw + k, 0);
-  for (int32_t v = 0; v < nt; ++v) {
-    hpw[hp[v]] += hv[v];
-    for (int32_t j = hx[v]; j < hx[v + 1]; ++j)
-      if (hp[ha[j]] != hp[v]) { hb[v] = 1; break; }
-  }
-  *hcut0 = cut0;
+  std::memset(hup, 0, state_bytes);
+  const State hs = state_at(hup);
+  hs.cut[nl - 1] = cut0;
+  *hs.cap = cap;
+  for (int32_t l = 0; l < nl; ++l) hs.voff[2 * l + 1] = L[l].g.n;
+  hs.pwoff[1] = k;
+  *hs.kk = k;
   S.init_cut = cut0;
   Buf<int32_t> partA, partB, bndA, bndB, pw;
   GK_TRY(partA.alloc(P, n0));
@@ -657,20 +704,31 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   GK_TRY(bndA.alloc(P, n0));
   GK_TRY(bndB.alloc(P, n0));
   GK_TRY(pw.alloc(P, k));
-  Buf<long long> dcut;
-  GK_TRY(dcut.alloc(P, 1));
-  if (nt > 0) {
-    GK_HIP(hipMemcpyAsync(partA.p, hp, sizeof(int32_t) * size_t(nt), hipMemcpyHostToDevice, st));
-    GK_HIP(hipMemcpyAsync(bndA.p, hb, sizeof(int32_t) * size_t(nt), hipMemcpyHostToDevice, st));
+  // Gain statistics: a (vertices, entries) pair per block of the gain launches
+  // (grids of at most kGainSlots blocks), and the selection kernels'
+  // algorithmic bytes, likewise per block slot; summed at the end.
+  constexpr int kGainSlots = gkd::kGainMaxBlocks;
+  constexpr int kWork = 2 * kGainSlots + gkd::kSelectByteSlots;
+  const int64_t nwords0 = (int64_t(n0) + 63) / 64;
+  Buf<char> dstate;
+  Buf<unsigned long long> work;
+  Buf<uint64_t> selbits;
+  GK_TRY(dstate.alloc(P, int64_t(state_bytes)));
+  const State ds = state_at(dstate.p);
+  gkd::Copies upc;
+  upc.add(dstate.p, hup, state_bytes);
+  upc.add(partA.p, hp, sizeof(int32_t) * size_t(nt));
+  if (nl > 1) {
+    GK_TRY(work.alloc(P, kWork));
+    GK_TRY(selbits.alloc(P, nwords0 + 1));
+    upc.add(pw.p, nullptr, sizeof(int32_t) * size_t(k));
+    upc.add(work.p, nullptr, sizeof(unsigned long long) * kWork);
+    upc.add(selbits.p, nullptr, sizeof(uint64_t) * size_t(nwords0 + 1));
   }
-  GK_HIP(hipMemcpyAsync(pw.p, hpw, sizeof(int32_t) * size_t(k), hipMemcpyHostToDevice, st));
-  GK_HIP(hipMemcpyAsync(dcut.p, hcut0, sizeof(long long), hipMemcpyHostToDevice, st));
-  GK_TRY(fetch(ctx, st, {{hmaxdeg.data(), dmaxall.p, sizeof(int32_t) * size_t(nl)}}));
-  const uint64_t hpart_top = trace ? fnv_host(std::vector<int32_t>(hp, hp + nt)) : 0;
-  ctx->dl.drained();  // the stream is synchronised: both staging arenas are free again
-  ctx->up.drained();
+  GK_TRY(gkd::launch_copies(upc, st));
+  if (nl > 1) GK_TRY(gkd::launch_part_state(top.g, k, partA.p, bndA.p, pw.p, st));
   S.levels[nl - 1].cut_after = cut0;
-  if (trace) S.levels[nl - 1].h_part = hpart_top;
+  if (trace) S.levels[nl - 1].h_part = fnv_host(std::vector<int32_t>(hp, hp + nt));
   const auto t2 = clk::now();
 
   // ---------------------------------------------------------- uncoarsening
@@ -681,23 +739,9 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   int32_t* oth_bnd = bndB.p;
   if (nl > 1) {
     const int32_t M = prm.max_moves;
-    Buf<int32_t> xlist, dthr, wpos, sscr, status;
-    Buf<int32_t> gain, dest, upd, heavy, hcnt, wl, list, active, drounds, lastcnt, dvoff, dpw_off, dkk;
-    Buf<long long> dcap, dmoved, dpaths, dabytes;
-    Buf<uint64_t> cand, movable, selbits, defbits;
+    Buf<int32_t> xlist, wpos, sscr, gain, dest, upd, heavy, wl, list;
+    Buf<uint64_t> cand, movable, defbits;
     Buf<uint32_t> hkey;
-    Buf<unsigned long long> work;
-    GK_TRY(dpaths.alloc(P, 3));
-    gkd::fill<long long>(dpaths.p, 0, 3, st);
-    // gain statistics: a (vertices, entries) pair per block of the gain
-    // launches (grids of at most kGainSlots blocks), summed at the end
-    constexpr int kGainSlots = gkd::kGainMaxBlocks;
-    GK_TRY(work.alloc(P, 2 * kGainSlots));
-    gkd::fill<unsigned long long>(work.p, 0ull, 2 * kGainSlots, st);
-    // the selection kernels' algorithmic bytes, likewise per block slot
-    Buf<unsigned long long> selbytes;
-    GK_TRY(selbytes.alloc(P, gkd::kSelectByteSlots));
-    gkd::fill<unsigned long long>(selbytes.p, 0ull, gkd::kSelectByteSlots, st);
     GK_TRY(gain.alloc(P, n0));
     GK_TRY(dest.alloc(P, n0));
     GK_TRY(upd.alloc(P, n0));
@@ -705,64 +749,36 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     GK_TRY(wl.alloc(P, n0));
     GK_TRY(list.alloc(P, n0));
     GK_TRY(hkey.alloc(P, n0));
-    GK_TRY(cand.alloc(P, (int64_t(n0) + 63) / 64 + 1));
-    const int64_t nwords0 = (int64_t(n0) + 63) / 64;
+    GK_TRY(cand.alloc(P, nwords0 + 1));
     GK_TRY(movable.alloc(P, nwords0 + 1));
-    GK_TRY(selbits.alloc(P, nwords0 + 1));
     GK_TRY(defbits.alloc(P, nwords0 + 1));
     GK_TRY(wpos.alloc(P, nwords0 + 1));
     GK_TRY(sscr.alloc(P, gkd::select_scratch_ints(n0)));
     GK_TRY(xlist.alloc(P, n0));
-    GK_TRY(dthr.alloc(P, 1));
-    GK_TRY(hcnt.alloc(P, 4));  // two pairs: [0] gain worklist count, [1] heavy-row count
-    GK_TRY(status.alloc(P, 4));
-    GK_TRY(active.alloc(P, 1));
-    // Per-level rounds, moves and cut after the level, read back once at the end.
-    Buf<long long> dcutlv;
-    GK_TRY(drounds.alloc(P, nl));
-    GK_TRY(lastcnt.alloc(P, 1));
-    GK_TRY(dmoved.alloc(P, nl));
-    GK_TRY(dabytes.alloc(P, nl));
-    GK_TRY(dcutlv.alloc(P, nl));
-    GK_TRY(dvoff.alloc(P, 2));
-    GK_TRY(dpw_off.alloc(P, 2));
-    GK_TRY(dkk.alloc(P, 1));
-    GK_TRY(dcap.alloc(P, 1));
-    gkd::fill<uint64_t>(selbits.p, 0ull, nwords0 + 1, st);
-    const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, selbytes.p};
-    gkd::fill<int32_t>(dvoff.p, 0, 1, st);
-    gkd::fill<int32_t>(dpw_off.p, 0, 1, st);
-    gkd::fill<int32_t>(dpw_off.p + 1, k, 1, st);
-    gkd::fill<int32_t>(dkk.p, k, 1, st);
-    gkd::fill<long long>(dcap.p, static_cast<long long>(cap), 1, st);
+    const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, work.p + 2 * kGainSlots};
     for (int32_t l = nl - 2; l >= 0; --l) {
       Level& f = L[l];
       const DGraph& g = f.g;
       gk_level_stats& ls = S.levels[l];
+      int32_t* hcnt = ds.hcnt + 4 * l;
+      // The projected boundary becomes the first gain worklist; every gain is
+      // 0, so there is no candidate yet.
       GK_STAGE(ctx, GK_ST_PROJECT, 32LL * g.n,
-               gkd::launch_project(g.n, f.cmap.p, cur_part, cur_bnd, oth_part, oth_bnd, gain.p, dest.p,
-                                   upd.p, st));
+               gkd::launch_level_start(g.n, f.cmap.p, cur_part, cur_bnd, oth_part, oth_bnd, gain.p, dest.p, upd.p,
+                                       cand.p, wl.p, hcnt, ds.cut + l + 1, ds.cut + l, ds.thr, ds.lastcnt, st));
       std::swap(cur_part, oth_part);
       std::swap(cur_bnd, oth_bnd);
       const int lanes = gain_lanes(g);
       // Rows longer than the lane count: the gain pass takes them itself for
       // k <= kGainInlineK, else they go to the heavy-row kernel, whose
       // launches are skipped when there are none.
-      const int32_t maxdeg = hmaxdeg[l];
-      const bool heavy_rows = maxdeg > lanes && gkd::gain_heavy_separate(k);
-      // After projection every gain is 0: no candidate yet.
-      gkd::fill<uint64_t>(cand.p, 0ull, (int64_t(g.n) + 63) / 64 + 1, st);
-      gkd::fill<int32_t>(dvoff.p + 1, g.n, 1, st);
-      GK_TRY(gkd::launch_rounds_init(1, lastcnt.p, dthr.p, drounds.p + l, dmoved.p + l, dabytes.p + l, hcnt.p, status.p,
-                                     st));
-      // The projected boundary becomes the first gain worklist.
-      GK_STAGE(ctx, GK_ST_PROJECT, 4LL * g.n, gkd::launch_compact(g.n, upd.p, wl.p, hcnt.p, st));
+      const bool heavy_rows = heavy_k && maxdeg_of[l] > lanes;
       GK_STAGE(ctx, GK_ST_GAIN, 0,
-               gkd::launch_gain_wl(g, k, lanes, wl.p, hcnt.p, heavy.p, cur_part, upd.p, cur_bnd, gain.p, dest.p,
+               gkd::launch_gain_wl(g, k, lanes, wl.p, hcnt, heavy.p, cur_part, upd.p, cur_bnd, gain.p, dest.p,
                                    work.p, g.n, cand.p, st, steal_of(ctx)));
       if (heavy_rows)
         GK_STAGE(ctx, GK_ST_GAIN_HEAVY, 0,
-                 gkd::launch_gain_heavy(g, k, heavy.p, hcnt.p, cur_part, upd.p, cur_bnd, gain.p, dest.p, work.p,
+                 gkd::launch_gain_heavy(g, k, heavy.p, hcnt, cur_part, upd.p, cur_bnd, gain.p, dest.p, work.p,
                                         cand.p, st));
       // A round updates at most M movers and their neighbours.
       const int64_t avg_deg = g.n > 0 ? (int64_t(g.nnz) + g.n - 1) / g.n : 0;
@@ -774,72 +790,41 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
       rs.lanes = lanes;
       rs.heavy_rows = heavy_rows;
       rs.wl_items = wl_items;
-      rs.v_off = dvoff.p;
-      rs.kk = dkk.p;
-      rs.pw_off = dpw_off.p;
-      rs.cap = dcap.p;
+      rs.v_off = ds.voff + 2 * l;
+      rs.kk = ds.kk;
+      rs.pw_off = ds.pwoff;
+      rs.cap = ds.cap;
       rs.part = cur_part;
       rs.bnd = cur_bnd;
       rs.gain = gain.p;
       rs.dest = dest.p;
       rs.pw = pw.p;
       rs.upd = upd.p;
-      rs.cut = dcut.p;
-      rs.moved = dmoved.p + l;
-      rs.paths = dpaths.p;
-      rs.abytes = dabytes.p + l;
-      rs.rounds = drounds.p + l;
-      rs.lastcnt = lastcnt.p;
-      rs.thr = dthr.p;
-      rs.active = active.p;
+      rs.cut = ds.cut + l;
+      rs.moved = ds.moved + l;
+      rs.paths = ds.paths;
+      rs.abytes = ds.abytes + l;
+      rs.rounds = ds.rounds + l;
+      rs.lastcnt = ds.lastcnt;
+      rs.thr = ds.thr;
+      rs.active = ds.active;
       rs.cand = cand.p;
       rs.sb = sb;
       rs.xlist = xlist.p;
       rs.wl = wl.p;
-      rs.hcnt = hcnt.p;
+      rs.hcnt = hcnt;
       rs.heavy = heavy.p;
-      rs.status = status.p;
+      rs.status = ds.status + 4 * l;
       rs.hkey = hkey.p;
       rs.work = work.p;
       GK_TRY(refine_rounds(ctx, st, rs, 0, false, (prm.flags & GK_FLAG_GRAPH_ROUNDS) != 0, nullptr));
-      GK_HIP(hipMemcpyAsync(dcutlv.p + l, dcut.p, sizeof(long long), hipMemcpyDeviceToDevice, st));
       if (trace) {
         std::vector<int32_t> h;
         GK_TRY(to_host(st, h, cur_part, g.n));
         ls.h_part = fnv_host(h);
       }
     }
-    std::vector<long long> hcutlv(nl), hmovedlv(nl), habytes(nl);
-    std::vector<int32_t> hroundslv(nl);
-    long long hpaths[3] = {0, 0, 0};
-    GK_TRY(fetch(ctx, st, {{hcutlv.data(), dcutlv.p, sizeof(long long) * size_t(nl - 1)},
-                           {hmovedlv.data(), dmoved.p, sizeof(long long) * size_t(nl - 1)},
-                           {habytes.data(), dabytes.p, sizeof(long long) * size_t(nl - 1)},
-                           {hroundslv.data(), drounds.p, sizeof(int32_t) * size_t(nl - 1)},
-                           {hpaths, dpaths.p, sizeof hpaths}}));
-    for (int i = 0; i < 3; ++i) S.round_paths[i] = hpaths[i];
-    for (int32_t l = 0; l + 1 < nl; ++l) {
-      gk_level_stats& ls = S.levels[l];
-      // The round kernel's algorithmic bytes, counted on the device.
-      S.stage_bytes[GK_ST_BALANCE] += habytes[l];
-      ls.rounds = hroundslv[l];
-      ls.moves = hmovedlv[l];
-      ls.cut_after = hcutlv[l];
-    }
-    // Data-dependent bytes of the gain passes from the device work counters.
-    std::vector<unsigned long long> wk;
-    GK_TRY(to_host(st, wk, work.p, 2 * kGainSlots));
-    unsigned long long wv = 0, we = 0;
-    for (int i = 0; i < kGainSlots; ++i) {
-      wv += wk[2 * i];
-      we += wk[2 * i + 1];
-    }
-    S.stage_bytes[GK_ST_GAIN] += int64_t(28 * wv + 12 * we);
-    std::vector<unsigned long long> sbk;
-    GK_TRY(to_host(st, sbk, selbytes.p, gkd::kSelectByteSlots));
-    for (unsigned long long b : sbk) S.stage_bytes[GK_ST_SELECT] += int64_t(b);
   }
-  GK_HIP(hipStreamSynchronize(st));
   const auto t3 = clk::now();
 
   // ---------------------------------------------------------- final metrics
@@ -850,21 +835,49 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     GK_TRY(cscr.alloc(P, gkd::cut_scratch(L[0].g.n, k)));
     GK_STAGE(ctx, GK_ST_CUT, 16LL * n0 + 12LL * L[0].g.nnz,
              gkd::launch_cut(L[0].g, k, cur_part, cut.p, pw64.p, cscr.p, st));
-    std::vector<unsigned long long> hpw64;
-    unsigned long long hcut = 0;
-    long long tracked = 0;
-    GK_TRY(fetch(ctx, st, {{&hcut, cut.p, sizeof hcut}, {&tracked, dcut.p, sizeof tracked}}));
-    GK_TRY(to_host(st, hpw64, pw64.p, k));
-    S.cut = static_cast<int64_t>(hcut);
-    S.cut_tracked = tracked;
+    // The partition, the metrics and the levels' figures, in one launch.
+    void* hend = nullptr;
+    GK_TRY(ctx->dl.get(st, state_bytes + 32 + sizeof(unsigned long long) * (size_t(k) + 2 + kWork), &hend));
+    unsigned long long* hcut = static_cast<unsigned long long*>(hend);
+    unsigned long long* hpw64 = hcut + 2;
+    unsigned long long* hwork = hpw64 + ((size_t(k) + 1) & ~size_t(1));
+    void* hstate = hwork + kWork;
+    gkd::Copies fin;
+    if (dpart_out != cur_part) fin.add(dpart_out, cur_part, sizeof(int32_t) * size_t(n0));
+    fin.add(hcut, cut.p, sizeof *hcut);
+    fin.add(hpw64, pw64.p, sizeof *hpw64 * size_t(k));
+    fin.add(hstate, dstate.p, state_bytes);
+    if (nl > 1) fin.add(hwork, work.p, sizeof *hwork * size_t(kWork));
+    GK_TRY(gkd::launch_copies(fin, st));
+    GK_HIP(hipStreamSynchronize(st));
+    const State fs = state_at(hstate);
+    S.cut = static_cast<int64_t>(*hcut);
+    S.cut_tracked = fs.cut[0];
+    for (int i = 0; i < 3; ++i) S.round_paths[i] = fs.paths[i];
+    for (int32_t l = 0; l + 1 < nl; ++l) {
+      gk_level_stats& ls = S.levels[l];
+      // The round kernel's algorithmic bytes, counted on the device.
+      S.stage_bytes[GK_ST_BALANCE] += fs.abytes[l];
+      ls.rounds = fs.rounds[l];
+      ls.moves = fs.moved[l];
+      ls.cut_after = fs.cut[l];
+    }
+    if (nl > 1) {
+      // Data-dependent bytes of the gain passes and the selection.
+      unsigned long long wv = 0, we = 0;
+      for (int i = 0; i < kGainSlots; ++i) {
+        wv += hwork[2 * i];
+        we += hwork[2 * i + 1];
+      }
+      S.stage_bytes[GK_ST_GAIN] += int64_t(28 * wv + 12 * we);
+      for (int i = 0; i < gkd::kSelectByteSlots; ++i) S.stage_bytes[GK_ST_SELECT] += int64_t(hwork[2 * kGainSlots + i]);
+    }
+    reset.done = true;
     unsigned long long mx = 0;
-    for (auto x : hpw64) mx = std::max(mx, x);
+    for (int32_t q = 0; q < k; ++q) mx = std::max(mx, hpw64[q]);
     S.max_part_wgt = static_cast<int64_t>(mx);
     S.imbalance = T > 0 ? double(mx) * k / double(T) : 1.0;
   }
-  if (dpart_out != cur_part)
-    GK_HIP(hipMemcpyAsync(dpart_out, cur_part, sizeof(int32_t) * n0, hipMemcpyDeviceToDevice, st));
-  GK_HIP(hipStreamSynchronize(st));
   S.nlevels = nl;
   S.coarsest_n = nt;
   for (int32_t l = 0; l < nl; ++l) {

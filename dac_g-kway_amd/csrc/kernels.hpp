@@ -38,6 +38,23 @@ struct DGraph {
   const int32_t* vw = nullptr;
 };
 
+// Copies of 32-bit words made by one launch, src null: zeros.  Either side may
+// be pinned host memory.  Distinct ranges.
+struct Copies {
+  static constexpr int kMax = 16;
+  int n = 0;
+  int32_t* dst[kMax];
+  const int32_t* src[kMax];
+  int64_t len[kMax];
+  void add(void* d, const void* s, size_t bytes) {
+    if (!bytes) return;
+    dst[n] = static_cast<int32_t*>(d);
+    src[n] = static_cast<const int32_t*>(s);
+    len[n++] = int64_t(bytes / sizeof(int32_t));
+  }
+};
+int launch_copies(const Copies& c, hipStream_t st);
+
 // Lanes per vertex for row-parallel kernels, from the average degree.
 int lanes_for_degree(double avg_deg);
 
@@ -171,6 +188,15 @@ int launch_project(int32_t n, const int32_t* cmap, const int32_t* cpart, const i
                    hipStream_t st);
 // Worklist of the v with flags[v] != 0 appended at list[*cnt...].
 int launch_compact(int32_t n, const int32_t* flags, int32_t* list, int32_t* cnt, hipStream_t st);
+// launch_project, launch_compact of the projected boundary (wl, cnt: zero
+// before), and the rest of a level's start: no candidates, *cut = *cut_in, the
+// first round's threshold and count.
+int launch_level_start(int32_t n, const int32_t* cmap, const int32_t* cpart, const int32_t* cbnd, int32_t* part,
+                       int32_t* bnd, int32_t* gain, int32_t* dest, int32_t* upd, uint64_t* cand, int32_t* wl,
+                       int32_t* cnt, const long long* cut_in, long long* cut, int32_t* thr, int32_t* lastcnt,
+                       hipStream_t st);
+// Boundary flags and part weights (pw: k words, zero before) of a partition.
+int launch_part_state(const DGraph& g, int32_t k, const int32_t* part, int32_t* bnd, int32_t* pw, hipStream_t st);
 // Gain pass over the worklist wl[0..wlc[0]); rows longer than `lanes` go
 // through heavy[] (count wlc[1]) to the LDS-histogram kernel.  Clears upd of
 // every processed vertex.  work (may be null) accumulates [0] vertices

@@ -88,6 +88,152 @@ int launch_compact(int32_t n, const int32_t* flags, int32_t* list, int32_t* cnt,
   return hip_status();
 }
 
+// Start of a level's rounds in one launch instead of six (projection, cleared
+// candidates, state words, compaction of the boundary, cut): on small levels
+// each was 2 us of launch and gap.  Every vertex is read once, so the boundary
+// is compacted where it is projected; four vertices a thread keep the gathers
+// of cpart and cbnd in flight together.
+constexpr int kStartIPT = 4;
+constexpr int kStartTile = 256 * kStartIPT;
+
+__global__ void __launch_bounds__(256) k_level_start(int32_t n, const int32_t* __restrict__ cmap,
+                                                     const int32_t* __restrict__ cpart,
+                                                     const int32_t* __restrict__ cbnd, int32_t* __restrict__ part,
+                                                     int32_t* __restrict__ bnd, int32_t* __restrict__ gain,
+                                                     int32_t* __restrict__ dest, int32_t* __restrict__ upd,
+                                                     uint64_t* __restrict__ cand, int32_t* __restrict__ wl,
+                                                     int32_t* __restrict__ cnt,
+                                                     const long long* __restrict__ cut_in,
+                                                     long long* __restrict__ cut, int32_t* __restrict__ thr,
+                                                     int32_t* __restrict__ lastcnt) {
+  __shared__ int wsum[4];
+  __shared__ int base_s;
+  const int wave = threadIdx.x >> 6;
+  const int64_t wbase = int64_t(xcd_block()) * kStartTile + int64_t(wave) * 64 * kStartIPT;
+  int32_t c[kStartIPT], p[kStartIPT], b[kStartIPT];
+#pragma unroll
+  for (int j = 0; j < kStartIPT; ++j) {
+    const int64_t v = wbase + j * 64 + lane_id();
+    c[j] = v < n ? cmap[v] : -1;
+  }
+#pragma unroll
+  for (int j = 0; j < kStartIPT; ++j) {
+    p[j] = c[j] >= 0 ? cpart[c[j]] : 0;
+    b[j] = c[j] >= 0 && cbnd[c[j]] ? 1 : 0;
+  }
+  uint64_t m[kStartIPT];
+  int tot = 0;
+#pragma unroll
+  for (int j = 0; j < kStartIPT; ++j) {
+    const int64_t v = wbase + j * 64 + lane_id();
+    m[j] = ballot(b[j] != 0);
+    tot += popc64(m[j]);
+    if (v < n) {
+      part[v] = p[j];
+      bnd[v] = b[j];
+      gain[v] = 0;
+      dest[v] = p[j];
+      upd[v] = b[j];
+      if (lane_id() == 0) cand[v >> 6] = 0;
+    }
+  }
+  if (lane_id() == 0) wsum[wave] = tot;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int t = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    base_s = t ? atomicAdd(cnt, t) : 0;
+    if (blockIdx.x == 0) {
+      cand[(int64_t(n) + 63) / 64] = 0;
+      *cut = *cut_in;
+      *thr = 1;
+      *lastcnt = 1;
+    }
+  }
+  __syncthreads();
+  int off = base_s;
+  for (int w = 0; w < wave; ++w) off += wsum[w];
+  const uint64_t lt = lanemask_lt();
+#pragma unroll
+  for (int j = 0; j < kStartIPT; ++j) {
+    if (b[j]) wl[off + popc64(m[j] & lt)] = int32_t(wbase + j * 64 + lane_id());
+    off += popc64(m[j]);
+  }
+}
+
+int launch_level_start(int32_t n, const int32_t* cmap, const int32_t* cpart, const int32_t* cbnd, int32_t* part,
+                       int32_t* bnd, int32_t* gain, int32_t* dest, int32_t* upd, uint64_t* cand, int32_t* wl,
+                       int32_t* cnt, const long long* cut_in, long long* cut, int32_t* thr, int32_t* lastcnt,
+                       hipStream_t st) {
+  if (n <= 0) return 0;
+  k_level_start<<<grid_for(n, kStartTile), 256, 0, st>>>(n, cmap, cpart, cbnd, part, bnd, gain, dest, upd, cand, wl,
+                                                         cnt, cut_in, cut, thr, lastcnt);
+  return hip_status();
+}
+
+// Boundary flags and part weights of the initial partition, which the host
+// used to walk the coarsest graph for: 16 lanes a vertex, part weights in an
+// LDS histogram per block.
+__global__ void __launch_bounds__(256) k_part_state(int32_t n, int32_t k, const int32_t* __restrict__ xadj,
+                                                    const int32_t* __restrict__ adj, const int32_t* __restrict__ vw,
+                                                    const int32_t* __restrict__ part, int32_t* __restrict__ bnd,
+                                                    int32_t* __restrict__ pw) {
+  extern __shared__ int32_t hist[];
+  for (int32_t q = threadIdx.x; q < k; q += 256) hist[q] = 0;
+  __syncthreads();
+  const int sub = threadIdx.x & 15;
+  const int base_lane = lane_id() & ~15;
+  // whole segments of 16 lanes stay together
+  for (int64_t v = (int64_t(blockIdx.x) * 256 + threadIdx.x) / 16; v < n; v += int64_t(gridDim.x) * 16) {
+    const int32_t p = part[v];
+    const int32_t s = xadj[v], e = xadj[v + 1];
+    bool other = false;
+    for (int32_t j = s + sub; j < e && !other; j += 16) other = part[adj[j]] != p;
+    const bool any = ((ballot(other) >> base_lane) & 0xffffull) != 0;
+    if (sub == 0) {
+      bnd[v] = any ? 1 : 0;
+      atomicAdd(&hist[p], vw[v]);
+    }
+  }
+  __syncthreads();
+  for (int32_t q = threadIdx.x; q < k; q += 256)
+    if (hist[q]) atomicAdd(&pw[q], hist[q]);
+}
+
+int launch_part_state(const DGraph& g, int32_t k, const int32_t* part, int32_t* bnd, int32_t* pw, hipStream_t st) {
+  if (g.n <= 0) return 0;
+  const unsigned grid = std::min(grid_for(int64_t(g.n) * 16, 256), 256u);
+  k_part_state<<<grid, 256, sizeof(int32_t) * k, st>>>(g.n, k, g.xadj, g.adj, g.vw, part, bnd, pw);
+  return hip_status();
+}
+
+// One launch for a set of copies: a copy by the runtime costs 5 to 10 us of
+// host time and a kernel of its own each, and the V-cycle's are small.
+__global__ void __launch_bounds__(256) k_copies(const Copies c) {
+  const int64_t at = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t step = int64_t(gridDim.x) * 256;
+  for (int i = 0; i < c.n; ++i) {
+    int32_t* d = c.dst[i];
+    const int32_t* s = c.src[i];
+    int64_t done = 0;
+    if (((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(s)) & 15) == 0) {
+      const int64_t n4 = c.len[i] / 4;
+      const int4 zero = make_int4(0, 0, 0, 0);
+      for (int64_t x = at; x < n4; x += step)
+        reinterpret_cast<int4*>(d)[x] = s ? reinterpret_cast<const int4*>(s)[x] : zero;
+      done = n4 * 4;
+    }
+    for (int64_t x = done + at; x < c.len[i]; x += step) d[x] = s ? s[x] : 0;
+  }
+}
+
+int launch_copies(const Copies& c, hipStream_t st) {
+  int64_t most = 0;
+  for (int i = 0; i < c.n; ++i) most = std::max(most, c.len[i]);
+  if (most == 0) return 0;
+  k_copies<<<std::min(grid_for(most, 1024), 2048u), 256, 0, st>>>(c);
+  return hip_status();
+}
+
 // update_vertex_info + calculate_gain (gkway/uncoarsen.hpp:175-237, 82-109)
 // over a worklist of updated vertices (wlc[0] entries), S lanes per vertex
 // (gain_pass), grid-stride.  Rows longer than S: with k <= kGainInlineK the

@@ -139,7 +139,14 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     a.next_status[0] = 0;
     a.next_status[1] = 0;
   }
-  if (a.lastcnt[j] == 0) return;  // converged in an earlier launch
+  if (a.lastcnt[j] == 0) {  // converged in an earlier launch
+    if (a.host && t == 0) {
+      a.host[0] = 0;
+      a.host[1] = 0;
+      a.host[2] = a.rounds[j];
+    }
+    return;
+  }
   const int32_t vb = a.v_off[j], ve = a.v_off[j + 1];
   const int32_t kj = a.kk[j];
   const long long cap = a.cap[j];
@@ -161,6 +168,11 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     if (t == 0) {
       atomicAdd(&a.status[0], 1);
       atomicAdd(&a.status[1], 1);
+      if (a.host) {
+        a.host[0] = 1;
+        a.host[1] = 1;
+        a.host[2] = a.rounds[j];
+      }
     }
     return;
   }
@@ -735,6 +747,11 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     a.moved[j] = moved0;
     a.lastcnt[j] = count;
     if (count) atomicAdd(&a.status[0], 1);
+    if (a.host) {
+      a.host[0] = count ? 1 : 0;
+      a.host[1] = 0;
+      a.host[2] = rounds0;
+    }
   }
 }
 
