@@ -55,6 +55,13 @@ struct Copies {
 };
 int launch_copies(const Copies& c, hipStream_t st);
 
+// Validity of a graph whose xadj begins with 0 and ends with nnz (weights may
+// be null: ones).  out (3 words, zero before): [0] != 0 for rows that do not
+// follow one another, neighbours out of range, self loops or weights below 1;
+// [1] the sum of the vertex weights, [2] of the entries'.  Reads no entry
+// outside [0, nnz).
+int launch_graph_check(const DGraph& g, unsigned long long* out, hipStream_t st);
+
 // Lanes per vertex for row-parallel kernels, from the average degree.
 int lanes_for_degree(double avg_deg);
 

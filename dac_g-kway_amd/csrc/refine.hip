@@ -206,6 +206,56 @@ int launch_part_state(const DGraph& g, int32_t k, const int32_t* part, int32_t* 
   return hip_status();
 }
 
+// The checks of a host graph, on its uploaded copy: a pass over the entries in
+// memory order, 8 lanes a vertex, one atomic per block and sum.  The host's pass
+// took 810 us for a mesh of 100 k vertices and 600 k entries.
+__global__ void __launch_bounds__(256) k_graph_check(int32_t n, int32_t nnz, const int32_t* __restrict__ xadj,
+                                                     const int32_t* __restrict__ adj, const int32_t* __restrict__ w,
+                                                     const int32_t* __restrict__ vw,
+                                                     unsigned long long* __restrict__ out) {
+  __shared__ long long sv[4], se[4];
+  const int sub = threadIdx.x & 7;
+  long long tv = 0, te = 0;
+  bool bad = false;
+  for (int64_t v = (int64_t(xcd_block()) * 256 + threadIdx.x) / 8; v < n; v += int64_t(gridDim.x) * 32) {
+    const int32_t s = xadj[v], e = xadj[v + 1];
+    if (s < 0 || e < s || e > nnz) {
+      bad = true;
+      continue;
+    }
+    for (int64_t j = int64_t(s) + sub; j < e; j += 8) {
+      const int32_t u = adj[j];
+      const int32_t x = w ? w[j] : 1;
+      bad |= uint32_t(u) >= uint32_t(n) || u == int32_t(v) || x < 1;
+      te += x;
+    }
+    if (sub == 0) {
+      const int32_t x = vw ? vw[v] : 1;
+      bad |= x < 1;
+      tv += x;
+    }
+  }
+  tv = wave_sum64(tv);
+  te = wave_sum64(te);
+  if (lane_id() == 0) {
+    sv[threadIdx.x >> 6] = tv;
+    se[threadIdx.x >> 6] = te;
+  }
+  if (ballot(bad) != 0 && lane_id() == 0) out[0] = 1;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicAdd(&out[1], (unsigned long long)(sv[0] + sv[1] + sv[2] + sv[3]));
+    atomicAdd(&out[2], (unsigned long long)(se[0] + se[1] + se[2] + se[3]));
+  }
+}
+
+int launch_graph_check(const DGraph& g, unsigned long long* out, hipStream_t st) {
+  if (g.n <= 0) return 0;
+  k_graph_check<<<std::min(grid_for(int64_t(g.n) * 8, 256), 512u), 256, 0, st>>>(g.n, g.nnz, g.xadj, g.adj, g.w, g.vw,
+                                                                                out);
+  return hip_status();
+}
+
 // One launch for a set of copies: a copy by the runtime costs 5 to 10 us of
 // host time and a kernel of its own each, and the V-cycle's are small.
 __global__ void __launch_bounds__(256) k_copies(const Copies c) {
