@@ -58,13 +58,12 @@ __device__ __forceinline__ void block_jobs(const int32_t* __restrict__ off, int3
 // ---------------------------------------------------------------- pack
 __global__ void __launch_bounds__(256) k_pack_vert(int32_t nj, const PackSrc* __restrict__ src,
                                                    const int32_t* __restrict__ v_off,
-                                                   const int32_t* __restrict__ e_off,
-                                                   const int32_t* __restrict__ c_off, int32_t ntot,
-                                                   int32_t* __restrict__ xadj, int32_t* __restrict__ vw,
-                                                   int32_t* __restrict__ vjob, int32_t* __restrict__ cmap) {
+                                                   const int32_t* __restrict__ e_off, int32_t ntot, int32_t etot,
+                                                   int32_t* __restrict__ xadj, int32_t* __restrict__ vw) {
   __shared__ int32_t sj[2];
   const int64_t i0 = int64_t(blockIdx.x) * kPackPer * 256;
   block_jobs(v_off, nj, ntot, i0, sj);
+  if (blockIdx.x == 0 && threadIdx.x == 0) xadj[ntot] = etot;
   for (int r = 0; r < kPackPer; ++r) {
     const int64_t i = i0 + r * 256 + threadIdx.x;
     if (i >= ntot) break;
@@ -73,9 +72,83 @@ __global__ void __launch_bounds__(256) k_pack_vert(int32_t nj, const PackSrc* __
     const int32_t li = int32_t(i - v_off[j]);
     xadj[i] = e_off[j] + (s.xadj[li] - s.xbase);
     vw[i] = s.vw[li];
-    if (vjob) vjob[i] = j;
-    // No source map: the coarse side has the fine level's ids (identity).
-    if (cmap) cmap[i] = c_off[j] + (s.cmap ? s.cmap[li] - s.cbase : li);
+  }
+}
+
+// The vertex side of a refinement pack, with the start of its rounds: rows and
+// weights, expand_partition (gkway/uncoarsen.hpp:325-356) straight from the
+// coarse level's arrays (levels entered by projection) or the carried state
+// (resumed ones), the candidate bits, the worklist of the projected boundary
+// and the jobs' state words.  Five kernels (pack, packed coarse arrays,
+// projection, candidates, compaction) took 18 + 12 + 4 + 2 + 9 us a step before,
+// most of it launches and chains of small loads (160 graphs of 500 to 50000
+// vertices).
+__global__ void __launch_bounds__(256) k_pack_refine(int32_t nj, const PackSrc* __restrict__ src,
+                                                     const int32_t* __restrict__ v_off,
+                                                     const int32_t* __restrict__ e_off, int32_t ntot, int32_t etot,
+                                                     int32_t* __restrict__ xadj, int32_t* __restrict__ vw,
+                                                     const RefineStart o) {
+  __shared__ int32_t sj[2];
+  __shared__ int wsum[4];
+  __shared__ int base_s;
+  const int64_t i0 = int64_t(blockIdx.x) * kPackPer * 256;
+  const int wave = threadIdx.x >> 6;
+  block_jobs(v_off, nj, ntot, i0, sj);
+  if (blockIdx.x == 0 && threadIdx.x == 0) xadj[ntot] = etot;
+  for (int64_t j = int64_t(blockIdx.x) * 256 + threadIdx.x; j < nj; j += int64_t(gridDim.x) * 256) {
+    o.lastcnt[j] = 1;
+    o.thr[j] = 1;
+  }
+  uint64_t m[kPackPer];
+  int tot = 0;
+#pragma unroll
+  for (int r = 0; r < kPackPer; ++r) {
+    const int64_t i = i0 + r * 256 + threadIdx.x;
+    bool up = false, cnd = false;
+    if (i < ntot) {
+      const int32_t j = sj[0] == sj[1] ? sj[0] : job_in(v_off, sj[0], sj[1] + 1, i);
+      const PackSrc& s = src[j];
+      const int32_t li = int32_t(i - v_off[j]);
+      xadj[i] = e_off[j] + (s.xadj[li] - s.xbase);
+      vw[i] = s.vw[li];
+      o.vjob[i] = j;
+      // No source map: the coarse side has the level's own ids (resumed).
+      const int32_t c = s.cmap ? s.cmap[li] - s.cbase : li;
+      const int32_t p = s.cpart[c];
+      const bool b = s.cbnd[c] != 0;
+      int32_t g = 0, d = p;
+      if (s.cgain) {
+        g = s.cgain[c];
+        d = s.cdest[c];
+      } else {
+        up = b;
+      }
+      o.part[i] = p;
+      o.bnd[i] = b ? 1 : 0;
+      o.gain[i] = g;
+      o.dest[i] = d;
+      o.upd[i] = up ? 1 : 0;
+      cnd = b && g > 0;
+    }
+    m[r] = ballot(up);
+    tot += popc64(m[r]);
+    const uint64_t cb = ballot(cnd);
+    if (lane_id() == 0 && i < ntot) o.cand[i >> 6] = cb;
+  }
+  if (lane_id() == 0) wsum[wave] = tot;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int t = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    base_s = t ? atomicAdd(o.cnt, t) : 0;
+  }
+  __syncthreads();
+  int off = base_s;
+  for (int w = 0; w < wave; ++w) off += wsum[w];
+  const uint64_t lt = lanemask_lt();
+#pragma unroll
+  for (int r = 0; r < kPackPer; ++r) {
+    if ((m[r] >> lane_id()) & 1ull) o.wl[off + popc64(m[r] & lt)] = int32_t(i0 + r * 256 + threadIdx.x);
+    off += popc64(m[r]);
   }
 }
 
@@ -113,76 +186,18 @@ __global__ void __launch_bounds__(256) k_pack_edge(int32_t nj, const PackSrc* __
   }
 }
 
-// Coarse-side arrays of a refinement pack (partition and boundary flags of
-// the next coarser level, one range per job).
-__global__ void __launch_bounds__(256) k_pack_coarse(int32_t nj, const PackSrc* __restrict__ src,
-                                                     const int32_t* __restrict__ c_off, int32_t ctot,
-                                                     int32_t* __restrict__ cpart, int32_t* __restrict__ cbnd,
-                                                     int32_t* __restrict__ cgain, int32_t* __restrict__ cdest) {
-  __shared__ int32_t sj[2];
-  const int64_t i0 = int64_t(blockIdx.x) * kPackPer * 256;
-  block_jobs(c_off, nj, ctot, i0, sj);
-  for (int r = 0; r < kPackPer; ++r) {
-    const int64_t i = i0 + r * 256 + threadIdx.x;
-    if (i >= ctot) break;
-    const int32_t j = sj[0] == sj[1] ? sj[0] : job_in(c_off, sj[0], sj[1] + 1, i);
-    const int32_t li = int32_t(i - c_off[j]);
-    const PackSrc& s = src[j];
-    cpart[i] = s.cpart[li];
-    cbnd[i] = s.cbnd[li];
-    if (cgain) {
-      cgain[i] = s.cgain ? s.cgain[li] : 0;
-      cdest[i] = s.cgain ? s.cdest[li] : -1;
-    }
-  }
-}
-
-int launch_pack(int32_t nj, const PackSrc* src, const int32_t* v_off, const int32_t* e_off, const int32_t* c_off,
-                int32_t ntot, int32_t etot, int32_t ctot, int32_t* xadj, int32_t* adj, int32_t* w, int32_t* vw,
-                int32_t* vjob, int32_t* cmap, int32_t* cpart, int32_t* cbnd, int32_t* cgain, int32_t* cdest,
-                hipStream_t st) {
+int launch_pack(int32_t nj, const PackSrc* src, const int32_t* v_off, const int32_t* e_off, int32_t ntot, int32_t etot,
+                int32_t* xadj, int32_t* adj, int32_t* w, int32_t* vw, const RefineStart* refine, hipStream_t st) {
   constexpr int kTile = kPackPer * 256;
-  if (ntot > 0)
-    k_pack_vert<<<grid_for(ntot, kTile), 256, 0, st>>>(nj, src, v_off, e_off, c_off, ntot, xadj, vw, vjob, cmap);
-  fill<int32_t>(xadj + ntot, etot, 1, st);
-  if (etot > 0) k_pack_edge<<<grid_for(etot, kTile), 256, 0, st>>>(nj, src, v_off, e_off, etot, adj, w);
-  if (cpart && ctot > 0)
-    k_pack_coarse<<<grid_for(ctot, kTile), 256, 0, st>>>(nj, src, c_off, ctot, cpart, cbnd, cgain, cdest);
-  return hip_status();
-}
-
-// expand_partition (gkway/uncoarsen.hpp:325-356) on a refinement pack, with
-// resumed levels taking their carried state.
-__global__ void __launch_bounds__(256) k_project_b(int32_t n, const int32_t* __restrict__ cmap,
-                                                   const int32_t* __restrict__ cpart,
-                                                   const int32_t* __restrict__ cbnd,
-                                                   const int32_t* __restrict__ cgain,
-                                                   const int32_t* __restrict__ cdest, int32_t* __restrict__ part,
-                                                   int32_t* __restrict__ bnd, int32_t* __restrict__ gain,
-                                                   int32_t* __restrict__ dest, int32_t* __restrict__ upd) {
-  const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
-  if (v >= n) return;
-  const int32_t c = cmap[v];
-  const int32_t p = cpart[c];
-  const int32_t b = cbnd[c] ? 1 : 0;
-  const int32_t d = cdest[c];
-  part[v] = p;
-  bnd[v] = b;
-  if (d >= 0) {
-    gain[v] = cgain[c];
-    dest[v] = d;
-    upd[v] = 0;
-  } else {
-    gain[v] = 0;
-    dest[v] = p;
-    upd[v] = b;
+  if (ntot <= 0) {
+    fill<int32_t>(xadj, 0, 1, st);
+    return hip_status();
   }
-}
-
-int launch_project_b(int32_t n, const int32_t* cmap, const int32_t* cpart, const int32_t* cbnd, const int32_t* cgain,
-                     const int32_t* cdest, int32_t* part, int32_t* bnd, int32_t* gain, int32_t* dest, int32_t* upd,
-                     hipStream_t st) {
-  if (n > 0) k_project_b<<<grid_for(n, 256), 256, 0, st>>>(n, cmap, cpart, cbnd, cgain, cdest, part, bnd, gain, dest, upd);
+  if (refine)
+    k_pack_refine<<<grid_for(ntot, kTile), 256, 0, st>>>(nj, src, v_off, e_off, ntot, etot, xadj, vw, *refine);
+  else
+    k_pack_vert<<<grid_for(ntot, kTile), 256, 0, st>>>(nj, src, v_off, e_off, ntot, etot, xadj, vw);
+  if (etot > 0) k_pack_edge<<<grid_for(etot, kTile), 256, 0, st>>>(nj, src, v_off, e_off, etot, adj, w);
   return hip_status();
 }
 
@@ -763,30 +778,40 @@ int launch_max_deg(const DGraph& g, int32_t* out, hipStream_t st) {
 // Final cut and part weights (calculate_cutsize + calculate_partition_wgt,
 // gkway/uncoarsen.hpp:398-424, gkway/cuda_check.hpp:61-73) per chunk of one
 // job's vertices: the block sums its vertex weights per part in an LDS
-// histogram and its cut edges in registers, then adds them to the job's
-// totals with one atomic per touched part and one for the cut.
+// histogram and its cut edges in registers (8 lanes a vertex), then adds them
+// to the job's totals with one atomic per touched part and one for the cut.
+// The finished partition goes to its job's destination on the way.  Few jobs
+// end in one step, so a chunk is short: with 2048 vertices of a chunk and one
+// lane a vertex a launch took 67 us, nearly all of it one block's chain.
 __global__ void __launch_bounds__(256) k_cut_chunks(const int32_t* __restrict__ cj, const int32_t* __restrict__ cs,
                                                     const int32_t* __restrict__ ce, const int32_t* __restrict__ kk,
+                                                    const int32_t* __restrict__ v_off,
                                                     const int32_t* __restrict__ xadj,
                                                     const int32_t* __restrict__ adj, const int32_t* __restrict__ w,
                                                     const int32_t* __restrict__ vw,
                                                     const int32_t* __restrict__ part,
                                                     const int32_t* __restrict__ pw_off,
+                                                    const UnpackDst* __restrict__ dst,
                                                     unsigned long long* __restrict__ cut,
                                                     unsigned long long* __restrict__ pw64) {
   extern __shared__ unsigned int hist[];
   __shared__ long long wsum[4];
   const int32_t c = static_cast<int32_t>(xcd_block());
-  const int32_t j = cj[c], k = kk[j];
+  const int32_t j = cj[c], k = kk[j], e0 = ce[c];
+  int32_t* out = dst[j].part - v_off[j];
   for (int32_t q = threadIdx.x; q < k; q += 256) hist[q] = 0;
   __syncthreads();
   long long cc = 0;
-  for (int32_t v = cs[c] + threadIdx.x; v < ce[c]; v += 256) {
+  const int sub = threadIdx.x & 7;
+  for (int32_t v = cs[c] + int32_t(threadIdx.x >> 3); v < e0; v += 32) {
     const int32_t p = part[v];
-    atomicAdd(&hist[p], (unsigned int)vw[v]);
-    for (int32_t e = xadj[v]; e < xadj[v + 1]; ++e) {
+    for (int32_t e = xadj[v] + sub; e < xadj[v + 1]; e += 8) {
       const int32_t u = adj[e];
       if (v < u && part[u] != p) cc += w[e];
+    }
+    if (sub == 0) {
+      atomicAdd(&hist[p], (unsigned int)vw[v]);
+      out[v] = p;
     }
   }
   cc = wave_sum64(cc);
@@ -801,11 +826,12 @@ __global__ void __launch_bounds__(256) k_cut_chunks(const int32_t* __restrict__ 
 }
 
 int launch_cut_chunks(int32_t nchunks, const int32_t* cj, const int32_t* cs, const int32_t* ce, int32_t kmax,
-                      const int32_t* kk, const DGraph& g, const int32_t* part, const int32_t* pw_off,
-                      unsigned long long* cut, unsigned long long* pw64, hipStream_t st) {
+                      const int32_t* kk, const int32_t* v_off, const DGraph& g, const int32_t* part,
+                      const int32_t* pw_off, const UnpackDst* dst, unsigned long long* cut, unsigned long long* pw64,
+                      hipStream_t st) {
   if (nchunks <= 0) return 0;
-  k_cut_chunks<<<nchunks, 256, sizeof(unsigned int) * kmax, st>>>(cj, cs, ce, kk, g.xadj, g.adj, g.w, g.vw, part,
-                                                                  pw_off, cut, pw64);
+  k_cut_chunks<<<nchunks, 256, sizeof(unsigned int) * kmax, st>>>(cj, cs, ce, kk, v_off, g.xadj, g.adj, g.w, g.vw,
+                                                                  part, pw_off, dst, cut, pw64);
   return hip_status();
 }
 

@@ -32,22 +32,22 @@ struct UnpackDst {
   int32_t* bnd;
 };
 
+// What a refinement pack's kernel writes besides the graph, per vertex of the
+// pack (cand: a bit each, worklist wl with its count cnt, zero before) and per
+// job (lastcnt and thr: 1).
+struct RefineStart {
+  int32_t *vjob, *part, *bnd, *gain, *dest, *upd, *wl, *cnt;
+  uint64_t* cand;
+  int32_t *lastcnt, *thr;
+};
+
 // Pack nj jobs: vertices at v_off, entries at e_off (nj+1 prefix arrays);
-// writes xadj[ntot+1], adj/w[etot], vw/vjob[ntot]; with cmap != null also the
-// packed fine->coarse map (+c_off) and, with cpart != null, the packed coarse
-// partition/boundary arrays (ctot entries).
-// With cgain != null also cgain/cdest: the carried values of resumed jobs, and
-// dest = -1 for the others.
-int launch_pack(int32_t nj, const PackSrc* src, const int32_t* v_off, const int32_t* e_off, const int32_t* c_off,
-                int32_t ntot, int32_t etot, int32_t ctot, int32_t* xadj, int32_t* adj, int32_t* w, int32_t* vw,
-                int32_t* vjob, int32_t* cmap, int32_t* cpart, int32_t* cbnd, int32_t* cgain, int32_t* cdest,
-                hipStream_t st);
-// Projection of a refinement pack: expand_partition for levels entered from
-// the coarser level (gain 0, dest = part, update = boundary); resumed levels
-// (cdest >= 0) take their carried gain and dest and need no update.
-int launch_project_b(int32_t n, const int32_t* cmap, const int32_t* cpart, const int32_t* cbnd, const int32_t* cgain,
-                     const int32_t* cdest, int32_t* part, int32_t* bnd, int32_t* gain, int32_t* dest, int32_t* upd,
-                     hipStream_t st);
+// writes xadj[ntot+1], adj/w[etot], vw[ntot], and with refine the start of the
+// rounds: levels entered by projection get gain 0, dest = part and an update
+// of their boundary, resumed ones (cgain != null) their carried gains and
+// destinations.
+int launch_pack(int32_t nj, const PackSrc* src, const int32_t* v_off, const int32_t* e_off, int32_t ntot, int32_t etot,
+                int32_t* xadj, int32_t* adj, int32_t* w, int32_t* vw, const RefineStart* refine, hipStream_t st);
 // cand bit v = (bnd[v] && gain[v] > 0), all (n + 63) / 64 words written.
 int launch_cand_init(int32_t n, const int32_t* bnd, const int32_t* gain, uint64_t* cand, hipStream_t st);
 // out[j] = total vertex weight of job j (v_off on the device, nj+1).
@@ -143,9 +143,11 @@ int launch_rounds_init(int32_t nj, int32_t* lastcnt, int32_t* thr, int32_t* roun
 int launch_max_deg(const DGraph& g, int32_t* out, hipStream_t st);
 // Final cut and part weights of the jobs covered by the chunk table: chunk c
 // is vertices [cs[c], ce[c]) of job cj[c] (pack ids); cut[job] and
-// pw64[pw_off[job] + q] accumulate (zeroed by the caller).
+// pw64[pw_off[job] + q] accumulate (zeroed by the caller); the vertices' parts
+// go to dst[job].part.
 int launch_cut_chunks(int32_t nchunks, const int32_t* cj, const int32_t* cs, const int32_t* ce, int32_t kmax,
-                      const int32_t* kk, const DGraph& g, const int32_t* part, const int32_t* pw_off,
-                      unsigned long long* cut, unsigned long long* pw64, hipStream_t st);
+                      const int32_t* kk, const int32_t* v_off, const DGraph& g, const int32_t* part,
+                      const int32_t* pw_off, const UnpackDst* dst, unsigned long long* cut, unsigned long long* pw64,
+                      hipStream_t st);
 
 }  // namespace gkd

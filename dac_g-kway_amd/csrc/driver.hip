@@ -447,13 +447,17 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
   int pair = 1;  // the compaction before the rounds used pair 0
   int done = 0, wide_done = 0, per_check = kWideRounds;
   // Jobs that go on, jobs left out, and with one job the ordering rounds so
-  // far, which its kernel writes to pinned memory: a wait instead of a copy.
+  // far; one job's kernel writes them to pinned memory itself.
   const bool one = s.nj == 1;
   auto status = [&](int p, int32_t* words) -> int {
-    if (!one) return fetch(ctx, st, {{words, s.status + 2 * p, 2 * sizeof(int32_t)}});
+    if (!one) {
+      gkd::Copies c;
+      c.add(ctx->hctl, s.status + 2 * p, 2 * sizeof(int32_t));
+      GK_TRY(gkd::launch_copies(c, st));
+    }
     GK_HIP(hipEventRecord(ctx->ev, st));
     GK_HIP(hipEventSynchronize(ctx->ev));
-    std::memcpy(words, ctx->hctl, 3 * sizeof(int32_t));
+    std::memcpy(words, ctx->hctl, (one ? 3 : 2) * sizeof(int32_t));
     return GK_OK;
   };
   while (max_rounds <= 0 || done < max_rounds) {
@@ -522,9 +526,6 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
 namespace {
 
 // ---------------------------------------------------------------- V-cycle
-// Host arrays of up to this size move through pinned staging memory.
-constexpr size_t kStageMax = size_t(16) << 20;
-
 // The partition goes to dpart_out (device) or, if that is null, to part (host).
 int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params& prm,
                int32_t* dpart_out, gk_stats* stats, int32_t* part = nullptr) {
@@ -927,7 +928,6 @@ constexpr int32_t kDeviceCheckEntries = 1 << 15;
 // from 2880 to 2031 us.
 int upload_graph(gk_ctx* ctx, hipStream_t st, const gk_csr& h, bool check, Buf<int32_t>& x, Buf<int32_t>& a,
                  Buf<int32_t>& w, Buf<int32_t>& v, DGraph* g) {
-  constexpr size_t kPiece = size_t(1) << 20;
   Pool& P = ctx->pool;
   const size_t nb = sizeof(int32_t) * size_t(h.n), eb = sizeof(int32_t) * size_t(h.nnz);
   struct Array {
@@ -954,13 +954,13 @@ int upload_graph(gk_ctx* ctx, hipStream_t st, const gk_csr& h, bool check, Buf<i
     size_t pending = 0;
     for (const Array& y : arrays) {
       if (!y.host || !y.bytes) continue;
-      for (size_t o = 0; o < y.bytes; o += kPiece) {
-        const size_t b = std::min(kPiece, y.bytes - o);
+      for (size_t o = 0; o < y.bytes; o += kStagePiece) {
+        const size_t b = std::min(kStagePiece, y.bytes - o);
         std::memcpy(to, reinterpret_cast<const char*>(y.host) + o, b);
         c.add(reinterpret_cast<char*>(y.dev.p) + o, to, b);
         to += (b + 15) & ~size_t(15);
         pending += b;
-        if (pending >= kPiece || c.n == gkd::Copies::kMax) {
+        if (pending >= kStagePiece || c.n == gkd::Copies::kMax) {
           GK_TRY(gkd::launch_copies(c, st));
           c = gkd::Copies{};
           pending = 0;

@@ -133,22 +133,44 @@ Engine::~Engine() {
 }
 
 int Engine::sync() {
+  GK_TRY(flush());
   GK_HIP(hipStreamSynchronize(st_));
   up_.drained();
   return GK_OK;
 }
 
+int Engine::stage(void* dst, const void* src, size_t bytes) {
+  if (!bytes) return GK_OK;
+  if (pending_.n == gkd::Copies::kMax || (src && !up_.fits(bytes))) GK_TRY(flush());
+  void* h = nullptr;
+  if (src) {
+    GK_TRY(up_.get(st_, bytes, &h));
+    std::memcpy(h, src, bytes);
+  }
+  pending_.add(dst, h, bytes);
+  return GK_OK;
+}
+
+int Engine::flush() {
+  const gkd::Copies c = pending_;
+  pending_ = gkd::Copies{};
+  return gkd::launch_copies(c, st_);
+}
+
 int Engine::download(std::initializer_list<Fetch> items) {
+  GK_TRY(flush());
   size_t tot = 0;
   for (const Fetch& f : items) tot += (f.bytes + 255) & ~size_t(255);
   void* h = nullptr;
   GK_TRY(dl_.get(st_, tot, &h));
   char* c = static_cast<char*>(h);
   size_t off = 0;
+  gkd::Copies back;
   for (const Fetch& f : items) {
-    if (f.bytes) GK_HIP(hipMemcpyAsync(c + off, f.dev, f.bytes, hipMemcpyDeviceToHost, st_));
+    back.add(c + off, f.dev, f.bytes);
     off += (f.bytes + 255) & ~size_t(255);
   }
+  GK_TRY(gkd::launch_copies(back, st_));
   GK_TRY(sync());
   off = 0;
   for (const Fetch& f : items) {
@@ -185,58 +207,48 @@ PackSrc Engine::src_of(const JLevel& lv) {
   return p;
 }
 
-int Engine::pack_copy(const std::vector<PackSrc>& src, const std::vector<int32_t>& nv,
-                      const std::vector<int32_t>& ne, const std::vector<int32_t>* ncv, StoreP& out,
-                      RefineSide* rs) {
-  const int32_t J = static_cast<int32_t>(src.size());
+int Engine::pack_store(const std::vector<int32_t>& nv, const std::vector<int32_t>& ne, StoreP& out) {
+  const int32_t J = static_cast<int32_t>(nv.size());
   auto S = std::make_shared<Store>();
   S->nj = J;
   S->v_off.assign(J + 1, 0);
   S->e_off.assign(J + 1, 0);
-  std::vector<int32_t> c_off(J + 1, 0);
   for (int32_t i = 0; i < J; ++i) {
     const int64_t a = int64_t(S->v_off[i]) + nv[i], b = int64_t(S->e_off[i]) + ne[i];
-    const int64_t c = int64_t(c_off[i]) + (ncv ? (*ncv)[i] : 0);
-    if (a >= INT32_MAX || b >= INT32_MAX || c >= INT32_MAX) {
+    if (a >= INT32_MAX || b >= INT32_MAX) {
       gkh::set_error("packed batch exceeds 2^31 vertices or entries");
       return GK_ERR_LIMIT;
     }
     S->v_off[i + 1] = int32_t(a);
     S->e_off[i + 1] = int32_t(b);
-    c_off[i + 1] = int32_t(c);
   }
   S->n = S->v_off[J];
   S->nnz = S->e_off[J];
-  const int32_t ctot = c_off[J];
-  Buf<PackSrc> dsrc;
-  Buf<int32_t> de_off, dc_off;
-  GK_TRY(upload(dsrc, src.data(), src.size()));
-  GK_TRY(upload(S->dv_off, S->v_off.data(), S->v_off.size()));
-  GK_TRY(upload(de_off, S->e_off.data(), S->e_off.size()));
-  GK_TRY(upload(dc_off, c_off.data(), c_off.size()));
   GK_TRY(S->bx.alloc(P_, int64_t(S->n) + 1));
   GK_TRY(S->ba.alloc(P_, S->nnz));
   GK_TRY(S->bw.alloc(P_, S->nnz));
   GK_TRY(S->bv.alloc(P_, S->n));
-  if (rs) {
-    GK_TRY(rs->vjob.alloc(P_, S->n));
-    GK_TRY(rs->cmap.alloc(P_, S->n));
-    GK_TRY(rs->cpart.alloc(P_, ctot));
-    GK_TRY(rs->cbnd.alloc(P_, ctot));
-    GK_TRY(rs->cgain.alloc(P_, ctot));
-    GK_TRY(rs->cdest.alloc(P_, ctot));
-    rs->c_off = c_off;
-  }
-  GK_STAGE(ctx_, GK_ST_PACK, 20LL * S->n + 16LL * S->nnz + (rs ? 16LL * S->n + 24LL * ctot : 0),
-           gkd::launch_pack(J, dsrc.p, S->dv_off.p, de_off.p, dc_off.p, S->n, S->nnz, ctot, S->bx.p, S->ba.p,
-                            S->bw.p, S->bv.p, rs ? rs->vjob.p : nullptr, rs ? rs->cmap.p : nullptr,
-                            rs ? rs->cpart.p : nullptr, rs ? rs->cbnd.p : nullptr, rs ? rs->cgain.p : nullptr,
-                            rs ? rs->cdest.p : nullptr, st_));
   S->xadj = S->bx.p;
   S->adj = S->ba.p;
   S->w = S->bw.p;
   S->vw = S->bv.p;
   out = std::move(S);
+  return GK_OK;
+}
+
+int Engine::pack_copy(const std::vector<PackSrc>& src, const std::vector<int32_t>& nv,
+                      const std::vector<int32_t>& ne, StoreP& out, const gkd::RefineStart* refine) {
+  const int32_t J = static_cast<int32_t>(src.size());
+  if (!out) GK_TRY(pack_store(nv, ne, out));
+  Store& S = *out;
+  Buf<PackSrc> dsrc;
+  Buf<int32_t> de_off;
+  GK_TRY(upload(dsrc, src.data(), src.size()));
+  GK_TRY(upload(S.dv_off, S.v_off.data(), S.v_off.size()));
+  GK_TRY(upload(de_off, S.e_off.data(), S.e_off.size()));
+  GK_TRY(flush());
+  GK_STAGE(ctx_, GK_ST_PACK, 20LL * S.n + 16LL * S.nnz + (refine ? 40LL * S.n : 0),
+           gkd::launch_pack(J, dsrc.p, S.dv_off.p, de_off.p, S.n, S.nnz, S.bx.p, S.ba.p, S.bw.p, S.bv.p, refine, st_));
   return GK_OK;
 }
 
@@ -286,7 +298,7 @@ int Engine::coarsen_step(bool* worked) {
       nv.push_back(l->n);
       ne.push_back(l->nnz);
     }
-    GK_TRY(pack_copy(src, nv, ne, nullptr, pk, nullptr));
+    GK_TRY(pack_copy(src, nv, ne, pk));
   }
   const Store& F = *pk;
   const DGraph g = F.graph();
@@ -369,7 +381,7 @@ int Engine::init_step(bool* worked) {
       nv.push_back(l->n);
       ne.push_back(l->nnz);
     }
-    GK_TRY(pack_copy(src, nv, ne, nullptr, pk, nullptr));
+    GK_TRY(pack_copy(src, nv, ne, pk));
   }
   const Store& Q = *pk;
   std::vector<int32_t> hx(int64_t(Q.n) + 1), ha(Q.nnz), hw(Q.nnz), hv(Q.n);
@@ -467,6 +479,7 @@ int Engine::collect_inits(bool block, bool* worked) {
     }
     GK_TRY(upload(*pb, hp.data(), hp.size()));
     GK_TRY(upload(*bb, hb.data(), hb.size()));
+    GK_TRY(flush());
   }
   // Jobs whose coarsest level is level 0 are finished by the initial partition.
   std::vector<UnpackDst> dst(ready.size());
@@ -502,6 +515,7 @@ int Engine::collect_inits(bool block, bool* worked) {
     Buf<int32_t> doff;
     GK_TRY(upload(ddst, dst.data(), dst.size()));
     GK_TRY(upload(doff, off.data(), off.size()));
+    GK_TRY(flush());
     GK_TRY(gkd::launch_unpack_part(static_cast<int32_t>(ready.size()), ddst.p, doff.p, int32_t(tot), pb->p,
                                    nullptr, st_));
     GK_TRY(sync());
@@ -534,8 +548,7 @@ int Engine::refine_step(bool* worked) {
   const int32_t J = static_cast<int32_t>(ids.size());
   const int32_t M = ids[0]->prm.max_moves;
   std::vector<PackSrc> src(J);
-  std::vector<int32_t> nv(J), ne(J), ncv(J), pw_off(J + 1, 0), kk(J);
-  std::vector<long long> cap(J), cut(J);
+  std::vector<int32_t> nv(J), ne(J), pw_off(J + 1, 0);
   int32_t kmax = 1;
   for (int32_t i = 0; i < J; ++i) {
     Job& j = *ids[i];
@@ -552,27 +565,67 @@ int Engine::refine_step(bool* worked) {
       src[i].cmap = nullptr;
       src[i].cgain = j.cgain->p + j.coff;
       src[i].cdest = j.cdest->p + j.coff;
-      ncv[i] = f.n;
-    } else {
-      ncv[i] = j.L[j.cur + 1].n;
     }
-    kk[i] = j.prm.k;
     kmax = std::max(kmax, j.prm.k);
     pw_off[i + 1] = pw_off[i] + j.prm.k;
-    cap[i] = j.cap;
-    cut[i] = j.cut;
   }
-  std::vector<int32_t> hpw(pw_off[J]);
-  for (int32_t i = 0; i < J; ++i) std::copy(ids[i]->hpw.begin(), ids[i]->hpw.end(), hpw.begin() + pw_off[i]);
-  RefineSide rs;
+  // The jobs' tables go up, and come back, as one block: cut and cap, then
+  // part weight offsets, numbers of parts, part weights.
+  struct Tables {
+    long long *cut, *cap;
+    int32_t *pw_off, *kk, *pw;
+  };
+  const size_t table_bytes = sizeof(long long) * 2 * size_t(J) + sizeof(int32_t) * (2 * size_t(J) + 1 + size_t(pw_off[J]));
+  auto tables_at = [&](void* base) {
+    Tables t;
+    t.cut = static_cast<long long*>(base);
+    t.cap = t.cut + J;
+    t.pw_off = reinterpret_cast<int32_t*>(t.cap + J);
+    t.kk = t.pw_off + J + 1;
+    t.pw = t.kk + J;
+    return t;
+  };
+  std::vector<char> htab(table_bytes);
+  const Tables ht = tables_at(htab.data());
+  for (int32_t i = 0; i < J; ++i) {
+    const Job& j = *ids[i];
+    ht.cut[i] = j.cut;
+    ht.cap[i] = j.cap;
+    ht.kk[i] = j.prm.k;
+    std::copy(j.hpw.begin(), j.hpw.end(), ht.pw + pw_off[i]);
+  }
+  std::copy(pw_off.begin(), pw_off.end(), ht.pw_off);
+  // So do the counters, zero before the rounds: gain statistics (a (vertices,
+  // entries) pair per block of the gain launches, grids of at most kGainSlots
+  // blocks) and the selection kernels' bytes per block slot, which end in the
+  // stages' algorithmic bytes, the round kernels' bytes, paths and moves per
+  // job; rounds per job, worklist counts, round loop status.
+  constexpr int kGainSlots = gkd::kGainMaxBlocks;
+  constexpr int kWork = 2 * kGainSlots + gkd::kSelectByteSlots;
+  struct Counters {
+    unsigned long long* work;
+    long long *abytes, *paths, *moved;
+    int32_t *rounds, *hcnt, *status;
+  };
+  const size_t counter_bytes = sizeof(long long) * (kWork + 5 * size_t(J)) + sizeof(int32_t) * (size_t(J) + 8);
+  auto counters_at = [&](void* base) {
+    Counters t;
+    t.work = static_cast<unsigned long long*>(base);
+    t.abytes = reinterpret_cast<long long*>(t.work + kWork);
+    t.paths = t.abytes + J;
+    t.moved = t.paths + 3 * size_t(J);
+    t.rounds = reinterpret_cast<int32_t*>(t.moved + J);
+    t.hcnt = t.rounds + J;
+    t.status = t.hcnt + 4;
+    return t;
+  };
   StoreP pk;
-  GK_TRY(pack_copy(src, nv, ne, &ncv, pk, &rs));
+  GK_TRY(pack_store(nv, ne, pk));
   const Store& F = *pk;
   const DGraph g = F.graph();
   const int32_t N = g.n;
-  Buf<int32_t> dpw_off, dkk, dpw, upd, wl, heavy, list, hcnt, active, drounds, lastcnt, dmax, xlist, dthr, wpos,
-      sscr, status;
-  Buf<long long> dcap, dcut, dmoved, dpaths;
+  Buf<char> dtab, dcnt;
+  Buf<int32_t> vjob, upd, wl, heavy, list, active, lastcnt, dmax, xlist, dthr, wpos, sscr;
   Buf<uint64_t> cand, movable, selbits, defbits;
   Buf<uint32_t> hkey;
   auto part = std::make_shared<Buf<int32_t>>();
@@ -581,11 +634,12 @@ int Engine::refine_step(bool* worked) {
   auto destp = std::make_shared<Buf<int32_t>>();
   Buf<int32_t>& gain = *gainp;
   Buf<int32_t>& dest = *destp;
-  GK_TRY(upload(dpw_off, pw_off.data(), pw_off.size()));
-  GK_TRY(upload(dkk, kk.data(), kk.size()));
-  GK_TRY(upload(dpw, hpw.data(), hpw.size()));
-  GK_TRY(upload(dcap, cap.data(), cap.size()));
-  GK_TRY(upload(dcut, cut.data(), cut.size()));
+  GK_TRY(upload(dtab, htab.data(), table_bytes));
+  GK_TRY(dcnt.alloc(P_, int64_t(counter_bytes)));
+  GK_TRY(stage(dcnt.p, nullptr, counter_bytes));
+  const Tables dt = tables_at(dtab.p);
+  const Counters dc = counters_at(dcnt.p);
+  GK_TRY(vjob.alloc(P_, N));
   GK_TRY(part->alloc(P_, N));
   GK_TRY(bnd->alloc(P_, N));
   GK_TRY(gain.alloc(P_, N));
@@ -603,34 +657,14 @@ int Engine::refine_step(bool* worked) {
   GK_TRY(sscr.alloc(P_, gkd::select_scratch_ints(N)));
   GK_TRY(xlist.alloc(P_, N));
   GK_TRY(dthr.alloc(P_, J));
-  gkd::fill<uint64_t>(selbits.p, 0ull, nwords + 1, st_);
-  Buf<unsigned long long> selbytes;  // the selection kernels' algorithmic bytes, per block slot
-  GK_TRY(selbytes.alloc(P_, gkd::kSelectByteSlots));
-  gkd::fill<unsigned long long>(selbytes.p, 0ull, gkd::kSelectByteSlots, st_);
-  const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, selbytes.p};
+  GK_TRY(stage(selbits.p, nullptr, sizeof(uint64_t) * size_t(nwords + 1)));
+  const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, dc.work + 2 * kGainSlots};
   GK_TRY(hkey.alloc(P_, N));
-  GK_TRY(hcnt.alloc(P_, 4));
-  GK_TRY(status.alloc(P_, 4));
   GK_TRY(active.alloc(P_, 1));
-  GK_TRY(drounds.alloc(P_, J));
   GK_TRY(lastcnt.alloc(P_, J));
   GK_TRY(dmax.alloc(P_, 1));
-  GK_TRY(dmoved.alloc(P_, J));
-  GK_TRY(dpaths.alloc(P_, 3LL * J));
-  gkd::fill<long long>(dpaths.p, 0, 3LL * J, st_);
-  Buf<long long> dab;  // the round kernel's algorithmic bytes per job
-  GK_TRY(dab.alloc(P_, J));
-  // Gain-pass statistics: a (vertices, entries) pair per block of the gain
-  // launches (grids of at most kGainSlots blocks), summed after the rounds
-  // into the stage's algorithmic bytes.
-  constexpr int kGainSlots = gkd::kGainMaxBlocks;
-  Buf<unsigned long long> gwork;
-  GK_TRY(gwork.alloc(P_, 2 * kGainSlots));
-  gkd::fill<unsigned long long>(gwork.p, 0ull, 2 * kGainSlots, st_);
-  GK_STAGE(ctx_, GK_ST_PROJECT, 44LL * N,
-           gkd::launch_project_b(N, rs.cmap.p, rs.cpart.p, rs.cbnd.p, rs.cgain.p, rs.cdest.p, part->p, bnd->p,
-                                 gain.p, dest.p, upd.p, st_));
-  GK_STAGE(ctx_, GK_ST_PROJECT, 8LL * N + N / 8, gkd::launch_cand_init(N, bnd->p, gain.p, cand.p, st_));
+  const gkd::RefineStart start{vjob.p, part->p, bnd->p, gain.p, dest.p, upd.p, wl.p, dc.hcnt, cand.p, lastcnt.p, dthr.p};
+  GK_TRY(pack_copy(src, nv, ne, pk, &start));
   const int lanes = gain_lanes(g);
   // Rows longer than the gain pass's lane count: the pass takes them itself
   // for k <= kGainInlineK; above it they go to the heavy-row kernel, whose
@@ -643,14 +677,12 @@ int Engine::refine_step(bool* worked) {
     GK_TRY(fetch(ctx_, st_, {{&maxdeg, dmax.p, sizeof maxdeg}}));
     heavy_rows = maxdeg > lanes;
   }
-  GK_TRY(gkd::launch_rounds_init(J, lastcnt.p, dthr.p, drounds.p, dmoved.p, dab.p, hcnt.p, status.p, st_));
-  GK_STAGE(ctx_, GK_ST_PROJECT, 4LL * N, gkd::launch_compact(N, upd.p, wl.p, hcnt.p, st_));
   GK_STAGE(ctx_, GK_ST_GAIN, 0,
-           gkd::launch_gain_wl(g, kmax, lanes, wl.p, hcnt.p, heavy.p, part->p, upd.p, bnd->p, gain.p, dest.p,
-                               gwork.p, N, cand.p, st_, steal_of(ctx_)));
+           gkd::launch_gain_wl(g, kmax, lanes, wl.p, dc.hcnt, heavy.p, part->p, upd.p, bnd->p, gain.p, dest.p,
+                               dc.work, N, cand.p, st_, steal_of(ctx_)));
   if (heavy_rows)
     GK_STAGE(ctx_, GK_ST_GAIN_HEAVY, 0,
-             gkd::launch_gain_heavy(g, kmax, heavy.p, hcnt.p, part->p, upd.p, bnd->p, gain.p, dest.p, gwork.p,
+             gkd::launch_gain_heavy(g, kmax, heavy.p, dc.hcnt, part->p, upd.p, bnd->p, gain.p, dest.p, dc.work,
                                     cand.p, st_));
   const int64_t avg_deg = N > 0 ? (int64_t(g.nnz) + N - 1) / N : 0;
   const int64_t wl_items = std::min<int64_t>(N, int64_t(J) * M * (1 + 2 * avg_deg));
@@ -669,22 +701,22 @@ int Engine::refine_step(bool* worked) {
   s.lanes = lanes;
   s.heavy_rows = heavy_rows;
   s.wl_items = wl_items;
-  s.vjob = rs.vjob.p;
+  s.vjob = vjob.p;
   s.v_off = F.dv_off.p;
-  s.kk = dkk.p;
-  s.pw_off = dpw_off.p;
-  s.cap = dcap.p;
+  s.kk = dt.kk;
+  s.pw_off = dt.pw_off;
+  s.cap = dt.cap;
   s.part = part->p;
   s.bnd = bnd->p;
   s.gain = gain.p;
   s.dest = dest.p;
-  s.pw = dpw.p;
+  s.pw = dt.pw;
   s.upd = upd.p;
-  s.cut = dcut.p;
-  s.moved = dmoved.p;
-  s.paths = dpaths.p;
-  s.abytes = dab.p;
-  s.rounds = drounds.p;
+  s.cut = dt.cut;
+  s.moved = dc.moved;
+  s.paths = dc.paths;
+  s.abytes = dc.abytes;
+  s.rounds = dc.rounds;
   s.lastcnt = lastcnt.p;
   s.thr = dthr.p;
   s.active = active.p;
@@ -692,39 +724,31 @@ int Engine::refine_step(bool* worked) {
   s.sb = sb;
   s.xlist = xlist.p;
   s.wl = wl.p;
-  s.hcnt = hcnt.p;
+  s.hcnt = dc.hcnt;
   s.heavy = heavy.p;
-  s.status = status.p;
+  s.status = dc.status;
   s.hkey = hkey.p;
-  s.work = gwork.p;
+  s.work = dc.work;
   const double tr0 = now_ms();
   int ran = 0;
   GK_TRY(refine_rounds(ctx_, st_, s, kMaxRounds, false, graph_rounds_, &ran));
   rounds_ += ran;
   prof_ms_[5] += now_ms() - tr0;
-  std::vector<long long> hcut(J), hmoved(J), hpaths(3 * size_t(J));
-  std::vector<int32_t> hrounds(J), hlast(J);
-  std::vector<unsigned long long> hwork(2 * kGainSlots);
-  std::vector<long long> hab(J);
-  std::vector<unsigned long long> hsel(gkd::kSelectByteSlots);
-  GK_TRY(download({{hwork.data(), gwork.p, sizeof(unsigned long long) * hwork.size()},
-                   {hsel.data(), selbytes.p, sizeof(unsigned long long) * hsel.size()},
-                   {hab.data(), dab.p, sizeof(long long) * J},
-                   {hpaths.data(), dpaths.p, sizeof(long long) * 3 * J},
-                   {hcut.data(), dcut.p, sizeof(long long) * J},
-                   {hpw.data(), dpw.p, sizeof(int32_t) * hpw.size()},
-                   {hrounds.data(), drounds.p, sizeof(int32_t) * J},
-                   {hmoved.data(), dmoved.p, sizeof(long long) * J},
+  std::vector<char> hcnts(counter_bytes);
+  std::vector<int32_t> hlast(J);
+  GK_TRY(download({{htab.data(), dtab.p, table_bytes},
+                   {hcnts.data(), dcnt.p, counter_bytes},
                    {hlast.data(), lastcnt.p, sizeof(int32_t) * J}}));
+  const Counters hc = counters_at(hcnts.data());
   if (ctx_->cur) {
     unsigned long long wv = 0, we = 0;
     for (int i = 0; i < kGainSlots; ++i) {
-      wv += hwork[2 * i];
-      we += hwork[2 * i + 1];
+      wv += hc.work[2 * i];
+      we += hc.work[2 * i + 1];
     }
     ctx_->cur->stage_bytes[GK_ST_GAIN] += int64_t(28 * wv + 12 * we);
-    for (int32_t i = 0; i < J; ++i) ctx_->cur->stage_bytes[GK_ST_BALANCE] += hab[i];
-    for (unsigned long long b : hsel) ctx_->cur->stage_bytes[GK_ST_SELECT] += int64_t(b);
+    for (int32_t i = 0; i < J; ++i) ctx_->cur->stage_bytes[GK_ST_BALANCE] += hc.abytes[i];
+    for (int i = 2 * kGainSlots; i < kWork; ++i) ctx_->cur->stage_bytes[GK_ST_SELECT] += int64_t(hc.work[i]);
   }
   std::vector<UnpackDst> dst(J);
   std::vector<int32_t> done(J, 0);
@@ -732,12 +756,12 @@ int Engine::refine_step(bool* worked) {
   for (int32_t i = 0; i < J; ++i) {
     Job& j = *ids[i];
     gk_level_stats& ls = j.S.levels[j.cur];
-    ls.rounds += hrounds[i];
-    ls.moves += hmoved[i];
-    for (int q = 0; q < 3; ++q) j.S.round_paths[q] += hpaths[3 * size_t(i) + q];
-    ls.cut_after = hcut[i];
-    j.cut = hcut[i];
-    std::copy(hpw.begin() + pw_off[i], hpw.begin() + pw_off[i + 1], j.hpw.begin());
+    ls.rounds += hc.rounds[i];
+    ls.moves += hc.moved[i];
+    for (int q = 0; q < 3; ++q) j.S.round_paths[q] += hc.paths[3 * size_t(i) + q];
+    ls.cut_after = ht.cut[i];
+    j.cut = ht.cut[i];
+    std::copy(ht.pw + pw_off[i], ht.pw + pw_off[i + 1], j.hpw.begin());
     std::memset(&dst[i], 0, sizeof dst[i]);
     if (hlast[i] > 0) {
       // Still moving after this step's rounds: the level resumes next step.
@@ -766,7 +790,7 @@ int Engine::refine_step(bool* worked) {
   }
   if (any_done) {
     // Chunks of at most kCutChunk vertices of each finished job.
-    constexpr int32_t kCutChunk = 2048;
+    constexpr int32_t kCutChunk = 512;
     std::vector<int32_t> cj, cs, ce;
     for (int32_t i = 0; i < J; ++i) {
       if (!done[i]) continue;
@@ -785,16 +809,16 @@ int Engine::refine_step(bool* worked) {
     GK_TRY(upload(dce, ce.data(), ce.size()));
     GK_TRY(c64.alloc(P_, J));
     GK_TRY(pw64.alloc(P_, pw_off[J]));
-    gkd::fill<unsigned long long>(c64.p, 0ull, J, st_);
-    gkd::fill<unsigned long long>(pw64.p, 0ull, pw_off[J], st_);
-    GK_TRY(gkd::launch_unpack_part(J, ddst.p, F.dv_off.p, N, part->p, nullptr, st_));
+    GK_TRY(stage(c64.p, nullptr, sizeof(unsigned long long) * size_t(J)));
+    GK_TRY(stage(pw64.p, nullptr, sizeof(unsigned long long) * size_t(pw_off[J])));
+    GK_TRY(flush());
     int64_t cut_bytes = 0;
     for (size_t c = 0; c < cj.size(); ++c)
       cut_bytes += 16LL * (ce[c] - cs[c]) + 12LL * (F.e_off[cj[c] + 1] - F.e_off[cj[c]]) * (ce[c] - cs[c]) /
                                                std::max<int64_t>(1, F.v_off[cj[c] + 1] - F.v_off[cj[c]]);
     GK_STAGE(ctx_, GK_ST_CUT, cut_bytes,
-             gkd::launch_cut_chunks(static_cast<int32_t>(cj.size()), dcj.p, dcs.p, dce.p, kmax, dkk.p, g, part->p,
-                                    dpw_off.p, c64.p, pw64.p, st_));
+             gkd::launch_cut_chunks(static_cast<int32_t>(cj.size()), dcj.p, dcs.p, dce.p, kmax, dt.kk,
+                                    F.dv_off.p, g, part->p, dt.pw_off, ddst.p, c64.p, pw64.p, st_));
     std::vector<unsigned long long> hc64(J), hpw64(pw_off[J]);
     GK_TRY(download({{hc64.data(), c64.p, sizeof(unsigned long long) * J},
                      {hpw64.data(), pw64.p, sizeof(unsigned long long) * hpw64.size()}}));
@@ -952,6 +976,7 @@ int run_packed(gk_ctx* ctx, hipStream_t st, const gk_packed_csr* pk, const gk_pa
   {
     Buf<long long> dT;
     GK_TRY(dT.alloc(P, G));
+    GK_TRY(E.flush());
     GK_TRY(gkd::launch_job_sum(G, S0->dv_off.p, S0->vw, dT.p, st));
     GK_TRY(E.download({{T.data(), dT.p, sizeof(long long) * G}}));
   }

@@ -108,13 +108,6 @@ struct Job {
   }
 };
 
-// Refinement pack extras: vertex -> job slot, packed projection map and the
-// packed coarse partition / boundary.
-struct RefineSide {
-  Buf<int32_t> vjob, cmap, cpart, cbnd, cgain, cdest;
-  std::vector<int32_t> c_off;
-};
-
 class Engine {
  public:
   Engine(gk_ctx* ctx, hipStream_t st, int workers);
@@ -134,15 +127,15 @@ class Engine {
   // Called for each job right after it is finished and its partition written.
   std::function<int(Job&)> done_cb_;
 
+  // Copies to the device (src null: zeros) gather until flush(), which comes
+  // before the first kernel that reads or writes them: a step's many small
+  // arrays go up in one launch.
+  int stage(void* dst, const void* src, size_t bytes);
+  int flush();
   template <class T>
   int upload(Buf<T>& dst, const T* src, size_t n) {
     GK_TRY(dst.alloc(P_, static_cast<int64_t>(n)));
-    if (n == 0) return GK_OK;
-    void* h = nullptr;
-    GK_TRY(up_.get(st_, sizeof(T) * n, &h));
-    std::memcpy(h, src, sizeof(T) * n);
-    GK_HIP(hipMemcpyAsync(dst.p, h, sizeof(T) * n, hipMemcpyHostToDevice, st_));
-    return GK_OK;
+    return stage(dst.p, src, sizeof(T) * n);
   }
   int download(std::initializer_list<Fetch> items);
   // Refinement rounds replayed from a captured hipGraph (GK_FLAG_GRAPH_ROUNDS).
@@ -152,7 +145,9 @@ class Engine {
   static StoreP whole_store(const std::vector<const JLevel*>& lv);
   static gkd::PackSrc src_of(const JLevel& lv);
   int pack_copy(const std::vector<gkd::PackSrc>& src, const std::vector<int32_t>& nv,
-                const std::vector<int32_t>& ne, const std::vector<int32_t>* ncv, StoreP& out, RefineSide* rs);
+                const std::vector<int32_t>& ne, StoreP& out, const gkd::RefineStart* refine = nullptr);
+  // A pack's offsets, with its arrays allocated.
+  int pack_store(const std::vector<int32_t>& nv, const std::vector<int32_t>& ne, StoreP& out);
   void mark(Job& j, int phase);
   void finish_stats(Job& j, int64_t cut, int64_t tracked, const std::vector<int64_t>& pw);
   int coarsen_step(bool* worked);
@@ -167,6 +162,7 @@ class Engine {
   std::chrono::steady_clock::time_point t0_;
   Pinned& up_;  // the context's staging arenas
   Pinned& dl_;
+  gkd::Copies pending_;
   size_t ndone_ = 0;
   bool graph_rounds_ = false;
   int64_t steps_ = 0, rounds_ = 0;

@@ -253,6 +253,8 @@ class Pinned {
   ~Pinned();
   int get(hipStream_t st, size_t bytes, void** out);
   void drained() { used_ = 0; }
+  // Whether get hands out this many bytes without starting over.
+  bool fits(size_t bytes) const { return used_ + ((bytes + 255) & ~size_t(255)) <= cap_; }
 
  private:
   char* base_ = nullptr;
@@ -367,6 +369,10 @@ class Tuner {
 }  // namespace gkrt
 
 namespace gkrt {
+// Host arrays of up to kStageMax bytes move through pinned staging memory, in
+// pieces of kStagePiece.
+constexpr size_t kStageMax = size_t(16) << 20;
+constexpr size_t kStagePiece = size_t(1) << 20;
 // Pinned bytes of a context: fetch() staging, then the control words.
 constexpr size_t kPinFetch = 4096;
 constexpr size_t kPinCtl = 256;

@@ -109,12 +109,21 @@ int admit(gk_server* s, Engine* E, Request* r) {
   GK_TRY(S0->bv.alloc(P, r->n));
   GK_TRY(r->dout.alloc(P, r->n));
   // The host copies stay alive until the request finishes.
-  GK_HIP(hipMemcpyAsync(S0->bx.p, r->x.data(), sizeof(int32_t) * (size_t(r->n) + 1), hipMemcpyHostToDevice, st));
-  if (r->nnz) {
-    GK_HIP(hipMemcpyAsync(S0->ba.p, r->a.data(), sizeof(int32_t) * size_t(r->nnz), hipMemcpyHostToDevice, st));
-    GK_HIP(hipMemcpyAsync(S0->bw.p, r->w.data(), sizeof(int32_t) * size_t(r->nnz), hipMemcpyHostToDevice, st));
+  const size_t nb = sizeof(int32_t) * size_t(r->n), eb = sizeof(int32_t) * size_t(r->nnz);
+  const struct {
+    int32_t* dev;
+    const int32_t* host;
+    size_t bytes;
+  } arrays[4] = {{S0->bx.p, r->x.data(), nb + sizeof(int32_t)},
+                 {S0->ba.p, r->a.data(), eb},
+                 {S0->bw.p, r->w.data(), eb},
+                 {S0->bv.p, r->v.data(), nb}};
+  const bool staged = 2 * (nb + eb) <= kStageMax;
+  for (const auto& y : arrays) {
+    if (staged) GK_TRY(E->stage(y.dev, y.host, y.bytes));
+    else if (y.bytes) GK_HIP(hipMemcpyAsync(y.dev, y.host, y.bytes, hipMemcpyHostToDevice, st));
   }
-  GK_HIP(hipMemcpyAsync(S0->bv.p, r->v.data(), sizeof(int32_t) * size_t(r->n), hipMemcpyHostToDevice, st));
+  GK_TRY(E->flush());
   S0->xadj = S0->bx.p;
   S0->adj = S0->ba.p;
   S0->w = S0->bw.p;
@@ -144,12 +153,17 @@ void serve_loop(gk_server* s) {
   std::vector<Request*> running;
   auto make_engine = [s, st, &wp, &running]() {
     auto E = std::make_unique<Engine>(s->ctx, st, batch_workers(wp));
-    E->done_cb_ = [s, st, &running](Job& j) -> int {
+    Engine* engine = E.get();
+    E->done_cb_ = [s, st, engine, &running](Job& j) -> int {
       Request* r = static_cast<Request*>(j.user);
       r->part.resize(r->n);
-      if (r->n)
-        GK_HIP(hipMemcpyAsync(r->part.data(), r->dout.p, sizeof(int32_t) * size_t(r->n), hipMemcpyDeviceToHost, st));
-      GK_HIP(hipStreamSynchronize(st));
+      const size_t bytes = sizeof(int32_t) * size_t(r->n);
+      if (bytes <= kStageMax) {
+        GK_TRY(engine->download({{r->part.data(), r->dout.p, bytes}}));
+      } else {
+        GK_HIP(hipMemcpyAsync(r->part.data(), r->dout.p, bytes, hipMemcpyDeviceToHost, st));
+        GK_HIP(hipStreamSynchronize(st));
+      }
       r->dout.release();
       r->S = j.S;
       std::lock_guard<std::mutex> lk(s->m);
