@@ -28,24 +28,40 @@ int lanes_for_degree(double avg) {
 static inline int hip_status() { return hipGetLastError() == hipSuccess ? 0 : GK_ERR_HIP; }
 
 // --------------------------------------------------------------- matching
+constexpr int32_t kDegMore = 255;
+
 // matching_with_score (gkway/coarsen.hpp:39-78) with S lanes per vertex: the
 // lanes stride over the row, then reduce the packed preference
 // (weight desc, neighbour degree asc, neighbour id asc) by xor-shuffles.
 // Global thread slot gt serves vertex gt / S as lane gt % S of its group.
+// deg (may be null): the neighbours' degrees as bytes, kDegMore for that many
+// or more.
 template <int S>
 __device__ __forceinline__ void match_slot(int64_t gt, int32_t n, const int32_t* __restrict__ xadj,
                                            const int32_t* __restrict__ adj, const int32_t* __restrict__ w,
-                                           int32_t* __restrict__ cand) {
+                                           const uint8_t* __restrict__ deg, int32_t* __restrict__ cand) {
   const int32_t v = static_cast<int32_t>(gt / S);
   const int sub = static_cast<int>(gt % S);
   if (v >= n) return;
   int bw = 0, bd = 0, bu = v;
   const int s = xadj[v], e = xadj[v + 1];
-  for (int j = s + sub; j < e; j += S) {
-    const int u = adj[j];
-    const int wj = w[j];
-    const int d = xadj[u + 1] - xadj[u];
+  auto better = [&](int wj, int d, int u) {
     if (wj > bw || (wj == bw && (d < bd || (d == bd && u < bu)))) { bw = wj; bd = d; bu = u; }
+  };
+  if (deg) {
+    for (int j = s + sub; j < e; j += S) {
+      const int u = adj[j];
+      const int wj = w[j];
+      int d = deg[u];
+      if (d == kDegMore) d = xadj[u + 1] - xadj[u];
+      better(wj, d, u);
+    }
+  } else {
+    for (int j = s + sub; j < e; j += S) {
+      const int u = adj[j];
+      const int wj = w[j];
+      better(wj, xadj[u + 1] - xadj[u], u);
+    }
   }
 #pragma unroll
   for (int o = S / 2; o > 0; o >>= 1) {
@@ -58,25 +74,26 @@ __device__ __forceinline__ void match_slot(int64_t gt, int32_t n, const int32_t*
 template <int S, int B>
 __global__ void __launch_bounds__(B) k_match(int32_t n, const int32_t* __restrict__ xadj,
                                              const int32_t* __restrict__ adj,
-                                             const int32_t* __restrict__ w, int32_t* __restrict__ cand) {
-  match_slot<S>(int64_t(xcd_block()) * B + threadIdx.x, n, xadj, adj, w, cand);
+                                             const int32_t* __restrict__ w, const uint8_t* __restrict__ deg,
+                                             int32_t* __restrict__ cand) {
+  match_slot<S>(int64_t(xcd_block()) * B + threadIdx.x, n, xadj, adj, w, deg, cand);
 }
 
 // The same slots, taken from the work-stealing queues.
 template <int S, int B>
 __global__ void __launch_bounds__(B) k_match_ws(int32_t n, const int32_t* __restrict__ xadj,
                                                 const int32_t* __restrict__ adj,
-                                                const int32_t* __restrict__ w, int32_t* __restrict__ cand,
-                                                unsigned long long* __restrict__ ctr) {
+                                                const int32_t* __restrict__ w, const uint8_t* __restrict__ deg,
+                                                int32_t* __restrict__ cand, unsigned long long* __restrict__ ctr) {
   const int64_t sweeps = (int64_t(n) * S + 63) / 64;
-  steal_sweeps(ctr, sweeps, [&](int64_t sw) { match_slot<S>(sw * 64 + lane_id(), n, xadj, adj, w, cand); });
+  steal_sweeps(ctr, sweeps, [&](int64_t sw) { match_slot<S>(sw * 64 + lane_id(), n, xadj, adj, w, deg, cand); });
 }
 
 template <int S, int B>
-static void match_go(const DGraph& g, int32_t* cand, const Steal* ws, hipStream_t st) {
+static void match_go(const DGraph& g, const uint8_t* deg, int32_t* cand, const Steal* ws, hipStream_t st) {
   const unsigned grid = grid_for(int64_t(g.n) * S, B);
   if (!ws) {
-    gk_launch(k_match<S, B>, dim3(grid), dim3(B), 0, st, g.n, g.xadj, g.adj, g.w, cand);
+    gk_launch(k_match<S, B>, dim3(grid), dim3(B), 0, st, g.n, g.xadj, g.adj, g.w, deg, cand);
     return;
   }
   const unsigned pg = steal_grid(reinterpret_cast<const void*>(&k_match_ws<S, B>), B, *ws, grid);
@@ -85,28 +102,54 @@ static void match_go(const DGraph& g, int32_t* cand, const Steal* ws, hipStream_
     fill<unsigned long long>(ws->ctr, 0ull, kStealWords, st);
     ctr = ws->ctr;
   }
-  gk_launch(k_match_ws<S, B>, dim3(pg), dim3(B), 0, st, g.n, g.xadj, g.adj, g.w, cand, ctr);
+  gk_launch(k_match_ws<S, B>, dim3(pg), dim3(B), 0, st, g.n, g.xadj, g.adj, g.w, deg, cand, ctr);
 }
 
 template <int B>
-static void match_block(const DGraph& g, int lanes, int32_t* cand, const Steal* ws, hipStream_t st) {
+static void match_block(const DGraph& g, int lanes, const uint8_t* deg, int32_t* cand, const Steal* ws,
+                        hipStream_t st) {
   switch (lanes) {
-    case 1: match_go<1, B>(g, cand, ws, st); break;
-    case 2: match_go<2, B>(g, cand, ws, st); break;
-    case 4: match_go<4, B>(g, cand, ws, st); break;
-    case 8: match_go<8, B>(g, cand, ws, st); break;
-    case 16: match_go<16, B>(g, cand, ws, st); break;
-    case 32: match_go<32, B>(g, cand, ws, st); break;
-    default: match_go<64, B>(g, cand, ws, st); break;
+    case 1: match_go<1, B>(g, deg, cand, ws, st); break;
+    case 2: match_go<2, B>(g, deg, cand, ws, st); break;
+    case 4: match_go<4, B>(g, deg, cand, ws, st); break;
+    case 8: match_go<8, B>(g, deg, cand, ws, st); break;
+    case 16: match_go<16, B>(g, deg, cand, ws, st); break;
+    case 32: match_go<32, B>(g, deg, cand, ws, st); break;
+    default: match_go<64, B>(g, deg, cand, ws, st); break;
   }
 }
 
-int launch_match(const DGraph& g, int lanes, int block, int32_t* cand, hipStream_t st, const Steal* ws) {
+// Every entry's degree is a random gather: the bound of the matching of a large
+// mesh numbered without locality (2^22 vertices, 25 M entries: 372 us, 67 G/s
+// out of 16 MB of row bounds).  From kDegTable vertices on the row bounds are
+// larger than an XCD's 4 MB L2 and a table of bytes pays (the same mesh: 209 us
+// and 9 for the table; a DAG of 1 M vertices, 32 us, is as fast without).
+__global__ void __launch_bounds__(256) k_deg_table(int32_t n, const int32_t* __restrict__ xadj,
+                                                   uint8_t* __restrict__ deg) {
+  const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  int32_t x[5];
+  uint32_t packed = 0;
+#pragma unroll
+  for (int j = 0; j < 5; ++j) x[j] = xadj[i + j <= n ? i + j : n];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) packed |= uint32_t(min(x[j + 1] - x[j], kDegMore)) << (8 * j);
+  *reinterpret_cast<uint32_t*>(deg + i) = packed;
+}
+
+int launch_deg_table(const DGraph& g, uint8_t* deg, hipStream_t st) {
+  if (g.n <= 0) return 0;
+  k_deg_table<<<grid_for(g.n, 1024), 256, 0, st>>>(g.n, g.xadj, deg);
+  return hip_status();
+}
+
+int launch_match(const DGraph& g, int lanes, int block, const uint8_t* deg, int32_t* cand, hipStream_t st,
+                 const Steal* ws) {
   if (g.n <= 0) return 0;
   switch (block) {
-    case 128: match_block<128>(g, lanes, cand, ws, st); break;
-    case 512: match_block<512>(g, lanes, cand, ws, st); break;
-    default: match_block<256>(g, lanes, cand, ws, st); break;
+    case 128: match_block<128>(g, lanes, deg, cand, ws, st); break;
+    case 512: match_block<512>(g, lanes, deg, cand, ws, st); break;
+    default: match_block<256>(g, lanes, deg, cand, ws, st); break;
   }
   return hip_status();
 }
@@ -163,11 +206,13 @@ int launch_jump_round(int32_t n, const int32_t* cand, const int32_t* next_in, co
   return hip_status();
 }
 
-// One vertex more in the component of key: its largest id in comp[key].x, its
-// members counted in comp[key].y; returns v's (arbitrary) place among them.
-// Components are small, so the atomics rarely collide; lanes that share the
-// first active lane's key (hubs, stars) are added with one atomic pair, since
-// same-address atomics serialise.
+// One vertex more in the component of key, its root pair's larger id and so one
+// of its members: the largest id above key in comp[key].x (0: none), its members
+// counted in comp[key].y; returns v's (arbitrary) place among them.  Most
+// vertices are not above their key, which saves their atomicMax (in a random
+// numbering four of five).  Components are small, so the atomics rarely collide;
+// lanes that share the first active lane's key (hubs, stars) are added with one
+// atomic pair, since same-address atomics serialise.
 __device__ __forceinline__ int32_t comp_add(int2* __restrict__ comp, int32_t key, int32_t v, bool live) {
   const uint64_t lm = ballot(live);
   if (lm == 0) return 0;
@@ -178,14 +223,14 @@ __device__ __forceinline__ int32_t comp_add(int2* __restrict__ comp, int32_t key
     int32_t base = 0;
     const int lead = 63 - __clzll(static_cast<long long>(same));  // ids grow with the lane: its id is the largest
     if (lane_id() == lead) {
-      atomicMax(&comp[key].x, v);
+      if (v > key) atomicMax(&comp[key].x, v);
       base = atomicAdd(&comp[key].y, popc64(same));
     }
     base = __shfl(base, lead, 64);
     if ((same >> lane_id()) & 1ull) return base + popc64(same & lanemask_lt());
   }
   if (live) {
-    atomicMax(&comp[key].x, v);
+    if (v > key) atomicMax(&comp[key].x, v);
     slot = atomicAdd(&comp[key].y, 1);
   }
   return slot;
@@ -197,11 +242,13 @@ __device__ __forceinline__ int32_t comp_add(int2* __restrict__ comp, int32_t key
 // rarely more than ten, so the walk reads cand[] about three times per vertex
 // where the jumping rounds read and write pointer and distance arrays four
 // times over.  On a 2^22-vertex mesh numbered at random (every read a cache
-// line): 327 us with the component atomics, which bound it, where init and
-// jumping rounds took 60 + 269 us and the label kernels 148 + 98 us (now 64).  flags[r] is set when some vertex is more than 2^r hops
-// away, which tells the jumping rounds that the walk replaces; a vertex more
-// than kWalkMax hops away sets flags[kWalkBits], and the caller falls back to
-// the jumping rounds (long chains would make the walk linear).
+// line): 244 us with the component atomics, which bound it (327 us with an
+// atomicMax for every vertex), where init and jumping rounds took 60 + 269 us
+// and the label kernels 148 + 98 us (now 64).  flags[r] is set when some vertex
+// is more than 2^r hops away, which tells the jumping rounds that the walk
+// replaces; a vertex more than kWalkMax hops away sets flags[kWalkBits], and
+// the caller falls back to the jumping rounds (long chains would make the walk
+// linear).
 __global__ void __launch_bounds__(256) k_walk(int32_t n, const int32_t* __restrict__ cand, int2* __restrict__ comp,
                                               int32_t* __restrict__ key_out, int32_t* __restrict__ dist,
                                               int32_t* __restrict__ slot, int32_t* __restrict__ flags) {
@@ -218,7 +265,12 @@ __global__ void __launch_bounds__(256) k_walk(int32_t n, const int32_t* __restri
       ++d;
     }
     key = max(a, b);
-    if (c != a) d = kWalkMax + 1;
+    if (c != a) {
+      // Unresolved: a component of its own.  A key must be a member of its
+      // component, or the members' places would not fit their groups.
+      key = v;
+      d = kWalkMax + 1;
+    }
     key_out[v] = key;
     dist[v] = d;
   }
@@ -270,9 +322,11 @@ __global__ void __launch_bounds__(256) k_label_size(int32_t n, const int32_t* ke
                                                     int32_t* label, int32_t* __restrict__ size) {
   const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
   if (v >= n) return;
-  const int2 c = comp[key[v]];
-  label[v] = c.x;
-  size[v] = c.x == int32_t(v) ? c.y : 0;
+  const int32_t k = key[v];
+  const int2 c = comp[k];
+  const int32_t l = max(c.x, k);
+  label[v] = l;
+  size[v] = l == int32_t(v) ? c.y : 0;
 }
 
 int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* label, int32_t* size,
@@ -1358,12 +1412,16 @@ __global__ void __launch_bounds__(256) k_contract_copy(int32_t nc, const int32_t
                                                        const int32_t* __restrict__ cxadj,
                                                        const int32_t* __restrict__ tadj,
                                                        const int32_t* __restrict__ tw,
-                                                       int32_t* __restrict__ cadj, int32_t* __restrict__ cw) {
+                                                       int32_t* cadj, int32_t* cw, int32_t* xout) {
   const int64_t gt = int64_t(blockIdx.x) * 256 + threadIdx.x;
   const int64_t c = gt / 8;
   const int sub = static_cast<int>(gt % 8);
   if (c >= nc) return;
   const int32_t s = toff[c], d = cxadj[c], l = len[c];
+  if (xout && sub == 0) {
+    xout[c] = d;
+    if (c == nc - 1) xout[nc] = d + l;
+  }
   for (int32_t t = sub; t < l; t += 8) {
     cadj[d + t] = tadj[s + t];
     cw[d + t] = tw[s + t];
@@ -1371,10 +1429,10 @@ __global__ void __launch_bounds__(256) k_contract_copy(int32_t nc, const int32_t
 }
 
 int launch_contract_copy(int32_t nc, const int32_t* toff, const int32_t* len, const int32_t* cxadj,
-                         const int32_t* tadj, const int32_t* tw, int32_t* cadj, int32_t* cw,
+                         const int32_t* tadj, const int32_t* tw, int32_t* cadj, int32_t* cw, int32_t* xout,
                          hipStream_t st) {
   if (nc <= 0) return 0;
-  k_contract_copy<<<grid_for(int64_t(nc) * 8, 256), 256, 0, st>>>(nc, toff, len, cxadj, tadj, tw, cadj, cw);
+  k_contract_copy<<<grid_for(int64_t(nc) * 8, 256), 256, 0, st>>>(nc, toff, len, cxadj, tadj, tw, cadj, cw, xout);
   return hip_status();
 }
 

@@ -231,9 +231,10 @@ int coarse_ids(gk_ctx* ctx, hipStream_t st, const DGraph& g, const int32_t* cand
 
 // Contraction of g under cmap, with its members by coarse id (m: first places,
 // rows, and, unless null, weights), into the coarse level c; with weights also
-// the coarse weights into c.vw (allocated by the caller).
+// the coarse weights into c.vw (allocated by the caller).  With out the coarse
+// CSR goes to its arrays, written after everything else has been read.
 int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, const int32_t* cmap, const Members& m,
-                   Level& c) {
+                   Level& c, const CsrOut* out) {
   Pool& P = ctx->pool;
   Buf<int32_t> toff, lists, scratch, tadj, tw, len;
   Buf<int2> desc;
@@ -339,13 +340,16 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
     GK_TRY(scan_lengths());
   }
   const int32_t cnnz = words[0];
-  GK_TRY(c.adj.alloc(P, cnnz));
-  GK_TRY(c.w.alloc(P, cnnz));
+  if (!out) {
+    GK_TRY(c.adj.alloc(P, cnnz));
+    GK_TRY(c.w.alloc(P, cnnz));
+  }
   // Row merge: member rows and the cmap gathers read once, merged rows
   // written once (known now that cnnz is).
   if (ctx->cur) ctx->cur->stage_bytes[GK_ST_CONTRACT] += 8LL * g.n + 20LL * nc + 12LL * g.nnz + 8LL * cnnz;
   GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc + 16LL * cnnz,
-           gkd::launch_contract_copy(nc, toff.p, len.p, c.xadj.p, tadj.p, tw.p, c.adj.p, c.w.p, st));
+           gkd::launch_contract_copy(nc, toff.p, len.p, c.xadj.p, tadj.p, tw.p, out ? out->adj : c.adj.p,
+                                     out ? out->w : c.w.p, out ? out->xadj : nullptr, st));
   c.g.n = nc;
   c.g.nnz = cnnz;
   c.g.xadj = c.xadj.p;
@@ -354,10 +358,21 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
   return GK_OK;
 }
 
+// Degrees as bytes, for graphs on which the matching is faster with them; left
+// out where the pool has no room (they only save time).
+int degree_table(gk_ctx* ctx, hipStream_t st, const DGraph& g, Buf<uint8_t>& deg) {
+  if (g.n < gkd::kDegTable || deg.alloc(ctx->pool, (int64_t(g.n) + 3) & ~int64_t(3)) != GK_OK) return GK_OK;
+  return gkd::launch_deg_table(g, deg.p, st);
+}
+
 int match_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t* cand) {
   const int def = gkd::lanes_for_degree(g.n ? double(g.nnz) / g.n : 0.0);
   Tuner::Shape shape{def, 256};
-  auto run = [&](const Tuner::Shape& x) { return gkd::launch_match(g, x.lanes, x.block, cand, st, steal_of(ctx)); };
+  Buf<uint8_t> deg;
+  GK_TRY(degree_table(ctx, st, g, deg));
+  auto run = [&](const Tuner::Shape& x) {
+    return gkd::launch_match(g, x.lanes, x.block, deg.p, cand, st, steal_of(ctx));
+  };
   if (ctx->autotune && g.nnz >= kTuneMinEntries) {
     const uint64_t key = Tuner::key(0, g.n, g.nnz);
     if (const Tuner::Shape* s = ctx->tuner.find(key)) {
@@ -1200,7 +1215,9 @@ int gk_k_match(gk_ctx* ctx, const gk_csr* dg, int32_t* cand, void* stream) {
   DeviceGuard guard(ctx->device);
   hipStream_t st = pick(ctx, stream);
   DGraph g = dview(dg);
-  GK_TRY(gkd::launch_match(g, gkd::lanes_for_degree(g.n ? double(g.nnz) / g.n : 0.0), 256, cand, st));
+  Buf<uint8_t> deg;
+  GK_TRY(gkrt::degree_table(ctx, st, g, deg));
+  GK_TRY(gkd::launch_match(g, gkd::lanes_for_degree(g.n ? double(g.nnz) / g.n : 0.0), 256, deg.p, cand, st));
   GK_HIP(hipStreamSynchronize(st));
   return GK_OK;
 }
@@ -1290,12 +1307,9 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   if (nc2 != nc) { gkh::set_error("cmap is not onto [0, nc)"); return GK_ERR_ARG; }
   Level c;
   DGraph g = dview(dg);
-  GK_TRY(contract_stage(ctx, st, g, nc, cmap, m, c));
-  GK_HIP(hipMemcpyAsync(cxadj, c.g.xadj, sizeof(int32_t) * (nc + 1), hipMemcpyDeviceToDevice, st));
-  if (c.g.nnz) {
-    GK_HIP(hipMemcpyAsync(cadjncy, c.g.adj, sizeof(int32_t) * c.g.nnz, hipMemcpyDeviceToDevice, st));
-    GK_HIP(hipMemcpyAsync(cadjwgt, c.g.w, sizeof(int32_t) * c.g.nnz, hipMemcpyDeviceToDevice, st));
-  }
+  const CsrOut out{cxadj, cadjncy, cadjwgt};
+  GK_TRY(contract_stage(ctx, st, g, nc, cmap, m, c, &out));
+  if (nc == 0) gkd::fill<int32_t>(cxadj, 0, 1, st);
   GK_HIP(hipStreamSynchronize(st));
   *cnnz = c.g.nnz;
   return GK_OK;

@@ -69,7 +69,11 @@ int lanes_for_degree(double avg_deg);
 // lanes per vertex (1..64) and block size (128, 256 or 512 threads) change
 // only the launch shape, never the result.
 // ws (may be null): run as a persistent work-stealing launch (same result).
-int launch_match(const DGraph& g, int lanes, int block, int32_t* cand, hipStream_t st,
+// deg (may be null): the neighbours' degrees from launch_deg_table (n bytes,
+// rounded up to a multiple of 4), worth while from kDegTable vertices on.
+constexpr int32_t kDegTable = 1 << 20;
+int launch_deg_table(const DGraph& g, uint8_t* deg, hipStream_t st);
+int launch_match(const DGraph& g, int lanes, int block, const uint8_t* deg, int32_t* cand, hipStream_t st,
                  const Steal* ws = nullptr);
 // Pointer jumping over the candidate pseudo-forest.
 int launch_jump_init(int32_t n, const int32_t* cand, int32_t* next, int32_t* dist, hipStream_t st);
@@ -177,8 +181,9 @@ int launch_contract_big_merge(const int32_t* rows, int32_t nrows, const int32_t*
                               const uint64_t* keys, const int32_t* vals, const int32_t* toff,
                               int32_t* tadj, int32_t* tw, int32_t* len, hipStream_t st);
 // Phase 3: copy the merged rows to their final CSR slots.
+// xout (may be null): cxadj's nc + 1 entries once more.
 int launch_contract_copy(int32_t nc, const int32_t* toff, const int32_t* len, const int32_t* cxadj,
-                         const int32_t* tadj, const int32_t* tw, int32_t* cadj, int32_t* cw,
+                         const int32_t* tadj, const int32_t* tw, int32_t* cadj, int32_t* cw, int32_t* xout,
                          hipStream_t st);
 // Big-row prefix (boff = exclusive scan of the big rows' bounds ub).
 int launch_big_offsets(const int32_t* rows, const int32_t* ub, int32_t nrows, int32_t* boff, int32_t* scratch,

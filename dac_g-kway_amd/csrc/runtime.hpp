@@ -561,6 +561,11 @@ struct Groups {
   static int32_t rounds(const int32_t* words);
 };
 
+// Where a caller wants a coarse CSR.
+struct CsrOut {
+  int32_t *xadj, *adj, *w;
+};
+
 // Members by coarse id: first place of every coarse id, and in member order
 // the vertices, their rows (start, length) and their weights; ctl: the
 // grouping's control words, then a contraction's row class counters (zero).
@@ -581,7 +586,8 @@ struct MemberOut {
 int coarse_ids(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, const int32_t* cand, int32_t G, bool want_order,
                int32_t* cmap, Members& m, int32_t* nc, int32_t* rounds);
 int contract_stage(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, int32_t nc, const int32_t* cmap,
-                   const Members& m, Level& c);
+                   const Members& m, Level& c, const CsrOut* out = nullptr);
+int degree_table(gk_ctx* ctx, hipStream_t st, const gkd::DGraph& g, Buf<uint8_t>& deg);
 // Lanes per vertex of the gain pass for this graph's average degree.
 int gain_lanes(const gkd::DGraph& g);
 // Candidate matching with the context's tuned launch shape (tuned on first
