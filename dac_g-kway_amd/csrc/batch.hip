@@ -289,14 +289,13 @@ int launch_unpack_part(int32_t nj, const UnpackDst* dst, const int32_t* v_off, i
 // (gkway/uncoarsen.hpp:111-173) with the cap and part weights of the vertex's
 // job, over the candidate bitmask kept by the gain kernels (boundary vertices
 // with positive gain), so vertices outside the mask cost one bit of a
-// coalesced load.  k_select_fit turns the candidates into the movable set
-// (move fits the cap); k_select_list keeps the movable vertices with no
-// smaller-id movable neighbour, as a bitmask; a scan turns
+// coalesced load.  k_select_list keeps the movable candidates (move fits the
+// cap) with no smaller-id movable neighbour, as a bitmask; a scan turns
 // the bitmask into a list ordered by vertex id, in which every job's selected
 // vertices form one slice.  No kernel of the selection shares a counter
 // between waves (same-address atomics serialise in L2).  vjob == null: one
 // job.
-// Candidate bitmask words read per wave by k_select_fit / k_select_list, and
+// Candidate bitmask words read per wave by k_select_list, and
 // per 256-thread block.
 constexpr int kSelectWords = 8;
 constexpr int kSelectBlockWords = 4 * kSelectWords;
@@ -333,24 +332,40 @@ __device__ __forceinline__ void deal_bit(int incl, uint64_t word, int r, int* wi
   *bit_out = nth_set_bit(wd, r - (wi > 0 ? before : 0));
 }
 
-// Movable set of a round: the candidates (boundary, positive gain) whose move
-// fits their job's cap, as a bitmask.  Each wave reads kSelectWords words of
-// the candidate mask with one load and deals their set bits out to its lanes,
-// 64 per pass; the movable bits are gathered in LDS and written back for
-// every word.  Thread 0 also clears the worklist counters and the round's
-// move counter, which only the round kernel adds to.
-__global__ void __launch_bounds__(256) k_select_fit(int32_t n, const int32_t* __restrict__ vw,
-                                                    const int32_t* __restrict__ vjob,
-                                                    const int32_t* __restrict__ dest,
-                                                    const int32_t* __restrict__ pw,
-                                                    const int32_t* __restrict__ pw_off,
-                                                    const long long* __restrict__ cap,
-                                                    const uint64_t* __restrict__ cand,
-                                                    uint64_t* __restrict__ movable, int32_t* __restrict__ reset,
-                                                    int32_t* __restrict__ active,
-                                                    unsigned long long* __restrict__ abytes) {
-  __shared__ unsigned long long mw[4][kSelectWords];
-  __shared__ int32_t wtot[4];
+// Selection of a round: a candidate (boundary, positive gain) is movable when
+// its move fits its job's cap, and a movable vertex is selected when no
+// smaller-id neighbour is movable.  Each wave reads kSelectWords words of the
+// candidate mask with one load and deals their set bits out to its lanes, 64
+// per pass.  A neighbour's candidate bit is looked up first, and only for the
+// few that are candidates whether their move fits, so no second launch over a
+// finished movable mask is needed (that took 5 us and a gap of 2 a round on a
+// mesh of 2 M vertices).  Only vertices with gain >= thr[job] are tested; the
+// others get a bit in defbits, and the round kernel tests them, against the
+// movable mask, only when fewer than M were selected (every key above the
+// threshold beats every key below it).  A lane tests a row of up to
+// kSelectShortRow entries itself; longer rows of a dealing pass are then tested
+// one after another by the whole wave, 64 neighbours per step.  Results are
+// bitmask words (movable, selbits, defbits), all written, so no counter is
+// shared between waves.  Thread 0 also clears the worklist counters and the
+// round's move counter, which only the round kernel adds to.
+__global__ void __launch_bounds__(256) k_select_list(int32_t n, const int32_t* __restrict__ xadj,
+                                                     const int32_t* __restrict__ adj,
+                                                     const int32_t* __restrict__ vw,
+                                                     const int32_t* __restrict__ vjob,
+                                                     const int32_t* __restrict__ gain,
+                                                     const int32_t* __restrict__ dest,
+                                                     const int32_t* __restrict__ pw,
+                                                     const int32_t* __restrict__ pw_off,
+                                                     const long long* __restrict__ cap,
+                                                     const int32_t* __restrict__ thr,
+                                                     const uint64_t* __restrict__ cand,
+                                                     uint64_t* __restrict__ movable, uint64_t* __restrict__ selbits,
+                                                     uint64_t* __restrict__ defbits, int32_t* __restrict__ bsum,
+                                                     int32_t* __restrict__ reset, int32_t* __restrict__ active,
+                                                     unsigned long long* __restrict__ abytes) {
+  __shared__ unsigned long long sw[4][3][kSelectWords];  // selected, deferred, movable
+  __shared__ int32_t wsum[4];
+  __shared__ long long wbytes[4];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     reset[0] = 0;
     reset[1] = 0;
@@ -358,7 +373,11 @@ __global__ void __launch_bounds__(256) k_select_fit(int32_t n, const int32_t* __
   }
   const int lane = lane_id();
   const int wv = threadIdx.x >> 6;
-  if (lane < kSelectWords) mw[wv][lane] = 0;
+  if (lane < kSelectWords) {
+    sw[wv][0][lane] = 0;
+    sw[wv][1][lane] = 0;
+    sw[wv][2][lane] = 0;
+  }
   __syncthreads();
   const int64_t nwords = (int64_t(n) + 63) >> 6;
   const int64_t w0 = ((int64_t(blockIdx.x) * 256 + threadIdx.x) >> 6) * kSelectWords;
@@ -366,62 +385,8 @@ __global__ void __launch_bounds__(256) k_select_fit(int32_t n, const int32_t* __
   if (lane < kSelectWords && w0 + lane < nwords) word = cand[w0 + lane];
   const int incl = wave_incl_scan(popc64(word));
   const int total = __shfl(incl, kSelectWords - 1, 64);
-  for (int base = 0; base < total; base += 64) {
-    const int r = base + lane;
-    int wi, bit;
-    deal_bit(incl, word, r, &wi, &bit);
-    if (r < total) {
-      const int32_t v = int32_t(((w0 + wi) << 6) + bit);
-      const int32_t j = vjob ? vjob[v] : 0;
-      if ((long long)pw[pw_off[j] + dest[v]] + vw[v] <= cap[j]) atomicOr(&mw[wv][wi], 1ull << bit);
-    }
-  }
-  if (lane == 0) wtot[wv] = total;
-  __syncthreads();
-  if (lane < kSelectWords && w0 + lane < nwords) movable[w0 + lane] = mw[wv][lane];
-  // Algorithmic bytes: the block's candidate and movable words, and per
-  // candidate its job, destination, part weight and vertex weight.
-  if (abytes && threadIdx.x == 0)
-    atomicAdd(&abytes[blockIdx.x % kSelectByteSlots],
-              (unsigned long long)(16 * kSelectBlockWords + 16 * (wtot[0] + wtot[1] + wtot[2] + wtot[3])));
-}
-
-// Selection proper: a movable vertex is selected when no smaller-id
-// neighbour is movable (one bit per neighbour).  Same dealing of the movable
-// mask's bits to lanes as k_select_fit.  Only vertices with gain >= thr[job]
-// are tested; the others get a bit in defbits, and the round kernel tests
-// them only when fewer than M were selected (every key above the threshold
-// beats every key below it).  A lane tests a row of up to kSelectShortRow
-// entries itself; longer rows of a dealing pass are then tested one after
-// another by the whole wave, 64 neighbours per step.  Results are bitmask
-// words (selbits, defbits), all written, so no counter is shared between
-// waves.
-__global__ void __launch_bounds__(256) k_select_list(int32_t n, const int32_t* __restrict__ xadj,
-                                                     const int32_t* __restrict__ adj,
-                                                     const int32_t* __restrict__ vjob,
-                                                     const int32_t* __restrict__ gain,
-                                                     const int32_t* __restrict__ thr,
-                                                     const uint64_t* __restrict__ movable,
-                                                     uint64_t* __restrict__ selbits, uint64_t* __restrict__ defbits,
-                                                     int32_t* __restrict__ bsum,
-                                                     unsigned long long* __restrict__ abytes) {
-  __shared__ unsigned long long sw[4][2][kSelectWords];
-  __shared__ int32_t wsum[4];
-  __shared__ long long wbytes[4];
-  const int lane = lane_id();
-  const int wv = threadIdx.x >> 6;
-  if (lane < kSelectWords) {
-    sw[wv][0][lane] = 0;
-    sw[wv][1][lane] = 0;
-  }
-  __syncthreads();
-  const int64_t nwords = (int64_t(n) + 63) >> 6;
-  const int64_t w0 = ((int64_t(blockIdx.x) * 256 + threadIdx.x) >> 6) * kSelectWords;
-  uint64_t word = 0;
-  if (lane < kSelectWords && w0 + lane < nwords) word = movable[w0 + lane];
-  const int incl = wave_incl_scan(popc64(word));
-  const int total = __shfl(incl, kSelectWords - 1, 64);
   long long tested = 0;  // row entries of the tested vertices
+  int fitting = 0;       // movable vertices
   for (int base = 0; base < total; base += 64) {
     const int r = base + lane;
     int wi, bit;
@@ -429,31 +394,45 @@ __global__ void __launch_bounds__(256) k_select_list(int32_t n, const int32_t* _
     int32_t v = 0, s = 0, e = 0;
     int which = -1;  // 0 selected, 1 deferred
     bool long_row = false;
+    const int32_t* pj = pw;  // part weights and cap of the vertex's job, and so of its neighbours'
+    long long cj = 0;
+    auto fits = [&](int32_t u) { return (long long)pj[dest[u]] + vw[u] <= cj; };
     if (r < total) {
       v = int32_t(((w0 + wi) << 6) + bit);
       const int32_t j = vjob ? vjob[v] : 0;
+      pj = pw + pw_off[j];
+      cj = cap[j];
       s = xadj[v];
       e = xadj[v + 1];
-      if (gain[v] < thr[j]) {
-        which = 1;
-      } else if (e - s > kSelectShortRow) {
-        tested += e - s;
-        long_row = true;
-      } else {
-        tested += e - s;
-        // eight neighbours per step: their ids, then their movable bits
-        bool sel = true;
-        for (int32_t x = s; x < e && sel; x += 8) {
-          int32_t u[8];
+      if (fits(v)) {
+        ++fitting;
+        atomicOr(&sw[wv][2][wi], 1ull << bit);
+        if (gain[v] < thr[j]) {
+          which = 1;
+        } else if (e - s > kSelectShortRow) {
+          tested += e - s;
+          long_row = true;
+        } else {
+          tested += e - s;
+          // eight neighbours per step: their ids, their candidate bits, and
+          // whether those that are candidates fit
+          bool sel = true;
+          for (int32_t x = s; x < e && sel; x += 8) {
+            int32_t u[8];
+            uint32_t c = 0;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) u[i] = x + i < e ? adj[x + i] : v;
+            for (int i = 0; i < 8; ++i) u[i] = x + i < e ? adj[x + i] : v;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint64_t mwd = movable[u[i] >> 6];
-            if (u[i] < v && ((mwd >> (u[i] & 63)) & 1ull)) sel = false;
+            for (int i = 0; i < 8; ++i) {
+              const uint64_t cw = cand[u[i] >> 6];
+              if (u[i] < v && ((cw >> (u[i] & 63)) & 1ull)) c |= 1u << i;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              if (((c >> i) & 1u) && sel && fits(u[i])) sel = false;
           }
+          if (sel) which = 0;
         }
-        if (sel) which = 0;
       }
     }
     // The pass's long rows, one at a time, by the whole wave.
@@ -462,13 +441,16 @@ __global__ void __launch_bounds__(256) k_select_list(int32_t n, const int32_t* _
       const int src = __ffsll(static_cast<long long>(lm)) - 1;
       lm &= lm - 1;
       const int32_t lv = __shfl(v, src, 64), ls = __shfl(s, src, 64), le = __shfl(e, src, 64);
+      const int32_t lj = vjob ? vjob[lv] : 0;
+      const int32_t* lp = pw + pw_off[lj];
+      const long long lc = cap[lj];
       bool blocked = false;
       for (int32_t x0 = ls; x0 < le && !blocked; x0 += 64) {
         const int32_t x = x0 + lane;
         bool b = false;
         if (x < le) {
           const int32_t u = adj[x];
-          b = u < lv && ((movable[u >> 6] >> (u & 63)) & 1ull);
+          b = u < lv && ((cand[u >> 6] >> (u & 63)) & 1ull) && (long long)lp[dest[u]] + vw[u] <= lc;
         }
         blocked = ballot(b) != 0;
       }
@@ -481,24 +463,27 @@ __global__ void __launch_bounds__(256) k_select_list(int32_t n, const int32_t* _
   if (lane < kSelectWords && w0 + lane < nwords) {
     selbits[w0 + lane] = sw[wv][0][lane];
     defbits[w0 + lane] = sw[wv][1][lane];
+    movable[w0 + lane] = sw[wv][2][lane];
     c = popc64(sw[wv][0][lane]);
   }
   // selected vertices of the block's kSelectBlockWords words
   c = wave_sum(c);
   tested = wave_sum64(tested);
+  fitting = wave_sum(fitting);
   if (lane == 0) {
     wsum[wv] = c;
-    // movable words read, selected and deferred words written; per movable
-    // vertex its row bounds, job and gain, per tested entry the neighbour id
-    // and one movable bit
-    wbytes[wv] = 8LL * total + 4LL * tested + tested / 8;
+    // per candidate its job, destination, part weight and vertex weight, per
+    // movable vertex its row bounds, job and gain, per tested entry the
+    // neighbour id and one movable bit
+    wbytes[wv] = 16LL * total + 8LL * fitting + 4LL * tested + tested / 8;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     bsum[blockIdx.x] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    // and the block's candidate, movable, selected and deferred words
     if (abytes)
       atomicAdd(&abytes[blockIdx.x % kSelectByteSlots],
-                (unsigned long long)(24LL * kSelectBlockWords + wbytes[0] + wbytes[1] + wbytes[2] + wbytes[3]));
+                (unsigned long long)(40LL * kSelectBlockWords + wbytes[0] + wbytes[1] + wbytes[2] + wbytes[3]));
   }
 }
 
@@ -570,10 +555,8 @@ int launch_select_list(const DGraph& g, const int32_t* vjob, const int32_t* gain
   const int64_t nwords = (int64_t(g.n) + 63) / 64;
   const int64_t waves = (nwords + kSelectWords - 1) / kSelectWords;
   const unsigned grid = grid_for(waves * 64, 256);
-  gk_launch(k_select_fit, dim3(grid), dim3(256), 0, st, g.n, g.vw, vjob, dest, pw, pw_off, cap, cand, sb.movable,
-            reset, active, sb.abytes);
-  gk_launch(k_select_list, dim3(grid), dim3(256), 0, st, g.n, g.xadj, g.adj, vjob, gain, thr, sb.movable, sb.selbits,
-            sb.defbits, sb.scratch, sb.abytes);
+  gk_launch(k_select_list, dim3(grid), dim3(256), 0, st, g.n, g.xadj, g.adj, g.vw, vjob, gain, dest, pw, pw_off, cap,
+            thr, cand, sb.movable, sb.selbits, sb.defbits, sb.scratch, reset, active, sb.abytes);
   gk_launch(k_sel_scatter, dim3(grid_for(nwords, kScatterWords)), dim3(256), 0, st, nwords, sb.selbits, sb.scratch,
             sb.wpos, sb.list, sb.abytes);
   return hip_status();
@@ -592,6 +575,7 @@ int launch_select_list(const DGraph& g, const int32_t* vjob, const int32_t* gain
 //      (apply_sequence_move, gkway/uncoarsen.hpp:290-323).
 // A job with nothing selected is left untouched, so extra rounds after the
 // last productive one change nothing.
+template <int kBigBits>
 __global__ void __launch_bounds__(kBalThreads) k_round_b(
     const int32_t* __restrict__ v_off, int32_t M, int32_t kmax, const int32_t* __restrict__ kk,
     const long long* __restrict__ cap,
@@ -602,8 +586,11 @@ __global__ void __launch_bounds__(kBalThreads) k_round_b(
     uint32_t* __restrict__ hkey, int32_t* __restrict__ upd, int32_t* __restrict__ wl, int32_t* __restrict__ wlc,
     int32_t* __restrict__ lastcnt, int32_t* __restrict__ active, uint64_t* __restrict__ cand,
     int32_t* __restrict__ thr, long long* __restrict__ paths, int32_t* __restrict__ order,
-    int32_t* __restrict__ hist, long long* __restrict__ abytes) {
+    int32_t* __restrict__ hist, long long* __restrict__ abytes, int32_t* __restrict__ movers) {
   __shared__ RoundLds R;
+  __shared__ int32_t big[1 << kBigBits];  // the apply's table for rounds of many moves
+  if (kBigBits > 0)
+    for (int i = threadIdx.x; i < (1 << kBigBits); i += kBalThreads) big[i] = -1;
   extern __shared__ int32_t dpw[];  // 2 * kmax ints: part weight changes, then the part weights
   int32_t* spw = dpw + kmax;
   const int t = threadIdx.x;
@@ -668,6 +655,7 @@ __global__ void __launch_bounds__(kBalThreads) k_round_b(
   }
   if (count == 0) {
     if (t == 0) thr[j] = 1;
+    if (movers && t == 0) movers[0] = 0;
     // Nothing selected: the job's state (partition, gains, part weights) is
     // unchanged, so every later round of this level selects nothing either.
     // The first time, its candidate bits are dropped so that the selection
@@ -687,7 +675,7 @@ __global__ void __launch_bounds__(kBalThreads) k_round_b(
   }
   const int32_t B = count < M ? count : M;
   // 2. and 3. the B best keys into R.b.sk, sorted; the balanced prefix
-  const bool narrow = order_moves(R, count, M, vb, ve, hkey + vb, SelectedList{seg, gain});
+  const bool narrow = order_moves<8>(R, count, M, vb, ve, hkey + vb, SelectedList{seg, gain});
   if (t < kj) spw[t] = pw_t;
   for (int32_t q = t + kBalThreads; q < kj; q += kBalThreads) spw[q] = pwj[q];
   BalanceOpt bo;
@@ -720,7 +708,24 @@ __global__ void __launch_bounds__(kBalThreads) k_round_b(
   // 4. the apply
   const bool sole = gridDim.x == 1;
   int32_t wrun = 0;
-  const int tot = apply_moves(R, pos, part, xadj, adj, upd, wl, wlc, sole, &wrun);
+  if (movers && t == 0) movers[0] = pos < 64 ? 0 : pos + 1;
+  if (movers && pos >= 64) {
+    // More than a wave's worth, and one job: the whole device expands them
+    // (k_expand_moves).
+    if (t <= pos) {
+      const int32_t v = R.b.sv[t];
+      part[v] = R.mdst[t];
+      movers[1 + t] = v;
+    }
+    if (t == 0) {
+      thr[j] = R.lz[2];
+      rounds[j] = rounds0 + 1;
+      moved[j] = moved0 + pos + 1;
+      if (abytes) abytes[j] = ab0 + 8LL * count + 16LL * B + 4LL * kj;
+    }
+    return;
+  }
+  const int tot = apply_moves(R, pos, part, xadj, adj, upd, wl, wlc, sole, &wrun, big, kBigBits);
   if (t == 0) {
     if (sole) wlc[0] = wrun;
     thr[j] = R.lz[2];
@@ -734,18 +739,95 @@ __global__ void __launch_bounds__(kBalThreads) k_round_b(
   }
 }
 
+// The movers of a round that moved 64 or more (movers[0] of them, else 0;
+// their parts are set): they and their neighbours, items dealt out over the
+// device, each once onto the gain worklist.  The round's own workgroup took 19
+// to 25 us for the 7100 items of 1024 movers, bound by the scattered accesses
+// of one compute unit.  Every block adds up the movers' rows for itself.
+__global__ void __launch_bounds__(256) k_expand_moves(const int32_t* __restrict__ movers,
+                                                      const int32_t* __restrict__ xadj,
+                                                      const int32_t* __restrict__ adj, int32_t* __restrict__ upd,
+                                                      int32_t* __restrict__ wl, int32_t* __restrict__ wlc,
+                                                      long long* __restrict__ abytes) {
+  __shared__ int32_t mv[kBalMax], rstart[kBalMax], istart[kBalMax];
+  __shared__ int lds[8];
+  constexpr int kPer = kBalMax / 256;
+  const int32_t cnt = movers[0];
+  if (cnt == 0) return;
+  const int t = threadIdx.x;
+  int32_t v[kPer], s[kPer], c[kPer];
+  int sum = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int m = t * kPer + i;
+    v[i] = m < cnt ? movers[1 + m] : -1;
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    s[i] = v[i] >= 0 ? xadj[v[i]] : 0;
+    c[i] = v[i] >= 0 ? xadj[v[i] + 1] - s[i] + 1 : 0;
+    sum += c[i];
+  }
+  int tot;
+  int run = block_excl_scan_256(sum, &tot, lds);
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int m = t * kPer + i;
+    mv[m] = v[i];
+    rstart[m] = s[i];
+    istart[m] = run;
+    run += c[i];
+  }
+  __syncthreads();
+  if (abytes && blockIdx.x == 0 && t == 0) atomicAdd(reinterpret_cast<unsigned long long*>(abytes), 12ull * tot);
+  const int64_t step = int64_t(gridDim.x) * 256;
+  // whole waves stay together
+  for (int64_t b = int64_t(blockIdx.x) * 256 + (t & ~63); b < tot; b += step) {
+    const int64_t x = b + lane_id();
+    bool first = false;
+    int32_t u = 0;
+    if (x < tot) {
+      int lo = 0, hi = cnt - 1;  // last mover m with istart[m] <= x
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (istart[mid] <= x) lo = mid; else hi = mid - 1;
+      }
+      const int off = int(x) - istart[lo];
+      u = off == 0 ? mv[lo] : adj[rstart[lo] + off - 1];
+      first = atomicExch(&upd[u], 1) == 0;
+    }
+    const uint64_t m = ballot(first);
+    int base = 0;
+    if (lane_id() == 0 && m) base = atomicAdd(wlc, popc64(m));
+    base = __shfl(base, 0, 64);
+    if (first) wl[base + popc64(m & lanemask_lt())] = u;
+  }
+}
+
 int launch_round_b(int32_t nj, int32_t kmax, const int32_t* v_off, int32_t M, const int32_t* kk, const long long* cap,
                    const int32_t* pw_off, const DGraph& g, int32_t* part, const int32_t* dest, const int32_t* gain,
                    int32_t* pw, long long* cut, int32_t* rounds, long long* moved, const SelectBufs& sb,
                    int32_t* xlist, uint32_t* hkey, int32_t* upd, int32_t* wl, int32_t* wlc, int32_t* lastcnt,
                    int32_t* active, uint64_t* cand, int32_t* thr, long long* paths, int32_t* order, int32_t* hist,
-                   long long* abytes, hipStream_t st) {
+                   long long* abytes, int32_t* movers, hipStream_t st) {
   if (nj <= 0) return 0;
   if (M > kBalMax) return GK_ERR_LIMIT;
-  gk_launch(k_round_b, dim3(nj), dim3(kBalThreads), uint32_t(2 * sizeof(int32_t) * kmax), st, v_off, M, kmax, kk, cap,
-            pw_off,
-            g.xadj, g.adj, part, dest, gain, g.vw, pw, cut, rounds, moved, sb, xlist, hkey, upd, wl, wlc, lastcnt,
-            active, cand, thr, paths, order, hist, abytes);
+  if (nj != 1) movers = nullptr;
+  // 64 KB of LDS for the apply's table, unless the device expands the moves,
+  // the jobs need to share a compute unit, or the part weights (8 kmax bytes)
+  // take the room.
+  if (!movers && nj <= 256 && kmax <= 4096)
+    gk_launch(k_round_b<14>, dim3(nj), dim3(kBalThreads), uint32_t(2 * sizeof(int32_t) * kmax), st, v_off, M, kmax, kk, cap,
+              pw_off,
+              g.xadj, g.adj, part, dest, gain, g.vw, pw, cut, rounds, moved, sb, xlist, hkey, upd, wl, wlc, lastcnt,
+              active, cand, thr, paths, order, hist, abytes, movers);
+  else
+    gk_launch(k_round_b<0>, dim3(nj), dim3(kBalThreads), uint32_t(2 * sizeof(int32_t) * kmax), st, v_off, M, kmax, kk, cap,
+              pw_off,
+              g.xadj, g.adj, part, dest, gain, g.vw, pw, cut, rounds, moved, sb, xlist, hkey, upd, wl, wlc, lastcnt,
+              active, cand, thr, paths, order, hist, abytes, movers);
+  if (movers)
+    gk_launch(k_expand_moves, dim3(64), dim3(256), 0, st, movers, g.xadj, g.adj, upd, wl, wlc, abytes);
   return hip_status();
 }
 

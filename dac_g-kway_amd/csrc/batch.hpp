@@ -100,12 +100,14 @@ int launch_select_list(const DGraph& g, const int32_t* vjob, const int32_t* gain
                        const int32_t* pw, const int32_t* pw_off, const long long* cap, const int32_t* thr,
                        const uint64_t* cand, const SelectBufs& sb, int32_t* reset, int32_t* active,
                        hipStream_t st);
+// movers (one job; may be null): 1 + M ints, through which the device expands
+// the moves of a round that makes 64 or more.
 int launch_round_b(int32_t nj, int32_t kmax, const int32_t* v_off, int32_t M, const int32_t* kk, const long long* cap,
                    const int32_t* pw_off, const DGraph& g, int32_t* part, const int32_t* dest, const int32_t* gain,
                    int32_t* pw, long long* cut, int32_t* rounds, long long* moved, const SelectBufs& sb,
                    int32_t* xlist, uint32_t* hkey, int32_t* upd, int32_t* wl, int32_t* wlc, int32_t* lastcnt,
                    int32_t* active, uint64_t* cand, int32_t* thr, long long* paths, int32_t* order, int32_t* hist,
-                   long long* abytes, hipStream_t st);
+                   long long* abytes, int32_t* movers, hipStream_t st);
 // All of a round, and many rounds, in one launch (one workgroup per job), for
 // k <= kGainInlineK.  A job stops when a round selects nothing (lastcnt[job] =
 // 0), after max_rounds rounds, when a round updates more vertices than one

@@ -407,7 +407,7 @@ int wide_round(gk_ctx* ctx, hipStream_t st, const RoundState& s) {
   GK_STAGE(ctx, GK_ST_BALANCE, 0,
            gkd::launch_round_b(s.nj, s.kmax, s.v_off, s.M, s.kk, s.cap, s.pw_off, s.g, s.part, s.dest, s.gain, s.pw,
                                s.cut, s.rounds, s.moved, s.sb, s.xlist, s.hkey, s.upd, s.wl, s.hcnt, s.lastcnt,
-                               s.active, s.cand, s.thr, s.paths, s.order, s.hist, s.abytes, st));
+                               s.active, s.cand, s.thr, s.paths, s.order, s.hist, s.abytes, s.movers, st));
   GK_STAGE(ctx, GK_ST_GAIN, 0,
            gkd::launch_gain_wl(s.g, s.kmax, s.lanes, s.wl, s.hcnt, s.heavy, s.part, s.upd, s.bnd, s.gain, s.dest,
                                s.work, s.wl_items, s.cand, st, steal_of(ctx)));
@@ -521,8 +521,12 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
       }
       done += rounds;
       wide_done += rounds;
-      int32_t live = 0;
-      GK_TRY(fetch(ctx, st, {{&live, s.active, sizeof live}}));
+      gkd::Copies look;
+      look.add(ctx->hctl, s.active, sizeof(int32_t));
+      GK_TRY(gkd::launch_copies(look, st));
+      GK_HIP(hipEventRecord(ctx->ev, st));
+      GK_HIP(hipEventSynchronize(ctx->ev));
+      const int32_t live = ctx->hctl[0];
       if (live == 0) break;
       if (can_loop && live <= kLoopSelected * s.nj) {
         loop = true;
@@ -553,20 +557,15 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   std::memset(&S, 0, sizeof S);
   ctx->cur = &S;
   ctx->clock.start((prm.flags & GK_FLAG_STAGE_TIME) != 0, st);
+  StageGuard stage_guard{ctx, st};
   struct Reset {
     gk_ctx* c;
-    hipStream_t st;
-    bool done = false;
     ~Reset() {
-      // An error may leave launches that read the staging memory.
-      if (!done) (void)hipStreamSynchronize(st);
-      c->dl.drained();
-      c->up.drained();
       c->cur = nullptr;
       c->clock.start(false, nullptr);
       gkrt::clear_launch_options(c);
     }
-  } reset{ctx, st};
+  } reset{ctx};
   GK_TRY(gkrt::set_launch_options(ctx, prm.flags));
 
   std::vector<Level> L;
@@ -759,7 +758,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   int32_t* oth_bnd = bndB.p;
   if (nl > 1) {
     const int32_t M = prm.max_moves;
-    Buf<int32_t> xlist, wpos, sscr, gain, dest, upd, heavy, wl, list;
+    Buf<int32_t> movers, xlist, wpos, sscr, gain, dest, upd, heavy, wl, list;
     Buf<uint64_t> cand, movable, defbits;
     Buf<uint32_t> hkey;
     GK_TRY(gain.alloc(P, n0));
@@ -775,6 +774,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     GK_TRY(wpos.alloc(P, nwords0 + 1));
     GK_TRY(sscr.alloc(P, gkd::select_scratch_ints(n0)));
     GK_TRY(xlist.alloc(P, n0));
+    GK_TRY(movers.alloc(P, int64_t(M) + 1));
     const gkd::SelectBufs sb{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, work.p + 2 * kGainSlots};
     for (int32_t l = nl - 2; l >= 0; --l) {
       Level& f = L[l];
@@ -831,6 +831,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
       rs.cand = cand.p;
       rs.sb = sb;
       rs.xlist = xlist.p;
+      rs.movers = movers.p;
       rs.wl = wl.p;
       rs.hcnt = hcnt;
       rs.heavy = heavy.p;
@@ -901,7 +902,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
       S.stage_bytes[GK_ST_GAIN] += int64_t(28 * wv + 12 * we);
       for (int i = 0; i < gkd::kSelectByteSlots; ++i) S.stage_bytes[GK_ST_SELECT] += int64_t(hwork[2 * kGainSlots + i]);
     }
-    reset.done = true;
+    stage_guard.done = true;
     unsigned long long mx = 0;
     for (int32_t q = 0; q < k; ++q) mx = std::max(mx, hpw64[q]);
     S.max_part_wgt = static_cast<int64_t>(mx);
@@ -1332,19 +1333,17 @@ int gk_k_gain(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* part, con
   hipStream_t st = pick(ctx, stream);
   DGraph g = dview(dg);
   const int lanes = gain_lanes(g);
-  Buf<int32_t> wl, heavy, cnt, flags;
+  Buf<int32_t> wl, heavy, cnt;
   GK_TRY(wl.alloc(ctx->pool, g.n));
   GK_TRY(heavy.alloc(ctx->pool, g.n));
   GK_TRY(cnt.alloc(ctx->pool, 2));
-  GK_TRY(flags.alloc(ctx->pool, g.n));
-  // The kernels clear the flags they consume: work on a copy.
-  if (g.n) GK_HIP(hipMemcpyAsync(flags.p, upd, sizeof(int32_t) * g.n, hipMemcpyDeviceToDevice, st));
   gkd::fill<int32_t>(cnt.p, 0, 2, st);
-  GK_TRY(gkd::launch_compact(g.n, flags.p, wl.p, cnt.p, st));
-  GK_TRY(gkd::launch_gain_wl(g, k, lanes, wl.p, cnt.p, heavy.p, part, flags.p, bnd, gain, dest, nullptr, g.n, nullptr,
+  // The caller's flags stay as they are (none given to the gain kernels).
+  GK_TRY(gkd::launch_compact(g.n, upd, wl.p, cnt.p, st));
+  GK_TRY(gkd::launch_gain_wl(g, k, lanes, wl.p, cnt.p, heavy.p, part, nullptr, bnd, gain, dest, nullptr, g.n, nullptr,
                               st));
   if (gkd::gain_heavy_separate(k))
-    GK_TRY(gkd::launch_gain_heavy(g, k, heavy.p, cnt.p, part, flags.p, bnd, gain, dest, nullptr, nullptr, st));
+    GK_TRY(gkd::launch_gain_heavy(g, k, heavy.p, cnt.p, part, nullptr, bnd, gain, dest, nullptr, nullptr, st));
   GK_HIP(hipStreamSynchronize(st));
   return GK_OK;
 }
@@ -1470,16 +1469,13 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   const int32_t n = g.n, M = max_moves;
   const int64_t nwords = (int64_t(n) + 63) / 64;
   // The round state of run_vcycle's refinement, for one job.
-  Buf<int32_t> upd, wl, heavy, hcnt, list, xlist, wpos, sscr, dthr, active, drounds, lastcnt, dvoff, dpw_off, dkk,
-      dorder, dmax, status, hist;
-  Buf<long long> dcap, dcut, dmoved, dpaths, dabytes;
+  Buf<int32_t> movers, upd, wl, heavy, list, xlist, wpos, sscr, dorder, dmax, hist;
+  Buf<char> state;
   Buf<uint64_t> cand, movable, selbits, defbits;
   Buf<uint32_t> hkey;
   GK_TRY(upd.alloc(P, n));
   GK_TRY(wl.alloc(P, n));
   GK_TRY(heavy.alloc(P, n));
-  GK_TRY(hcnt.alloc(P, 4));
-  GK_TRY(status.alloc(P, 4));
   GK_TRY(hist.alloc(P, 2 * int64_t(nrounds)));
   GK_TRY(list.alloc(P, n));
   GK_TRY(xlist.alloc(P, n));
@@ -1490,31 +1486,33 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   GK_TRY(movable.alloc(P, nwords + 1));
   GK_TRY(selbits.alloc(P, nwords + 1));
   GK_TRY(defbits.alloc(P, nwords + 1));
-  GK_TRY(dthr.alloc(P, 1));
-  GK_TRY(active.alloc(P, 1));
-  GK_TRY(drounds.alloc(P, 1));
-  GK_TRY(lastcnt.alloc(P, 1));
-  GK_TRY(dvoff.alloc(P, 2));
-  GK_TRY(dpw_off.alloc(P, 2));
-  GK_TRY(dkk.alloc(P, 1));
+  GK_TRY(movers.alloc(P, int64_t(M) + 1));
   GK_TRY(dorder.alloc(P, int64_t(M) + 2));
   GK_TRY(dmax.alloc(P, 1));
-  GK_TRY(dcap.alloc(P, 1));
-  GK_TRY(dcut.alloc(P, 1));
-  GK_TRY(dmoved.alloc(P, 1));
-  GK_TRY(dpaths.alloc(P, 3));
-  GK_TRY(dabytes.alloc(P, 1));
-  gkd::fill<int32_t>(upd.p, 0, n, st);
-  gkd::fill<uint64_t>(selbits.p, 0ull, nwords + 1, st);
-  gkd::fill<int32_t>(dvoff.p, 0, 1, st);
-  gkd::fill<int32_t>(dvoff.p + 1, n, 1, st);
-  gkd::fill<int32_t>(dpw_off.p, 0, 1, st);
-  gkd::fill<int32_t>(dpw_off.p + 1, k, 1, st);
-  gkd::fill<int32_t>(dkk.p, k, 1, st);
-  gkd::fill<long long>(dcap.p, static_cast<long long>(cap), 1, st);
-  gkd::fill<long long>(dcut.p, 0, 1, st);
-  gkd::fill<long long>(dpaths.p, 0, 3, st);
-  GK_TRY(gkd::launch_rounds_init(1, lastcnt.p, dthr.p, drounds.p, dmoved.p, dabytes.p, hcnt.p, status.p, st));
+  // The words of the one job's state, which go up and come back as one block.
+  struct State {
+    long long cut, cap, moved, abytes, paths[3], pad;
+    int32_t voff[2], pwoff[2], hcnt[4], status[4], kk, thr, lastcnt, rounds, active, pad2[3];
+  };
+  static_assert(sizeof(State) % 16 == 0, "whole 16-byte words");
+  GK_TRY(state.alloc(P, sizeof(State)));
+  State* ds = reinterpret_cast<State*>(state.p);
+  StageGuard staged{ctx, st};
+  void* hup = nullptr;
+  GK_TRY(ctx->up.get(st, sizeof(State), &hup));
+  State* hs = static_cast<State*>(hup);
+  std::memset(hs, 0, sizeof *hs);
+  hs->cap = cap;
+  hs->voff[1] = n;
+  hs->pwoff[1] = k;
+  hs->kk = k;
+  hs->thr = 1;
+  hs->lastcnt = 1;
+  gkd::Copies begin;
+  begin.add(ds, hs, sizeof *hs);
+  begin.add(upd.p, nullptr, sizeof(int32_t) * size_t(n));
+  begin.add(selbits.p, nullptr, sizeof(uint64_t) * size_t(nwords + 1));
+  GK_TRY(gkd::launch_copies(begin, st));
   GK_TRY(gkd::launch_cand_init(n, bnd, gain, cand.p, st));
   RoundState rs;
   rs.g = g;
@@ -1528,42 +1526,50 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
     rs.heavy_rows = maxdeg > rs.lanes;
   }
   rs.wl_items = n;
-  rs.v_off = dvoff.p;
-  rs.kk = dkk.p;
-  rs.pw_off = dpw_off.p;
-  rs.cap = dcap.p;
+  rs.v_off = ds->voff;
+  rs.kk = &ds->kk;
+  rs.pw_off = ds->pwoff;
+  rs.cap = &ds->cap;
   rs.part = part;
   rs.bnd = bnd;
   rs.gain = gain;
   rs.dest = dest;
   rs.pw = pw;
   rs.upd = upd.p;
-  rs.cut = dcut.p;
-  rs.moved = dmoved.p;
-  rs.paths = dpaths.p;
-  rs.abytes = dabytes.p;
-  rs.rounds = drounds.p;
-  rs.lastcnt = lastcnt.p;
-  rs.thr = dthr.p;
-  rs.active = active.p;
+  rs.cut = &ds->cut;
+  rs.moved = &ds->moved;
+  rs.paths = ds->paths;
+  rs.abytes = &ds->abytes;
+  rs.rounds = &ds->rounds;
+  rs.lastcnt = &ds->lastcnt;
+  rs.thr = &ds->thr;
+  rs.active = &ds->active;
   rs.cand = cand.p;
   rs.sb = gkd::SelectBufs{movable.p, selbits.p, defbits.p, wpos.p, list.p, sscr.p, nullptr};
   rs.xlist = xlist.p;
+  rs.movers = movers.p;
   rs.wl = wl.p;
-  rs.hcnt = hcnt.p;
+  rs.hcnt = ds->hcnt;
   rs.heavy = heavy.p;
-  rs.status = status.p;
+  rs.status = ds->status;
   rs.hkey = hkey.p;
   rs.order = dorder.p;
   rs.hist = hist.p;
   GK_TRY(refine_rounds(ctx, st, rs, nrounds, true, false, nullptr));
   // Rounds that ordered no move came after those that did (an unchanged state
   // stays so): no moves, position -1.
-  long long hcut = 0, hp[3] = {0, 0, 0};
-  int32_t made = 0;
-  GK_TRY(fetch(ctx, st, {{&hcut, dcut.p, sizeof hcut}, {hp, dpaths.p, sizeof hp}, {&made, drounds.p, sizeof made}}));
-  std::vector<int32_t> hh;
-  GK_TRY(to_host(st, hh, hist.p, 2 * int64_t(made)));
+  const size_t hist_bytes = sizeof(int32_t) * 2 * size_t(nrounds);
+  void* hend = nullptr;
+  GK_TRY(ctx->dl.get(st, sizeof(State) + hist_bytes, &hend));
+  const State* he = static_cast<const State*>(hend);
+  const int32_t* hh = reinterpret_cast<const int32_t*>(he + 1);
+  gkd::Copies end;
+  end.add(hend, ds, sizeof *ds);
+  end.add(static_cast<char*>(hend) + sizeof *ds, hist.p, hist_bytes);
+  GK_TRY(gkd::launch_copies(end, st));
+  GK_HIP(hipStreamSynchronize(st));
+  staged.done = true;
+  const int32_t made = he->rounds;
   for (int32_t r = 0; r < nrounds; ++r) {
     if (nmoves) nmoves[r] = r < made ? hh[2 * r] : 0;
     if (pos) pos[r] = r < made ? hh[2 * r + 1] : -1;
@@ -1571,9 +1577,9 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   if (order && made > 0)
     GK_HIP(hipMemcpyAsync(order, dorder.p + 2, sizeof(int32_t) * size_t(hh[2 * made - 2]), hipMemcpyDeviceToDevice, st));
   GK_HIP(hipStreamSynchronize(st));
-  *gain_sum = -hcut;
+  *gain_sum = -he->cut;
   if (paths)
-    for (int i = 0; i < 3; ++i) paths[i] = hp[i];
+    for (int i = 0; i < 3; ++i) paths[i] = he->paths[i];
   return GK_OK;
 }
 
@@ -1588,14 +1594,18 @@ int gk_k_cut(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* part, int6
   GK_TRY(p.alloc(ctx->pool, k));
   GK_TRY(cscr.alloc(ctx->pool, gkd::cut_scratch(g.n, k)));
   GK_TRY(gkd::launch_cut(g, k, part, c.p, p.p, cscr.p, st));
-  unsigned long long hc = 0;
-  GK_TRY(fetch(ctx, st, {{&hc, c.p, sizeof hc}}));
-  *cut = static_cast<int64_t>(hc);
-  if (pw) {
-    std::vector<unsigned long long> hp;
-    GK_TRY(to_host(st, hp, p.p, k));
-    for (int32_t q = 0; q < k; ++q) pw[q] = static_cast<int64_t>(hp[q]);
-  }
+  void* h = nullptr;
+  GK_TRY(ctx->dl.get(st, sizeof(unsigned long long) * (size_t(k) + 2), &h));
+  unsigned long long* hc = static_cast<unsigned long long*>(h);
+  gkd::Copies back;
+  back.add(hc, c.p, sizeof *hc);
+  if (pw) back.add(hc + 2, p.p, sizeof *hc * size_t(k));
+  GK_TRY(gkd::launch_copies(back, st));
+  GK_HIP(hipStreamSynchronize(st));
+  ctx->dl.drained();
+  *cut = static_cast<int64_t>(*hc);
+  if (pw)
+    for (int32_t q = 0; q < k; ++q) pw[q] = static_cast<int64_t>(hc[2 + q]);
   return GK_OK;
 }
 

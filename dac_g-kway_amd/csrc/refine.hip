@@ -331,7 +331,7 @@ __device__ __forceinline__ void gain_wl_body(const int32_t* __restrict__ wl, int
                    gain[u] = up ? g : 0;
                    dest[u] = up ? q : p;
                    if (cand) set_cand(cand, u, up);
-                   upd[u] = 0;
+                   if (upd) upd[u] = 0;
                    ++done_v;
                    done_e += du;
                  });
@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(64) k_gain_heavy(const int32_t* __restrict__ h
       if (any && g > 0) { gain[v] = g; dest[v] = bq; }
       else { gain[v] = 0; dest[v] = p; }
       if (cand) set_cand(cand, v, any && g > 0);
-      upd[v] = 0;
+      if (upd) upd[v] = 0;
       done_v += 1;
       done_e += (unsigned long long)(e - s);
     }

@@ -543,7 +543,7 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
       }
       // the best moves in order, and their balanced prefix
       const int32_t B = count < a.M ? count : a.M;
-      const bool narrow = order_moves(R, count, a.M, vb, ve, nullptr, SelectedIndex<CAP>{&L});
+      const bool narrow = order_moves<4>(R, count, a.M, vb, ve, nullptr, SelectedIndex<CAP>{&L});
       BalanceOpt bo;
       bo.spw = L.spw;
       bo.mdst = R.mdst;
@@ -596,8 +596,16 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     if (pos >= 64 || L.tot > kLoopItems) {
       // More than this workgroup should update: the worklist in memory, and
       // out, for the gain pass over the whole device.
+      // Its table of first occurrences lies over the candidates' gains and
+      // weights, which nobody reads any more.
+      static_assert(offsetof(LoopLds<CAP>, lw) == offsetof(LoopLds<CAP>, lg) + sizeof(L.lg), "one array of 2 * CAP");
+      constexpr int kBits = CAP == 4096 ? 13 : 11;
+      static_assert((1 << kBits) == 2 * CAP, "slots");
+      int32_t* table = &L.lg[0];
+      for (int i = t; i < 2 * CAP; i += kBalThreads) table[i] = -1;
+      __syncthreads();
       int32_t unused = 0;
-      const int tot = apply_moves(R, pos, a.part, a.xadj, a.adj, a.upd, a.wl, a.wlc, false, &unused);
+      const int tot = apply_moves(R, pos, a.part, a.xadj, a.adj, a.upd, a.wl, a.wlc, false, &unused, table, kBits);
       if (t == 0) rounds_bytes += 12LL * tot;
       break;
     }

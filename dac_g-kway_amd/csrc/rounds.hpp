@@ -46,11 +46,12 @@ struct SelectedList {
 // [vb, ve), by (gain desc, id asc), sorted into R.b.sk as (gain key << 32 |
 // vertex), slots behind them the largest key.  sel.vertex(i) and
 // sel.gain_key(i, vertex) give the selected vertices.  hk: scratch for count
-// keys, used beyond 4 * kBalThreads selected.  R.lz[2] gets the gain threshold
+// keys, used beyond kKeep * kBalThreads selected (kKeep a thread stay in
+// registers).  R.lz[2] gets the gain threshold
 // of the job's next round when one is due.  Returns whether the keys were
 // sorted as 32-bit words.  Every thread of the block calls it after a barrier;
 // it ends with one.
-template <class Sel>
+template <int kKeep, class Sel>
 __device__ __forceinline__ bool order_moves(RoundLds& R, int32_t count, int32_t M, int32_t vb, int32_t ve, uint32_t* hk,
                                             const Sel& sel) {
   const int t = threadIdx.x;
@@ -70,7 +71,6 @@ __device__ __forceinline__ bool order_moves(RoundLds& R, int32_t count, int32_t 
     // use 11-bit digits from the top.  Up to kKeep keys per thread stay in
     // registers across the passes (with their vertices); more go through the
     // scratch hk.
-    constexpr int kKeep = 4;
     const bool inreg = count <= kKeep * kBalThreads;
     uint32_t hr[kKeep];
     int32_t vr[kKeep];
@@ -218,10 +218,11 @@ __device__ __forceinline__ bool order_moves(RoundLds& R, int32_t count, int32_t 
 // its last barrier) and appends the movers and their neighbours to the gain
 // worklist, each once: wl at *wlc, by an atomic per pass, or with sole (one
 // workgroup owns the list, empty before) at a running offset whose end thread
-// 0 gets in *wrun_out.  R.ht is all -1 before.  Returns the items looked at.
+// 0 gets in *wrun_out.  R.ht is all -1 before, and so are the 2^big_bits slots
+// of LDS at big, if there are any (big_bits > 0).  Returns the items looked at.
 __device__ __forceinline__ int apply_moves(RoundLds& R, int pos, int32_t* part, const int32_t* __restrict__ xadj,
                                            const int32_t* __restrict__ adj, int32_t* upd, int32_t* wl, int32_t* wlc,
-                                           bool sole, int32_t* wrun_out) {
+                                           bool sole, int32_t* wrun_out, int32_t* big, int big_bits) {
   const int t = threadIdx.x;
   // The movers and their neighbours are items [0, tot) -- mover m owns
   // [istart[m], istart[m] + deg + 1), first itself, then its row -- dealt out
@@ -235,14 +236,15 @@ __device__ __forceinline__ int apply_moves(RoundLds& R, int pos, int32_t* part, 
   int32_t* rstart = R.b.cover;  // likewise
   int tot = 0;
   // Items [a0, a0 + kApplyPer) of [0, tot): their vertices (-1 past the end)
-  // and the bit mask of the first occurrences.  With a table ht (LDS, kHt
-  // slots, all -1, more than twice the items): first occurrences within the
+  // and the bit mask of the first occurrences.  With a table ht (LDS, 2^bits
+  // slots, all -1, at least twice the items): first occurrences within the
   // round by insertion into ht, the update flag then set by a plain store --
   // every flag is clear when a round starts (the gain pass of the previous
-  // round cleared those it set).  Without: by the update flag's atomic swap.
+  // round cleared those it set).  Without: by the update flag's atomic swap,
+  // which a workgroup waits for (7100 items: 25 us, with the table 19).
   constexpr int kHt = sizeof(R.ht) / sizeof(int32_t);
   static_assert(kHt == 1024, "10-bit table index");
-  auto take = [&](int a0, int32_t (&us)[kApplyPer], int32_t* ht) -> uint32_t {
+  auto take = [&](int a0, int32_t (&us)[kApplyPer], int32_t* ht, int bits) -> uint32_t {
     uint32_t win = 0;
 #pragma unroll
     for (int i = 0; i < kApplyPer; ++i) us[i] = -1;
@@ -266,7 +268,7 @@ __device__ __forceinline__ int apply_moves(RoundLds& R, int pos, int32_t* part, 
 #pragma unroll
       for (int i = 0; i < kApplyPer; ++i) {
         if (us[i] < 0) continue;
-        uint32_t sl = (uint32_t(us[i]) * 0x9E3779B1u) >> 22;  // 10 bits: kHt slots
+        uint32_t sl = (uint32_t(us[i]) * 0x9E3779B1u) >> (32 - bits);
         while (true) {
           const int32_t o = atomicCAS(&ht[sl], -1, us[i]);
           if (o == -1) {
@@ -275,7 +277,7 @@ __device__ __forceinline__ int apply_moves(RoundLds& R, int pos, int32_t* part, 
             break;
           }
           if (o == us[i]) break;
-          sl = (sl + 1) & (kHt - 1);
+          sl = (sl + 1) & ((1u << bits) - 1);
         }
       }
     } else {
@@ -306,11 +308,16 @@ __device__ __forceinline__ int apply_moves(RoundLds& R, int pos, int32_t* part, 
       }
       // first occurrences in LDS when the items fit the table
       int32_t* ht = tot <= kHt / 2 ? R.ht : nullptr;
+      int bits = 10;
+      if (!ht && big_bits > 0 && 2 * int64_t(tot) <= (int64_t(1) << big_bits)) {
+        ht = big;
+        bits = big_bits;
+      }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
       for (int pb = 0; pb < tot; pb += kApplyPer * 64) {
         int32_t us[kApplyPer];
-        const uint32_t win = take(pb + kApplyPer * t, us, ht);
+        const uint32_t win = take(pb + kApplyPer * t, us, ht, bits);
         const int c = __popc(win);
         const int wincl = seg_incl_scan<64>(c);
         const int wtot = __shfl(wincl, 63, 64);
@@ -342,9 +349,10 @@ __device__ __forceinline__ int apply_moves(RoundLds& R, int pos, int32_t* part, 
       rstart[t] = es;
     }
     __syncthreads();
+    int32_t* ht = big_bits > 0 && 2 * int64_t(tot) <= (int64_t(1) << big_bits) ? big : nullptr;
     for (int pb = 0; pb < tot; pb += kApplyPer * kBalThreads) {
       int32_t us[kApplyPer];
-      const uint32_t win = take(pb + kApplyPer * t, us, nullptr);
+      const uint32_t win = take(pb + kApplyPer * t, us, ht, big_bits);
       int wtot;
       const int wex = block_excl_scan_1024(__popc(win), &wtot, R.ws);
       if (t == 0) {

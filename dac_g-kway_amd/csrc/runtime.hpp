@@ -566,6 +566,19 @@ struct CsrOut {
   int32_t *xadj, *adj, *w;
 };
 
+// Frees the staging arenas at the end of a call, after a wait if the call ends
+// early: an error may leave launches that read or write them.
+struct StageGuard {
+  gk_ctx* ctx;
+  hipStream_t st;
+  bool done = false;  // the stream has been waited for
+  ~StageGuard() {
+    if (!done) (void)hipStreamSynchronize(st);
+    ctx->dl.drained();
+    ctx->up.drained();
+  }
+};
+
 // Members by coarse id: first place of every coarse id, and in member order
 // the vertices, their rows (start, length) and their weights; ctl: the
 // grouping's control words, then a contraction's row class counters (zero).
@@ -616,6 +629,7 @@ struct RoundState {
   uint32_t* hkey = nullptr;
   unsigned long long* work = nullptr;
   int32_t *order = nullptr, *hist = nullptr;
+  int32_t* movers = nullptr;  // one job: 1 + M ints (launch_round_b)
 };
 // Runs rounds until every job has converged, at most about max_rounds per job
 // (0: no bound; with exact, exactly so many at most); *ran gets the rounds
