@@ -134,7 +134,7 @@ struct RoundsArgs {
   int32_t *upd, *wl, *wlc, *next_wlc, *lastcnt, *status, *next_status, *thr;
   long long *paths, *abytes;
   int32_t *order, *hist;
-  int32_t* host;  // pinned, one job: live, left out, ordering rounds so far (may be null)
+  HostWords host;  // one job: live, left out, ordering rounds so far
 };
 int launch_rounds(const RoundsArgs& a, int32_t nj, int lanes, hipStream_t st);
 // Per-job state before a level's first round (rounds, moved and abytes 0,

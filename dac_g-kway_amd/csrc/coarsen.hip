@@ -426,12 +426,12 @@ __global__ void __launch_bounds__(256) k_size_mid(int64_t nb, int2* __restrict__
 }
 
 // offc[l] = first place and first coarse id of label l's group, offc[n] the
-// totals; ctl[0] (and the host's copy) = the number of coarse ids; host[1..]
+// totals; ctl[0] (and the host's copy) = the number of coarse ids; words 1.. of host
 // = the flags.
 __global__ void __launch_bounds__(256) k_size_apply(int32_t n, const int32_t* __restrict__ size, int32_t G,
                                                     const int2* __restrict__ partial, int scanned,
                                                     int2* __restrict__ offc, int32_t* __restrict__ ctl,
-                                                    int32_t* __restrict__ host) {
+                                                    const HostWords host) {
   __shared__ int lds[8];
   int32_t pm = 0, pc = 0;
   if (scanned) {
@@ -472,16 +472,19 @@ __global__ void __launch_bounds__(256) k_size_apply(int32_t n, const int32_t* __
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) {
     offc[n] = make_int2(rm, rc);
     ctl[0] = rc;
-    host[0] = rc;
+    int32_t word[kCtlInts];  // read first: the loads would wait for the stores
+    word[0] = rc;
 #pragma unroll
-    for (int i = 1; i < kCtlInts; ++i) host[i] = ctl[i];
+    for (int i = 1; i < kCtlInts; ++i) word[i] = ctl[i];
+#pragma unroll
+    for (int i = 0; i < kCtlInts; ++i) tell(host, i, word[i]);
   }
 }
 
 int64_t size_partials(int64_t n) { return (n + kSizeTile - 1) / kSizeTile; }
 
-int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl, int32_t* host,
-                     hipStream_t st) {
+int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl,
+                     const HostWords& host, hipStream_t st) {
   if (n <= 0) return 0;
   const int64_t nb = size_partials(n);
   k_size_reduce<<<unsigned(nb), 256, 0, st>>>(n, size, G, partial, ctl);
@@ -1362,7 +1365,7 @@ __global__ void __launch_bounds__(256) k_len_mid(int64_t nb, int32_t* __restrict
 __global__ void __launch_bounds__(256) k_len_apply(int32_t nc, const int32_t* __restrict__ len,
                                                    const int32_t* __restrict__ partial, int scanned,
                                                    int32_t* __restrict__ cxadj, const int32_t* __restrict__ cnt,
-                                                   int32_t* __restrict__ host) {
+                                                   const HostWords host) {
   __shared__ int lds[8];
   int32_t pre = 0;
   int t;
@@ -1390,14 +1393,17 @@ __global__ void __launch_bounds__(256) k_len_apply(int32_t nc, const int32_t* __
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) {
     cxadj[nc] = run;
-    host[0] = run;
+    int32_t word[kRowCtlWords];
 #pragma unroll
-    for (int k = 0; k < kRowCtlWords; ++k) host[1 + k] = cnt[k * kRowCtlStride];
+    for (int k = 0; k < kRowCtlWords; ++k) word[k] = cnt[k * kRowCtlStride];
+    tell(host, 0, run);
+#pragma unroll
+    for (int k = 0; k < kRowCtlWords; ++k) tell(host, 1 + k, word[k]);
   }
 }
 
-int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt, int32_t* host,
-                    hipStream_t st) {
+int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt,
+                    const HostWords& host, hipStream_t st) {
   const int64_t nb = std::max<int64_t>(1, size_partials(nc));
   k_len_reduce<<<unsigned(nb), 256, 0, st>>>(nc, len, partial);
   const bool mid = nb > kSizeDirect;

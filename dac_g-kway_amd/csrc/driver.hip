@@ -45,6 +45,33 @@ namespace gkrt {
 constexpr int64_t kTuneMinEntries = int64_t(1) << 20;
 constexpr int32_t kTuneMinRows = 1 << 14;
 
+int wait_words(gk_ctx* ctx, hipStream_t st, const gkd::HostWords& h, int n, int32_t* out) {
+  bool ended = false;  // the stream has run out
+  for (int i = 0, spins = 0; i < n;) {
+    const unsigned long long w = __atomic_load_n(&ctx->hctl[i], __ATOMIC_ACQUIRE);
+    if (uint32_t(w >> 32) == h.number) {
+      out[i++] = int32_t(uint32_t(w));
+      continue;
+    }
+    if (ended) {
+      gkh::set_error("a kernel did not report to the host");
+      return GK_ERR_INTERNAL;
+    }
+    __builtin_ia32_pause();
+    if (++spins % 4096) continue;
+    const hipError_t e = hipStreamQuery(st);
+    if (e == hipSuccess) {
+      ended = true;
+    } else if (e == hipErrorNotReady) {
+      (void)hipGetLastError();  // no error, but remembered as one
+    } else {
+      gkh::set_error(std::string("waiting for a kernel: ") + hipGetErrorString(e));
+      return GK_ERR_HIP;
+    }
+  }
+  return GK_OK;
+}
+
 // ---------------------------------------------------------------- stages
 // Labels, hops and member counts of the groups by walking to the root pairs.
 // The control words (zeroed here) hold whether every vertex reached its pair.
@@ -141,18 +168,16 @@ static int count_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* 
                          int32_t* words) {
   Buf<int2> partial;
   Buf<int4> memb;
+  const gkd::HostWords told = host_words(ctx);
   GK_TRY(partial.alloc(ctx->pool, gkd::size_partials(n)));
   GK_TRY(memb.alloc(ctx->pool, 2 * int64_t(n)));
   GK_STAGE(ctx, GK_ST_SORT, 16LL * n,
-           gkd::launch_size_scan(n, gr.size.p, G, partial.p, gr.comp.p, gr.ctl.p, ctx->hctl, st));
+           gkd::launch_size_scan(n, gr.size.p, G, partial.p, gr.comp.p, gr.ctl.p, told, st));
   // The counts come back while the members are ordered.
-  GK_HIP(hipEventRecord(ctx->ev, st));
   GK_STAGE(ctx, GK_ST_SORT, 120LL * n,
            gkd::launch_members(n, label, stamp, gr.slot.p, gr.comp.p, xadj, vw, memb.p, G, gr.ctl.p, out.order,
                                out.cmap, out.cptr, out.mrow, out.mvw, st));
-  GK_HIP(hipEventSynchronize(ctx->ev));
-  std::memcpy(words, ctx->hctl, sizeof(int32_t) * gkd::kCtlInts);
-  return GK_OK;
+  return wait_words(ctx, st, told, gkd::kCtlInts, words);
 }
 
 // The same by a radix sort of (label, stamp), stamps below 2^sbits.
@@ -304,12 +329,10 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
   // The entry count comes back with the class counters; rows for the global
   // sort, if there are any, are merged then, and the lengths scanned again.
   auto scan_lengths = [&]() -> int {
+    const gkd::HostWords told = host_words(ctx);
     GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc,
-             gkd::launch_len_scan(nc, len.p, scratch.p, c.xadj.p, cnt, ctx->hctl, st));
-    GK_HIP(hipEventRecord(ctx->ev, st));
-    GK_HIP(hipEventSynchronize(ctx->ev));
-    std::memcpy(words, ctx->hctl, sizeof words);
-    return GK_OK;
+             gkd::launch_len_scan(nc, len.p, scratch.p, c.xadj.p, cnt, told, st));
+    return wait_words(ctx, st, told, 1 + gkd::kRowCtlWords, words);
   };
   GK_TRY(scan_lengths());
   if (hc[4] > 0) {
@@ -420,13 +443,14 @@ int wide_round(gk_ctx* ctx, hipStream_t st, const RoundState& s) {
 
 // A launch of the round loop; pair: which pair of counts and status words it
 // uses.
-int loop_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, int pair) {
+int loop_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, int pair,
+                const gkd::HostWords& told) {
   const int o = 2 * pair, e = 2 * (1 - pair);
   const gkd::RoundsArgs a{s.v_off,     s.M,        max_rounds, s.kk,         s.cap,        s.pw_off,  s.g.xadj,
                           s.g.adj,     s.g.w,      s.g.vw,     s.part,       s.bnd,        s.gain,    s.dest,
                           s.pw,        s.cut,      s.rounds,   s.moved,      s.cand,       s.upd,     s.wl,
                           s.hcnt + o,  s.hcnt + e, s.lastcnt,  s.status + o, s.status + e, s.thr,     s.paths,
-                          s.abytes,    s.order,    s.hist,     s.nj == 1 ? ctx->hctl : nullptr};
+                          s.abytes,    s.order,    s.hist,     told};
   GK_STAGE(ctx, GK_ST_BALANCE, 0, gkd::launch_rounds(a, s.nj, s.lanes, st));
   return GK_OK;
 }
@@ -464,17 +488,13 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
   // Jobs that go on, jobs left out, and with one job the ordering rounds so
   // far; one job's kernel writes them to pinned memory itself.
   const bool one = s.nj == 1;
-  auto status = [&](int p, int32_t* words) -> int {
-    if (!one) {
-      gkd::Copies c;
-      c.add(ctx->hctl, s.status + 2 * p, 2 * sizeof(int32_t));
-      GK_TRY(gkd::launch_copies(c, st));
-    }
-    GK_HIP(hipEventRecord(ctx->ev, st));
-    GK_HIP(hipEventSynchronize(ctx->ev));
-    std::memcpy(words, ctx->hctl, (one ? 3 : 2) * sizeof(int32_t));
-    return GK_OK;
+  auto status = [&](int p, const gkd::HostWords& told, int32_t* words) -> int {
+    if (one) return wait_words(ctx, st, told, 3, words);
+    const gkd::HostWords t2 = host_words(ctx);
+    GK_TRY(gkd::launch_tell(s.status + 2 * p, 2, t2, st));
+    return wait_words(ctx, st, t2, 2, words);
   };
+  auto listen = [&]() { return one ? host_words(ctx) : gkd::HostWords{}; };
   while (max_rounds <= 0 || done < max_rounds) {
     if (loop) {
       const int left = max_rounds > 0 ? max_rounds - done : kLoopRounds;
@@ -483,20 +503,23 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
         // both pairs, so that every replay begins with the same one
         if (!loop_graph.ready())
           GK_TRY(loop_graph.capture(ctx, st, [&]() -> int {
-            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, pair));
+            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, pair, gkd::HostWords{}));
             GK_TRY(loop_gains(ctx, st, s, pair));
-            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, 1 - pair));
+            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, 1 - pair, gkd::HostWords{}));
             return loop_gains(ctx, st, s, 1 - pair);
           }));
         GK_TRY(loop_graph.replay(ctx, st));
-        GK_TRY(status(1 - pair, words));
+        const gkd::HostWords told = host_words(ctx);
+        GK_TRY(gkd::launch_tell(s.status + 2 * (1 - pair), 2, told, st));
+        GK_TRY(wait_words(ctx, st, told, 2, words));
         done += kLoopRounds;
       } else {
         const int rounds = std::min(left, kLoopRounds);
-        GK_TRY(loop_rounds(ctx, st, s, rounds, pair));
+        const gkd::HostWords told = listen();
+        GK_TRY(loop_rounds(ctx, st, s, rounds, pair, told));
         // Of several jobs some usually go on, and the wait is the longer part.
         if (!one) GK_TRY(loop_gains(ctx, st, s, pair));
-        GK_TRY(status(pair, words));
+        GK_TRY(status(pair, told, words));
         if (one && words[0] != 0) GK_TRY(loop_gains(ctx, st, s, pair));
         done = exact ? words[2] : done + rounds;  // exact: one job
         pair = 1 - pair;
@@ -521,12 +544,10 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
       }
       done += rounds;
       wide_done += rounds;
-      gkd::Copies look;
-      look.add(ctx->hctl, s.active, sizeof(int32_t));
-      GK_TRY(gkd::launch_copies(look, st));
-      GK_HIP(hipEventRecord(ctx->ev, st));
-      GK_HIP(hipEventSynchronize(ctx->ev));
-      const int32_t live = ctx->hctl[0];
+      int32_t live = 0;
+      const gkd::HostWords told = host_words(ctx);
+      GK_TRY(gkd::launch_tell(s.active, 1, told, st));
+      GK_TRY(wait_words(ctx, st, told, 1, &live));
       if (live == 0) break;
       if (can_loop && live <= kLoopSelected * s.nj) {
         loop = true;
@@ -996,14 +1017,13 @@ int upload_graph(gk_ctx* ctx, hipStream_t st, const gk_csr& h, bool check, Buf<i
   g->w = h.adjwgt ? w.p : nullptr;
   g->vw = h.vwgt ? v.p : nullptr;
   if (!check) return GK_OK;
-  gkd::Copies back;
-  back.add(ctx->hctl, verdict.p, 3 * sizeof(unsigned long long));
   GK_TRY(gkd::launch_graph_check(*g, verdict.p, st));
-  GK_TRY(gkd::launch_copies(back, st));
-  GK_HIP(hipEventRecord(ctx->ev, st));
-  GK_HIP(hipEventSynchronize(ctx->ev));
   unsigned long long r[3];
-  std::memcpy(r, ctx->hctl, sizeof r);
+  int32_t halves[6];
+  const gkd::HostWords told = host_words(ctx);
+  GK_TRY(gkd::launch_tell(reinterpret_cast<const int32_t*>(verdict.p), 6, told, st));
+  GK_TRY(wait_words(ctx, st, told, 6, halves));
+  std::memcpy(r, halves, sizeof r);
   const unsigned long long limit = 1ull << 31;
   if (r[0] != 0 || r[1] >= limit || r[2] / 2 >= limit) {
     gkh::set_error("graph changed while it was read");  // unless the host's check names its fault
@@ -1092,14 +1112,8 @@ int gk_ctx_create(int device, gk_ctx** out) {
     gkh::set_error("hipHostMalloc failed");
     return GK_ERR_NOMEM;
   }
-  c->hctl = reinterpret_cast<int32_t*>(c->hpin + kPinFetch);
-  if (hipEventCreateWithFlags(&c->ev, hipEventDisableTiming) != hipSuccess) {
-    (void)hipHostFree(c->hpin);
-    (void)hipStreamDestroy(c->stream);
-    delete c;
-    gkh::set_error("hipEventCreate failed");
-    return GK_ERR_HIP;
-  }
+  c->hctl = reinterpret_cast<unsigned long long*>(c->hpin + kPinFetch);
+  std::memset(c->hctl, 0, kPinCtl);
   *out = c;
   return GK_OK;
 }
@@ -1121,7 +1135,6 @@ int gk_ctx_destroy(gk_ctx* c) {
   DeviceGuard dg(c->device);
   (void)hipStreamSynchronize(c->stream);
   c->pool.release_all();
-  (void)hipEventDestroy(c->ev);
   (void)hipHostFree(c->hpin);
   (void)hipStreamDestroy(c->stream);
   delete c;
@@ -1296,11 +1309,10 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   int32_t nc2 = 0;
   GK_TRY(gr.count(ctx, st, n, cmap));
   if (n > 0) {
-    GK_TRY(gkd::launch_size_scan(n, gr.size.p, INT32_MAX, partial.p, gr.comp.p, gr.ctl.p, ctx->hctl, st));
-    GK_HIP(hipEventRecord(ctx->ev, st));
+    const gkd::HostWords told = gkrt::host_words(ctx);
+    GK_TRY(gkd::launch_size_scan(n, gr.size.p, INT32_MAX, partial.p, gr.comp.p, gr.ctl.p, told, st));
     GK_TRY(gkd::launch_member_place(n, cmap, gr.slot.p, gr.comp.p, dg->xadj, gr.ctl.p, m.cptr.p, m.mrow.p, st));
-    GK_HIP(hipEventSynchronize(ctx->ev));
-    nc2 = ctx->hctl[0];
+    GK_TRY(gkrt::wait_words(ctx, st, told, 1, &nc2));
   }
   m.ctl = std::move(gr.ctl);
   // With G = INT32_MAX every label is one chunk, so chunks are the coarse

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
+#include "dev_common.hpp"
 #include "steal.hpp"
 
 namespace gkd {
@@ -54,6 +55,8 @@ struct Copies {
   }
 };
 int launch_copies(const Copies& c, hipStream_t st);
+// Tells the host words[0, n), n <= 64.
+int launch_tell(const int32_t* words, int n, const HostWords& host, hipStream_t st);
 
 // Validity of a graph whose xadj begins with 0 and ends with nnz (weights may
 // be null: ones).  out (3 words, zero before): [0] != 0 for rows that do not
@@ -119,11 +122,11 @@ int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* 
 // size and slot of labels in [0, n) that come without a grouping.
 int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, hipStream_t st);
 // offc[l] = (first place, first coarse id) of label l's group; coarse ids and
-// flags to ctl and to host (pinned, kCtlInts ints).  partial: size_partials(n),
+// flags to ctl and, kCtlInts words, to host.  partial: size_partials(n),
 // offc: n + 1 (the last one the totals).
 int64_t size_partials(int64_t n);
-int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl, int32_t* host,
-                     hipStream_t st);
+int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl,
+                     const HostWords& host, hipStream_t st);
 // Vertices in (label, stamp, id) order, chunks of at most G, the members' rows
 // and weights in that order.  memb: 2n records; stamp, xadj, vw and the
 // outputs order, cmap, mrow, mvw may be null.  Groups of more than kRankMax members
@@ -189,10 +192,10 @@ int launch_contract_copy(int32_t nc, const int32_t* toff, const int32_t* len, co
 int launch_big_offsets(const int32_t* rows, const int32_t* ub, int32_t nrows, int32_t* boff, int32_t* scratch,
                        hipStream_t st);
 // cxadj = exclusive scan of len (nc + 1 entries); the entry count and the
-// kRowCtlWords class counters to host (pinned).  partial: size_partials(nc)
+// kRowCtlWords class counters to host.  partial: size_partials(nc)
 // ints (at least one).
-int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt, int32_t* host,
-                    hipStream_t st);
+int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt,
+                    const HostWords& host, hipStream_t st);
 
 // ---- refinement (refine.hip)
 int launch_project(int32_t n, const int32_t* cmap, const int32_t* cpart, const int32_t* cbnd,

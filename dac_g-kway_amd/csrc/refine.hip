@@ -276,6 +276,15 @@ __global__ void __launch_bounds__(256) k_copies(const Copies c) {
   }
 }
 
+__global__ void __launch_bounds__(64) k_tell(const int32_t* __restrict__ words, int n, const HostWords host) {
+  if (int(threadIdx.x) < n) tell(host, threadIdx.x, words[threadIdx.x]);
+}
+
+int launch_tell(const int32_t* words, int n, const HostWords& host, hipStream_t st) {
+  k_tell<<<1, 64, 0, st>>>(words, n, host);
+  return hip_status();
+}
+
 int launch_copies(const Copies& c, hipStream_t st) {
   int64_t most = 0;
   for (int i = 0; i < c.n; ++i) most = std::max(most, c.len[i]);

@@ -140,10 +140,10 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     a.next_status[1] = 0;
   }
   if (a.lastcnt[j] == 0) {  // converged in an earlier launch
-    if (a.host && t == 0) {
-      a.host[0] = 0;
-      a.host[1] = 0;
-      a.host[2] = a.rounds[j];
+    if (a.host.host && t == 0) {
+      tell(a.host, 0, 0);
+      tell(a.host, 1, 0);
+      tell(a.host, 2, a.rounds[j]);
     }
     return;
   }
@@ -168,10 +168,10 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     if (t == 0) {
       atomicAdd(&a.status[0], 1);
       atomicAdd(&a.status[1], 1);
-      if (a.host) {
-        a.host[0] = 1;
-        a.host[1] = 1;
-        a.host[2] = a.rounds[j];
+      if (a.host.host) {
+        tell(a.host, 0, 1);
+        tell(a.host, 1, 1);
+        tell(a.host, 2, a.rounds[j]);
       }
     }
     return;
@@ -755,10 +755,10 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
     a.moved[j] = moved0;
     a.lastcnt[j] = count;
     if (count) atomicAdd(&a.status[0], 1);
-    if (a.host) {
-      a.host[0] = count ? 1 : 0;
-      a.host[1] = 0;
-      a.host[2] = rounds0;
+    if (a.host.host) {
+      tell(a.host, 0, count ? 1 : 0);
+      tell(a.host, 1, 0);
+      tell(a.host, 2, rounds0);
     }
   }
 }

@@ -376,7 +376,7 @@ constexpr size_t kStagePiece = size_t(1) << 20;
 // Pinned bytes of a context: fetch() staging, then the control words.
 constexpr size_t kPinFetch = 4096;
 constexpr size_t kPinCtl = 256;
-static_assert(sizeof(int32_t) * gkd::kCtlInts <= kPinCtl && sizeof(int32_t) * (1 + gkd::kRowCtlWords) <= kPinCtl,
+static_assert(sizeof(uint64_t) * gkd::kCtlInts <= kPinCtl && sizeof(uint64_t) * (1 + gkd::kRowCtlWords) <= kPinCtl,
               "control words fit");
 }  // namespace gkrt
 
@@ -385,8 +385,8 @@ struct gk_ctx {
   hipStream_t stream = nullptr;
   gkrt::Pool pool;
   char* hpin = nullptr;  // pinned staging for small read-backs
-  int32_t* hctl = nullptr;  // pinned: control words that kernels write to the host themselves
-  hipEvent_t ev = nullptr;  // marks when they are written
+  unsigned long long* hctl = nullptr;  // pinned: control words that kernels tell the host
+  uint32_t told = 0;                   // numbers the calls that do
   gkrt::StageClock clock;
   gk_stats* cur = nullptr;  // stats of the running partition (stage counters)
   gkrt::Pinned up, dl;      // pinned staging of the batched form (uploads / read-backs)
@@ -578,6 +578,13 @@ struct StageGuard {
     ctx->up.drained();
   }
 };
+
+// Words that the next launch tells the host, and the wait for them (the first n
+// of them): the host watches the words themselves, and the stream now and then
+// in case they never come.  (Not for launches that are replayed from a graph:
+// those would carry an old number.)
+inline gkd::HostWords host_words(gk_ctx* ctx) { return gkd::HostWords{ctx->hctl, ++ctx->told}; }
+int wait_words(gk_ctx* ctx, hipStream_t st, const gkd::HostWords& h, int n, int32_t* out);
 
 // Members by coarse id: first place of every coarse id, and in member order
 // the vertices, their rows (start, length) and their weights; ctl: the
