@@ -285,9 +285,14 @@ __global__ void __launch_bounds__(256) k_walk(int32_t n, const int32_t* __restri
 }
 
 int launch_walk(int32_t n, const int32_t* cand, int2* comp, int32_t* key, int32_t* dist, int32_t* slot,
-                int32_t* flags, hipStream_t st) {
+                int32_t* ctl, hipStream_t st) {
   if (n <= 0) return 0;
-  fill<int2>(comp, int2{0, 0}, n, st);
+  Copies zero;
+  zero.add(comp, nullptr, sizeof(int2) * size_t(n));
+  zero.add(ctl, nullptr, sizeof(int32_t) * (kCtlInts + kRowCtlInts));
+  const int rc = launch_copies(zero, st);
+  if (rc) return rc;
+  int32_t* flags = ctl + kCtlFlags;
   k_walk<<<grid_for(n, 256), 256, 0, st>>>(n, cand, comp, key, dist, slot, flags);
   return hip_status();
 }
@@ -552,6 +557,167 @@ int launch_members(int32_t n, const int32_t* label, const int32_t* stamp, const 
   if (n <= 0) return 0;
   k_member_scatter<<<grid_for(n, 256), 256, 0, st>>>(n, label, stamp, slot, offc, xadj, vw, memb);
   k_member_rank<<<grid_for(n, 256), 256, 0, st>>>(n, memb, G, ctl, order, cmap, cptr, mrow, mvw);
+  return hip_status();
+}
+
+// Grouping, coarse ids and members of a small graph by one workgroup, in LDS:
+// the walk, the component counts, the scan over the labels, the places and the
+// ranks are the steps of the kernels above.  Their eight launches on a few
+// thousand vertices took 24 us and the gaps between them as much again.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallPer = kSmallGroup / kSmallThreads;
+static_assert(kSmallPer == 4 && kSmallGroup <= 65536, "16-bit ids, four vertices a thread");
+
+// Exclusive scan over the block (16 waves); *tot the sum.  ws: 16 ints, not
+// read by the scan before after this one's first barrier.
+__device__ __forceinline__ int small_scan(int x, int* tot, int32_t* ws) {
+  const int wave = threadIdx.x >> 6;
+  const int incl = wave_incl_scan(x);
+  if (lane_id() == 63) ws[wave] = incl;
+  __syncthreads();
+  int below = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < kSmallThreads / 64; ++w) {
+    below += w < wave ? ws[w] : 0;
+    all += ws[w];
+  }
+  *tot = all;
+  return incl - x + below;
+}
+
+__global__ void __launch_bounds__(kSmallThreads) k_group_small(int32_t n, const int32_t* __restrict__ cand, int32_t G,
+                                                               const int32_t* __restrict__ xadj,
+                                                               const int32_t* __restrict__ vw,
+                                                               int32_t* __restrict__ order,
+                                                               int32_t* __restrict__ cmap, int32_t* __restrict__ cptr,
+                                                               int2* __restrict__ mrow, int32_t* __restrict__ mvw,
+                                                               int32_t* __restrict__ ctl, const HostWords host) {
+  __shared__ uint16_t cd[kSmallGroup];                     // candidates; then the vertices by place
+  __shared__ int32_t mx[kSmallGroup], ct[kSmallGroup];     // by key: largest id above it, members
+  __shared__ uint16_t sz[kSmallGroup];                     // by label: members,
+  __shared__ uint16_t off[kSmallGroup], ch[kSmallGroup];   // first place, first coarse id
+  __shared__ uint8_t ds[kSmallGroup];
+  __shared__ int32_t wsm[16], wsc[16];
+  __shared__ int32_t deepest, largest;
+  const int t = threadIdx.x;
+  int32_t row[kSmallPer], len[kSmallPer], wt[kSmallPer];
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j) {
+    const int32_t v = t + j * kSmallThreads;
+    mx[v] = 0;
+    ct[v] = 0;
+    row[j] = len[j] = wt[j] = 0;
+    if (v < n) {
+      cd[v] = uint16_t(cand[v]);
+      row[j] = xadj[v];
+      len[j] = xadj[v + 1] - row[j];
+      wt[j] = vw[v];
+    }
+  }
+  if (t == 0) deepest = largest = 0;
+  for (int i = t; i < kCtlInts + kRowCtlInts; i += kSmallThreads) ctl[i] = 0;
+  __syncthreads();
+  int32_t key[kSmallPer], slot[kSmallPer];
+  int far = 0;
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j) {
+    const int32_t v = t + j * kSmallThreads;
+    key[j] = slot[j] = 0;
+    if (v >= n) continue;
+    int32_t a = v, d = 0, b = cd[a], c = cd[b];
+    while (c != a && d <= kWalkMax) {
+      a = b;
+      b = c;
+      c = cd[b];
+      ++d;
+    }
+    int32_t k = max(a, b);
+    if (c != a) {
+      k = v;
+      d = kWalkMax + 1;
+    }
+    key[j] = k;
+    ds[v] = uint8_t(d);
+    far = max(far, d);
+    if (v > k) atomicMax(&mx[k], v);
+    slot[j] = atomicAdd(&ct[k], 1);
+  }
+  far = wave_max(far);
+  if (lane_id() == 0) atomicMax(&deepest, far);
+  __syncthreads();
+  int32_t label[kSmallPer];
+  int big = 0;
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j) {
+    const int32_t v = t + j * kSmallThreads;
+    label[j] = max(mx[key[j]], key[j]);
+    const int32_t s = v < n && label[j] == v ? ct[key[j]] : 0;
+    sz[v] = uint16_t(s);
+    big = max(big, s);
+  }
+  big = wave_max(big);
+  if (lane_id() == 0) atomicMax(&largest, big);
+  __syncthreads();
+  {
+    int32_t s[kSmallPer];
+    int m = 0, c = 0;
+#pragma unroll
+    for (int j = 0; j < kSmallPer; ++j) {
+      s[j] = sz[t * kSmallPer + j];
+      m += s[j];
+      c += chunks_of(s[j], G);
+    }
+    int tm, tc;
+    int32_t rm = small_scan(m, &tm, wsm), rc = small_scan(c, &tc, wsc);
+#pragma unroll
+    for (int j = 0; j < kSmallPer; ++j) {
+      off[t * kSmallPer + j] = uint16_t(rm);
+      ch[t * kSmallPer + j] = uint16_t(rc);
+      rm += s[j];
+      rc += chunks_of(s[j], G);
+    }
+    if (t == 0) {
+      cptr[tc] = n;
+      ctl[0] = tc;
+      tell(host, 0, tc);
+      tell(host, 1, largest > kRankMax ? 1 : 0);
+#pragma unroll
+      for (int b = 0; b <= kWalkBits; ++b) tell(host, kCtlFlags + b, deepest > (1 << b) ? 1 : 0);
+    }
+  }
+  __syncthreads();
+  uint16_t* mem = cd;  // the walk has ended
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j) {
+    const int32_t v = t + j * kSmallThreads;
+    if (v < n) mem[off[label[j]] + slot[j]] = uint16_t(v);
+  }
+  __syncthreads();
+  if (largest > kRankMax) return;
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j) {
+    const int32_t v = t + j * kSmallThreads;
+    if (v >= n) continue;
+    const int32_t l = label[j], base = off[l], d = ds[v];
+    int32_t r = 0;
+    for (int32_t i = base; i < base + sz[l]; ++i) {
+      const int32_t u = mem[i];
+      r += (ds[u] < d || (ds[u] == d && u < v)) ? 1 : 0;
+    }
+    const int32_t p = base + r, q = r / G;
+    cmap[v] = ch[l] + q;
+    if (r - q * G == 0) cptr[ch[l] + q] = p;
+    if (order) order[p] = v;
+    mrow[p] = make_int2(row[j], len[j]);
+    mvw[p] = wt[j];
+  }
+}
+
+int launch_group_small(int32_t n, const int32_t* cand, int32_t G, const int32_t* xadj, const int32_t* vw,
+                       int32_t* order, int32_t* cmap, int32_t* cptr, int2* mrow, int32_t* mvw, int32_t* ctl,
+                       const HostWords& host, hipStream_t st) {
+  if (n <= 0 || n > kSmallGroup) return GK_ERR_LIMIT;
+  k_group_small<<<1, kSmallThreads, 0, st>>>(n, cand, G, xadj, vw, order, cmap, cptr, mrow, mvw, ctl, host);
   return hip_status();
 }
 
@@ -1332,7 +1498,8 @@ int launch_contract_big_merge(const int32_t* rows, int32_t nrows, const int32_t*
 }
 
 // Row starts of the coarse CSR from the rows' lengths: per-tile sums, then
-// every tile adds up the sums before it (many tiles: scanned by one block).
+// every tile adds up the sums before it (many tiles: scanned by one block; up to
+// kLenDirect tiles: the lengths before it, which saves the first launch).
 // The last tile writes the entry count and the row class counters to the host.
 __global__ void __launch_bounds__(256) k_len_reduce(int32_t nc, const int32_t* __restrict__ len,
                                                     int32_t* __restrict__ partial) {
@@ -1372,8 +1539,11 @@ __global__ void __launch_bounds__(256) k_len_apply(int32_t nc, const int32_t* __
   if (scanned) {
     pre = partial[blockIdx.x];
   } else {
+    // partial: the sums of the tiles before this one, or null and the lengths themselves
+    const int64_t nb = partial ? int64_t(blockIdx.x) : int64_t(blockIdx.x) * kSizeTile;
+    const int32_t* from = partial ? partial : len;
     int32_t s = 0;
-    for (int64_t b = threadIdx.x; b < int64_t(blockIdx.x); b += 256) s += partial[b];
+    for (int64_t b = threadIdx.x; b < nb; b += 256) s += from[b];
     (void)block_excl_scan_256(s, &t, lds);
     pre = t;
   }
@@ -1405,6 +1575,11 @@ __global__ void __launch_bounds__(256) k_len_apply(int32_t nc, const int32_t* __
 int launch_len_scan(int32_t nc, const int32_t* len, int32_t* partial, int32_t* cxadj, const int32_t* cnt,
                     const HostWords& host, hipStream_t st) {
   const int64_t nb = std::max<int64_t>(1, size_partials(nc));
+  constexpr int64_t kLenDirect = 4;
+  if (nb <= kLenDirect) {
+    k_len_apply<<<unsigned(nb), 256, 0, st>>>(nc, len, nullptr, 0, cxadj, cnt, host);
+    return hip_status();
+  }
   k_len_reduce<<<unsigned(nb), 256, 0, st>>>(nc, len, partial);
   const bool mid = nb > kSizeDirect;
   if (mid) k_len_mid<<<1, 256, 0, st>>>(nb, partial);

@@ -74,7 +74,7 @@ int wait_words(gk_ctx* ctx, hipStream_t st, const gkd::HostWords& h, int n, int3
 
 // ---------------------------------------------------------------- stages
 // Labels, hops and member counts of the groups by walking to the root pairs.
-// The control words (zeroed here) hold whether every vertex reached its pair.
+// The control words hold whether every vertex reached its pair.
 int Groups::walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label) {
   Pool& P = ctx->pool;
   GK_TRY(ctl.alloc(P, gkd::kCtlInts + gkd::kRowCtlInts));
@@ -82,9 +82,8 @@ int Groups::walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, in
   GK_TRY(dist.alloc(P, n));
   GK_TRY(slot.alloc(P, n));
   GK_TRY(size.alloc(P, n));
-  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts + gkd::kRowCtlInts, st);
   GK_STAGE(ctx, GK_ST_GROUP, 52LL * n,
-           (gkd::launch_walk(n, cand, comp.p, label, dist.p, slot.p, ctl.p + gkd::kCtlFlags, st) ||
+           (gkd::launch_walk(n, cand, comp.p, label, dist.p, slot.p, ctl.p, st) ||
                     gkd::launch_label_size(n, label, comp.p, label, size.p, st)
                 ? GK_ERR_HIP
                 : GK_OK));
@@ -233,13 +232,25 @@ int coarse_ids(gk_ctx* ctx, hipStream_t st, const DGraph& g, const int32_t* cand
   const int32_t n = g.n;
   Buf<int32_t> label;
   Groups gr;
-  GK_TRY(label.alloc(P, n));
   if (want_order) GK_TRY(m.order.alloc(P, n));
   GK_TRY(m.cptr.alloc(P, int64_t(n) + 1));
   GK_TRY(m.mrow.alloc(P, n));
   GK_TRY(m.mvw.alloc(P, n));
-  const MemberOut out{m.order.p, cmap, m.cptr.p, m.mrow.p, m.mvw.p};
   int32_t words[gkd::kCtlInts];
+  // Small graphs in one launch, unless a tree is too deep or a group too large.
+  if (n > 0 && n <= gkd::kSmallGroup) {
+    GK_TRY(m.ctl.alloc(P, gkd::kCtlInts + gkd::kRowCtlInts));
+    const gkd::HostWords told = host_words(ctx);
+    GK_STAGE(ctx, GK_ST_GROUP, 40LL * n,
+             gkd::launch_group_small(n, cand, G, g.xadj, g.vw, m.order.p, cmap, m.cptr.p, m.mrow.p, m.mvw.p, m.ctl.p,
+                                     told, st));
+    GK_TRY(wait_words(ctx, st, told, gkd::kCtlInts, words));
+    *rounds = Groups::rounds(words);
+    *nc = words[0];
+    if (!words[1] && !words[gkd::kCtlFlags + gkd::kWalkBits]) return GK_OK;
+  }
+  GK_TRY(label.alloc(P, n));
+  const MemberOut out{m.order.p, cmap, m.cptr.p, m.mrow.p, m.mvw.p};
   GK_TRY(gr.walk(ctx, st, n, cand, label.p));
   GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, words));
   *rounds = Groups::rounds(words);
@@ -328,10 +339,25 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
   }
   // The entry count comes back with the class counters; rows for the global
   // sort, if there are any, are merged then, and the lengths scanned again.
+  // Graphs of up to kEarlyEntries get arrays as large as their own, so that the
+  // rows are copied while the host still waits for their number.  (A caller's
+  // arrays need not be so large.)  Rows for the global sort are then copied
+  // twice, first up to their bounds.
+  constexpr int32_t kEarlyEntries = 1 << 20;
+  const bool early = !out && g.nnz <= kEarlyEntries;
+  auto copy_rows = [&](int32_t room) -> int {
+    if (!out) {
+      GK_TRY(c.adj.alloc(P, room));
+      GK_TRY(c.w.alloc(P, room));
+    }
+    return gkd::launch_contract_copy(nc, toff.p, len.p, c.xadj.p, tadj.p, tw.p, out ? out->adj : c.adj.p,
+                                     out ? out->w : c.w.p, out ? out->xadj : nullptr, st);
+  };
   auto scan_lengths = [&]() -> int {
     const gkd::HostWords told = host_words(ctx);
     GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc,
              gkd::launch_len_scan(nc, len.p, scratch.p, c.xadj.p, cnt, told, st));
+    if (early) GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc, copy_rows(g.nnz));
     return wait_words(ctx, st, told, 1 + gkd::kRowCtlWords, words);
   };
   GK_TRY(scan_lengths());
@@ -363,16 +389,14 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
     GK_TRY(scan_lengths());
   }
   const int32_t cnnz = words[0];
-  if (!out) {
-    GK_TRY(c.adj.alloc(P, cnnz));
-    GK_TRY(c.w.alloc(P, cnnz));
-  }
   // Row merge: member rows and the cmap gathers read once, merged rows
   // written once (known now that cnnz is).
   if (ctx->cur) ctx->cur->stage_bytes[GK_ST_CONTRACT] += 8LL * g.n + 20LL * nc + 12LL * g.nnz + 8LL * cnnz;
-  GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc + 16LL * cnnz,
-           gkd::launch_contract_copy(nc, toff.p, len.p, c.xadj.p, tadj.p, tw.p, out ? out->adj : c.adj.p,
-                                     out ? out->w : c.w.p, out ? out->xadj : nullptr, st));
+  if (early) {
+    if (ctx->cur) ctx->cur->stage_bytes[GK_ST_CONTRACT_AUX] += 16LL * cnnz;
+  } else {
+    GK_STAGE(ctx, GK_ST_CONTRACT_AUX, 12LL * nc + 16LL * cnnz, copy_rows(cnnz));
+  }
   c.g.n = nc;
   c.g.nnz = cnnz;
   c.g.xadj = c.xadj.p;

@@ -109,9 +109,9 @@ constexpr int32_t kRowsAllMax = 1 << 16;
 constexpr int32_t kRankMax = 512;
 // Grouping by walking to the root pair: key of v's component, hops, and comp
 // [key] = (largest id, members); slot[v] = v's place among the members
-// (arbitrary).  flags: the control words from kCtlFlags on.
+// (arbitrary).  ctl: kCtlInts + kRowCtlInts control words, zeroed here.
 int launch_walk(int32_t n, const int32_t* cand, int2* comp, int32_t* key, int32_t* dist, int32_t* slot,
-                int32_t* flags, hipStream_t st);
+                int32_t* ctl, hipStream_t st);
 // The same (without hops) from the pointers of the jumping rounds.
 int launch_comp_count(int32_t n, const int32_t* cand, const int32_t* next, int2* comp, int32_t* key, int32_t* slot,
                       hipStream_t st);
@@ -127,6 +127,16 @@ int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* 
 int64_t size_partials(int64_t n);
 int launch_size_scan(int32_t n, const int32_t* size, int32_t G, int2* partial, int2* offc, int32_t* ctl,
                      const HostWords& host, hipStream_t st);
+// The whole of it, from the walk to the members' order, for graphs of up to
+// kSmallGroup vertices in one workgroup: order (may be null), cmap, cptr, mrow
+// and mvw as launch_members, rows and weights from xadj and vw.  ctl: kCtlInts +
+// kRowCtlInts words, all written, the first kCtlInts also told the host; with
+// [1] or the flag of kWalkBits set the other results are void (the kernels
+// above take over).
+constexpr int32_t kSmallGroup = 4096;
+int launch_group_small(int32_t n, const int32_t* cand, int32_t G, const int32_t* xadj, const int32_t* vw,
+                       int32_t* order, int32_t* cmap, int32_t* cptr, int2* mrow, int32_t* mvw, int32_t* ctl,
+                       const HostWords& host, hipStream_t st);
 // Vertices in (label, stamp, id) order, chunks of at most G, the members' rows
 // and weights in that order.  memb: 2n records; stamp, xadj, vw and the
 // outputs order, cmap, mrow, mvw may be null.  Groups of more than kRankMax members
