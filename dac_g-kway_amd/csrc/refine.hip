@@ -685,15 +685,24 @@ int launch_boundary(const DGraph& g, const int32_t* part, int32_t* bnd, hipStrea
 }
 
 // calculate_cutsize + calculate_partition_wgt (gkway/uncoarsen.hpp:398-424,
-// gkway/cuda_check.hpp:61-73): grid-stride, 8 lanes per vertex; part weights
-// gathered in an LDS histogram per block, then one global atomic per block
-// and part (a block's share of the total weight fits 32 bits, the total
-// being below 2^31); the cut reduced per wave in 64 bits.
-// Blocks of the cut kernel: at most 2048, and at most 4 Mi part-weight slots.
+// gkway/cuda_check.hpp:61-73): grid-stride, 4 lanes per vertex, two entries a
+// lane and kCutPer vertices of a group in flight (one where there is but one);
+// part weights gathered in an LDS histogram per block (a block's share of the
+// total weight fits 32 bits, the total being below 2^31); the cut reduced per
+// wave in 64 bits.  With 8 lanes, one entry and one vertex the chain row,
+// neighbours, their parts was the time: a call on 2 M vertices in order (72 MB)
+// took 48 us, on 500 k 16.4; with four vertices 38 and 12.8, as it is here 30
+// and 9.8.  Blocks of 1024 threads, at most 512 of them, and at most 4 Mi
+// part-weight slots: a quarter of the slots that blocks of 256 write and
+// k_cut_sum adds up (a call on 65 k vertices 8.1 us with those, 6.5 with these,
+// which is the host's time for two launches).
+constexpr int kCutThreads = 1024;
+constexpr int kCutLanes = 4;
+
 inline unsigned cut_grid(int64_t n, int32_t k) {
-  unsigned grid = grid_for(n * 8, 256);
+  unsigned grid = grid_for(n * kCutLanes, kCutThreads);
   const int64_t cap = std::max<int64_t>(1, (int64_t(1) << 22) / std::max<int32_t>(k, 1));
-  if (grid > 2048) grid = 2048;
+  if (grid > 512) grid = 512;
   if (grid > cap) grid = static_cast<unsigned>(cap);
   return grid;
 }
@@ -703,32 +712,67 @@ int64_t cut_scratch(int64_t n, int32_t k) { return int64_t(cut_grid(n, k)) * (in
 // Each block writes its share of the cut and its part-weight histogram to its
 // own slots (bcut[b], bpw[b * k + q]); k_cut_sum adds them up.  No counter is
 // shared between blocks.
-__global__ void __launch_bounds__(256) k_cut(int32_t n, int32_t k, const int32_t* __restrict__ xadj,
-                                             const int32_t* __restrict__ adj,
-                                             const int32_t* __restrict__ w,
-                                             const int32_t* __restrict__ vw,
-                                             const int32_t* __restrict__ part,
-                                             unsigned long long* __restrict__ bcut,
-                                             unsigned long long* __restrict__ bpw) {
+template <int kCutPer>
+__global__ void __launch_bounds__(kCutThreads) k_cut(int32_t n, int32_t k, const int32_t* __restrict__ xadj,
+                                                     const int32_t* __restrict__ adj,
+                                                     const int32_t* __restrict__ w,
+                                                     const int32_t* __restrict__ vw,
+                                                     const int32_t* __restrict__ part,
+                                                     unsigned long long* __restrict__ bcut,
+                                                     unsigned long long* __restrict__ bpw) {
   extern __shared__ unsigned int hist32[];
-  __shared__ long long wc[4];
-  for (int32_t q = threadIdx.x; q < k; q += 256) hist32[q] = 0;
+  __shared__ long long wc[kCutThreads / 64];
+  for (int32_t q = threadIdx.x; q < k; q += kCutThreads) hist32[q] = 0;
   __syncthreads();
   long long c = 0;
-  const int sub = threadIdx.x & 7;
-  for (int64_t v = (int64_t(xcd_block()) * 256 + threadIdx.x) / 8; v < n; v += int64_t(gridDim.x) * 32) {
-    const int32_t p = part[v];
-    for (int32_t j = xadj[v] + sub; j < xadj[v + 1]; j += 8) {
-      const int32_t u = adj[j];
-      if (v < u && part[u] != p) c += w[j];
+  const int sub = threadIdx.x % kCutLanes;
+  const int64_t stride = int64_t(gridDim.x) * (kCutThreads / kCutLanes);
+  for (int64_t v0 = (int64_t(xcd_block()) * kCutThreads + threadIdx.x) / kCutLanes; v0 < n; v0 += kCutPer * stride) {
+    int32_t s[kCutPer], e[kCutPer], p[kCutPer], x[kCutPer], u[kCutPer][2], q[kCutPer][2];
+#pragma unroll
+    for (int i = 0; i < kCutPer; ++i) {
+      const int64_t v = v0 + i * stride;
+      s[i] = e[i] = p[i] = x[i] = 0;
+      if (v < n) {
+        s[i] = xadj[v];
+        e[i] = xadj[v + 1];
+        p[i] = part[v];
+        if (sub == 0) x[i] = vw[v];
+      }
     }
-    if (sub == 0) atomicAdd(&hist32[p], (unsigned int)vw[v]);
+#pragma unroll
+    for (int i = 0; i < kCutPer; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int32_t j = s[i] + sub + h * kCutLanes;
+        u[i][h] = j < e[i] ? adj[j] : -1;
+      }
+#pragma unroll
+    for (int i = 0; i < kCutPer; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) q[i][h] = u[i][h] > v0 + i * stride ? part[u[i][h]] : p[i];
+#pragma unroll
+    for (int i = 0; i < kCutPer; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (q[i][h] != p[i]) c += w[s[i] + sub + h * kCutLanes];
+      if (sub == 0 && x[i]) atomicAdd(&hist32[p[i]], (unsigned int)x[i]);
+      for (int32_t j = s[i] + sub + 2 * kCutLanes; j < e[i]; j += kCutLanes) {
+        const int32_t y = adj[j];
+        if (y > v0 + i * stride && part[y] != p[i]) c += w[j];
+      }
+    }
   }
   c = wave_sum64(c);
   if (lane_id() == 0) wc[threadIdx.x >> 6] = c;
   __syncthreads();
-  if (threadIdx.x == 0) bcut[blockIdx.x] = (unsigned long long)(wc[0] + wc[1] + wc[2] + wc[3]);
-  for (int32_t q = threadIdx.x; q < k; q += 256) bpw[int64_t(blockIdx.x) * k + q] = hist32[q];
+  if (threadIdx.x == 0) {
+    long long t = 0;
+#pragma unroll
+    for (int i = 0; i < kCutThreads / 64; ++i) t += wc[i];
+    bcut[blockIdx.x] = (unsigned long long)t;
+  }
+  for (int32_t q = threadIdx.x; q < k; q += kCutThreads) bpw[int64_t(blockIdx.x) * k + q] = hist32[q];
 }
 
 // Block q < k: pw64[q] = sum of the blocks' slots for part q; block k: the
@@ -768,7 +812,8 @@ int launch_cut(const DGraph& g, int32_t k, const int32_t* part, unsigned long lo
   if (int64_t(grid) > fit) grid = static_cast<unsigned>(fit);
   unsigned long long* bcut = scratch;
   unsigned long long* bpw = scratch + grid;
-  k_cut<<<grid, 256, sizeof(unsigned int) * k, st>>>(g.n, k, g.xadj, g.adj, g.w, g.vw, part, bcut, bpw);
+  const auto kernel = int64_t(g.n) * kCutLanes <= int64_t(grid) * kCutThreads ? k_cut<1> : k_cut<2>;
+  kernel<<<grid, kCutThreads, sizeof(unsigned int) * k, st>>>(g.n, k, g.xadj, g.adj, g.w, g.vw, part, bcut, bpw);
   k_cut_sum<<<k + 1, 256, 0, st>>>(int32_t(grid), k, bcut, bpw, cut, pw64);
   return hip_status();
 }
