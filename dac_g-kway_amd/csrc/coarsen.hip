@@ -361,9 +361,12 @@ __global__ void __launch_bounds__(256) k_label_count(int32_t n, const int32_t* _
   if (live) slot[v] = atomicAdd(&size[l], 1);
 }
 
-int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, hipStream_t st) {
-  if (n <= 0) return 0;
-  fill<int32_t>(size, 0, n, st);
+int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, int32_t* ctl, hipStream_t st) {
+  Copies zero;
+  zero.add(ctl, nullptr, sizeof(int32_t) * (kCtlInts + kRowCtlInts));
+  if (n > 0) zero.add(size, nullptr, sizeof(int32_t) * size_t(n));
+  const int rc = launch_copies(zero, st);
+  if (rc || n <= 0) return rc;
   k_label_count<<<grid_for(n, 256), 256, 0, st>>>(n, label, size, slot);
   return hip_status();
 }
@@ -533,10 +536,10 @@ __global__ void __launch_bounds__(256) k_member_rank(int32_t n, const int4* __re
                                                      int2* __restrict__ mrow, int32_t* __restrict__ mvw) {
   const int64_t i = int64_t(xcd_block()) * 256 + threadIdx.x;
   if (i >= n) return;
+  if (ctl[1]) return;  // some group is too large: the caller sorts
   if (i == n - 1) cptr[ctl[0]] = n;
   const int4 a = memb[2 * i], b = memb[2 * i + 1];
   const int32_t cnt = b.w;
-  if (cnt > kRankMax) return;  // ctl[1] is set: the caller sorts
   int32_t r = 0;
   for (int32_t j = 0; j < cnt; ++j) {
     const int4 o = memb[2 * (int64_t(a.z) + j)];
@@ -841,19 +844,24 @@ int launch_cluster(int32_t n, const uint64_t* skeys, const int32_t* sids, int sb
 
 // cal_coarsen_vwgt (gkway/coarsen.hpp:157-171) as an ordered sum over the
 // (at most G) members of each chunk, their weights in member order; no
-// atomics, destination fully written.
-__global__ void __launch_bounds__(256) k_cvwgt(int32_t nc, const int32_t* __restrict__ cptr,
+// atomics, destination fully written.  With ctl the chunks are counted there
+// (nc: no more than that), and nothing is done where the members are not in
+// order (ctl[1]).
+__global__ void __launch_bounds__(256) k_cvwgt(int32_t nc, const int32_t* __restrict__ ctl,
+                                               const int32_t* __restrict__ cptr,
                                                const int32_t* __restrict__ mvw, int32_t* __restrict__ cvw) {
   const int64_t c = int64_t(xcd_block()) * 256 + threadIdx.x;
+  if (ctl) nc = ctl[1] ? 0 : min(nc, ctl[0]);
   if (c >= nc) return;
   int32_t s = 0;
   for (int32_t j = cptr[c]; j < cptr[c + 1]; ++j) s += mvw[j];
   cvw[c] = s;
 }
 
-int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* mvw, int32_t* cvw, hipStream_t st) {
+int launch_cvwgt(int32_t nc, const int32_t* ctl, const int32_t* cptr, const int32_t* mvw, int32_t* cvw,
+                 hipStream_t st) {
   if (nc <= 0) return 0;
-  k_cvwgt<<<grid_for(nc, 256), 256, 0, st>>>(nc, cptr, mvw, cvw);
+  k_cvwgt<<<grid_for(nc, 256), 256, 0, st>>>(nc, ctl, cptr, mvw, cvw);
   return hip_status();
 }
 

@@ -73,17 +73,18 @@ int wait_words(gk_ctx* ctx, hipStream_t st, const gkd::HostWords& h, int n, int3
 }
 
 // ---------------------------------------------------------------- stages
-// Labels, hops and member counts of the groups by walking to the root pairs.
+// Labels, hops (to dist_out, or dist) and member counts of the groups by
+// walking to the root pairs.
 // The control words hold whether every vertex reached its pair.
-int Groups::walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label) {
+int Groups::walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* dist_out) {
   Pool& P = ctx->pool;
   GK_TRY(ctl.alloc(P, gkd::kCtlInts + gkd::kRowCtlInts));
   GK_TRY(comp.alloc(P, int64_t(n) + 1));
-  GK_TRY(dist.alloc(P, n));
+  if (!dist_out) GK_TRY(dist.alloc(P, n));
   GK_TRY(slot.alloc(P, n));
   GK_TRY(size.alloc(P, n));
   GK_STAGE(ctx, GK_ST_GROUP, 52LL * n,
-           (gkd::launch_walk(n, cand, comp.p, label, dist.p, slot.p, ctl.p, st) ||
+           (gkd::launch_walk(n, cand, comp.p, label, dist_out ? dist_out : dist.p, slot.p, ctl.p, st) ||
                     gkd::launch_label_size(n, label, comp.p, label, size.p, st)
                 ? GK_ERR_HIP
                 : GK_OK));
@@ -154,17 +155,16 @@ int Groups::count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label) 
   GK_TRY(comp.alloc(P, int64_t(n) + 1));
   GK_TRY(slot.alloc(P, n));
   GK_TRY(size.alloc(P, n));
-  gkd::fill<int32_t>(ctl.p, 0, gkd::kCtlInts + gkd::kRowCtlInts, st);
-  GK_STAGE(ctx, GK_ST_SORT, 16LL * n, gkd::launch_label_count(n, label, size.p, slot.p, st));
+  GK_STAGE(ctx, GK_ST_SORT, 16LL * n, gkd::launch_label_count(n, label, size.p, slot.p, ctl.p, st));
   return GK_OK;
 }
 
 // Order, coarse ids and member records by counting, from the groups' sizes
-// and slots.  words (kCtlInts) receives the control words; words[1] != 0: some
+// and slots.  The control words (kCtlInts) are told the host; [1] != 0: some
 // group is too large, the results are incomplete and sort_members is needed.
 static int count_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* stamp,
                          Groups& gr, const int32_t* xadj, const int32_t* vw, int32_t G, const MemberOut& out,
-                         int32_t* words) {
+                         gkd::HostWords* told_out) {
   Buf<int2> partial;
   Buf<int4> memb;
   const gkd::HostWords told = host_words(ctx);
@@ -176,7 +176,8 @@ static int count_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* 
   GK_STAGE(ctx, GK_ST_SORT, 120LL * n,
            gkd::launch_members(n, label, stamp, gr.slot.p, gr.comp.p, xadj, vw, memb.p, G, gr.ctl.p, out.order,
                                out.cmap, out.cptr, out.mrow, out.mvw, st));
-  return wait_words(ctx, st, told, gkd::kCtlInts, words);
+  *told_out = told;
+  return GK_OK;
 }
 
 // The same by a radix sort of (label, stamp), stamps below 2^sbits.
@@ -251,12 +252,15 @@ int coarse_ids(gk_ctx* ctx, hipStream_t st, const DGraph& g, const int32_t* cand
   }
   GK_TRY(label.alloc(P, n));
   const MemberOut out{m.order.p, cmap, m.cptr.p, m.mrow.p, m.mvw.p};
+  gkd::HostWords told;
   GK_TRY(gr.walk(ctx, st, n, cand, label.p));
-  GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, words));
+  GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, &told));
+  GK_TRY(wait_words(ctx, st, told, gkd::kCtlInts, words));
   *rounds = Groups::rounds(words);
   if (words[gkd::kCtlFlags + gkd::kWalkBits]) {
     GK_TRY(gr.jump(ctx, st, n, cand, label.p, rounds));
-    GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, words));
+    GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, &told));
+    GK_TRY(wait_words(ctx, st, told, gkd::kCtlInts, words));
   }
   *nc = words[0];
   // Distances are at most 2^rounds.
@@ -1268,9 +1272,20 @@ int gk_k_group(gk_ctx* ctx, int32_t n, const int32_t* cand, int32_t* label, int3
   if (n <= 0) { if (sweeps) *sweeps = 0; return GK_OK; }
   Groups gr;
   int32_t words[gkd::kCtlInts];
-  GK_TRY(gr.walk(ctx, st, n, cand, label));
-  GK_HIP(hipMemcpyAsync(stamp, gr.dist.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
-  GK_TRY(fetch(ctx, st, {{words, gr.ctl.p, sizeof words}}));
+  // The walk writes labels and hops while it reads candidates: where those lie
+  // in the same place, it works on a copy.
+  Buf<int32_t> own;
+  auto apart = [&](const int32_t* x) { return x + n <= cand || cand + n <= x; };
+  if (!apart(stamp) || !apart(label)) {
+    GK_TRY(own.alloc(ctx->pool, n));
+    GK_HIP(hipMemcpyAsync(own.p, cand, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
+    cand = own.p;
+  }
+  const gkd::HostWords told = gkrt::host_words(ctx);
+  GK_TRY(gr.walk(ctx, st, n, cand, label, stamp));
+  GK_TRY(gkd::launch_tell(gr.ctl.p, gkd::kCtlInts, told, st));
+  GK_HIP(hipStreamSynchronize(st));
+  GK_TRY(gkrt::wait_words(ctx, st, told, gkd::kCtlInts, words));
   int32_t rounds = Groups::rounds(words);
   if (words[gkd::kCtlFlags + gkd::kWalkBits]) {
     GK_TRY(gr.jump(ctx, st, n, cand, label, &rounds));
@@ -1298,7 +1313,11 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
   const MemberOut out{order, cmap, cptr.p, nullptr, mvw.p};
   int32_t words[gkd::kCtlInts];
   GK_TRY(gr.count(ctx, st, n, label));
-  GK_TRY(count_members(ctx, st, n, label, stamp, gr, nullptr, vwgt, max_group, out, words));
+  gkd::HostWords told;
+  GK_TRY(count_members(ctx, st, n, label, stamp, gr, nullptr, vwgt, max_group, out, &told));
+  GK_TRY(gkd::launch_cvwgt(n, gr.ctl.p, cptr.p, mvw.p, cvwgt, st));
+  GK_HIP(hipStreamSynchronize(st));
+  GK_TRY(gkrt::wait_words(ctx, st, told, gkd::kCtlInts, words));
   *nc = words[0];
   if (words[1]) {
     // The stamp bit width is taken from the data (max stamp).
@@ -1307,9 +1326,9 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
     int32_t mx = 0;
     for (int32_t x : hs) mx = std::max(mx, x);
     GK_TRY(sort_members(ctx, st, n, label, stamp, bits_for(mx), nullptr, vwgt, max_group, out, nc));
+    GK_TRY(gkd::launch_cvwgt(*nc, nullptr, cptr.p, mvw.p, cvwgt, st));
+    GK_HIP(hipStreamSynchronize(st));
   }
-  GK_TRY(gkd::launch_cvwgt(*nc, cptr.p, mvw.p, cvwgt, st));
-  GK_HIP(hipStreamSynchronize(st));
   return GK_OK;
 }
 

@@ -119,8 +119,9 @@ int launch_comp_count(int32_t n, const int32_t* cand, const int32_t* next, int2*
 // where l is no label).  key may be label.
 int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* label, int32_t* size,
                       hipStream_t st);
-// size and slot of labels in [0, n) that come without a grouping.
-int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, hipStream_t st);
+// size and slot of labels in [0, n) that come without a grouping; ctl as in
+// launch_walk.
+int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, int32_t* ctl, hipStream_t st);
 // offc[l] = (first place, first coarse id) of label l's group; coarse ids and
 // flags to ctl and, kCtlInts words, to host.  partial: size_partials(n),
 // offc: n + 1 (the last one the totals).
@@ -273,6 +274,7 @@ int launch_cut(const DGraph& g, int32_t k, const int32_t* part, unsigned long lo
                int64_t max_slots = INT64_MAX);
 
 int launch_sum(const int32_t* a, int64_t n, unsigned long long* out, hipStream_t st);
-int launch_cvwgt(int32_t nc, const int32_t* cptr, const int32_t* mvw, int32_t* cvw, hipStream_t st);
+int launch_cvwgt(int32_t nc, const int32_t* ctl, const int32_t* cptr, const int32_t* mvw, int32_t* cvw,
+                 hipStream_t st);
 
 }  // namespace gkd

@@ -555,7 +555,7 @@ struct Level;
 struct Groups {
   Buf<int32_t> ctl, dist, slot, size;
   Buf<int2> comp;
-  int walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label);
+  int walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* dist_out = nullptr);
   int jump(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* rounds);
   int count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label);
   static int32_t rounds(const int32_t* words);
