@@ -162,27 +162,34 @@ int Groups::count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label) 
 // Order, coarse ids and member records by counting, from the groups' sizes
 // and slots.  The control words (kCtlInts) are told the host; [1] != 0: some
 // group is too large, the results are incomplete and sort_members is needed.
+// So it is with *no_room: the pool had none for the members' records (32 bytes
+// a vertex beside the counts; the sort's arrays come after the counts are
+// given back), and nothing but the control words is written.
 static int count_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* stamp,
                          Groups& gr, const int32_t* xadj, const int32_t* vw, int32_t G, const MemberOut& out,
-                         gkd::HostWords* told_out) {
+                         gkd::HostWords* told_out, bool* no_room) {
   Buf<int2> partial;
   Buf<int4> memb;
   const gkd::HostWords told = host_words(ctx);
   GK_TRY(partial.alloc(ctx->pool, gkd::size_partials(n)));
-  GK_TRY(memb.alloc(ctx->pool, 2 * int64_t(n)));
+  *no_room = memb.alloc(ctx->pool, 2 * int64_t(n)) != GK_OK;
   GK_STAGE(ctx, GK_ST_SORT, 16LL * n,
            gkd::launch_size_scan(n, gr.size.p, G, partial.p, gr.comp.p, gr.ctl.p, told, st));
+  *told_out = told;
+  if (*no_room) return GK_OK;
   // The counts come back while the members are ordered.
   GK_STAGE(ctx, GK_ST_SORT, 120LL * n,
            gkd::launch_members(n, label, stamp, gr.slot.p, gr.comp.p, xadj, vw, memb.p, G, gr.ctl.p, out.order,
                                out.cmap, out.cptr, out.mrow, out.mvw, st));
-  *told_out = told;
   return GK_OK;
 }
 
-// The same by a radix sort of (label, stamp), stamps below 2^sbits.
+// The same by a radix sort of (label, stamp), stamps below 2^sbits.  The rows
+// and weights (out.mrow and out.mvw are not used) are allocated when the keys
+// have been given back: 12 bytes a vertex less at the peak.
 static int sort_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label, const int32_t* stamp, int sbits,
-                        const int32_t* xadj, const int32_t* vw, int32_t G, const MemberOut& out, int32_t* nc) {
+                        const int32_t* xadj, const int32_t* vw, int32_t G, const MemberOut& out, Buf<int2>* mrow,
+                        Buf<int32_t>* mvw, int32_t* nc) {
   Pool& P = ctx->pool;
   const int lbits = bits_for(n > 0 ? n - 1 : 0);
   Buf<uint64_t> keys, keys2;
@@ -192,6 +199,8 @@ static int sort_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* l
     gkd::fill<int32_t>(zero.p, 0, n, st);
     stamp = zero.p;
   }
+  if (mrow) mrow->release();
+  mvw->release();
   int32_t* cmap = out.cmap;
   if (!cmap) {
     GK_TRY(cm.alloc(P, n));
@@ -213,12 +222,22 @@ static int sort_members(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* l
                 ? GK_ERR_HIP
                 : GK_OK));
   const int32_t* sid = alt ? ids2.p : ids.p;
-  GK_STAGE(ctx, GK_ST_CLUSTER, 80LL * n,
-           (gkd::launch_cluster(n, alt ? keys2.p : keys.p, sid, sbits, G, gstart.p, flagscan.p, cmap, out.cptr, ncd.p,
-                                scratch.p, st) ||
-                    (out.mrow || out.mvw ? gkd::launch_member_rows(n, sid, xadj, vw, out.mrow, out.mvw, st) : 0)
-                ? GK_ERR_HIP
-                : GK_OK));
+  auto rows = [&]() -> int {
+    keys.release();
+    keys2.release();
+    gstart.release();
+    flagscan.release();
+    if (mrow) GK_TRY(mrow->alloc(P, n));
+    GK_TRY(mvw->alloc(P, n));
+    return gkd::launch_member_rows(n, sid, xadj, vw, mrow ? mrow->p : nullptr, mvw->p, st);
+  };
+  ctx->clock.begin(GK_ST_CLUSTER);
+  int rc = gkd::launch_cluster(n, alt ? keys2.p : keys.p, sid, sbits, G, gstart.p, flagscan.p, cmap, out.cptr, ncd.p,
+                               scratch.p, st);
+  if (!rc) rc = rows();
+  ctx->clock.end(GK_ST_CLUSTER);
+  if (rc) return rc;
+  count_stage(ctx, GK_ST_CLUSTER, 80LL * n);
   if (out.order)
     GK_HIP(hipMemcpyAsync(out.order, sid, sizeof(int32_t) * size_t(n), hipMemcpyDeviceToDevice, st));
   GK_TRY(fetch(ctx, st, {{nc, ncd.p, sizeof(int32_t)}}));
@@ -253,18 +272,22 @@ int coarse_ids(gk_ctx* ctx, hipStream_t st, const DGraph& g, const int32_t* cand
   GK_TRY(label.alloc(P, n));
   const MemberOut out{m.order.p, cmap, m.cptr.p, m.mrow.p, m.mvw.p};
   gkd::HostWords told;
+  bool no_room = false;
   GK_TRY(gr.walk(ctx, st, n, cand, label.p));
-  GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, &told));
+  GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, &told, &no_room));
   GK_TRY(wait_words(ctx, st, told, gkd::kCtlInts, words));
   *rounds = Groups::rounds(words);
   if (words[gkd::kCtlFlags + gkd::kWalkBits]) {
     GK_TRY(gr.jump(ctx, st, n, cand, label.p, rounds));
-    GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, &told));
+    GK_TRY(count_members(ctx, st, n, label.p, gr.dist.p, gr, g.xadj, g.vw, G, out, &told, &no_room));
     GK_TRY(wait_words(ctx, st, told, gkd::kCtlInts, words));
   }
   *nc = words[0];
   // Distances are at most 2^rounds.
-  if (words[1]) GK_TRY(sort_members(ctx, st, n, label.p, gr.dist.p, *rounds + 1, g.xadj, g.vw, G, out, nc));
+  if (words[1] || no_room) {
+    gr.counts_done();
+    GK_TRY(sort_members(ctx, st, n, label.p, gr.dist.p, *rounds + 1, g.xadj, g.vw, G, out, &m.mrow, &m.mvw, nc));
+  }
   m.ctl = std::move(gr.ctl);
   return GK_OK;
 }
@@ -345,12 +368,20 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
   // sort, if there are any, are merged then, and the lengths scanned again.
   // Graphs of up to kEarlyEntries get arrays as large as their own, so that the
   // rows are copied while the host still waits for their number.  (A caller's
-  // arrays need not be so large.)  Rows for the global sort are then copied
-  // twice, first up to their bounds.
+  // arrays need not be so large.)  They stay as large as that (levels of 8 MB at
+  // most): under a pool limit, without room, or with rows for the global sort,
+  // which needs the room, the rows are copied once it is known.
   constexpr int32_t kEarlyEntries = 1 << 20;
-  const bool early = !out && g.nnz <= kEarlyEntries;
+  bool early = !out && !P.limited() && g.nnz <= kEarlyEntries && c.adj.alloc(P, g.nnz) == GK_OK &&
+               c.w.alloc(P, g.nnz) == GK_OK;
+  auto not_early = [&]() {
+    early = false;
+    c.adj.release();
+    c.w.release();
+  };
+  if (!early) not_early();
   auto copy_rows = [&](int32_t room) -> int {
-    if (!out) {
+    if (!out && !early) {
       GK_TRY(c.adj.alloc(P, room));
       GK_TRY(c.w.alloc(P, room));
     }
@@ -367,6 +398,7 @@ int contract_stage(gk_ctx* ctx, hipStream_t st, const DGraph& g, int32_t nc, con
   GK_TRY(scan_lengths());
   if (hc[4] > 0) {
     const int32_t nbig = hc[4], eb = hc[gkd::kRowBigEntries];
+    not_early();
     const int32_t* rows = lists.p + int64_t(4) * nc;
     Buf<int32_t> boff, bscr;
     GK_TRY(boff.alloc(P, int64_t(nbig) + 1));
@@ -671,6 +703,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     Level c;
     GK_TRY(c.vw.alloc(P, nc));
     c.g.vw = c.vw.p;
+    if (!trace) cand.release();
     GK_TRY(contract_stage(ctx, st, f.g, nc, cmap.p, mem, c));
     ls.sweeps = rounds;
     if (trace) {
@@ -1327,18 +1360,20 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
   int32_t words[gkd::kCtlInts];
   GK_TRY(gr.count(ctx, st, n, label));
   gkd::HostWords told;
-  GK_TRY(count_members(ctx, st, n, label, stamp, gr, nullptr, vwgt, max_group, out, &told));
-  GK_TRY(gkd::launch_cvwgt(n, gr.ctl.p, cptr.p, mvw.p, cvwgt, st));
+  bool no_room = false;
+  GK_TRY(count_members(ctx, st, n, label, stamp, gr, nullptr, vwgt, max_group, out, &told, &no_room));
+  if (!no_room) GK_TRY(gkd::launch_cvwgt(n, gr.ctl.p, cptr.p, mvw.p, cvwgt, st));
   GK_HIP(hipStreamSynchronize(st));
   GK_TRY(gkrt::wait_words(ctx, st, told, gkd::kCtlInts, words));
   *nc = words[0];
-  if (words[1]) {
+  if (words[1] || no_room) {
+    gr.counts_done();
     // The stamp bit width is taken from the data (max stamp).
     std::vector<int32_t> hs;
     GK_TRY(to_host(st, hs, stamp, n));
     int32_t mx = 0;
     for (int32_t x : hs) mx = std::max(mx, x);
-    GK_TRY(sort_members(ctx, st, n, label, stamp, bits_for(mx), nullptr, vwgt, max_group, out, nc));
+    GK_TRY(sort_members(ctx, st, n, label, stamp, bits_for(mx), nullptr, vwgt, max_group, out, nullptr, &mvw, nc));
     GK_TRY(gkd::launch_cvwgt(*nc, nullptr, cptr.p, mvw.p, cvwgt, st));
     GK_HIP(hipStreamSynchronize(st));
   }

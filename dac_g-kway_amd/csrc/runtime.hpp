@@ -74,6 +74,7 @@ class Pool {
   // Bytes the pool may hand out at once (0 = no limit); a request beyond it
   // fails with GK_ERR_NOMEM.
   void set_limit(int64_t bytes) { limit_ = bytes > 0 ? bytes : 0; }
+  bool limited() const { return limit_ > 0; }
   void reset_peak() { peak_ = in_use_; }
   void trim() {
     for (auto& kv : free_) {
@@ -558,6 +559,11 @@ struct Groups {
   int walk(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* dist_out = nullptr);
   int jump(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, int32_t* label, int32_t* rounds);
   int count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label);
+  void counts_done() {  // the control words and distances stay
+    slot.release();
+    size.release();
+    comp.release();
+  }
   static int32_t rounds(const int32_t* words);
 };
 
