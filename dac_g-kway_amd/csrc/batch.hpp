@@ -137,10 +137,6 @@ struct RoundsArgs {
   HostWords host;  // one job: live, left out, ordering rounds so far
 };
 int launch_rounds(const RoundsArgs& a, int32_t nj, int lanes, hipStream_t st);
-// Per-job state before a level's first round (rounds, moved and abytes 0,
-// lastcnt and thr 1) and the 4 words each of wlc and status.
-int launch_rounds_init(int32_t nj, int32_t* lastcnt, int32_t* thr, int32_t* rounds, long long* moved,
-                       long long* abytes, int32_t* wlc, int32_t* status, hipStream_t st);
 // *out = largest row length of g.
 int launch_max_deg(const DGraph& g, int32_t* out, hipStream_t st);
 // Final cut and part weights of the jobs covered by the chunk table: chunk c

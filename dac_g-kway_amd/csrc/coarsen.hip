@@ -1,10 +1,10 @@
 // Coarsening kernels for gfx950: heavy-edge candidate matching, grouping of
-// the candidate pseudo-forest by pointer jumping, chunking into coarse
-// vertices, and CSR contraction (relabel, per-row sort, merge of parallel
-// edges) -- the work of gkway/coarsen.hpp.  Every kernel is integer-exact and
-// writes results that do not depend on the launch schedule: atomics are used
-// only for commutative integer max/add or for slot reservation whose order is
-// discarded by a later sort.
+// the candidate pseudo-forest by walking to the root pairs (pointer jumping in
+// deep trees), chunking into coarse vertices, and CSR contraction (relabel,
+// per-row sort, merge of parallel edges) -- the work of gkway/coarsen.hpp.
+// Every kernel is integer-exact and writes results that do not depend on the
+// launch schedule: atomics are used only for commutative integer max/add or for
+// slot reservation whose order is discarded by a later rank or sort.
 #include <algorithm>
 
 #include "kernels.hpp"

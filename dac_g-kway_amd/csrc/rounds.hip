@@ -24,8 +24,6 @@
 // more vertices than one workgroup should (a large graph's first rounds)
 // appends them to the worklist and leaves, for the gain pass over the whole
 // device and another launch.
-#include <algorithm>
-
 #include "balance.hpp"
 #include "batch.hpp"
 #include "gain.hpp"
@@ -777,31 +775,6 @@ int launch_rounds(const RoundsArgs& a, int32_t nj, int lanes, hipStream_t st) {
   if (lanes <= 8) rounds_go<8>(a, nj, st);
   else if (lanes <= 16) rounds_go<16>(a, nj, st);
   else rounds_go<32>(a, nj, st);
-  return hip_status();
-}
-
-// State of a level's rounds before the first one: per job the counters, and
-// the words that the launches share.
-__global__ void __launch_bounds__(256) k_rounds_init(int32_t nj, int32_t* __restrict__ lastcnt,
-                                                     int32_t* __restrict__ thr, int32_t* __restrict__ rounds,
-                                                     long long* __restrict__ moved, long long* __restrict__ abytes,
-                                                     int32_t* __restrict__ wlc, int32_t* __restrict__ status) {
-  const int32_t j = blockIdx.x * 256 + threadIdx.x;
-  if (j < 4) {
-    wlc[j] = 0;
-    status[j] = 0;
-  }
-  if (j >= nj) return;
-  lastcnt[j] = 1;
-  thr[j] = 1;
-  rounds[j] = 0;
-  moved[j] = 0;
-  abytes[j] = 0;
-}
-
-int launch_rounds_init(int32_t nj, int32_t* lastcnt, int32_t* thr, int32_t* rounds, long long* moved,
-                       long long* abytes, int32_t* wlc, int32_t* status, hipStream_t st) {
-  k_rounds_init<<<grid_for(std::max(nj, 4), 256), 256, 0, st>>>(nj, lastcnt, thr, rounds, moved, abytes, wlc, status);
   return hip_status();
 }
 

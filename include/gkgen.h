@@ -1,8 +1,8 @@
 /* gkgen.h — seeded synthetic workload generators (libgkgen.so, host only).
  *
  * The reference ships one sample input (simple_test/delaunay_n11.graph) and
- * no generator; these produce the benchmark's graph families from a seed so
- * the GPU box can rebuild any workload without files:
+ * no generator; these produce the benchmark's graph families from a seed, so
+ * that any workload can be rebuilt without files:
  *   - 2-D Delaunay triangulations of uniform random points (exact integer
  *     predicates on a 2^24 x 2^24 grid, duplicates redrawn);
  *   - road-like graphs: Euclidean MST of uniform points plus the shortest

@@ -106,8 +106,8 @@ typedef struct gk_params {
 
 /* Stage ids of gk_stats.stage_ms / stage_launches / stage_bytes. */
 #define GK_ST_MATCH 0      /* candidate matching                           */
-#define GK_ST_GROUP 1      /* pointer jumping + component labels           */
-#define GK_ST_SORT 2       /* radix sort by (label, stamp, id)             */
+#define GK_ST_GROUP 1      /* grouping (walk to the root pairs) + labels    */
+#define GK_ST_SORT 2       /* order by (label, stamp, id)                  */
 #define GK_ST_CLUSTER 3    /* chunking, coarse ids, coarse vertex weights  */
 #define GK_ST_CONTRACT 4   /* per-row sort + merge (rows <= 64 entries)    */
 #define GK_ST_CONTRACT_BIG 5 /* gather + sort + merge of rows > 64 entries */
