@@ -42,6 +42,7 @@ constexpr int kTop = 256;              // best movable vertices that the short w
 constexpr int kTopMin = 32;            // fewer than this many in its gain classes: the long way
 constexpr int kTopIdBits = 21;         // vertex ids of a job in a sort key of the short way
 constexpr int kGainClasses = 512;
+constexpr int32_t kNoClass = -1;       // too few in the classes that fit: the long way
 
 static_assert(kLoopItems <= 1024 / 2, "the table of first occurrences stays half empty");
 static_assert(kGainClasses <= kBalMax, "the class counts lie in the cover array");
@@ -366,15 +367,14 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
           // lanes that hold a class that fits are the first ones
           const uint64_t m = ballot(code < kGainClasses);
           const int last = m ? 63 - __clzll(static_cast<long long>(m)) : 0;
-          if (lane == last) {
-            L.code = code;
-            L.ntop = cnt >= kTopMin ? 0 : -1;
-          }
+          if (lane == last) L.code = cnt >= kTopMin ? code : kNoClass;
         }
         __syncthreads();
         ntop = 0;
-        if (L.ntop == 0) {
-          const int32_t code = L.code;
+        // decided by a word that nobody writes again before the next round's
+        // barriers: L.ntop counts up below while other waves still arrive here
+        const int32_t code = L.code;
+        if (code != kNoClass) {
           for (int32_t i0 = wave * 64; i0 < npick; i0 += kBalThreads) {
             const int32_t idx = i0 + lane < npick ? pick[i0 + lane] : -1;
             wave_append(idx >= 0 && gain_class(L.lg[idx]) >= code, uint16_t(idx), L.tj, &L.ntop);
