@@ -1321,6 +1321,7 @@ int gk_k_group(gk_ctx* ctx, int32_t n, const int32_t* cand, int32_t* label, int3
   // The walk writes labels and hops while it reads candidates: where those lie
   // in the same place, it works on a copy.
   Buf<int32_t> own;
+  StageGuard drain{ctx, st};  // an early end leaves nothing queued on memory that goes back
   auto apart = [&](const int32_t* x) { return x + n <= cand || cand + n <= x; };
   if (!apart(stamp) || !apart(label)) {
     GK_TRY(own.alloc(ctx->pool, n));
@@ -1338,6 +1339,7 @@ int gk_k_group(gk_ctx* ctx, int32_t n, const int32_t* cand, int32_t* label, int3
     GK_HIP(hipMemcpyAsync(stamp, gr.dist.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
     GK_HIP(hipStreamSynchronize(st));
   }
+  drain.done = true;
   if (sweeps) *sweeps = rounds;
   return GK_OK;
 }
@@ -1358,6 +1360,7 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
   GK_TRY(mvw.alloc(ctx->pool, n));
   const MemberOut out{order, cmap, cptr.p, nullptr, mvw.p};
   int32_t words[gkd::kCtlInts];
+  StageGuard drain{ctx, st};
   GK_TRY(gr.count(ctx, st, n, label));
   gkd::HostWords told;
   bool no_room = false;
@@ -1377,6 +1380,7 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
     GK_TRY(gkd::launch_cvwgt(*nc, nullptr, cptr.p, mvw.p, cvwgt, st));
     GK_HIP(hipStreamSynchronize(st));
   }
+  drain.done = true;
   return GK_OK;
 }
 
@@ -1398,6 +1402,7 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   GK_TRY(m.mrow.alloc(P, n));
   GK_TRY(partial.alloc(P, gkd::size_partials(n)));
   int32_t nc2 = 0;
+  StageGuard drain{ctx, st};
   GK_TRY(gr.count(ctx, st, n, cmap));
   if (n > 0) {
     const gkd::HostWords told = gkrt::host_words(ctx);
@@ -1415,6 +1420,7 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   GK_TRY(contract_stage(ctx, st, g, nc, cmap, m, c, &out));
   if (nc == 0) gkd::fill<int32_t>(cxadj, 0, 1, st);
   GK_HIP(hipStreamSynchronize(st));
+  drain.done = true;
   *cnnz = c.g.nnz;
   return GK_OK;
 }
@@ -1696,6 +1702,7 @@ int gk_k_cut(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* part, int6
   GK_TRY(c.alloc(ctx->pool, 1));
   GK_TRY(p.alloc(ctx->pool, k));
   GK_TRY(cscr.alloc(ctx->pool, gkd::cut_scratch(g.n, k)));
+  StageGuard drain{ctx, st};
   GK_TRY(gkd::launch_cut(g, k, part, c.p, p.p, cscr.p, st));
   void* h = nullptr;
   GK_TRY(ctx->dl.get(st, sizeof(unsigned long long) * (size_t(k) + 2), &h));
@@ -1705,7 +1712,7 @@ int gk_k_cut(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* part, int6
   if (pw) back.add(hc + 2, p.p, sizeof *hc * size_t(k));
   GK_TRY(gkd::launch_copies(back, st));
   GK_HIP(hipStreamSynchronize(st));
-  ctx->dl.drained();
+  drain.done = true;
   *cut = static_cast<int64_t>(*hc);
   if (pw)
     for (int32_t q = 0; q < k; ++q) pw[q] = static_cast<int64_t>(hc[2 + q]);

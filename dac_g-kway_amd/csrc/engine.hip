@@ -947,6 +947,7 @@ int run_packed(gk_ctx* ctx, hipStream_t st, const gk_packed_csr* pk, const gk_pa
       gkrt::clear_launch_options(c);
     }
   } reset{ctx};
+  StageGuard drain{ctx, st};  // an early end leaves nothing queued on the caller's pack or on staging memory
   GK_TRY(gkrt::set_launch_options(ctx, prm[0].flags));
   // Level 0 of every graph is a slice of the caller's pack.
   auto S0 = std::make_shared<Store>();
@@ -1002,6 +1003,7 @@ int run_packed(gk_ctx* ctx, hipStream_t st, const gk_packed_csr* pk, const gk_pa
     GK_TRY(E.step(&worked));
   }
   GK_TRY(E.sync());
+  drain.done = true;
   GK_TRY(ctx->clock.collect(SB));
   for (int i = 0; i < GK_ST_COUNT; ++i) SB.alg_bytes += SB.stage_bytes[i];
   int rc = GK_OK;
