@@ -342,17 +342,29 @@ int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* 
 }
 
 // size[l] = vertices with label l, slot[v] = v's (arbitrary) place among them,
-// for labels that come without a grouping.
+// for labels that come without a grouping and so from a caller: those outside
+// [0, n) are left out and flagged (kCtlFlags, and [1], so that nobody orders
+// the members).
 __global__ void __launch_bounds__(256) k_label_count(int32_t n, const int32_t* __restrict__ label,
-                                                     int32_t* __restrict__ size, int32_t* __restrict__ slot) {
+                                                     int32_t* __restrict__ size, int32_t* __restrict__ slot,
+                                                     int32_t* __restrict__ ctl) {
   const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
-  const bool live = v < n;
-  const int32_t l = live ? label[v] : -1;
-  const uint64_t same = ballot(live && l == __builtin_amdgcn_readfirstlane(l));
-  if (popc64(same) > 4) {  // one atomic for the lanes that share the first lane's label
+  const int32_t l = v < n ? label[v] : -1;
+  const bool live = uint32_t(l) < uint32_t(n);
+  const uint64_t lm = ballot(live);
+  if (ballot(v < n && !live) != 0 && lane_id() == 0) {
+    ctl[1] = 1;
+    ctl[kCtlFlags] = 1;
+  }
+  if (lm == 0) return;
+  // one atomic, by the first live lane, for the lanes that share its label
+  const int first = __ffsll(static_cast<long long>(lm)) - 1;
+  const int32_t lf = __shfl(l, first, 64);
+  const uint64_t same = ballot(live && l == lf);
+  if (popc64(same) > 4) {
     int32_t base = 0;
-    if (lane_id() == 0) base = atomicAdd(&size[l], popc64(same));
-    base = __shfl(base, 0, 64);
+    if (lane_id() == first) base = atomicAdd(&size[lf], popc64(same));
+    base = __shfl(base, first, 64);
     if ((same >> lane_id()) & 1ull) {
       slot[v] = base + popc64(same & lanemask_lt());
       return;
@@ -367,7 +379,7 @@ int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* 
   if (n > 0) zero.add(size, nullptr, sizeof(int32_t) * size_t(n));
   const int rc = launch_copies(zero, st);
   if (rc || n <= 0) return rc;
-  k_label_count<<<grid_for(n, 256), 256, 0, st>>>(n, label, size, slot);
+  k_label_count<<<grid_for(n, 256), 256, 0, st>>>(n, label, size, slot, ctl);
   return hip_status();
 }
 
@@ -515,6 +527,7 @@ __global__ void __launch_bounds__(256) k_member_scatter(int32_t n, const int32_t
   const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
   if (v >= n) return;
   const int32_t l = label[v];
+  if (uint32_t(l) >= uint32_t(n)) return;  // flagged by k_label_count
   const int2 oc = offc[l];
   const int32_t cnt = offc[l + 1].x - oc.x;
   int32_t a = 0, d = 0;
@@ -734,8 +747,8 @@ __global__ void __launch_bounds__(256) k_member_place(int32_t n, const int32_t* 
                                                       int2* __restrict__ mrow) {
   const int64_t v = int64_t(xcd_block()) * 256 + threadIdx.x;
   if (v >= n) return;
-  const int32_t a = xadj[v];
-  mrow[int64_t(offc[label[v]].x) + slot[v]] = make_int2(a, xadj[v + 1] - a);
+  const int32_t a = xadj[v], l = label[v];
+  if (uint32_t(l) < uint32_t(n)) mrow[int64_t(offc[l].x) + slot[v]] = make_int2(a, xadj[v + 1] - a);
   // index v as a label: the first place of its group, if it has members
   const int2 o = offc[v];
   if (offc[v + 1].x > o.x) cptr[o.y] = o.x;

@@ -148,7 +148,8 @@ int Groups::jump(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* cand, in
   return GK_OK;
 }
 
-// Labels in [0, n) that come without a grouping: member counts only.
+// Labels that come without a grouping: member counts only.  The control word
+// kCtlFlags tells of labels outside [0, n).
 int Groups::count(gk_ctx* ctx, hipStream_t st, int32_t n, const int32_t* label) {
   Pool& P = ctx->pool;
   GK_TRY(ctl.alloc(P, gkd::kCtlInts + gkd::kRowCtlInts));
@@ -1368,6 +1369,7 @@ int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* st
   if (!no_room) GK_TRY(gkd::launch_cvwgt(n, gr.ctl.p, cptr.p, mvw.p, cvwgt, st));
   GK_HIP(hipStreamSynchronize(st));
   GK_TRY(gkrt::wait_words(ctx, st, told, gkd::kCtlInts, words));
+  if (words[gkd::kCtlFlags]) { gkh::set_error("label outside [0, n)"); return GK_ERR_ARG; }
   *nc = words[0];
   if (words[1] || no_room) {
     gr.counts_done();
@@ -1401,19 +1403,19 @@ int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc
   GK_TRY(m.cptr.alloc(P, int64_t(n) + 1));
   GK_TRY(m.mrow.alloc(P, n));
   GK_TRY(partial.alloc(P, gkd::size_partials(n)));
-  int32_t nc2 = 0;
+  int32_t words[gkd::kCtlFlags + 1] = {};  // coarse vertices counted, flags
   StageGuard drain{ctx, st};
   GK_TRY(gr.count(ctx, st, n, cmap));
   if (n > 0) {
     const gkd::HostWords told = gkrt::host_words(ctx);
     GK_TRY(gkd::launch_size_scan(n, gr.size.p, INT32_MAX, partial.p, gr.comp.p, gr.ctl.p, told, st));
     GK_TRY(gkd::launch_member_place(n, cmap, gr.slot.p, gr.comp.p, dg->xadj, gr.ctl.p, m.cptr.p, m.mrow.p, st));
-    GK_TRY(gkrt::wait_words(ctx, st, told, 1, &nc2));
+    GK_TRY(gkrt::wait_words(ctx, st, told, gkd::kCtlFlags + 1, words));
   }
   m.ctl = std::move(gr.ctl);
   // With G = INT32_MAX every label is one chunk, so chunks are the coarse
   // vertices in id order exactly when cmap is onto [0, nc).
-  if (nc2 != nc) { gkh::set_error("cmap is not onto [0, nc)"); return GK_ERR_ARG; }
+  if (words[0] != nc || words[gkd::kCtlFlags]) { gkh::set_error("cmap is not onto [0, nc)"); return GK_ERR_ARG; }
   Level c;
   DGraph g = dview(dg);
   const CsrOut out{cxadj, cadjncy, cadjwgt};

@@ -119,8 +119,8 @@ int launch_comp_count(int32_t n, const int32_t* cand, const int32_t* next, int2*
 // where l is no label).  key may be label.
 int launch_label_size(int32_t n, const int32_t* key, const int2* comp, int32_t* label, int32_t* size,
                       hipStream_t st);
-// size and slot of labels in [0, n) that come without a grouping; ctl as in
-// launch_walk.
+// size and slot of labels that come without a grouping; ctl as in launch_walk,
+// with [1] and [kCtlFlags] set when some label is outside [0, n).
 int launch_label_count(int32_t n, const int32_t* label, int32_t* size, int32_t* slot, int32_t* ctl, hipStream_t st);
 // offc[l] = (first place, first coarse id) of label l's group; coarse ids and
 // flags to ctl and, kCtlInts words, to host.  partial: size_partials(n),

@@ -326,12 +326,14 @@ int gk_k_match(gk_ctx* ctx, const gk_csr* dg, int32_t* cand, void* stream);
 int gk_k_group(gk_ctx* ctx, int32_t n, const int32_t* cand, int32_t* label,
                int32_t* stamp, int32_t* sweeps, void* stream);
 /* order: vertices sorted by (label, stamp, id); cmap: coarse id per vertex;
- * cvwgt: coarse vertex weights; returns nc in *nc. */
+ * cvwgt: coarse vertex weights; returns nc in *nc.  Labels are vertex ids, in
+ * [0, n); GK_ERR_ARG otherwise. */
 int gk_k_cluster(gk_ctx* ctx, int32_t n, const int32_t* label, const int32_t* stamp,
                  const int32_t* vwgt, int32_t max_group, int32_t* order, int32_t* cmap,
                  int32_t* cvwgt, int32_t* nc, void* stream);
 /* Coarse CSR of the contraction; cxadj needs nc+1 entries, cadjncy/cadjwgt
- * need dg->nnz entries (upper bound); *cnnz receives the coarse entry count. */
+ * need dg->nnz entries (upper bound); *cnnz receives the coarse entry count.
+ * GK_ERR_ARG unless cmap is onto [0, nc). */
 int gk_k_contract(gk_ctx* ctx, const gk_csr* dg, const int32_t* cmap, int32_t nc,
                   int32_t* cxadj, int32_t* cadjncy, int32_t* cadjwgt, int32_t* cnnz,
                   void* stream);
