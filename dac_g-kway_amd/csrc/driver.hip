@@ -1587,7 +1587,10 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   GK_TRY(upd.alloc(P, n));
   GK_TRY(wl.alloc(P, n));
   GK_TRY(heavy.alloc(P, n));
-  GK_TRY(hist.alloc(P, 2 * int64_t(nrounds)));
+  // The round loop orders all of a round's moves when a caller wants to see
+  // them, and else only as many as decide the round.
+  const bool want_hist = nmoves || pos;
+  if (want_hist) GK_TRY(hist.alloc(P, 2 * int64_t(nrounds)));
   GK_TRY(list.alloc(P, n));
   GK_TRY(xlist.alloc(P, n));
   GK_TRY(hkey.alloc(P, n));
@@ -1598,7 +1601,7 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   GK_TRY(selbits.alloc(P, nwords + 1));
   GK_TRY(defbits.alloc(P, nwords + 1));
   GK_TRY(movers.alloc(P, int64_t(M) + 1));
-  GK_TRY(dorder.alloc(P, int64_t(M) + 2));
+  if (order) GK_TRY(dorder.alloc(P, int64_t(M) + 2));
   GK_TRY(dmax.alloc(P, 1));
   // The words of the one job's state, which go up and come back as one block.
   struct State {
@@ -1669,7 +1672,7 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   GK_TRY(refine_rounds(ctx, st, rs, nrounds, true, false, nullptr));
   // Rounds that ordered no move came after those that did (an unchanged state
   // stays so): no moves, position -1.
-  const size_t hist_bytes = sizeof(int32_t) * 2 * size_t(nrounds);
+  const size_t hist_bytes = want_hist ? sizeof(int32_t) * 2 * size_t(nrounds) : 0;
   void* hend = nullptr;
   GK_TRY(ctx->dl.get(st, sizeof(State) + hist_bytes, &hend));
   const State* he = static_cast<const State*>(hend);
@@ -1685,8 +1688,11 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
     if (nmoves) nmoves[r] = r < made ? hh[2 * r] : 0;
     if (pos) pos[r] = r < made ? hh[2 * r + 1] : -1;
   }
-  if (order && made > 0)
-    GK_HIP(hipMemcpyAsync(order, dorder.p + 2, sizeof(int32_t) * size_t(hh[2 * made - 2]), hipMemcpyDeviceToDevice, st));
+  if (order && made > 0) {
+    int32_t ordered = 0;
+    GK_TRY(fetch(ctx, st, {{&ordered, dorder.p, sizeof ordered}}));
+    GK_HIP(hipMemcpyAsync(order, dorder.p + 2, sizeof(int32_t) * size_t(ordered), hipMemcpyDeviceToDevice, st));
+  }
   GK_HIP(hipStreamSynchronize(st));
   *gain_sum = -he->cut;
   if (paths)

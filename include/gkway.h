@@ -361,8 +361,8 @@ int gk_k_balance(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* moves,
 int gk_k_apply(gk_ctx* ctx, const gk_csr* dg, const int32_t* moves, int32_t pos,
                const int32_t* gain, const int32_t* dest, int32_t* part, int32_t* updated,
                int64_t* gain_sum, void* stream);
-/* nrounds refinement rounds exactly as the V-cycle runs them, with the
- * product's round kernels: per round the movable set and its independent
+/* nrounds refinement rounds with the product's round kernels: per round the
+ * movable set and its independent
  * selection, the best min(selected, max_moves) moves by (gain desc, id asc)
  * (all of them, or a top-max_moves radix select), the largest balanced
  * prefix, the apply, then the gain pass over the updated vertices.  The state
@@ -374,7 +374,10 @@ int gk_k_apply(gk_ctx* ctx, const gk_csr* dg, const int32_t* moves, int32_t pos,
  * none was selected), pos[r] = last applied position (-1: none).
  * *gain_sum = summed gain of every applied move.  order (device, may be
  * NULL): max_moves ints, the ordered moves of the last round that selected
- * any.  paths (host, may be NULL): as gk_stats.round_paths over these rounds. */
+ * any.  paths (host, may be NULL): as gk_stats.round_paths over these rounds.
+ * The state after the rounds is that of the V-cycle's in any case.  With
+ * nmoves, pos and order all NULL the rounds are also decided as there, many by
+ * their best moves alone; with any of them every round orders all its moves. */
 int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t max_moves, int32_t nrounds,
                int32_t* part, int32_t* bnd, int32_t* gain, int32_t* dest, int32_t* pw, int32_t* nmoves,
                int32_t* pos, int64_t* gain_sum, int32_t* order, int64_t* paths, void* stream);
