@@ -58,32 +58,41 @@ def check(gk, oracle, ctx, g, k, M, R, gbits, slack, flip, seed=5):
         now = tuple(exp[name] for name in STATE)
 
 
+# The list of the round loop holds 3584 candidates: graphs of fewer vertices, or
+# compact blocks of a mesh numbered along a curve, whose borders are short.
 @pytest.mark.parametrize("slack", [1, 4, 30, 1000, None])
-@pytest.mark.parametrize("flip", [0.0005, 0.004, 0.02])
 @pytest.mark.parametrize("gbits", [1, 4, 14])
-def test_caps_and_gains(gk, oracle, ctx, slack, flip, gbits):
-    check(gk, oracle, ctx, gk.dag(20000, 60, 3), 32, 1024, 40, gbits, slack, flip)
+@pytest.mark.parametrize("name", ["dag", "mesh"])
+def test_caps_and_gains(gk, oracle, ctx, name, slack, gbits):
+    g = gk.dag(3500, 30, 3) if name == "dag" else gk.delaunay_hilbert(30000, 3)
+    check(gk, oracle, ctx, g, 16, 1024, 40, gbits, slack, 0.002)
 
 
 @pytest.mark.parametrize("M", [1, 4, 63, 64, 65, 128, 256])
 @pytest.mark.parametrize("slack", [3, 500])
 def test_move_caps(gk, oracle, ctx, M, slack):
-    check(gk, oracle, ctx, gk.delaunay(12000, 6), 16, M, 40, 10, slack, 0.003)
+    check(gk, oracle, ctx, gk.delaunay_hilbert(12000, 6), 8, M, 40, 10, slack, 0.003)
 
 
-@pytest.mark.parametrize("n,k", [(65535, 2), (65537, 256), (200000, 64)])
-def test_sizes(gk, oracle, ctx, n, k):
-    check(gk, oracle, ctx, gk.delaunay(n, 9), k, 1024, 20, 12, 6, 0.001)
+@pytest.mark.parametrize("n,k,flip", [(65535, 2, 0.004), (65536, 8, 0.0005), (65537, 8, 0.0005), (200000, 4, 0.0002)])
+def test_sizes(gk, oracle, ctx, n, k, flip):
+    check(gk, oracle, ctx, gk.delaunay_hilbert(n, 9), k, 1024, 20, 12, 6, flip)
+
+
+# from a handful of movable vertices to beyond the 256 that it looks at
+@pytest.mark.parametrize("n,k", [(300, 2), (700, 4), (1500, 4), (2500, 256), (3400, 100)])
+def test_few(gk, oracle, ctx, n, k):
+    check(gk, oracle, ctx, gk.dag(n, 20, 9), k, 1024, 30, 8, 4, 0.01)
 
 
 @pytest.mark.parametrize("fan,k", [(40, 8), (300, 16)])
 def test_hubs(gk, oracle, ctx, fan, k):
-    check(gk, oracle, ctx, hub_graph(gk, n=6000, hubs=30, fan=fan, seed=fan), k, 1024, 20, 9, 5, 0.01)
+    check(gk, oracle, ctx, hub_graph(gk, n=3000, hubs=20, fan=fan, seed=fan), k, 1024, 20, 9, 5, 0.01)
 
 
 def test_same_as_seen(gk, ctx):
     """Asked for or not, the rounds leave the same state."""
-    g, k, M, R = gk.dag(30000, 80, 4), 48, 200, 25
+    g, k, M, R = gk.delaunay_hilbert(30000, 4), 12, 200, 25
     start = state(gk, g, k, seed=8, gain_bits=11, flip=0.004)
     cap = int(start[4].max()) + 10
     seen = gpu_rounds(gk, ctx, g, k, cap, M, R, *start)
