@@ -59,7 +59,7 @@ struct LoopLds {
   uint16_t ti[kTop], tj[kTop];                   // the best selected; the best movable, not yet tested
   int32_t wv[kLoopItems], ws[kLoopItems], wd[kLoopItems], ww[kLoopItems];  // worklist: vertex, row, weight
   long long cut;
-  int32_t n, nmov, nsel, ntop, nts, nshort, nlong, tot, thr, pos, code, hmin, hmax;
+  int32_t n, nmov, nsel, ntop, nts, nshort, nlong, tot, thr, pos, code;
 };
 
 // Selected candidates by list index.
@@ -502,33 +502,6 @@ __global__ void __launch_bounds__(kBalThreads) k_rounds(const RoundsArgs a) {
         }
         __syncthreads();
         pos = L.pos;
-        if (pos >= 0 && a.paths && count > a.M && tested_all) {
-          // what order_moves would have said of the round: more than M
-          // selected, and whether their compressed keys fit 32 bits
-          if (t == 0) {
-            L.hmin = INT32_MAX;
-            L.hmax = 0;
-          }
-          __syncthreads();
-          int32_t lo = INT32_MAX, hi = 0;
-          for (int32_t i = t; i < count; i += kBalThreads) {
-            const int32_t g = L.lg[L.si[i]];
-            lo = g < lo ? g : lo;
-            hi = g > hi ? g : hi;
-          }
-          lo = -wave_max(-lo);
-          hi = wave_max(hi);
-          if (lane == 0) {
-            atomicMin(&L.hmin, lo);
-            atomicMax(&L.hmax, hi);
-          }
-          __syncthreads();
-          if (t == 0) {
-            a.paths[3 * int64_t(j)] += 1;
-            if (bits_of(uint32_t(L.hmax - L.hmin)) + bits_of(uint32_t(ve - vb - 1)) > 32)
-              a.paths[3 * int64_t(j) + 1] += 1;
-          }
-        }
       }
     }
     if (!tested_all) count = nmov;  // some are selected: the movable vertex of smallest id is

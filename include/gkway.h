@@ -160,10 +160,12 @@ typedef struct gk_stats {
   double stage_ms[GK_ST_COUNT];
   int32_t stage_launches[GK_ST_COUNT];
   int64_t stage_bytes[GK_ST_COUNT];
-  /* Refinement rounds by the ordering path they took (all levels): [0] more
-   * than max_moves selected (exact top-max_moves radix select), [1] of those,
-   * compressed keys wider than 32 bits (64-bit key sort), [2] rounds that
-   * tested vertices deferred by the previous round's gain threshold. */
+  /* Refinement rounds by the ordering path they took (all levels): [0] rounds
+   * with more than max_moves selected, ordered by the exact top-max_moves
+   * radix select (rounds that their best few moves decide order no others and
+   * are not counted), [1] of those, compressed keys wider than 32 bits (64-bit
+   * key sort), [2] rounds that tested vertices deferred by the previous
+   * round's gain threshold. */
   int64_t round_paths[3];
 } gk_stats;
 

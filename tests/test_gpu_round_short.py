@@ -100,3 +100,21 @@ def test_same_as_seen(gk, ctx):
     assert got["gain_sum"] == seen["gain_sum"]
     for name in STATE:
         assert np.array_equal(got[name], seen[name]), name
+
+
+@pytest.mark.parametrize("M,slack", [(64, 30), (60, 1000), (45, 30)])
+def test_paths_count_what_ran(gk, ctx, M, slack):
+    """More than M vertices are selected in most rounds: asked for, their moves
+    are ordered by the radix select every time; decided by the best ones alone,
+    the rounds are not among those that the select ordered."""
+    g, k, R = gk.delaunay_hilbert(30000, 3), 16, 60
+    start = state(gk, g, k, seed=5, gain_bits=4, flip=0.002)
+    cap = int(start[4].max()) + slack
+    seen = gpu_rounds(gk, ctx, g, k, cap, M, R, *start)
+    got = unseen_rounds(gk, ctx, g, k, cap, M, 1, R, start)[0]
+    print(f"M={M} nmoves={seen['nmoves']} pos={seen['pos']} paths: seen {seen['paths']} unseen {got['paths']}", flush=True)
+    for name in STATE:
+        assert np.array_equal(got[name], seen[name]), name
+    assert sum(m == M for m in seen["nmoves"]) >= seen["paths"][0] > 0
+    assert got["paths"][0] < seen["paths"][0]
+    assert got["paths"][1] <= got["paths"][0]
