@@ -27,6 +27,7 @@
 #include "batch.hpp"
 #include "kernels.hpp"
 #include "prim.hpp"
+#include "round_plan.hpp"
 #include "runtime.hpp"
 
 
@@ -527,25 +528,11 @@ int loop_gains(gk_ctx* ctx, hipStream_t st, const RoundState& s, int pair) {
 
 }  // namespace
 
-// Two ways to run rounds, which leave the same state.  The round loop (one
-// workgroup per job, k <= kGainInlineK) is the faster one while a job has up
-// to some thousand candidates; the separate kernels select over the whole
-// device, and start on graphs so large that their first rounds will have more.
-// The host looks at the end of a round loop's launch, and every 4 rounds of
-// the separate kernels (every 8, 16, then 32 once they ran 32: a look costs a
-// copy and a synchronisation; a round with nothing selected changes nothing).
 int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_rounds, bool exact, bool graph, int* ran) {
-  constexpr int kWideRounds = 4;
-  constexpr int kLoopRounds = 64;
-  constexpr int64_t kLoopVertices = int64_t(1) << 20;  // per job, to begin with the loop
-  constexpr int32_t kLoopSelected = 1024;              // selected per round, to come back to it
-  const bool can_loop = s.kmax <= gkd::kGainInlineK;
-  bool loop = can_loop && int64_t(s.g.n) <= kLoopVertices * s.nj;
   graph = graph && !exact && !ctx->clock.timed(GK_ST_SELECT) && !ctx->clock.timed(GK_ST_BALANCE) &&
           !ctx->clock.timed(GK_ST_GAIN) && !ctx->clock.timed(GK_ST_GAIN_HEAVY);
+  RoundPlan plan(s.kmax <= gkd::kGainInlineK, s.g.n, s.nj, max_rounds, exact, graph);
   RoundGraph wide_graph, loop_graph;
-  int pair = 1;  // the compaction before the rounds used pair 0
-  int done = 0, wide_done = 0, per_check = kWideRounds;
   // Jobs that go on, jobs left out, and with one job the ordering rounds so
   // far; one job's kernel writes them to pinned memory itself.
   const bool one = s.nj == 1;
@@ -556,82 +543,54 @@ int refine_rounds(gk_ctx* ctx, hipStream_t st, const RoundState& s, int max_roun
     return wait_words(ctx, st, t2, 2, words);
   };
   auto listen = [&]() { return one ? host_words(ctx) : gkd::HostWords{}; };
-  // A step of a batch: new requests wait for its end.  A launch of the loop that
-  // leaves a job out gives its rounds back, so max_rounds alone does not bound
-  // the rounds by the separate kernels; they get a quarter of it, and the loop
-  // is tried again only while each attempt leaves out at most half as many jobs
-  // as the last.  Poisson arrivals at 200 a second, 500 graphs of up to 2 M
-  // vertices, 20 s: without the bound 3000 such rounds and 100 attempts in a step
-  // of 350 ms, half of the requests later than 3.4-3.6 s; with it 46-47 ms.
-  const bool step = max_rounds > 0 && !exact;
-  const int wide_most = std::max(kWideRounds, max_rounds / 4);
-  int left_out = INT32_MAX;
-  bool may_return = can_loop;
-  while (max_rounds <= 0 || done < max_rounds) {
-    if (loop) {
-      const int left = max_rounds > 0 ? max_rounds - done : kLoopRounds;
+  while (!plan.ended()) {
+    const int rounds = plan.rounds();
+    if (plan.loop()) {
+      const int pair = plan.pair();
       int32_t words[3] = {0, 0, 0};
-      if (graph && left >= kLoopRounds) {
-        // both pairs, so that every replay begins with the same one
+      if (plan.captured()) {
         if (!loop_graph.ready())
           GK_TRY(loop_graph.capture(ctx, st, [&]() -> int {
-            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, pair, gkd::HostWords{}));
+            GK_TRY(loop_rounds(ctx, st, s, rounds / 2, pair, gkd::HostWords{}));
             GK_TRY(loop_gains(ctx, st, s, pair));
-            GK_TRY(loop_rounds(ctx, st, s, kLoopRounds / 2, 1 - pair, gkd::HostWords{}));
+            GK_TRY(loop_rounds(ctx, st, s, rounds / 2, 1 - pair, gkd::HostWords{}));
             return loop_gains(ctx, st, s, 1 - pair);
           }));
         GK_TRY(loop_graph.replay(ctx, st));
         const gkd::HostWords told = host_words(ctx);
         GK_TRY(gkd::launch_tell(s.status + 2 * (1 - pair), 2, told, st));
         GK_TRY(wait_words(ctx, st, told, 2, words));
-        done += kLoopRounds;
       } else {
-        const int rounds = std::min(left, kLoopRounds);
         const gkd::HostWords told = listen();
         GK_TRY(loop_rounds(ctx, st, s, rounds, pair, told));
         // Of several jobs some usually go on, and the wait is the longer part.
         if (!one) GK_TRY(loop_gains(ctx, st, s, pair));
         GK_TRY(status(pair, told, words));
         if (one && words[0] != 0) GK_TRY(loop_gains(ctx, st, s, pair));
-        done = exact ? words[2] : done + rounds;  // exact: one job
-        pair = 1 - pair;
       }
-      if (words[0] == 0) break;
-      if (words[1] != 0) {
-        loop = false;
-        if (!exact) done -= std::min(done, kLoopRounds);  // jobs left out did none
-        if (step && words[1] > left_out / 2) may_return = false;
-        left_out = words[1];
-      }
+      plan.loop_ran(words[0], words[1], words[2]);
     } else {
-      const int left = max_rounds > 0 ? max_rounds - done : per_check;
-      const int rounds = std::min(left, per_check);
-      if (graph && rounds % kWideRounds == 0) {
+      if (plan.captured()) {
         if (!wide_graph.ready())
           GK_TRY(wide_graph.capture(ctx, st, [&]() -> int {
-            for (int r = 0; r < kWideRounds; ++r) GK_TRY(wide_round(ctx, st, s));
+            for (int r = 0; r < RoundPlan::kWideRounds; ++r) GK_TRY(wide_round(ctx, st, s));
             return GK_OK;
           }));
-        for (int r = 0; r < rounds; r += kWideRounds) GK_TRY(wide_graph.replay(ctx, st));
+        for (int r = 0; r < rounds; r += RoundPlan::kWideRounds) GK_TRY(wide_graph.replay(ctx, st));
       } else {
         for (int r = 0; r < rounds; ++r) GK_TRY(wide_round(ctx, st, s));
       }
-      done += rounds;
-      wide_done += rounds;
       int32_t live = 0;
       const gkd::HostWords told = host_words(ctx);
       GK_TRY(gkd::launch_tell(s.active, 1, told, st));
       GK_TRY(wait_words(ctx, st, told, 1, &live));
-      if (live == 0 || (step && wide_done >= wide_most)) break;
-      if (may_return && live <= kLoopSelected * s.nj) {
-        loop = true;
+      if (plan.wide_ran(live)) {
         gkd::fill<int32_t>(s.hcnt, 0, 4, st);
         gkd::fill<int32_t>(s.status, 0, 4, st);
       }
-      if (wide_done >= 32 && per_check < 32) per_check *= 2;
     }
   }
-  if (ran) *ran = done;
+  if (ran) *ran = plan.done();
   return GK_OK;
 }
 

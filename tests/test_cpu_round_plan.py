@@ -1,0 +1,102 @@
+"""The bookkeeping of a level's refinement rounds (csrc/round_plan.hpp), compiled
+for the host and driven through made-up answers of the device: which launches
+follow, how many rounds are accounted for, and what bounds them."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "dac_g-kway_amd", "csrc")
+SHIM = r"""
+#include "round_plan.hpp"
+using P = gkrt::RoundPlan;
+extern "C" {
+P* make(int can_loop, long long n, int nj, int max_rounds, int exact, int graph) {
+  return new P(can_loop, n, nj, max_rounds, exact, graph);
+}
+void drop(P* p) { delete p; }
+int ended(P* p) { return p->ended(); }
+int loop(P* p) { return p->loop(); }
+int rounds(P* p) { return p->rounds(); }
+int captured(P* p) { return p->captured(); }
+int pair_of(P* p) { return p->pair(); }
+int done(P* p) { return p->done(); }
+void loop_ran(P* p, int live, int left_out, int ordered) { p->loop_ran(live, left_out, ordered); }
+int wide_ran(P* p, int live) { return p->wide_ran(live); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    d = tmp_path_factory.mktemp("round_plan")
+    (d / "shim.cpp").write_text(SHIM)
+    so = d / "shim.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-I", CSRC, str(d / "shim.cpp"), "-o", str(so)],
+                   check=True, timeout=120)
+    L = ctypes.CDLL(str(so))
+    L.make.restype = ctypes.c_void_p
+    L.make.argtypes = [ctypes.c_int, ctypes.c_longlong] + [ctypes.c_int] * 4
+    for f in ("ended", "loop", "rounds", "captured", "pair_of", "done", "drop"):
+        getattr(L, f).argtypes = [ctypes.c_void_p]
+    L.loop_ran.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 3
+    L.wide_ran.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    return L
+
+
+class Plan:
+    def __init__(self, shim, can_loop=True, n=100000, nj=1, max_rounds=0, exact=False, graph=False):
+        self.L, self.p = shim, shim.make(can_loop, n, nj, max_rounds, exact, graph)
+
+    def __del__(self):
+        self.L.drop(self.p)
+
+    def __getattr__(self, name):
+        return getattr(self.L, {"pair": "pair_of"}.get(name, name))(self.p)
+
+    def loop_ran(self, live, left_out, ordered=0):
+        self.L.loop_ran(self.p, live, left_out, ordered)
+
+    def wide_ran(self, live):
+        return self.L.wide_ran(self.p, live)
+
+
+def test_rounds_given_back_are_those_of_the_launch(shim):
+    """A launch that leaves a job out gives back its own rounds, not those that
+    the separate kernels have run before it."""
+    p = Plan(shim, nj=3, max_rounds=64)
+    assert p.loop and p.rounds == 64
+    p.loop_ran(3, 3)
+    assert not p.loop and p.done == 0 and p.rounds == 4
+    assert p.wide_ran(900) == 1
+    assert p.loop and p.done == 4 and p.rounds == 60
+    p.loop_ran(2, 1)
+    assert not p.loop and p.done == 4
+    assert p.wide_ran(100000) == 0
+    assert p.done == 8
+
+
+@pytest.mark.parametrize("seed", range(60))
+def test_every_round_is_accounted_for_once(shim, seed):
+    rng = random.Random(seed)
+    nj = rng.choice([1, 2, 9, 300])
+    p = Plan(shim, can_loop=rng.random() < 0.9, n=rng.choice([1000, 3_000_000]), nj=nj,
+             max_rounds=rng.choice([1, 3, 64, 100, 128, 256]), graph=rng.random() < 0.5)
+    told = 0
+    for _ in range(10000):
+        if p.ended:
+            break
+        n = p.rounds
+        assert n > 0
+        if p.loop:
+            left_out = rng.choice([0, 0, 1, nj])
+            live = max(left_out, rng.choice([0, 1, nj]))
+            told += n if live == 0 or left_out == 0 else 0
+            p.loop_ran(live, left_out)
+        else:
+            told += n
+            p.wide_ran(rng.choice([0, 500, 5000, 5000, 10**6]))
+        assert p.done == told
+    assert p.ended
