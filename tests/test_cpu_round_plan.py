@@ -100,3 +100,30 @@ def test_every_round_is_accounted_for_once(shim, seed):
             p.wide_ran(rng.choice([0, 500, 5000, 5000, 10**6]))
         assert p.done == told
     assert p.ended
+
+
+# A step of a batch ends soon whatever its jobs do: at most a quarter of its
+# rounds by the separate kernels (to the next look), and so many launches of the
+# loop that leave jobs out as that number can be halved.  The answers are those
+# that once kept a step going for 3000 rounds: selections small enough to go
+# back to the loop, which leaves out the same jobs again.
+@pytest.mark.parametrize("max_rounds", [4, 16, 64, 128, 256])
+@pytest.mark.parametrize("nj", [1, 5, 64, 500])
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("left", ["same", "one", "halves", "random"])
+def test_a_step_is_bounded(shim, max_rounds, nj, graph, left):
+    rng = random.Random(nj)
+    p = Plan(shim, nj=nj, max_rounds=max_rounds, graph=graph)
+    wide = attempts = 0
+    out = nj
+    while not p.ended and wide + attempts < 10000:
+        if p.loop:
+            attempts += 1
+            p.loop_ran(nj, out)
+            out = {"same": out, "one": 1, "halves": max(1, out // 2), "random": rng.randint(1, nj)}[left]
+        else:
+            wide += p.rounds
+            p.wide_ran(rng.randint(1, 1024 * nj))
+    assert p.ended
+    assert wide < max(4, max_rounds // 4) + 32
+    assert attempts <= 2 + nj.bit_length()
