@@ -36,8 +36,12 @@ class RoundPlan {
   // Whether they are replayed from a graph: two launches of half the loop's
   // rounds each, so that every replay begins with the same pair of counts; or
   // kWideRounds rounds of the separate kernels at a time.
-  bool captured() const { return graph_ && (loop_ ? rounds() == kLoopRounds : rounds() % kWideRounds == 0); }
-  // The pair of counts and status words that the next launch of the loop uses.
+  bool captured() const {
+    return graph_ && (loop_ ? rounds() == kLoopRounds && pair_ == kFirstPair : rounds() % kWideRounds == 0);
+  }
+  // The pair of counts and status words that the next launch of the loop uses,
+  // zero before it; the launch clears the other pair for the next one.  A graph
+  // holds the pair it was captured with, so only the first pair is captured.
   int pair() const { return pair_; }
   int done() const { return done_; }
 
@@ -66,7 +70,10 @@ class RoundPlan {
       ended_ = true;
       return false;
     }
-    if (may_return_ && live <= kLoopSelected * jobs_) loop_ = true;
+    if (may_return_ && live <= kLoopSelected * jobs_) {
+      loop_ = true;
+      pair_ = kFirstPair;  // both are cleared
+    }
     if (wide_done_ >= 32 && per_check_ < 32) per_check_ *= 2;
     return loop_;
   }
@@ -74,6 +81,7 @@ class RoundPlan {
  private:
   static constexpr int64_t kLoopVertices = int64_t(1) << 20;  // per job, to begin with the loop
   static constexpr int32_t kLoopSelected = 1024;              // selected per round, to come back to it
+  static constexpr int kFirstPair = 1;                        // the compaction before the rounds uses pair 0
   const int max_;
   const bool exact_, graph_;
   // A step of a batch: new requests wait for its end.  Launches of the loop
@@ -90,7 +98,7 @@ class RoundPlan {
   bool may_return_;  // from the separate kernels to the loop
   bool loop_;
   bool ended_ = false;
-  int pair_ = 1;  // the compaction before the rounds used pair 0
+  int pair_ = kFirstPair;
   int done_ = 0, wide_done_ = 0, per_check_ = kWideRounds;
   int32_t left_out_ = INT32_MAX;  // by the loop's last launch that left any
 };

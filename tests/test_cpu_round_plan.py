@@ -127,3 +127,40 @@ def test_a_step_is_bounded(shim, max_rounds, nj, graph, left):
     assert p.ended
     assert wide < max(4, max_rounds // 4) + 32
     assert attempts <= 2 + nj.bit_length()
+
+
+@pytest.mark.parametrize("seed", range(60))
+def test_launches_find_their_words_cleared(shim, seed):
+    """Pairs of counts and status words: a launch of the loop raises its own
+    pair, which must be zero, and clears the other; a replay is two launches
+    that begin with the pair they were captured with; the separate kernels raise
+    pair 0, and both pairs are cleared on the way back to the loop."""
+    rng = random.Random(seed)
+    nj = rng.choice([1, 4, 100])
+    exact = nj == 1 and rng.random() < 0.3
+    p = Plan(shim, n=rng.choice([1000, 3_000_000]), nj=nj, max_rounds=0 if rng.random() < 0.3 else rng.randint(1, 256),
+             exact=exact, graph=not exact and rng.random() < 0.7)
+    zero, held, ordered = [False, True], None, 0
+
+    def launch(pair):
+        assert zero[pair]
+        zero[pair], zero[1 - pair] = False, True
+
+    for _ in range(300):
+        if p.ended:
+            break
+        if p.loop:
+            if p.captured:
+                held = p.pair if held is None else held
+                launch(held)
+                launch(1 - held)
+            else:
+                launch(p.pair)
+            ordered += rng.randint(1, p.rounds)
+            live = rng.choice([0, nj, nj, nj])
+            p.loop_ran(live, rng.choice([0, 0, 1]) if live else 0, ordered)
+        else:
+            zero[0] = False
+            ordered += p.rounds
+            if p.wide_ran(rng.choice([1, 900, 10**6])):
+                zero = [True, True]
