@@ -611,6 +611,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   std::memset(&S, 0, sizeof S);
   ctx->cur = &S;
   ctx->clock.start((prm.flags & GK_FLAG_STAGE_TIME) != 0, st);
+  HostBlock top_down, part_up;
   StageGuard stage_guard{ctx, st};
   struct Reset {
     gk_ctx* c;
@@ -695,13 +696,12 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     GK_TRY(dmaxall.alloc(P, nl));
     for (int32_t l = 0; l + 1 < nl; ++l) GK_TRY(gkd::launch_max_deg(L[l].g, dmaxall.p + l, st));
   }
-  // The coarsest graph comes back through the context's pinned staging in one
+  // The coarsest graph comes back into the context's pinned staging in one
   // launch, which writes there, and is partitioned from there.
   const int64_t tn = top.g.nnz;
   auto up4 = [](size_t ints) { return (ints + 3) & ~size_t(3); };  // 16-byte places
-  void* hdn = nullptr;
-  GK_TRY(ctx->dl.get(st, sizeof(int32_t) * (4 + up4(nl) + up4(size_t(nt) + 1) + 2 * up4(tn) + up4(nt)), &hdn));
-  unsigned long long* ht = static_cast<unsigned long long*>(hdn);
+  GK_TRY(top_down.get(ctx->dl, st, sizeof(int32_t) * (4 + up4(nl) + up4(size_t(nt) + 1) + 2 * up4(tn) + up4(nt))));
+  unsigned long long* ht = static_cast<unsigned long long*>(top_down.p());
   int32_t* hmaxdeg = reinterpret_cast<int32_t*>(ht + 2);
   int32_t* hx = hmaxdeg + up4(nl);
   int32_t* ha = hx + up4(size_t(nt) + 1);
@@ -709,12 +709,15 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   int32_t* hv = hw + up4(tn);
   std::memset(hmaxdeg, 0, sizeof(int32_t) * size_t(nl));
   gkd::Copies dn;
-  dn.add(ht, tw.p, sizeof *ht);
-  if (heavy_k) dn.add(hmaxdeg, dmaxall.p, sizeof(int32_t) * size_t(nl - 1));
-  dn.add(hx, top.g.xadj, sizeof(int32_t) * (size_t(nt) + 1));
-  dn.add(ha, top.g.adj, sizeof(int32_t) * size_t(tn));
-  dn.add(hw, top.g.w, sizeof(int32_t) * size_t(tn));
-  dn.add(hv, top.g.vw, sizeof(int32_t) * size_t(nt));
+  auto down = [&](void* dst, const void* src, size_t words) -> int {
+    return top_down.copy(dn, st, dst, src, sizeof(int32_t) * words, hipMemcpyDeviceToHost);
+  };
+  GK_TRY(down(ht, tw.p, 2));
+  if (heavy_k) GK_TRY(down(hmaxdeg, dmaxall.p, size_t(nl - 1)));
+  GK_TRY(down(hx, top.g.xadj, size_t(nt) + 1));
+  GK_TRY(down(ha, top.g.adj, size_t(tn)));
+  GK_TRY(down(hw, top.g.w, size_t(tn)));
+  GK_TRY(down(hv, top.g.vw, size_t(nt)));
   GK_TRY(gkd::launch_copies(dn, st));
   GK_HIP(hipStreamSynchronize(st));
   const std::vector<int32_t> maxdeg_of(hmaxdeg, hmaxdeg + nl);
@@ -759,9 +762,9 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
     s.active = s.lastcnt + 1;
     return s;
   };
-  void* hup = nullptr;
-  GK_TRY(ctx->up.get(st, state_bytes + 16 + sizeof(int32_t) * size_t(nt), &hup));
-  int32_t* hp = reinterpret_cast<int32_t*>(static_cast<char*>(hup) + ((state_bytes + 15) & ~size_t(15)));
+  GK_TRY(part_up.get(ctx->up, st, sizeof(int32_t) * size_t(nt), state_bytes));
+  void* hup = part_up.head();
+  int32_t* hp = static_cast<int32_t*>(part_up.p());
   int64_t cut0 = 0;
   GK_TRY(gk_initpart(&hc, k, cap, prm.seed, prm.initpart_threads, hp, &cut0));
   std::memset(hup, 0, state_bytes);
@@ -791,7 +794,7 @@ int run_vcycle(gk_ctx* ctx, hipStream_t st, const DGraph& g0in, const gk_params&
   const State ds = state_at(dstate.p);
   gkd::Copies upc;
   upc.add(dstate.p, hup, state_bytes);
-  upc.add(partA.p, hp, sizeof(int32_t) * size_t(nt));
+  GK_TRY(part_up.copy(upc, st, partA.p, hp, sizeof(int32_t) * size_t(nt), hipMemcpyHostToDevice));
   if (nl > 1) {
     GK_TRY(work.alloc(P, kWork));
     GK_TRY(selbits.alloc(P, nwords0 + 1));
@@ -1570,6 +1573,7 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   static_assert(sizeof(State) % 16 == 0, "whole 16-byte words");
   GK_TRY(state.alloc(P, sizeof(State)));
   State* ds = reinterpret_cast<State*>(state.p);
+  HostBlock hist_down;
   StageGuard staged{ctx, st};
   void* hup = nullptr;
   GK_TRY(ctx->up.get(st, sizeof(State), &hup));
@@ -1632,13 +1636,13 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
   // Rounds that ordered no move came after those that did (an unchanged state
   // stays so): no moves, position -1.
   const size_t hist_bytes = want_hist ? sizeof(int32_t) * 2 * size_t(nrounds) : 0;
-  void* hend = nullptr;
-  GK_TRY(ctx->dl.get(st, sizeof(State) + hist_bytes, &hend));
+  GK_TRY(hist_down.get(ctx->dl, st, hist_bytes, sizeof(State)));
+  void* hend = hist_down.head();
   const State* he = static_cast<const State*>(hend);
-  const int32_t* hh = reinterpret_cast<const int32_t*>(he + 1);
+  const int32_t* hh = static_cast<const int32_t*>(hist_down.p());
   gkd::Copies end;
   end.add(hend, ds, sizeof *ds);
-  end.add(static_cast<char*>(hend) + sizeof *ds, hist.p, hist_bytes);
+  GK_TRY(hist_down.copy(end, st, hist_down.p(), hist.p, hist_bytes, hipMemcpyDeviceToHost));
   GK_TRY(gkd::launch_copies(end, st));
   GK_HIP(hipStreamSynchronize(st));
   staged.done = true;

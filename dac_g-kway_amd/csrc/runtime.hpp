@@ -10,6 +10,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
+#include <new>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -583,6 +585,45 @@ struct StageGuard {
     ctx->dl.drained();
     ctx->up.drained();
   }
+};
+
+// Host memory for one transfer of a call: of up to kStageMax bytes it lies in a
+// staging arena, where kernels read and write it (launch_copies); larger ones
+// get ordinary memory, which copies by the runtime fill or send, so that no call
+// leaves a context holding much pinned memory.
+class HostBlock {
+ public:
+  // head: so many bytes in the arena in any case (a second request of the
+  // arena could take back what the first one got).
+  int get(Pinned& arena, hipStream_t st, size_t bytes, size_t head = 0) {
+    head = (head + 15) & ~size_t(15);
+    const bool staged = bytes <= kStageMax;
+    if (head || staged) GK_TRY(arena.get(st, head + (staged ? bytes : 0), &head_));
+    if (staged) {
+      p_ = static_cast<char*>(head_) + head;
+      return GK_OK;
+    }
+    own_.reset(new (std::nothrow) int4[(bytes + 15) / 16]);
+    p_ = own_.get();
+    if (p_) return GK_OK;
+    gkh::set_error("host allocation of " + std::to_string(bytes) + " bytes failed");
+    return GK_ERR_NOMEM;
+  }
+  void* p() const { return p_; }
+  void* head() const { return head_; }
+  // Adds a copy to c, or makes it (dir: which way) after those already in c.
+  int copy(gkd::Copies& c, hipStream_t st, void* dst, const void* src, size_t bytes, hipMemcpyKind dir) const {
+    if (!own_) {
+      c.add(dst, src, bytes);
+      return GK_OK;
+    }
+    if (bytes) GK_HIP(hipMemcpyAsync(dst, src, bytes, dir, st));
+    return GK_OK;
+  }
+
+ private:
+  void *p_ = nullptr, *head_ = nullptr;
+  std::unique_ptr<int4[]> own_;
 };
 
 // Words that the next launch tells the host, and the wait for them (the first n
