@@ -1666,6 +1666,11 @@ int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t ma
 int gk_k_cut(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* part, int64_t* cut, int64_t* pw,
              void* stream) {
   if (!ctx || !dg || !dg->adjwgt || !dg->vwgt || !cut || k < 1) { gkh::set_error("bad argument"); return GK_ERR_ARG; }
+  if (k > gkd::kCutMaxK) {
+    gkh::set_error("k = " + std::to_string(k) + " exceeds " + std::to_string(gkd::kCutMaxK) +
+                   ", the part weights that fit a compute unit's LDS");
+    return GK_ERR_LIMIT;
+  }
   DeviceGuard guard(ctx->device);
   hipStream_t st = pick(ctx, stream);
   DGraph g = dview(dg);

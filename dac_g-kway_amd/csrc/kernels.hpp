@@ -269,6 +269,9 @@ int launch_boundary(const DGraph& g, const int32_t* part, int32_t* bnd, hipStrea
 // cut_scratch(n, k) values, or fewer when max_slots caps it (fewer blocks;
 // the sums do not depend on the block count).
 int64_t cut_scratch(int64_t n, int32_t k);
+// Parts whose weights fit a compute unit's 160 KB of LDS beside the kernel's
+// own words (a launch that asks for more is not refused but ends the queue).
+constexpr int32_t kCutMaxK = (160 * 1024 - 32) / 4;
 int launch_cut(const DGraph& g, int32_t k, const int32_t* part, unsigned long long* cut,
                unsigned long long* pw64, unsigned long long* scratch, hipStream_t st,
                int64_t max_slots = INT64_MAX);

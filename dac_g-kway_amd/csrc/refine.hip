@@ -721,8 +721,9 @@ __global__ void __launch_bounds__(kCutThreads) k_cut(int32_t n, int32_t k, const
                                                      unsigned long long* __restrict__ bcut,
                                                      unsigned long long* __restrict__ bpw) {
   extern __shared__ unsigned int hist32[];
-  __shared__ long long wc[kCutThreads / 64];
+  __shared__ unsigned long long total;  // the waves' shares of the cut
   for (int32_t q = threadIdx.x; q < k; q += kCutThreads) hist32[q] = 0;
+  if (threadIdx.x == 0) total = 0;
   __syncthreads();
   long long c = 0;
   const int sub = threadIdx.x % kCutLanes;
@@ -764,14 +765,9 @@ __global__ void __launch_bounds__(kCutThreads) k_cut(int32_t n, int32_t k, const
     }
   }
   c = wave_sum64(c);
-  if (lane_id() == 0) wc[threadIdx.x >> 6] = c;
+  if (lane_id() == 0 && c) atomicAdd(&total, (unsigned long long)c);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    long long t = 0;
-#pragma unroll
-    for (int i = 0; i < kCutThreads / 64; ++i) t += wc[i];
-    bcut[blockIdx.x] = (unsigned long long)t;
-  }
+  if (threadIdx.x == 0) bcut[blockIdx.x] = total;
   for (int32_t q = threadIdx.x; q < k; q += kCutThreads) bpw[int64_t(blockIdx.x) * k + q] = hist32[q];
 }
 
@@ -806,6 +802,7 @@ int launch_cut(const DGraph& g, int32_t k, const int32_t* part, unsigned long lo
     fill<unsigned long long>(pw64, 0ull, k, st);
     return hip_status();
   }
+  if (k > kCutMaxK) return GK_ERR_LIMIT;
   unsigned grid = cut_grid(g.n, k);
   const int64_t fit = max_slots / (int64_t(k) + 1);  // blocks whose slots fit
   if (fit < 1) return GK_ERR_LIMIT;

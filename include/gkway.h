@@ -383,7 +383,9 @@ int gk_k_apply(gk_ctx* ctx, const gk_csr* dg, const int32_t* moves, int32_t pos,
 int gk_k_round(gk_ctx* ctx, const gk_csr* dg, int32_t k, int64_t cap, int32_t max_moves, int32_t nrounds,
                int32_t* part, int32_t* bnd, int32_t* gain, int32_t* dest, int32_t* pw, int32_t* nmoves,
                int32_t* pos, int64_t* gain_sum, int32_t* order, int64_t* paths, void* stream);
-/* Weighted cut over entries (v,u), v<u, part differs; part weights pw[k]. */
+/* Weighted cut over entries (v,u), v<u, part differs; part weights pw[k].
+ * k above 40952 (what fits a compute unit's LDS) is rejected with
+ * GK_ERR_LIMIT. */
 int gk_k_cut(gk_ctx* ctx, const gk_csr* dg, int32_t k, const int32_t* part,
              int64_t* cut, int64_t* pw, void* stream);
 /* gk_k_cut without any allocation, for callers that cannot allocate device
