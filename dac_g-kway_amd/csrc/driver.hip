@@ -3,14 +3,20 @@
 //
 // Flow of one gk_partition_device call (the reference's graph_partitioner,
 // gkway/graph_partitioner.hpp:222-365):
-//   coarsening levels  -> match, pointer-jump grouping, radix sort by
-//                         (label, stamp, id), chunking, contraction
+//   coarsening levels  -> match, grouping by a walk to the root pairs (deep
+//                         trees: pointer jumping), order, chunks and coarse ids
+//                         by counting (large groups: a radix sort by (label,
+//                         stamp, id)), contraction
 //   coarsest level     -> copy to host, gk_initpart (METIS's role), copy back
-//   uncoarsening       -> per finer level: projection, gain pass, rounds of
-//                         select / balance / apply / gain until no move
+//   uncoarsening       -> per finer level: projection and gain pass, then rounds
+//                         by the round loop or by separate kernels (select,
+//                         order and balance, apply, gain) until no move
 //   final              -> weighted cut and part weights of level 0
-// One stream per context; the host synchronises once per level and once per
-// refinement round to read the counts that size the next launches.
+// One stream per context.  The host waits for the counts that size a coarsening
+// level's next launches (two or three of them), for the coarsest graph, and in
+// refinement at the end of a launch of the round loop (up to 64 rounds) or every
+// 4 to 32 rounds of the separate kernels; kernels tell it most counts in words
+// it watches.
 #include <algorithm>
 #include <chrono>
 #include <cstdlib>

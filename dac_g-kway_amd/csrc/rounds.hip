@@ -14,7 +14,7 @@
 // weights stay in LDS.  Jobs of a batch share no vertex and no part, so each
 // runs at its own pace and none waits for another's rounds.  Refinement of a
 // DAG of 300k vertices, k = 256 (375 rounds): 15.8 ms with separate kernels,
-// 7.9 ms here; a late round takes 25k to 35k cycles, about a quarter of them
+// 7.9 ms here; a late round takes 22k to 35k cycles, about a quarter of them
 // the gains of the updated vertices (three dependent reads), the rest shared
 // between finding the movable vertices, their best, the tests and the sort.
 //
